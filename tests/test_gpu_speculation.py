@@ -192,6 +192,23 @@ def test_stale_guess_both_kinds_of_guarded_launch(K, oracle, fallback, w32, monk
         K.lib.zk_reload_env()
 
 
+def test_stale_guess_with_more_calls_under_way_than_reports_fit(K, oracle):
+    """a host hundreds of calls ahead of the device: the ring the reports travel in holds 256, calls beyond it go without
+    one, and every one of them is still checked and computed again where its guess does not hold"""
+    rng = np.random.default_rng(970)
+    A, W = Operand(rand_i64(rng, (1, 40, 96), 20)), Operand(rand_i64(rng, (130, 96), 16))
+    call = _bmm(K, A, W, 11)
+    call()
+    torch.cuda.synchronize()
+    torch.cuda._sleep(200_000_000)              # (some 0.1 s: nothing below runs before all of it is queued)
+    for _ in range(300):
+        C, R = call()
+    A.poke((0, 39, 95), WIDE)
+    C, R = call()
+    Ce, Re = oracle.int64_bmm_broadcast(A.h, W.h, 1, 1, 11)
+    assert np.array_equal(host(C), Ce) and np.array_equal(host(R), Re)
+
+
 def test_stale_guess_long_k_falls_back_to_the_vector_alu(K, oracle):
     """nine digits over K = 16384 do not fit the int32 accumulators of one pass (the guarded MFMA form does not split K):
     the vector-ALU tiles stand behind such a product"""

@@ -26,9 +26,61 @@ struct GemmDesc {
 
 enum GemmPath { kPathAuto = 0, kPathValu = 1, kPathMfma = 2 };
 
-// Native 64-bit multiply-add chains on the vector ALU; handles every descriptor.  With a `guard` (device
-// pointer) the launch is conditional: its workgroups return at once unless *guard is non-zero when they start.
-void gemm_valu_launch(const GemmDesc &d, const unsigned long long *guard = nullptr);
+// A guarded launch stands behind a speculative one on the stream and computes every output again if some workgroup of
+// that launch raised the verdict; otherwise its workgroups return at once.  Its first workgroup also reports what the
+// speculative launch saw, so that no launch, no event and no wait is needed for that alone.
+struct GuardArgs {
+    const unsigned *verdict;         // device word; null: an unconditional launch
+    unsigned *next;                  // device word cleared for the next speculative launch (the calls take turns with two)
+    const unsigned *seen;            // per-workgroup digit counts of the speculative launch: byte 0 A, byte 1 B
+    long seen_count;
+    unsigned long long *host;        // receives seq << 32 | verdict << 16 | digits of B << 8 | digits of A in one store (may be null)
+    unsigned seq;
+};
+
+// by one whole workgroup of at most 1024 threads
+__device__ __forceinline__ void guard_report(const GuardArgs &g)
+{
+    __shared__ int report_red[16];
+    unsigned a = 0, b = 0;
+    // (four loads under way per thread: the launch waits for this workgroup)
+    for (long i0 = threadIdx.x; i0 < g.seen_count; i0 += 4L * blockDim.x) {
+        unsigned w[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const long i = i0 + (long)j * blockDim.x;
+            w[j] = i < g.seen_count ? g.seen[i] : 0;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const unsigned wa = w[j] & 0xFFu, wb = (w[j] >> 8) & 0xFFu;
+            a = wa > a ? wa : a;
+            b = wb > b ? wb : b;
+        }
+    }
+    unsigned ab = a << 16 | b;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned o = (unsigned)__shfl_xor((int)ab, off, kWave);
+        const unsigned oa = o >> 16, ob = o & 0xFFFFu, ma = ab >> 16, mb = ab & 0xFFFFu;
+        ab = (oa > ma ? oa : ma) << 16 | (ob > mb ? ob : mb);
+    }
+    if ((threadIdx.x & 63) == 0) report_red[threadIdx.x >> 6] = (int)ab;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    a = b = 0;
+    for (unsigned w = 0; w < blockDim.x / 64; w++) {
+        const unsigned o = (unsigned)report_red[w];
+        a = (o >> 16) > a ? (o >> 16) : a;
+        b = (o & 0xFFFFu) > b ? (o & 0xFFFFu) : b;
+    }
+    const unsigned v = __atomic_load_n(g.verdict, __ATOMIC_RELAXED);
+    if (g.host) __hip_atomic_store(g.host, (unsigned long long)g.seq << 32 | v << 16 | b << 8 | a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (g.next) __atomic_store_n(g.next, 0u, __ATOMIC_RELAXED);
+}
+
+// Native 64-bit multiply-add chains on the vector ALU; handles every descriptor.
+void gemm_valu_launch(const GemmDesc &d, const GuardArgs &guard = GuardArgs());
 
 // Matrix-vector kernel of the same family for one or two rows of A against k-contiguous B: one launch, nothing
 // guessed.  Returns false (nothing launched) for any other descriptor.
@@ -86,9 +138,8 @@ struct GroupedDesc {
 bool gemm_gemv_grouped_launch(const GroupedDesc &d);
 
 // The grouped product on the 16-row MFMA tiles (see gemm_rows16_launch): one launch, no wait.  0 / 1 / -1 as there.
-// `guard`: a device word; when given, the launch's workgroups return at once unless it is non-zero (the fallback behind
-// a speculative launch of the 32-row kernels).
-int gemm_rows16_grouped(const GroupedDesc &d, const unsigned long long *guard = nullptr);
+// `guard`: see GuardArgs (the fallback behind a speculative launch of the 32-row kernels).
+int gemm_rows16_grouped(const GroupedDesc &d, const GuardArgs &guard = GuardArgs());
 
 // One launch of the 32-row-tile MFMA kernels over all groups.  Returns 0 when done, 1 when the operands need
 // more digits than those kernels are built for (nothing valid was written: the caller takes another route),

@@ -17,13 +17,13 @@
 // RUN*OCTS apart.  Adjacent lanes then read adjacent 16-byte pieces and every 64-byte line of the tile is
 // fetched by exactly one load instruction.
 //
-// The digit counts are speculated from a cached or sampled range.  The kernels track the exact min and max of
-// everything they load (every workgroup leaves its share in a slot of its own, a few workgroups fold
-// them and compare with the digit counts used).  The first call for an operand reads the verdict back and
-// reruns with wider digits if the guess was too small.  Later calls do not wait: a guarded launch of the
-// vector-ALU kernel follows, which recomputes everything if the verdict is bad and returns at once otherwise,
-// and the exact range travels to the host behind the stream to refresh the cache.  Results never depend on
-// the guess, and a call whose operands were seen before never blocks the host.
+// The digit counts are speculated from a cached or sampled range.  The kernels track the digits that everything they
+// load needs.  A workgroup that meets an element its digit counts do not hold raises the verdict, a word on the device
+// that nobody writes otherwise; a guarded launch follows on the stream, which recomputes everything if the verdict is
+// raised and returns at once otherwise.  Its first workgroup also folds what every workgroup saw into one 8-byte store
+// to pinned host memory, marked with the call's number: that refreshes the cache at a later call.  (A fold kernel
+// between the two and an event behind them cost 10 us per call: 5 for the kernel, 5.5 of idle device at the event.)
+// Results never depend on the guess, and a call whose operands were seen before never blocks the host.
 #include "gemm_mfma_kernels.h"
 
 #include <map>
@@ -90,37 +90,35 @@ static const Instance *pick_instance(int na, int nb, bool b32, bool skinny, int 
 
 typedef std::tuple<const void *, long, long, int> OperandKey;     // (pointer, rows, K, element size)
 
-// A range on its way from the device to the host behind the stream (calls that do not wait for their verdict).
+// Digit counts on their way from the device to the host behind the stream (calls that do not wait for their verdict).
 struct PendingRange {
-    hipEvent_t ev = nullptr;
-    unsigned long long *host = nullptr;      // pinned: [minA, maxA, minB, maxB, verdict]
     OperandKey key_a, key_b;
     int nb_fixed = 0;                        // B came from prepared planes with this many digits (nothing of it was tracked)
-    bool busy = false;
+    unsigned seq = 0;                        // the call's number: its report has arrived when the slot's pinned word carries it
 };
 
-constexpr int kPendingSlots = 16;
+constexpr unsigned kPendingSlots = 256;      // (a host this many calls ahead of the device skips the report, not the check)
 
 struct RangeCache {
     std::mutex mu;
     std::map<OperandKey, int> limbs;         // operand -> digits its values needed when last seen
     std::map<OperandKey, int> partner_a;     // B operand -> digits of the A operand it was last multiplied with
     std::map<std::tuple<long, long, int>, int> by_shape;      // (rows, K, element size) -> digits of the last operand of that shape, wherever it lay
-    unsigned long long *dev = nullptr;       // [minA, maxA, minB, maxB, verdict]
+    unsigned long long *dev = nullptr;       // [minA, maxA, minB, maxB] of a sample, [4] a report that is waited for, [5] the two verdict words
+    int turn = 0;                            // which verdict word the next speculative launch uses; it is clear
     unsigned char *planes = nullptr;         // digit planes of A, grown on demand, kept for the process lifetime
     size_t planes_bytes = 0;
-    unsigned long long *mm = nullptr;        // per-workgroup ranges of the plane pre-pass
-    size_t mm_count = 0;
-    unsigned long long *wg = nullptr;        // per-workgroup ranges of the GEMM kernel
-    size_t wg_count = 0;
+    unsigned *seen = nullptr;                // per-workgroup digit counts of the GEMM kernel and of the plane pre-pass
+    size_t seen_count = 0;
     unsigned long long *partials = nullptr;  // partial sums of split tiles
     size_t partials_bytes = 0;
     int64_t *b_rows = nullptr;               // a small n-contiguous B rewritten with contiguous rows
     size_t b_rows_count = 0;
     int cus = 0;                             // compute units of the device
     PendingRange pending[kPendingSlots];
-    unsigned long long *pinned = nullptr;
-    int pending_head = 0;                    // next slot to use; slots are used and drained in ring order
+    volatile unsigned long long *pinned = nullptr;      // one word per slot
+    unsigned pending_head = 0, pending_tail = 0;        // slots used and drained so far, in ring order; head - tail are on their way
+    unsigned seq = 0;
     long guard_hits = 0;                     // calls whose speculation failed after they had returned
     int lookup(const OperandKey &k)
     {
@@ -211,24 +209,67 @@ static bool read_range(unsigned long long *dev, int64_t (&out)[4])
     return true;
 }
 
-// Takes in the ranges that have arrived since the last call, oldest first.
+// Takes in the reports that have arrived since the last call, oldest first (the stream delivers them in that order).
 static void drain_pending()
 {
-    for (int n = 0; n < kPendingSlots; n++) {
-        PendingRange &s = g_cache.pending[(g_cache.pending_head + n) % kPendingSlots];
-        if (!s.busy) continue;
-        const hipError_t st = hipEventQuery(s.ev);
-        if (st != hipSuccess) { (void)hipGetLastError(); if (st == hipErrorNotReady) continue; }
-        if (st == hipSuccess) {
-            const int64_t b_lo = (int64_t)(s.host[2] ^ kSignFlip), b_hi = (int64_t)(s.host[3] ^ kSignFlip);
-            const int na_seen = limbs_needed((int64_t)(s.host[0] ^ kSignFlip), (int64_t)(s.host[1] ^ kSignFlip));
-            if (b_lo <= b_hi) g_cache.store_pair(s.key_a, na_seen, s.key_b, limbs_needed(b_lo, b_hi));
-            else if (s.nb_fixed) g_cache.store_pair(s.key_a, na_seen, s.key_b, s.nb_fixed);      // (a grouped launch on prepared planes)
-            else g_cache.store(s.key_a, na_seen);            // B came from prepared planes: nothing of it was tracked
-            if (s.host[4]) g_cache.guard_hits++;
-        }
-        s.busy = false;
+    while (g_cache.pending_tail != g_cache.pending_head) {
+        const PendingRange &s = g_cache.pending[g_cache.pending_tail % kPendingSlots];
+        const unsigned long long w = g_cache.pinned[g_cache.pending_tail % kPendingSlots];
+        if ((unsigned)(w >> 32) != s.seq) return;
+        const int na = (int)(w & 0xFF), nb = (int)(w >> 8 & 0xFF);
+        if (nb) g_cache.store_pair(s.key_a, na ? na : 1, s.key_b, nb);
+        else if (s.nb_fixed) g_cache.store_pair(s.key_a, na ? na : 1, s.key_b, s.nb_fixed);      // (a grouped launch on prepared planes)
+        else g_cache.store(s.key_a, na ? na : 1);        // B came from prepared planes: nothing of it was tracked
+        if (w >> 16 & 0xFF) g_cache.guard_hits++;
+        g_cache.pending_tail++;
     }
+}
+
+// The guard of the call being launched: its verdict word, the word cleared for the next call, and, while a slot is free,
+// where the report goes.  guard_taken() once the guarded launch is on the stream.
+static GuardArgs make_guard(long seen_count)
+{
+    unsigned *words = reinterpret_cast<unsigned *>(g_cache.dev + 5);
+    GuardArgs g = {};
+    g.verdict = words + g_cache.turn;
+    g.next = words + (g_cache.turn ^ 1);
+    g.seen = g_cache.seen;
+    g.seen_count = seen_count;
+    if (g_cache.pending_head - g_cache.pending_tail < kPendingSlots) {
+        g.host = const_cast<unsigned long long *>(g_cache.pinned) + g_cache.pending_head % kPendingSlots;
+        if (++g_cache.seq == 0) g_cache.seq = 1;
+        g.seq = g_cache.seq;
+    }
+    return g;
+}
+
+static void guard_taken(const GuardArgs &g, const OperandKey &key_a, const OperandKey &key_b, int nb_fixed)
+{
+    g_cache.turn ^= 1;
+    if (!g.host) return;
+    PendingRange &s = g_cache.pending[g_cache.pending_head % kPendingSlots];
+    s.key_a = key_a;
+    s.key_b = key_b;
+    s.nb_fixed = nb_fixed;
+    s.seq = g.seq;
+    g_cache.pending_head++;
+}
+
+// Waits for the digits the launch just issued has seen, and clears its verdict word (its caller launches again).
+static bool wait_digits(long seen_count, int *need_a, int *need_b)
+{
+    GuardArgs g = {};
+    unsigned *word = reinterpret_cast<unsigned *>(g_cache.dev + 5) + g_cache.turn;
+    g.verdict = word; g.next = word; g.seen = g_cache.seen; g.seen_count = seen_count;
+    g.host = g_cache.dev + 4;
+    digits_report_kernel<<<1, 256, 0, 0>>>(g);
+    unsigned long long w;
+    if (hipMemcpy(&w, g_cache.dev + 4, sizeof(w), hipMemcpyDeviceToHost) != hipSuccess) return false;
+    *need_a = (int)(w & 0xFF);
+    *need_b = (int)(w >> 8 & 0xFF);
+    if (!*need_a) *need_a = 1;
+    if (!*need_b) *need_b = 1;
+    return true;
 }
 
 static int g_last_pairs = 0, g_last_prepared = 0;
@@ -248,8 +289,7 @@ long gemm_mfma_guard_hits()
 static bool init_cache()
 {
     if (g_cache.dev) return true;
-    // [minA, maxA, minB, maxB, verdict, fold ticket, -, -] and the partial results of the folding workgroups
-    const size_t dev_bytes = (8 + 4 * kFoldParts) * sizeof(unsigned long long);
+    const size_t dev_bytes = 8 * sizeof(unsigned long long);
     if (hipMalloc(&g_cache.dev, dev_bytes) != hipSuccess || hipMemset(g_cache.dev, 0, dev_bytes) != hipSuccess) {
         g_cache.dev = nullptr;
         set_error(kLaunchFailure, "gemm: cannot allocate the range buffer");
@@ -258,25 +298,16 @@ static bool init_cache()
     int dev = 0, n = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
     g_cache.cus = n;
-    // without the pinned slots every call simply waits for its own verdict
-    if (hipHostMalloc(&g_cache.pinned, kPendingSlots * 8 * sizeof(unsigned long long), hipHostMallocDefault) == hipSuccess) {
-        for (int i = 0; i < kPendingSlots; i++) {
-            g_cache.pending[i].host = g_cache.pinned + 8 * i;
-            if (hipEventCreateWithFlags(&g_cache.pending[i].ev, hipEventDisableTiming) != hipSuccess) g_cache.pending[i].ev = nullptr;
-        }
+    // without the pinned words every call simply waits for its own verdict
+    void *pinned = nullptr;
+    if (hipHostMalloc(&pinned, kPendingSlots * sizeof(unsigned long long), hipHostMallocDefault) == hipSuccess) {
+        g_cache.pinned = reinterpret_cast<volatile unsigned long long *>(pinned);
+        for (unsigned i = 0; i < kPendingSlots; i++) g_cache.pinned[i] = 0;
     } else {
         (void)hipGetLastError();
         g_cache.pinned = nullptr;
     }
     return true;
-}
-
-static FoldArgs make_fold(const unsigned long long *mm, long mm_count, const unsigned long long *wg, long wg_count,
-                          unsigned long long *range, int na, int nb, unsigned long long *host_copy)
-{
-    long parts = (mm_count + wg_count + kFoldSlotsPerPart - 1) / kFoldSlotsPerPart;
-    parts = parts < 1 ? 1 : (parts > kFoldParts ? kFoldParts : parts);
-    return FoldArgs{ mm, mm_count, wg, wg_count, range, na, nb, host_copy, (int)parts, g_cache.dev + 8 };
 }
 
 // ---- weights prepared once ------------------------------------------------------------------------------
@@ -404,21 +435,16 @@ int gemm_mfma_prepare(const void *B, int b32, int groups, int N, int K)
     // the pre-pass that splits A in fragment order does the same for the rows of a weight matrix (64 rows per workgroup)
     const int rows_per_wg = 256 / (4 * pb.kk);
     const dim3 grid((unsigned)(pb.ksteps / pb.kk), (unsigned)((pb.nsub * 32 + rows_per_wg - 1) / rows_per_wg), 1);
-    if (grow(g_cache.mm, g_cache.mm_count, (size_t)grid.x * grid.y * 2, "range scratch") != kDone) {
-        release_prepared(pb);
-        set_error(kLaunchFailure, "%s: cannot allocate the range scratch", name);
-        return 1;
-    }
     MfmaParams q = {};
     q.lda = K; q.sA = 0; q.M = N; q.K = K;
     for (int i = 0; i < count; i++) {
         q.A = reinterpret_cast<const int64_t *>(mats[i]);
         unsigned char *dst = pb.planes + per * i;
-#define ZK_PLANES(NB_) do { if (b32) a_planes_kernel<NB_, 2, 1, true><<<grid, dim3(256), 0, 0>>>(q, dst, pb.nsub, pb.ksteps, g_cache.mm); \
-                           else a_planes_kernel<NB_, 2, 1, false><<<grid, dim3(256), 0, 0>>>(q, dst, pb.nsub, pb.ksteps, g_cache.mm); } while (0)
+#define ZK_PLANES(NB_) do { if (b32) a_planes_kernel<NB_, 2, 1, true><<<grid, dim3(256), 0, 0>>>(q, dst, pb.nsub, pb.ksteps, nullptr); \
+                           else a_planes_kernel<NB_, 2, 1, false><<<grid, dim3(256), 0, 0>>>(q, dst, pb.nsub, pb.ksteps, nullptr); } while (0)
         switch (pb.nb) {
-#define ZK_PLANES2(NB_) do { if (b32) a_planes_kernel<NB_, 2, 2, true><<<grid, dim3(256), 0, 0>>>(q, dst, pb.nsub, pb.ksteps, g_cache.mm); \
-                            else a_planes_kernel<NB_, 2, 2, false><<<grid, dim3(256), 0, 0>>>(q, dst, pb.nsub, pb.ksteps, g_cache.mm); } while (0)
+#define ZK_PLANES2(NB_) do { if (b32) a_planes_kernel<NB_, 2, 2, true><<<grid, dim3(256), 0, 0>>>(q, dst, pb.nsub, pb.ksteps, nullptr); \
+                            else a_planes_kernel<NB_, 2, 2, false><<<grid, dim3(256), 0, 0>>>(q, dst, pb.nsub, pb.ksteps, nullptr); } while (0)
         case 3: if (pb.kk == 2) ZK_PLANES2(3); else ZK_PLANES(3); break;
         case 4: if (pb.kk == 2) ZK_PLANES2(4); else ZK_PLANES(4); break;
 #undef ZK_PLANES2
@@ -440,8 +466,8 @@ int gemm_mfma_prepare(const void *B, int b32, int groups, int N, int K)
 size_t gemm_mfma_workspace_bytes(size_t *prepared_bytes)
 {
     std::lock_guard<std::mutex> lock(g_cache.mu);
-    size_t scratch = g_cache.dev ? (8 + 4 * kFoldParts) * sizeof(unsigned long long) : 0;
-    scratch += g_cache.planes_bytes + (g_cache.mm_count + g_cache.wg_count + g_cache.partials_bytes) * sizeof(unsigned long long) +
+    size_t scratch = g_cache.dev ? 8 * sizeof(unsigned long long) : 0;
+    scratch += g_cache.planes_bytes + g_cache.seen_count * sizeof(unsigned) + g_cache.partials_bytes * sizeof(unsigned long long) +
                g_cache.b_rows_count * sizeof(int64_t);
     size_t prepared = 0;
     for (const auto &kv : g_prepared) {
@@ -461,13 +487,11 @@ void gemm_mfma_release_workspace()
     (void)hipDeviceSynchronize();
     drain_pending();
     if (g_cache.planes) (void)hipFree(g_cache.planes);
-    if (g_cache.mm) (void)hipFree(g_cache.mm);
-    if (g_cache.wg) (void)hipFree(g_cache.wg);
+    if (g_cache.seen) (void)hipFree(g_cache.seen);
     if (g_cache.partials) (void)hipFree(g_cache.partials);
     if (g_cache.b_rows) (void)hipFree(g_cache.b_rows);
     g_cache.planes = nullptr; g_cache.planes_bytes = 0;
-    g_cache.mm = nullptr; g_cache.mm_count = 0;
-    g_cache.wg = nullptr; g_cache.wg_count = 0;
+    g_cache.seen = nullptr; g_cache.seen_count = 0;
     g_cache.partials = nullptr; g_cache.partials_bytes = 0;
     g_cache.b_rows = nullptr; g_cache.b_rows_count = 0;
 }
@@ -503,7 +527,7 @@ constexpr long kBRowsMaxElements = 8L << 20;         // 64 MB
 // digits hold every int64, five every int32; config 4 with stale three-digit guesses: 4 ms where the vector-ALU tiles
 // take 35), one workgroup per compute unit walking the tiles.  Everything else, and a K beyond what its int32
 // accumulators take in one piece: the vector-ALU tiles.
-static Outcome launch_guarded_fallback(const GemmDesc &d, const MfmaParams &spec, int b_shift)
+static Outcome launch_guarded_fallback(const GemmDesc &d, const MfmaParams &spec, int b_shift, const GuardArgs &guard)
 {
     // (an n-contiguous B that the speculative launch read through its row-major copy is read through that copy here too)
     const bool b_copied = spec.B == (const void *)g_cache.b_rows && g_cache.b_rows != nullptr;
@@ -527,17 +551,13 @@ static Outcome launch_guarded_fallback(const GemmDesc &d, const MfmaParams &spec
         if (total > 0x7FFFFFFFL / 8) fn = nullptr;
         else {
             q.main_tiles = (int)total; q.split = 1; q.tail_xcd = 0; q.partials = nullptr; q.part64 = 0; q.n_fastest = 0;
-            q.guard = spec.range + 4;
+            q.guard = guard;
+            q.seen = nullptr;                  // (its digit counts hold whatever raised the verdict)
             q.walk_blocks = (int)total;
-            // (the range slots of the speculative launch have been folded by now: the fallback's tracking may overwrite them)
-            const Outcome got = grow(g_cache.wg, g_cache.wg_count, (size_t)total * 4, "range slots");
-            if (got == kFailed) return kFailed;
-            if (got == kDeclined) fn = nullptr;
-            q.wg_range = g_cache.wg;
         }
     }
     if (!fn) {
-        gemm_valu_launch(d, spec.range + 4);
+        gemm_valu_launch(d, guard);
         return kDone;
     }
     const size_t lds = 2 * (size_t)wide->kk * ((wide->bm / 32) * wide->na + (wide->bn / 32) * wide->nb) * 1024 + 9 * 1024 + 16;
@@ -619,13 +639,9 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         if (!na) na = g_cache.lookup_shape(key_a);
         if (!nb) nb = g_cache.lookup_shape(key_b);
     }
-    // No call waits for its verdict (unless no slot is free for the range to travel in, or ZK_GEMM_SYNC asks for it): a
-    // guarded launch behind the product redoes it with digits that cover everything if the verdict is bad.
-    PendingRange *slot = nullptr;
-    if (g_cache.pinned && !g_switches.sync_verdict) {
-        PendingRange &s = g_cache.pending[g_cache.pending_head];
-        if (!s.busy && s.ev) slot = &s;
-    }
+    // No call waits for its verdict (unless there is no pinned memory, or ZK_GEMM_SYNC asks for it): a guarded launch
+    // behind the product redoes it with digits that cover everything if the verdict is raised.
+    const bool speculate = g_cache.pinned && !g_switches.sync_verdict;
     if (!na || !nb) {
         p.tiles_m = p.tiles_n = 1;
         range_reset_kernel<<<1, 64, 0, 0>>>(p.range);
@@ -751,12 +767,9 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             else if (k_over) return kDeclined;
         }
         const long blocks = (long)p.main_tiles + (total - p.main_tiles) * p.split;
-        // (room for the guarded fallback's 64 x 64 tiles as well, so that it never has to regrow the buffer)
-        const long fb_blocks = (long)((d.M + 63) / 64) * ((d.N + 63) / 64) * d.G;
-        if (const Outcome got = grow(g_cache.wg, g_cache.wg_count, (size_t)(blocks > fb_blocks ? blocks : fb_blocks) * 4, "range slots")) return got;
-        p.wg_range = g_cache.wg;
-
         long plane_wgs = 0;
+        p.fail_class = inst->na > 5 || inst->nb > 5 ? 2 : 1;
+        p.verdict = reinterpret_cast<unsigned *>(g_cache.dev + 5) + g_cache.turn;
         p.a_planes = nullptr; p.a_msub = 0; p.a_ksteps = 0;
         if (use_planes) {
             const int msub = p.tiles_m * (BM / 32);
@@ -767,10 +780,11 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             const int rows_per_wg = 256 / (4 * inst->kk);
             const dim3 pgrid((unsigned)(ksteps / inst->kk), (unsigned)((msub * 32 + rows_per_wg - 1) / rows_per_wg), (unsigned)d.G);
             plane_wgs = (long)pgrid.x * pgrid.y * pgrid.z;
-            if (const Outcome got = grow(g_cache.mm, g_cache.mm_count, (size_t)plane_wgs * 2, "range scratch")) return got;
+            if (const Outcome got = grow(g_cache.seen, g_cache.seen_count, (size_t)(blocks + plane_wgs), "digit counts")) return got;
             // (the owned-k pattern of the planes of A follows the kernel that reads them: prepared planes of B go with the int64 forms)
-            inst->planes[(d.b32 && !prep) ? 1 : 0]<<<pgrid, dim3(256), 0, 0>>>(p, g_cache.planes, msub, ksteps, g_cache.mm);
-        }
+            inst->planes[(d.b32 && !prep) ? 1 : 0]<<<pgrid, dim3(256), 0, 0>>>(p, g_cache.planes, msub, ksteps, g_cache.seen + blocks);
+        } else if (const Outcome got = grow(g_cache.seen, g_cache.seen_count, (size_t)blocks, "digit counts")) return got;
+        p.seen = g_cache.seen;
         const size_t lds = pipe_lds ? pipe_lds : 2 * (size_t)inst->kk * ((BM / 32) * inst->na + (BN / 32) * inst->nb) * 1024 + 9 * 1024 + 16;
         static std::set<const void *> lds_raised;
         if (lds > 64 * 1024 && !lds_raised.count((const void *)fn)) {
@@ -792,32 +806,22 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
                 return kFailed;
             }
         }
-        const FoldArgs fold = make_fold(g_cache.mm, plane_wgs, g_cache.wg, blocks, p.range, inst->na, inst->nb, slot ? slot->host : nullptr);
         if (p.split > 1) {
-            inst->finish<<<dim3((unsigned)((total - p.main_tiles) * p.finish_rq + fold.parts)), dim3((unsigned)inst->threads), 0, 0>>>(p, fold);
+            inst->finish<<<dim3((unsigned)((total - p.main_tiles) * p.finish_rq)), dim3((unsigned)inst->threads), 0, 0>>>(p);
             if (hipGetLastError() != hipSuccess) { set_error(kLaunchFailure, "gemm: split finish launch failed"); return kFailed; }
-        } else {
-            range_fold_kernel<<<dim3((unsigned)fold.parts), 256, 0, 0>>>(fold);
         }
         *limbs_a = inst->na;
         *limbs_b = inst->nb;
-        if (slot) {
-            // no waiting: a guarded launch redoes the product if the verdict is bad, the range follows later
-            if (const Outcome got = launch_guarded_fallback(d, p, b_shift)) return got;
-            if (hipEventRecord(slot->ev, 0) == hipSuccess) {
-                slot->key_a = key_a;
-                slot->key_b = key_b;
-                slot->nb_fixed = prep ? prep->nb : 0;       // (the slots are shared with the grouped launches, which set it too)
-                slot->busy = true;
-                g_cache.pending_head = (g_cache.pending_head + 1) % kPendingSlots;
-            } else {
-                (void)hipGetLastError();
-            }
+        if (speculate) {
+            // no waiting: a guarded launch redoes the product if the verdict is raised, the digits seen follow later
+            const GuardArgs guard = make_guard(blocks + plane_wgs);
+            if (const Outcome got = launch_guarded_fallback(d, p, b_shift, guard)) return got;
+            guard_taken(guard, key_a, key_b, prep ? prep->nb : 0);       // (the slots are shared with the grouped launches, which set it too)
             return kDone;
         }
-        int64_t r[4];
-        if (!read_range(p.range, r)) { set_error(kLaunchFailure, "gemm: range readback failed"); return kFailed; }
-        const int need_a = limbs_needed(r[0], r[1]), need_b = prep ? prep->nb : limbs_needed(r[2], r[3]);
+        int need_a, need_b;
+        if (!wait_digits(blocks + plane_wgs, &need_a, &need_b)) { set_error(kLaunchFailure, "gemm: digit readback failed"); return kFailed; }
+        if (prep) need_b = prep->nb;
         g_cache.store_pair(key_a, need_a, key_b, need_b);
         if (need_a <= inst->na && need_b <= inst->nb) return kDone;
         na = need_a;
@@ -867,11 +871,7 @@ int gemm_mfma_grouped(const GroupedDesc &d, int *limbs_a, int *limbs_b)
     // unless the verdict is bad, in which case they compute every output again.  What the kernels saw travels to pinned
     // host memory behind an event and reaches the cache at a later call.  Otherwise (first sight of the weights, no
     // free slot) the verdict is read back before the call returns, as it used to be for every grouped launch.
-    PendingRange *slot = nullptr;
-    if (informed && g_cache.pinned && !g_switches.sync_verdict) {
-        PendingRange &s = g_cache.pending[g_cache.pending_head];
-        if (!s.busy && s.ev) slot = &s;
-    }
+    bool speculate = informed && g_cache.pinned && !g_switches.sync_verdict;
 
     for (int attempt = 0; attempt < 3; attempt++) {
         const Instance *inst = nullptr;
@@ -908,8 +908,10 @@ int gemm_mfma_grouped(const GroupedDesc &d, int *limbs_a, int *limbs_b)
         const long blocks = (max_mtiles + 7) / 8 * 8 * p.tiles_n;       // (whole rounds of the 8 XCDs: see the kernels' tile order)
         if (blocks > 0x7FFFFFFFL / 8) return 1;
         p.main_tiles = (int)blocks;
-        if (const Outcome got = grow(g_cache.wg, g_cache.wg_count, (size_t)blocks * 4, "range slots")) return got;
-        p.wg_range = g_cache.wg;
+        if (const Outcome got = grow(g_cache.seen, g_cache.seen_count, (size_t)blocks, "digit counts")) return got;
+        p.seen = g_cache.seen;
+        p.fail_class = inst->na > 5 || inst->nb > 5 ? 2 : 1;
+        p.verdict = reinterpret_cast<unsigned *>(g_cache.dev + 5) + g_cache.turn;
         const size_t lds = stream_lds ? stream_lds : 2 * (size_t)inst->kk * ((inst->bm / 32) * inst->na + (inst->bn / 32) * inst->nb) * 1024 + 9 * 1024 + 16;
         static std::set<const void *> lds_raised;
         if (lds > 64 * 1024 && !lds_raised.count((const void *)fn)) {
@@ -930,30 +932,21 @@ int gemm_mfma_grouped(const GroupedDesc &d, int *limbs_a, int *limbs_b)
                 return -1;
             }
         }
-        const FoldArgs fold = make_fold(nullptr, 0, g_cache.wg, blocks, p.range, inst->na, inst->nb, slot ? slot->host : nullptr);
-        range_fold_kernel<<<dim3((unsigned)fold.parts), 256, 0, 0>>>(fold);
-        if (slot) {
-            const int rc = gemm_rows16_grouped(d, p.range + 4);
+        if (speculate) {
+            const GuardArgs guard = make_guard(blocks);
+            const int rc = gemm_rows16_grouped(d, guard);
             if (rc < 0) return -1;
             if (rc == 0) {
                 *limbs_a = inst->na;
                 *limbs_b = inst->nb;
-                if (hipEventRecord(slot->ev, 0) == hipSuccess) {
-                    slot->key_a = key_a;
-                    slot->key_b = key_b;
-                    slot->nb_fixed = prep ? prep->nb : 0;
-                    slot->busy = true;
-                    g_cache.pending_head = (g_cache.pending_head + 1) % kPendingSlots;
-                } else {
-                    (void)hipGetLastError();
-                }
+                guard_taken(guard, key_a, key_b, prep ? prep->nb : 0);
                 return 0;
             }
-            slot = nullptr;         // the 16-row kernels do not take this product: wait for the verdict after all
+            speculate = false;      // the 16-row kernels do not take this product: wait for the verdict after all
         }
-        int64_t r[4];
-        if (!read_range(p.range, r)) { set_error(kLaunchFailure, "grouped gemm: range readback failed"); return -1; }
-        const int need_a = limbs_needed(r[0], r[1]), need_b = prep ? prep->nb : limbs_needed(r[2], r[3]);
+        int need_a, need_b;
+        if (!wait_digits(blocks, &need_a, &need_b)) { set_error(kLaunchFailure, "grouped gemm: digit readback failed"); return -1; }
+        if (prep) need_b = prep->nb;
         g_cache.store_pair(key_a, need_a, key_b, need_b);
         *limbs_a = inst->na;
         *limbs_b = inst->nb;

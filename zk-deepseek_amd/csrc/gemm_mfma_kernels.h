@@ -34,8 +34,10 @@ struct MfmaParams {
     int M, N, K, shift;
     int64_t init;
     int tiles_m, tiles_n;
-    unsigned long long *range;      // [minA, maxA, minB, maxB], order-preserving unsigned images of int64; [4] verdict
-    unsigned long long *wg_range;   // one such quadruple per workgroup of the GEMM kernel
+    unsigned long long *range;      // sampling only: [minA, maxA, minB, maxB], order-preserving unsigned images of int64
+    unsigned *seen;                 // one word per workgroup: digits its share of A (byte 0) and of B (byte 1) needs, 0 = nothing seen; may be null
+    unsigned *verdict;              // 0 unless some workgroup met an element its digit counts do not hold (see raise_verdict)
+    int fail_class;                 // what such a workgroup reports at least: 1, or 2 when a digit count of this launch is above five
     int verify_b_all_batches;       // B differs per batch: every batch's first tile row tracks its range
     const unsigned char *a_planes;  // pre-split digits of A (planes variants only)
     int a_msub, a_ksteps;           // 32-row groups and 32-k steps the planes were written for
@@ -55,9 +57,9 @@ struct MfmaParams {
     const void *const *grp_b;       // [groups] B of every group
     int b_shift;                    // BRS kernels: every element of B is divided by 2^b_shift first, truncating toward zero
     int finish_rq;                  // workgroups per tile of the finishing kernel (4 or 16)
-    // guarded launches (the fallback behind a speculative launch): the kernel does nothing unless *guard is non-zero, and
-    // its workgroups, one per compute unit, walk the `walk_blocks` workgroup ids of an ordinary launch
-    const unsigned long long *guard;
+    // guarded launches (the fallback behind a speculative launch): the kernel does nothing unless the verdict is non-zero,
+    // and its workgroups, one per compute unit, walk the `walk_blocks` workgroup ids of an ordinary launch
+    GuardArgs guard;
     int walk_blocks;
 };
 
@@ -147,10 +149,8 @@ __device__ __forceinline__ void mm_update(MinMax &r, int64_t v)
 // element; measured on the 512 x 7168 x 18432 product, 5.5 % of the kernel's time went into tracking B that way): the
 // digit count itself.  In balanced base-256 digits x + 0x8080...80 has byte j equal to 0x80 wherever digit j is zero,
 // so the OR over all elements of (x + 0x80..80) ^ 0x80..80 has its highest non-zero byte at the highest digit any
-// element needs: six full-rate 32-bit instructions per element.  The range reported for n digits is the widest one n
-// digits hold, [-0x80..80, 0x7F..7F] (n bytes each), which is all that the digit choice of the next call reads from it.
-// (An element beyond eight digits wraps the sum; it leaves a non-zero top byte like one that needs eight, and both are
-// reported as the full range: nine digits.)
+// element needs: six full-rate 32-bit instructions per element.  (An element beyond eight digits wraps the sum; it leaves
+// a non-zero top byte like one that needs eight, and both count as nine digits.)
 struct DigitsSeen {
     uint32_t lo = 0, hi = 0;
     bool seen = false;
@@ -160,21 +160,34 @@ struct DigitsSeen {
         lo |= (uint32_t)t;
         hi |= (uint32_t)(t >> 32);
     }
-    __device__ __forceinline__ MinMax range() const
+    // digits that hold everything added (0: nothing was)
+    __device__ __forceinline__ int digits() const
     {
-        if (!seen) return MinMax{ INT64_MAX, INT64_MIN };
+        if (!seen) return 0;
         const uint64_t e = ((uint64_t)hi << 32) | lo;
-        if (e >> 56) return MinMax{ INT64_MIN, INT64_MAX };
-        const int n = e ? (71 - __clzll((long long)e)) >> 3 : 1;          // bytes up to the highest non-zero one
-        const uint64_t mask = ~0ull >> (64 - 8 * n);
-        return MinMax{ -(int64_t)(0x8080808080808080ull & mask), (int64_t)(0x7F7F7F7F7F7F7F7Full & mask) };
+        if (e >> 56) return 9;
+        return e ? (71 - __clzll((long long)e)) >> 3 : 1;                 // bytes up to the highest non-zero one
     }
 };
 
-__device__ __forceinline__ void mm_merge(MinMax &r, const MinMax &o)
+// the same for int32 values between lo and hi (0: lo > hi, nothing was seen)
+__device__ __forceinline__ int digits_i32(int lo, int hi)
 {
-    r.lo = o.lo < r.lo ? o.lo : r.lo;
-    r.hi = o.hi > r.hi ? o.hi : r.hi;
+    if (lo > hi) return 0;
+    if (lo >= -0x80 && hi <= 0x7F) return 1;
+    if (lo >= -0x8080 && hi <= 0x7F7F) return 2;
+    if (lo >= -0x808080 && hi <= 0x7F7F7F) return 3;
+    return hi <= 0x7F7F7F7F ? 4 : 5;
+}
+
+__device__ __forceinline__ int wave_max_i32(int v)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const int o = __shfl_xor(v, off, kWave);
+        v = o > v ? o : v;
+    }
+    return v;
 }
 
 __device__ __forceinline__ MinMax mm_wave(MinMax r)
@@ -203,6 +216,19 @@ __device__ __forceinline__ void mm_publish(MinMax r, unsigned long long *slot)
 static __global__ void range_reset_kernel(unsigned long long *range)
 {
     if (threadIdx.x < 4) range[threadIdx.x] = (threadIdx.x & 1) ? 0ull : ~0ull;
+}
+
+// What a workgroup leaves about the digits of its share: its word for the report (see guard_report), and, only when an
+// element did not fit the launch's digit counts, the verdict that makes the guarded launch behind compute everything
+// again: 1 when five digits hold what it saw (and every digit count of the launch is at most five), else 2.  Nothing is
+// written to the shared word in the ordinary case, so thousands of workgroups do not queue up for one address.
+__device__ __forceinline__ void leave_digits(unsigned *seen_slot, unsigned *verdict, int fail_class, int na, int nb, int need_a, int need_b)
+{
+    if (seen_slot) *seen_slot = (unsigned)need_a | ((unsigned)need_b << 8);
+    if (need_a > na || need_b > nb) {
+        const unsigned v = (need_a > 5 || need_b > 5) ? 2u : (unsigned)fail_class;
+        atomicMax(verdict, v);
+    }
 }
 
 // Strided sample of both operands for the first guess (at most `rows_s` rows x `cols_s` k each).
@@ -295,14 +321,13 @@ __device__ __forceinline__ int frag_offset(int row, int j, int n_limbs, int subs
 // When A is reused by many column tiles it is split once, into digit planes stored in MFMA fragment order:
 // block (g, sub, ks32, i) of 1 KB holds digit i of rows [32*sub, 32*sub+32) for the 32 owned-k slots of MFMA
 // depth ks32, lane-major.  Rows >= M and k >= K are written as zero digits.  Each workgroup also leaves the
-// min and max of what it read in mm[2*block .. 2*block+1].
+// digits of what it read needs in seen[block] (when that is given).
 // IN32: the matrix holds int32 elements (weights prepared once; lda and sA count elements as they do for int64).
 template <int NA, int RUN, int KK, bool IN32 = false>
-__global__ __launch_bounds__(256) void a_planes_kernel(MfmaParams p, unsigned char *planes, int msub, int ksteps32,
-                                                       unsigned long long *mm)
+__global__ __launch_bounds__(256) void a_planes_kernel(MfmaParams p, unsigned char *planes, int msub, int ksteps32, unsigned *seen)
 {
     constexpr int OCTS = 4 * KK, ROWS = 256 / OCTS;
-    __shared__ MinMax red[4];
+    __shared__ int red[4];
     const int tid = threadIdx.x;
     const int g = blockIdx.z, ks = blockIdx.x;
     const int row = blockIdx.y * ROWS + tid / OCTS, j = tid % OCTS;
@@ -315,7 +340,6 @@ __global__ __launch_bounds__(256) void a_planes_kernel(MfmaParams p, unsigned ch
 #pragma unroll
     for (int q = 0; q < 8; q++) bound.add(x[q]);
     bound.seen = true;
-    MinMax r = bound.range();
     uint2 dg[NA];
     limb_split8<NA>(x, dg);
     // plane step layout: [g][sub][ks32][digit][1 KB]; a step of KK depths is contiguous per sub
@@ -325,100 +349,21 @@ __global__ __launch_bounds__(256) void a_planes_kernel(MfmaParams p, unsigned ch
 #pragma unroll
         for (int i = 0; i < NA; i++) *reinterpret_cast<uint2 *>(dst + i * 1024) = dg[i];
     }
-    r = mm_wave(r);
-    if ((tid & 63) == 0) red[tid >> 6] = r;
+    if (!seen) return;
+    const int need = wave_max_i32(bound.digits());
+    if ((tid & 63) == 0) red[tid >> 6] = need;
     __syncthreads();
     if (tid == 0) {
+        int n = red[0];
 #pragma unroll
-        for (int w = 1; w < 4; w++) mm_merge(r, red[w]);
+        for (int w = 1; w < 4; w++) n = red[w] > n ? red[w] : n;
         const long b = ((long)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
-        mm[2 * b] = (unsigned long long)r.lo ^ kSignFlip;
-        mm[2 * b + 1] = (unsigned long long)r.hi ^ kSignFlip;
+        leave_digits(seen + b, p.verdict, p.fail_class, NA, NA, n, 0);
     }
 }
 
-// Folds the per-workgroup ranges of the plane pre-pass (`mm`, A only) and of the GEMM kernel (`wg`, A and B) into
-// range[0..3] and leaves the verdict in range[4]: 0 when `na` and `nb` digits covered them, otherwise 1 when five digits
-// cover both operands and 2 when they do not (what the guarded launch behind the product multiplies with).
-// `host_copy`, when set, is pinned host memory that receives the same five words.
-// `parts` workgroups (of any size) share the slots; each leaves its partial result in `scratch` and takes a ticket, and
-// the one that arrives last folds the partials (a launch with tens of thousands of tiles would otherwise spend longer
-// in a one-workgroup fold than some GEMMs take).  range[5] is the ticket counter; it is zero between launches.
-constexpr int kFoldParts = 64;        // at most this many workgroups fold
-constexpr long kFoldSlotsPerPart = 1024;
-
-struct FoldArgs {
-    const unsigned long long *mm;
-    long mm_count;
-    const unsigned long long *wg;
-    long wg_count;
-    unsigned long long *range;
-    int na, nb;
-    unsigned long long *host_copy;
-    int parts;
-    unsigned long long *scratch;      // 4 * kFoldParts words
-};
-
-__host__ __device__ inline unsigned long long fold_pick(int q, unsigned long long a, unsigned long long b)
-{
-    return (q & 1) ? (a > b ? a : b) : (a < b ? a : b);       // words 1 and 3 are maxima, 0 and 2 minima
-}
-
-__device__ __forceinline__ void range_fold_body(const FoldArgs &f, int part)
-{
-    __shared__ unsigned long long red[16][4];
-    const int nthreads = blockDim.x;
-    const long first = (long)part * nthreads + threadIdx.x, stride = (long)f.parts * nthreads;
-    unsigned long long v[4] = { ~0ull, 0ull, ~0ull, 0ull };
-    for (long i = first; i < f.mm_count; i += stride) {
-        v[0] = fold_pick(0, f.mm[2 * i], v[0]);
-        v[1] = fold_pick(1, f.mm[2 * i + 1], v[1]);
-    }
-    for (long i = first; i < f.wg_count; i += stride) {
-#pragma unroll
-        for (int q = 0; q < 4; q++) v[q] = fold_pick(q, f.wg[4 * i + q], v[q]);
-    }
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1)
-            v[q] = fold_pick(q, (unsigned long long)__shfl_xor((long long)v[q], off, kWave), v[q]);
-    }
-    if ((threadIdx.x & 63) == 0) {
-#pragma unroll
-        for (int q = 0; q < 4; q++) red[threadIdx.x >> 6][q] = v[q];
-    }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    for (int w = 1; w < nthreads / 64; w++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) v[q] = fold_pick(q, red[w][q], v[q]);
-    if (f.parts > 1) {
-#pragma unroll
-        for (int q = 0; q < 4; q++) __hip_atomic_store(&f.scratch[4 * part + q], v[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // release the partial, then count in; whoever sees everyone else counted in acquires their partials
-        const unsigned long long ticket = __hip_atomic_fetch_add(&f.range[5], 1ull, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if (ticket != (unsigned long long)(f.parts - 1)) return;
-        for (int w = 0; w < f.parts; w++)
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                v[q] = fold_pick(q, __hip_atomic_load(&f.scratch[4 * w + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), v[q]);
-        __hip_atomic_store(&f.range[5], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-#pragma unroll
-    for (int q = 0; q < 4; q++) f.range[q] = v[q];
-    const int need_a = limbs_needed((int64_t)(v[0] ^ kSignFlip), (int64_t)(v[1] ^ kSignFlip));
-    const int need_b = limbs_needed((int64_t)(v[2] ^ kSignFlip), (int64_t)(v[3] ^ kSignFlip));
-    const unsigned long long verdict = (need_a <= f.na && need_b <= f.nb) ? 0ull : ((need_a <= 5 && need_b <= 5) ? 1ull : 2ull);
-    f.range[4] = verdict;
-    if (f.host_copy) {
-#pragma unroll
-        for (int q = 0; q < 4; q++) f.host_copy[q] = v[q];
-        f.host_copy[4] = verdict;
-    }
-}
-
-static __global__ __launch_bounds__(256) void range_fold_kernel(FoldArgs f) { range_fold_body(f, (int)blockIdx.x); }
+// The report of a launch that has no guarded launch behind it (its caller waits for the digits instead).
+static __global__ __launch_bounds__(256) void digits_report_kernel(GuardArgs g) { guard_report(g); }
 
 // Number of digit pairs (i', j') with i' + j' < d that come before (i, j) in row order (i' < i, or i' == i and j' < j).
 __host__ __device__ constexpr int kept_pairs_before(int na, int nb, int d, int i, int j)
@@ -479,10 +424,7 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
         const int xcd = lin & 7, w = lin >> 3, wq = w / p.tiles_n;
         const int mt = wq * 8 + xcd;
         if (mt >= *p.grp_ntiles) {                 // the grid covers the worst case: nothing to do, an empty range
-            if (tid == 0) {
-                unsigned long long *slot = p.wg_range + 4 * (long)block;
-                slot[0] = ~0ull; slot[1] = 0ull; slot[2] = ~0ull; slot[3] = 0ull;
-            }
+            if (tid == 0 && p.seen) p.seen[block] = 0;
             return;
         }
         tn = w - wq * p.tiles_n;
@@ -890,30 +832,23 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
     for (; ks + 1 < ks_end; ks++) step_body(ks, std::false_type());
     compute_all((ks_end - 1 - ks_begin) & 1);
 
-    // every workgroup leaves its ranges (empty ones included) in its own slot; the waves' ranges meet in LDS
-    // (the stages are free by now)
-    MinMax ra = { INT64_MAX, INT64_MIN }, rb = { INT64_MAX, INT64_MIN };
+    // every workgroup leaves the digits of what it saw in its own word; the waves meet in LDS (the stages are free by now)
+    int need_a = 0, need_b = 0;
     if (verify_a || verify_b) {
         __syncthreads();
-        MinMax *red = reinterpret_cast<MinMax *>(smem);
-        ra = oa.range();
-        rb = ob.range();
-        if (B32 && !BRS && rb32_lo <= rb32_hi) mm_merge(rb, MinMax{ (int64_t)rb32_lo, (int64_t)rb32_hi });
-        ra = mm_wave(ra);
-        rb = mm_wave(rb);
-        if (lane == 0) { red[2 * wave] = ra; red[2 * wave + 1] = rb; }
+        int *red = reinterpret_cast<int *>(smem);
+        need_a = wave_max_i32(oa.digits());
+        need_b = wave_max_i32(B32 && !BRS ? digits_i32(rb32_lo, rb32_hi) : ob.digits());
+        if (lane == 0) { red[2 * wave] = need_a; red[2 * wave + 1] = need_b; }
         __syncthreads();
         if (tid == 0) {
-            for (int w = 1; w < T / 64; w++) { mm_merge(ra, red[2 * w]); mm_merge(rb, red[2 * w + 1]); }
+            for (int w = 1; w < T / 64; w++) {
+                need_a = red[2 * w] > need_a ? red[2 * w] : need_a;
+                need_b = red[2 * w + 1] > need_b ? red[2 * w + 1] : need_b;
+            }
         }
     }
-    if (tid == 0) {
-        unsigned long long *slot = p.wg_range + 4 * (long)block;
-        slot[0] = (unsigned long long)ra.lo ^ kSignFlip;
-        slot[1] = (unsigned long long)ra.hi ^ kSignFlip;
-        slot[2] = (unsigned long long)rb.lo ^ kSignFlip;
-        slot[3] = (unsigned long long)rb.hi ^ kSignFlip;
-    }
+    if (tid == 0) leave_digits(p.seen ? p.seen + block : nullptr, p.verdict, p.fail_class, NA, NB, need_a, need_b);
 
     // epilogue: diagonals -> 128-bit sum -> shift.  Accumulator register r of lane l holds
     // row 8*(r/4) + 4*(l/32) + r%4, column l%32 of its 32x32 tile.
@@ -994,7 +929,8 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_mfma_kernel(MfmaParams p)
 template <int NA, int NB, int WVM, int WVN, int WM, int WN, int KK, bool B32, int DMAX = 16>
 __global__ __launch_bounds__(64 * WVM * WVN) void gemm_mfma_guarded_kernel(MfmaParams p)
 {
-    const unsigned long long verdict = __atomic_load_n(p.guard, __ATOMIC_RELAXED);            // (the same for every thread of the launch)
+    const unsigned verdict = __atomic_load_n(p.guard.verdict, __ATOMIC_RELAXED);            // (the same for every thread of the launch)
+    if (blockIdx.x == 0) guard_report(p.guard);
     if (verdict == 0) return;
     if (verdict == 1 && (NA > 5 || NB > 5)) {
         // five digits cover both operands (the fold kernel has seen every element): a third of the digit pairs of (9,9)
@@ -1013,14 +949,9 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_mfma_guarded_kernel(MfmaP
 
 // Adds the `split` partial sums of every tail tile, applies the rounding term and the shift, and stores C and R.
 // Thread layout and element order are those of the GEMM kernel's epilogue.
-// The last `fold.parts` workgroups fold the ranges (the GEMM kernel has left them by then), which saves a launch.
 template <int WVM, int WVN, int WM, int WN>
-__global__ __launch_bounds__(64 * WVM * WVN) void gemm_split_finish_kernel(MfmaParams p, FoldArgs fold)
+__global__ __launch_bounds__(64 * WVM * WVN) void gemm_split_finish_kernel(MfmaParams p)
 {
-    if (blockIdx.x >= gridDim.x - fold.parts) {
-        range_fold_body(fold, (int)(blockIdx.x - (gridDim.x - fold.parts)));
-        return;
-    }
     constexpr int T = 64 * WVM * WVN, BM = 32 * WM * WVM, BN = 32 * WN * WVN;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WVN, wn = wave % WVN;
@@ -1099,8 +1030,8 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_split_finish_kernel(MfmaP
 
 // ---- kernel tables -------------------------------------------------------------------------------------
 typedef void (*MfmaKernel)(MfmaParams);
-typedef void (*FinishKernel)(MfmaParams, FoldArgs);
-typedef void (*PlanesKernel)(MfmaParams, unsigned char *, int, int, unsigned long long *);
+typedef void (*FinishKernel)(MfmaParams);
+typedef void (*PlanesKernel)(MfmaParams, unsigned char *, int, int, unsigned *);
 
 enum Variant { kB64Fly = 0, kB64Planes, kB32Fly, kB32Planes, kB64KmajorFly, kB32KmajorFly, kB64Group, kB32Group, kB64FlyRs, kB32FlyRs,
                kB64PlanesBoth, kB64FlyBPlanes, kB64GroupBPlanes, kVariants };     // the last three: B from prepared digit planes
@@ -1111,7 +1042,7 @@ struct Instance {
     int dmax;                    // diagonals from this one up are left out (16: none but the 2^128 one)
     MfmaKernel fn[kVariants];
     PlanesKernel planes[2];      // [b32]: the owned-k pattern follows the element size of B
-    FinishKernel finish;         // adds up the partial sums of split tail tiles (and folds the ranges)
+    FinishKernel finish;         // adds up the partial sums of split tail tiles
     MfmaKernel guarded[2];       // [b32]: the guarded form for row-major B, A split on the fly (the widest instances only)
 };
 

@@ -8,8 +8,8 @@
 //     registers at the start of the step, A's digit by digit into the registers whose last use has just been issued
 //     (the MFMAs go through A's digits in order), so that the matrix pipe has its operands the moment the step's one
 //     barrier opens.
-// Eight wavefronts as 2 x 4, 64 x 32 outputs each, as in the general kernel; tiles, split tail tiles, partial sums, range
-// slots and outputs are the general kernel's (gemm_mfma_block with APL and BPL), which this one replaces for three digits
+// Eight wavefronts as 2 x 4, 64 x 32 outputs each, as in the general kernel; tiles, split tail tiles, partial sums, digit
+// words and outputs are the general kernel's (gemm_mfma_block with APL and BPL), which this one replaces for three digits
 // a side.
 #pragma once
 #include "lds_dma.h"
@@ -163,11 +163,8 @@ __global__ __launch_bounds__(512) void gemm_mfma_pipe_kernel(MfmaParams p)
     wait_vmcnt<0>();                                       // (the loads past the end)
     asm volatile("" ::: "memory");
 
-    // both operands' ranges were fixed when their planes were written: an empty range from here
-    if (tid == 0) {
-        unsigned long long *slot = p.wg_range + 4 * (long)blockIdx.x;
-        slot[0] = ~0ull; slot[1] = 0ull; slot[2] = ~0ull; slot[3] = 0ull;
-    }
+    // both operands' digits were counted when their planes were written: nothing seen here
+    if (tid == 0 && p.seen) p.seen[blockIdx.x] = 0;
 
     // epilogue: diagonals -> 128-bit sum -> shift, as in gemm_mfma_block (accumulator register r of lane l holds
     // row 8*(r/4) + 4*(l/32) + r%4, column l%32 of its 32 x 32 tile)

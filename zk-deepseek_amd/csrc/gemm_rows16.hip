@@ -44,7 +44,7 @@ struct Rows16Params {
     // grouped mode: rows of A and C form one segment per group, every group has its own B (see GroupedDesc)
     const int *grp_seg, *grp_tiles, *grp_ntiles;
     const void *const *grp_b;
-    const unsigned long long *guard;     // when set: do nothing unless this word is non-zero
+    GuardArgs guard;                     // with a verdict word: do nothing unless it is non-zero
     unsigned items;                      // work items of the launch (the grid may be smaller: workgroups walk them)
 };
 
@@ -432,7 +432,11 @@ __device__ __forceinline__ void rows16_item(const Rows16Params &p, unsigned item
 template <bool B32, bool GRP>
 __global__ __launch_bounds__(64 * kR16Waves) void gemm_rows16_kernel(Rows16Params p)
 {
-    if (p.guard && *p.guard == 0) return;            // (the same for every thread of the launch)
+    if (p.guard.verdict) {
+        const unsigned verdict = __atomic_load_n(p.guard.verdict, __ATOMIC_RELAXED);       // (the same for every thread of the launch)
+        if (blockIdx.x == 0) guard_report(p.guard);
+        if (verdict == 0) return;
+    }
     for (unsigned item = blockIdx.x; item < p.items; item += gridDim.x) {
         rows16_item<B32, GRP>(p, item);
         if (item + gridDim.x < p.items) __syncthreads();           // (the rings are used again)
@@ -590,7 +594,7 @@ static int r16_run(Rows16Kernel fn, const Rows16Params &params, long blocks)
     constexpr int lds = kR16LdsBytes;
     Rows16Params p = params;
     p.items = (unsigned)blocks;
-    if (p.guard && blocks > r16_cus()) blocks = r16_cus();
+    if (p.guard.verdict && blocks > r16_cus()) blocks = r16_cus();
     static const void *raised[4] = {};
     bool seen = false;
     for (const void *f : raised) seen = seen || f == (const void *)fn;
@@ -654,7 +658,7 @@ int gemm_rows16_launch(const GemmDesc &d, unsigned long long *acc, size_t max_sl
     return 0;
 }
 
-int gemm_rows16_grouped(const GroupedDesc &d, const unsigned long long *guard)
+int gemm_rows16_grouped(const GroupedDesc &d, const GuardArgs &guard)
 {
     if (d.K < 0 || d.N < 1 || d.rows < 1 || d.groups < 1) return 1;
     std::lock_guard<std::mutex> lock(g_r16_mu);

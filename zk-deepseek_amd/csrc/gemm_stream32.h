@@ -46,9 +46,9 @@ __global__ __launch_bounds__(512) void gemm_stream32_grouped_kernel(MfmaParams p
     // (the tile columns of one 32-row tile on one XCD, as in gemm_mfma_block's grouped form: its rows of A come from memory once)
     const int xcd = (int)blockIdx.x & 7, w = (int)blockIdx.x >> 3, wq = w / p.tiles_n;
     const int mt = wq * 8 + xcd;
-    unsigned long long *slot = p.wg_range + 4 * (long)blockIdx.x;
-    if (mt >= *p.grp_ntiles) {                   // the grid covers the worst case: nothing to do, an empty range
-        if (tid == 0) { slot[0] = ~0ull; slot[1] = 0ull; slot[2] = ~0ull; slot[3] = 0ull; }
+    unsigned *slot = p.seen ? p.seen + blockIdx.x : nullptr;
+    if (mt >= *p.grp_ntiles) {                   // the grid covers the worst case: nothing to do, nothing seen
+        if (tid == 0 && slot) *slot = 0;
         return;
     }
     const int tn = w - wq * p.tiles_n;
@@ -57,9 +57,9 @@ __global__ __launch_bounds__(512) void gemm_stream32_grouped_kernel(MfmaParams p
     const int32_t *b_base = reinterpret_cast<const int32_t *>(p.grp_b[e]);
     if ((uintptr_t)b_base & 15) {
         // a matrix that does not start on a 16-byte boundary: the loads into LDS cannot take it.  The workgroup reports
-        // the full range for B instead of computing (and nothing for A, which it has not looked at): no digit count
-        // covers that, so the guarded launch behind this one (or the caller's next route) computes these outputs.
-        if (tid == 0) { slot[0] = ~0ull; slot[1] = 0ull; slot[2] = 0ull; slot[3] = ~0ull; }
+        // nine digits for B instead of computing (and nothing for A, which it has not looked at): no digit count of this
+        // kernel covers that, so the guarded launch behind it (or the caller's next route) computes these outputs.
+        if (tid == 0) leave_digits(slot, p.verdict, p.fail_class, NA, NB, 0, 9);
         return;
     }
     const int n0 = tn * 256 + wave * 32;
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(512) void gemm_stream32_grouped_kernel(MfmaParams p
         for (int q = 0; q < 4; q++) lds_dma16(bq[q] + 32 * (long)t, ring_b_lds + st * 4096 + q * 1024);
     };
 
-    // ---- range tracking (see gemm_mfma_block): A is shared out over the first tile columns, B is all this workgroup's ----
+    // ---- digit tracking (see gemm_mfma_block): A is shared out over the first tile columns, B is all this workgroup's ----
     const int vmod_a = p.tiles_n < 8 ? p.tiles_n : 8;
     const bool verify_a = tn < vmod_a;
     DigitsSeen oa;
@@ -305,20 +305,17 @@ __global__ __launch_bounds__(512) void gemm_stream32_grouped_kernel(MfmaParams p
         }
     }
 
-    // every workgroup leaves its ranges in its own slot; the waves' ranges meet in LDS (the rings are free by now)
-    MinMax ra = oa.range(), rb = { INT64_MAX, INT64_MIN };
-    if (rb_lo <= rb_hi) rb = MinMax{ (int64_t)rb_lo, (int64_t)rb_hi };
-    ra = mm_wave(ra);
-    rb = mm_wave(rb);
-    MinMax *red = reinterpret_cast<MinMax *>(s32_smem);
-    if (lane == 0) { red[2 * wave] = ra; red[2 * wave + 1] = rb; }
+    // every workgroup leaves the digits of what it saw in its own word; the waves meet in LDS (the rings are free by now)
+    int need_a = wave_max_i32(oa.digits()), need_b = wave_max_i32(digits_i32(rb_lo, rb_hi));
+    int *red = reinterpret_cast<int *>(s32_smem);
+    if (lane == 0) { red[2 * wave] = need_a; red[2 * wave + 1] = need_b; }
     __syncthreads();
     if (tid == 0) {
-        for (int w = 1; w < 8; w++) { mm_merge(ra, red[2 * w]); mm_merge(rb, red[2 * w + 1]); }
-        slot[0] = (unsigned long long)ra.lo ^ kSignFlip;
-        slot[1] = (unsigned long long)ra.hi ^ kSignFlip;
-        slot[2] = (unsigned long long)rb.lo ^ kSignFlip;
-        slot[3] = (unsigned long long)rb.hi ^ kSignFlip;
+        for (int w = 1; w < 8; w++) {
+            need_a = red[2 * w] > need_a ? red[2 * w] : need_a;
+            need_b = red[2 * w + 1] > need_b ? red[2 * w + 1] : need_b;
+        }
+        leave_digits(slot, p.verdict, p.fail_class, NA, NB, need_a, need_b);
     }
 }
 

@@ -30,7 +30,7 @@ struct ValuParams {
     int a_shift, b_shift;                     // log2 of a divisor that is a positive power of two, else -1
     int tiles_m, tiles_n;
     long tiles;                               // tiles_m * tiles_n * G, walked by a 1-D grid
-    const unsigned long long *guard;          // when set: do nothing unless *guard != 0
+    GuardArgs guard;                          // with a verdict word: do nothing unless it is non-zero
     // grouped matrix-vector launches: blockIdx.y is a row of A, whose B is that of the segment the row lies in
     const void *const *grp_b;                 // device array of `groups` device pointers
     const int *grp_seg;                       // device [groups + 1]: first row of every segment
@@ -61,7 +61,11 @@ __global__ __launch_bounds__(256) void gemm_valu_kernel(ValuParams p)
     __shared__ int64_t Bs[kVK][kVP];
 
     const int tid = threadIdx.x;
-    if (p.guard && __atomic_load_n(p.guard, __ATOMIC_RELAXED) == 0) return;
+    if (p.guard.verdict) {
+        const unsigned verdict = __atomic_load_n(p.guard.verdict, __ATOMIC_RELAXED);
+        if (blockIdx.x == 0) guard_report(p.guard);
+        if (verdict == 0) return;
+    }
     for (long tile = blockIdx.x; tile < p.tiles; tile += gridDim.x) {
     const int g = (int)(tile / ((long)p.tiles_m * p.tiles_n));
     const int rem = (int)(tile - (long)g * p.tiles_m * p.tiles_n);
@@ -147,7 +151,7 @@ static void launch2(const ValuParams &p, dim3 grid, bool rescale)
     else gemm_valu_kernel<B32, KMAJOR, false><<<grid, dim3(256), 0, 0>>>(p);
 }
 
-void gemm_valu_launch(const GemmDesc &d, const unsigned long long *guard)
+void gemm_valu_launch(const GemmDesc &d, const GuardArgs &guard)
 {
     ValuParams p;
     p.A = d.A; p.B = d.B; p.C = d.C; p.R = d.R;
@@ -169,7 +173,7 @@ void gemm_valu_launch(const GemmDesc &d, const unsigned long long *guard)
     const bool rescale = d.a_rs != 1 || d.b_rs != 1;
     const bool kmajor = d.ldbn == 1 && d.ldbk != 1;
     // a guarded launch normally finds nothing to do, so it is kept small; either way workgroups stride over the tiles
-    const long cap = guard ? 2048 : (1L << 22);
+    const long cap = guard.verdict ? 2048 : (1L << 22);
     dim3 grid((unsigned)(p.tiles < cap ? p.tiles : cap));
     if (d.b32) { if (kmajor) launch2<true, true>(p, grid, rescale); else launch2<true, false>(p, grid, rescale); }
     else { if (kmajor) launch2<false, true>(p, grid, rescale); else launch2<false, false>(p, grid, rescale); }
