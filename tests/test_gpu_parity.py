@@ -98,6 +98,27 @@ def test_gemm_many_digit_operands_at_every_shift(K, oracle, bits_a, bits_w, w32,
     K.lib.zk_gemm_set_path(0)
 
 
+@pytest.mark.parametrize("w32", [False, True])
+@pytest.mark.parametrize("bits_a,bits_w,digits", [(20, 16, (3, 3)), (20, 28, (3, 4)), (28, 20, (4, 3)), (28, 28, (4, 4)), (36, 28, (5, 4)),
+                                                  (28, 30.99, (4, 5)), (20, 30.99, (3, 5)), (36, 30.99, (5, 5)), (44, 20, (6, 3))])
+def test_gemm_two_depths_per_step(K, oracle, bits_a, bits_w, digits, w32):
+    """the 128-row tiles by digit counts, two MFMA depths per step: K around whole steps of 64, row counts whose last tile
+    has one, two or three live groups of 32 rows, launches smaller than the device with short slices of K (A split in the
+    kernel) and long ones (A from planes), and larger than the device"""
+    rng = np.random.default_rng(int(bits_a * 7 + bits_w) + w32)
+    top = (1 << 31) - 1 if bits_w > 30 else None          # (an int32 needs a fifth digit at the top of its range)
+    for M, Kd, N in ((129, 64, 66), (160, 127, 300), (225, 129, 130), (97, 2050, 320), (70, 1, 256), (260, 192, 6000)):
+        A = rand_i64(rng, (1, M, Kd), bits_a)
+        W = rand_i32(rng, (N, Kd), int(bits_w)) if w32 else rand_i64(rng, (N, Kd), int(bits_w))
+        if top:
+            W[N - 1, Kd - 1] = top
+        W[0, 0], A[0, M - 1, Kd - 1] = W[0, 0] | (1 << (int(bits_w) - 1)), (1 << bits_a) - 1
+        for _ in range(2):      # (a first call may run on digits remembered for other operands at these addresses)
+            _gemm_case(K, oracle, 2, A, W, 1, 1, 23)
+    assert K.gemm_last_plan()[1:] == digits
+    K.lib.zk_gemm_set_path(0)
+
+
 @pytest.mark.parametrize("Kd", [14560, 14600, 16384, 18432])
 def test_gemm_long_k_with_nine_digit_operands(K, oracle, Kd):
     """the int32 accumulators of the MFMA path hold min(NA, NB) * K * 2^14: with nine digits that ends at K = 14563.

@@ -53,6 +53,7 @@ static const Instance *instances(int *count)
         mfma_instances_narrow(t);
         mfma_instances_mid(t);
         mfma_instances_wide(t);
+        mfma_instances_both(t);
         mfma_instances_pruned(t);
         mfma_instances_rows32(t);
         mfma_instances_rows32b(t);
@@ -75,7 +76,7 @@ static const Instance *pick_instance(int na, int nb, bool b32, bool skinny, int 
     const Instance *best = nullptr;
     long best_cost = 0;
     for (int i = 0; i < count; i++) {
-        if (t[i].na < na || t[i].nb < nb || t[i].skinny != skinny) continue;
+        if (t[i].na < na || t[i].nb < nb || t[i].skinny != skinny || t[i].alt) continue;
         if (t[i].dmax < 16 && t[i].dmax < need_diag) continue;
         if (exact_nb && (t[i].nb != exact_nb || t[i].kk != exact_kk)) continue;
         if (variant >= 0 && !t[i].fn[variant]) continue;
@@ -86,6 +87,24 @@ static const Instance *pick_instance(int na, int nb, bool b32, bool skinny, int 
         if (!best || cost < best_cost || (cost == best_cost && t[i].kk > best->kk)) { best = &t[i]; best_cost = cost; }
     }
     return best;
+}
+
+// The 128x64 form of an instance with 128x128 tiles, for launches of fewer 128x128 tiles than compute units: twice the
+// tiles, so half the slices of K per tile (half the partial sums), and two depths per step.  With (3,3) digits on int64
+// weights, 128x128 against 128x64 tiles, both on planes of A: 128 rows x [2048,7168] (16 tiles) 39.0 / 36.9 us, 128 x
+// [7168,2048] (56) 41.7 / 38.0, 200 x [7168,7168] (112) 159 / 147, 300 x [7168,7168] (168) 217 / 202.  Not where the
+// halves fill a round and three quarters (their last round is then not split): 500 x [7168,2048] (224) 69.5 / 80; nor for
+// launches larger than the device, which are bound by operand traffic: 512 x [18432,7168] 607 / 666.
+static const Instance *smaller_tiles(const Instance *inst, const GemmDesc &d, int cus)
+{
+    const long tiles = (long)((d.M + inst->bm - 1) / inst->bm) * ((d.N + inst->bn - 1) / inst->bn) * d.G;
+    if (inst->bm != 128 || inst->bn != 128 || tiles >= cus) return inst;
+    if (2 * tiles > cus && 2 * tiles - cus > cus / 2) return inst;
+    int count;
+    const Instance *t = instances(&count);
+    for (int i = 0; i < count; i++)
+        if (t[i].alt && t[i].na == inst->na && t[i].nb == inst->nb) return t + i;
+    return inst;
 }
 
 typedef std::tuple<const void *, long, long, int> OperandKey;     // (pointer, rows, K, element size)
@@ -669,6 +688,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             if (!inst) inst = pick_instance(na, nb, d.b32 != 0, false, need_diag);
         }
         if (!inst) return kDeclined;
+        if (!prep && !inst->skinny) inst = smaller_tiles(inst, d, g_cache.cus);
         // int32 accumulators: at most min(NA,NB) digit pairs per diagonal, each product at most 2^14 in magnitude
         const long pairs = inst->na < inst->nb ? inst->na : inst->nb;
         const int ksteps = ((d.K + 32 * inst->kk - 1) / (32 * inst->kk)) * inst->kk;     // 32-k steps, padded
@@ -685,11 +705,19 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         if (per_batch > 0x7FFFFFFFL) return kDeclined;
         const long total = per_batch * d.G;
         if (total > 0x7FFFFFFFL / 8) return kDeclined;
+        const int steps = (d.K + 32 * inst->kk - 1) / (32 * inst->kk);
+        // slices of K per tile of a launch smaller than the device
+        int small_split = total < g_cache.cus ? (int)(g_cache.cus / total) : 1;
+        if (small_split > 64) small_split = 64;
+        if (small_split > steps / 4) small_split = steps / 4;
         // A is pre-split into digit planes when enough column tiles reuse it to pay for the extra pass (never for the
-        // 32-row tiles: splitting a handful of rows on the fly is cheaper than another kernel in front)
-        // (nor for a launch with fewer tiles than compute units: its tiles are cut along K, every workgroup splits a short
-        // slice of A, and the pre-pass would be a launch of its own in front: 128 rows x [2048,7168] 43.8 -> 42.4 us)
-        const bool use_planes = !kmajor && ((p.tiles_n >= g_switches.planes_min_tiles_n && total >= g_cache.cus) || prep) && !inst->skinny;
+        // 32-row tiles: splitting a handful of rows on the fly is cheaper than another kernel in front; nor where the
+        // slices of a small launch are so short that the launch in front costs more than three bytes instead of eight per
+        // element of A save.  On the fly against planes, by K per workgroup: 256 (512 rows x [1024,1024] int32) 34.6 / 36.6
+        // us, 448 (243 x [512,7168]) 35.6 / 39.4, 896 (128 x [2048,7168]) 46.7 / 46.2, 1024 (128 x [7168,2048]) 49.5 /
+        // 47.1, 1434 (243 x [1536,7168]) 54.7 / 52.2, 16384 (243 x [7168,16384]) 449 / 353.)
+        const bool long_slices = (long)steps * 32 * inst->kk >= 800L * (small_split > 1 ? small_split : 1);
+        const bool use_planes = !kmajor && !inst->skinny && (prep || (p.tiles_n >= g_switches.planes_min_tiles_n && (total >= g_cache.cus || long_slices)));
         if (b_shift && (kmajor || !inst->skinny)) return kDeclined;
         const int variant = prep ? (inst->skinny ? kB64FlyBPlanes : kB64PlanesBoth)
                           : b_shift ? (d.b32 ? kB32FlyRs : kB64FlyRs)
@@ -707,7 +735,6 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         // Split-K: a launch smaller than the device is cut into `split` slices of K per tile, each a workgroup of
         // its own; with more tiles than compute units the same is done for the tiles of the last, partial round
         // only.  The slices leave raw partial sums and a small kernel adds them.
-        const int steps = (d.K + 32 * inst->kk - 1) / (32 * inst->kk);
         int tail = (int)(total % g_cache.cus), split = 1;
         p.main_tiles = (int)total;
         p.split = 1;
@@ -718,9 +745,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         if (!g_switches.no_tail_split) {
             if (total < g_cache.cus) {
                 tail = (int)total;
-                split = g_cache.cus / tail;
-                if (split > 64) split = 64;
-                if (split > steps / 4) split = steps / 4;
+                split = small_split;
                 p.finish_rq = 16;
             } else if (inst->skinny && total < 8L * g_cache.cus) {
                 // a few rows against many columns is a weight stream: more, shorter workgroups keep more of it in

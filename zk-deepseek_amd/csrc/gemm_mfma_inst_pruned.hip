@@ -5,10 +5,10 @@ namespace zk {
 
 void mfma_instances_pruned(std::vector<Instance> &out)
 {
-    out.push_back(make_instance<9, 9, false, 12>());
-    out.push_back(make_instance<9, 9, false, 8>());
-    out.push_back(make_instance<9, 5, false, 8>());
-    out.push_back(make_instance<5, 9, false, 8>());
+    out.push_back(make_instance<9, 9, kTileAuto, 12>());
+    out.push_back(make_instance<9, 9, kTileAuto, 8>());
+    out.push_back(make_instance<9, 5, kTileAuto, 8>());
+    out.push_back(make_instance<5, 9, kTileAuto, 8>());
 }
 
 }  // namespace zk

@@ -6,10 +6,10 @@ namespace zk {
 
 void mfma_instances_rows32(std::vector<Instance> &out)
 {
-    out.push_back(make_instance<3, 3, true>());
-    out.push_back(make_instance<5, 5, true>());
-    out.push_back(make_instance<4, 4, true>());
-    out.push_back(make_instance<4, 5, true>());
+    out.push_back(make_instance<3, 3, kTileRows32>());
+    out.push_back(make_instance<5, 5, kTileRows32>());
+    out.push_back(make_instance<4, 4, kTileRows32>());
+    out.push_back(make_instance<4, 5, kTileRows32>());
 }
 
 }  // namespace zk

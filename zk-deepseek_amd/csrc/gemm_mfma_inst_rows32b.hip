@@ -7,10 +7,10 @@ namespace zk {
 
 void mfma_instances_rows32b(std::vector<Instance> &out)
 {
-    out.push_back(make_instance<3, 3, true, 16, 2, true>());
-    out.push_back(make_instance<4, 4, true, 16, 2, true>());
-    out.push_back(make_instance<4, 3, true>());
-    out.push_back(make_instance<5, 3, true>());
+    out.push_back(make_instance<3, 3, kTileRows32, 16, 2, kUseB32>());
+    out.push_back(make_instance<4, 4, kTileRows32, 16, 2, kUseB32>());
+    out.push_back(make_instance<4, 3, kTileRows32>());
+    out.push_back(make_instance<5, 3, kTileRows32>());
 }
 
 }  // namespace zk

@@ -6,9 +6,9 @@ namespace zk {
 
 void mfma_instances_rows32c(std::vector<Instance> &out)
 {
-    out.push_back(make_instance<3, 3, true, 16, 2, false, true>());
-    out.push_back(make_instance<4, 3, true, 16, 2, false, true>());
-    out.push_back(make_instance<5, 3, true, 16, 2, false, true>());
+    out.push_back(make_instance<3, 3, kTileRows32, 16, 2, kUseGroupPlanes>());
+    out.push_back(make_instance<4, 3, kTileRows32, 16, 2, kUseGroupPlanes>());
+    out.push_back(make_instance<5, 3, kTileRows32, 16, 2, kUseGroupPlanes>());
 }
 
 }  // namespace zk

@@ -6,8 +6,8 @@ namespace zk {
 
 void mfma_instances_rows32d(std::vector<Instance> &out)
 {
-    out.push_back(make_instance<4, 4, true, 16, 2, false, true>());
-    out.push_back(make_instance<5, 4, true, 16, 2, false, true>());
+    out.push_back(make_instance<4, 4, kTileRows32, 16, 2, kUseGroupPlanes>());
+    out.push_back(make_instance<5, 4, kTileRows32, 16, 2, kUseGroupPlanes>());
 }
 
 }  // namespace zk

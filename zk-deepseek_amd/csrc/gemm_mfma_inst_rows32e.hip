@@ -7,7 +7,7 @@ namespace zk {
 
 void mfma_instances_rows32e(std::vector<Instance> &out)
 {
-    out.push_back(make_instance<3, 4, true, 16, 2, true>());
+    out.push_back(make_instance<3, 4, kTileRows32, 16, 2, kUseB32>());
 }
 
 }  // namespace zk

@@ -9,16 +9,12 @@
 #include <type_traits>
 #include <vector>
 
-// Tuning knobs: MFMA depths (32 k each) per pipeline step by diagonal count, and how many vector-ALU
-// instructions of the digit split are scheduled behind each MFMA of a step's last depth.  (A 32x32x32 MFMA holds the
+// Tuning knob: how many vector-ALU instructions of the digit split are scheduled behind each MFMA of a step's last depth.  (A 32x32x32 MFMA holds the
 // matrix pipe for 32 cycles, a vector instruction its own for 4; with two wavefronts on a SIMD up to four or five
 // vector instructions per MFMA run in its shade, eight cost a quarter more time per MFMA: measured with a probe, and
 // on the 512 x 7168 x 18432 product 0.631-0.638 ms with 5 against 0.642-0.643 with 8.)
 #ifndef ZK_VALU_PER_MFMA
 #define ZK_VALU_PER_MFMA 5
-#endif
-#ifndef ZK_KK
-#define ZK_KK(DD) 1
 #endif
 
 namespace zk {
@@ -459,6 +455,9 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
         m0 = tm * BM;
     }
     const int n0 = tn * BN;
+    // A wavefront whose rows all lie past the last one (the last tile of a row count that is no multiple of the tile)
+    // loads and splits its share and leaves the matrix pipe to the others.
+    const bool rows_live = __builtin_amdgcn_readfirstlane(m0 + wm * (32 * WM) < m_lim ? 1 : 0) != 0;
 
     // Range tracking is shared out: the tiles_m workgroups that load the same B tile each check every
     // tiles_m-th k-step of it (likewise for A across the workgroups of a tile row), so no workgroup is slower
@@ -468,16 +467,6 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
     const bool verify_b = !BPL && tm < vmod_b && (g == 0 || p.verify_b_all_batches);
     DigitsSeen oa, ob;
     int rb32_lo = INT32_MAX, rb32_hi = INT32_MIN;        // the range of an int32 B is tracked in 32 bits and joins rb at the end
-
-    v16i acc[WM][WN][D];
-#pragma unroll
-    for (int a = 0; a < WM; a++)
-#pragma unroll
-        for (int b = 0; b < WN; b++)
-#pragma unroll
-            for (int d = 0; d < D; d++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[a][b][d][r] = 0;
 
     // Work items of the loaders: (row, j) pairs owning 8 elements each, or 16-byte chunks of digit planes.
     constexpr int A_ITEMS = BM * OCTS, B_ITEMS = BN * OCTS;
@@ -675,35 +664,6 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
             for (int j = 0; j < NB; j++)
                 fb[b][j] = *reinterpret_cast<const v4i *>(base + ((A_BLOCKS + (wn * WN + b) * NB + j) * 1024) + lane * 16);
     };
-    // the digit pairs (i, j) with i + j < D are numbered in row order; a slice issues those numbered LO..HI-1
-    constexpr int MFMAS = WM * WN * kept_pairs_before(NA, NB, D, NA, 0);
-    auto mfma_slice = [&](auto lo_tag, auto hi_tag, const v4i (&fa)[WM][NA], const v4i (&fb)[WN][NB]) {
-        constexpr int LO = decltype(lo_tag)::value, HI = decltype(hi_tag)::value;
-#pragma unroll
-        for (int i = 0; i < NA; i++)
-#pragma unroll
-            for (int j = 0; j < NB; j++)
-#pragma unroll
-                for (int a = 0; a < WM; a++)
-#pragma unroll
-                    for (int b = 0; b < WN; b++) {
-                        const int idx = (kept_pairs_before(NA, NB, D, i, j) * WM + a) * WN + b;
-                        if (idx >= LO && idx < HI && i + j < D)
-                            acc[a][b][i + j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[a][i], fb[b][j], acc[a][b][i + j], 0, 0, 0);
-                    }
-    };
-    typedef std::integral_constant<int, 0> I0;
-    typedef std::integral_constant<int, MFMAS / 2> IH;
-    typedef std::integral_constant<int, MFMAS> IF;
-    auto compute_all = [&](int buf) {
-#pragma unroll
-        for (int kk = 0; kk < KK; kk++) {
-            v4i fa[WM][NA], fb[WN][NB];
-            load_frags(buf, kk, fa, fb);
-            mfma_slice(I0(), IF(), fa, fb);
-        }
-    };
-
     const int ksteps = (p.K + BK - 1) / BK;
     const int full_steps = (a_vec || APL) && (b_vec || BKM) ? p.K / BK : 0;     // steps that can use unguarded loads
     // this workgroup's slice of the k-steps (everything unless it is one of the split workgroups of a tail tile)
@@ -744,6 +704,88 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
                     }
                 }
             ob.seen = true;
+        }
+    };
+
+    // every workgroup leaves the digits of what it saw in its own word; the waves meet in LDS (the stages are free by now)
+    auto leave = [&]() {
+        int need_a = 0, need_b = 0;
+        if (verify_a || verify_b) {
+            __syncthreads();
+            int *red = reinterpret_cast<int *>(smem);
+            need_a = wave_max_i32(oa.digits());
+            need_b = wave_max_i32(B32 && !BRS ? digits_i32(rb32_lo, rb32_hi) : ob.digits());
+            if (lane == 0) { red[2 * wave] = need_a; red[2 * wave + 1] = need_b; }
+            __syncthreads();
+            if (tid == 0) {
+                for (int w = 1; w < T / 64; w++) {
+                    need_a = red[2 * w] > need_a ? red[2 * w] : need_a;
+                    need_b = red[2 * w + 1] > need_b ? red[2 * w + 1] : need_b;
+                }
+            }
+        }
+        if (tid == 0) leave_digits(p.seen ? p.seen + block : nullptr, p.verdict, p.fail_class, NA, NB, need_a, need_b);
+    };
+
+    // prologue: stage 0 holds the first step, the staging registers hold the second
+    if (ks_begin < full_steps) fetch(ks_begin, std::true_type(), PAll()); else fetch(ks_begin, std::false_type(), PAll());
+    track(PAll());
+    stash(0, PAll());
+    if (ks_begin + 1 < ks_end) {
+        if (ks_begin + 1 < full_steps) fetch(ks_begin + 1, std::true_type(), PAll()); else fetch(ks_begin + 1, std::false_type(), PAll());
+    }
+    __syncthreads();
+    int ks = ks_begin;
+    const int fast_end = full_steps < ks_end ? full_steps : ks_end;
+    // (411 rows x [18432,7168] int32, (4,4): 846 -> 805 us.  The 128x128 tiles keep the one loop: with two, the registers of
+    // the hot one were dealt worse and 512 x 7168 x 18432 went from 622 to 634.)
+    if (WM == 1 && WVM > 1 && !rows_live) {
+        auto dead_step = [&](int step, auto fast_tag) {
+            stash(((step - ks_begin) & 1) ^ 1, PAll());
+            track(PAll());
+            if (step + 2 < ks_end) fetch(step + 2, fast_tag, PAll());
+            __syncthreads();
+        };
+        for (; ks + 2 < fast_end; ks++) dead_step(ks, std::true_type());
+        for (; ks + 1 < ks_end; ks++) dead_step(ks, std::false_type());
+        leave();
+        return;
+    }
+    v16i acc[WM][WN][D];
+#pragma unroll
+    for (int a = 0; a < WM; a++)
+#pragma unroll
+        for (int b = 0; b < WN; b++)
+#pragma unroll
+            for (int d = 0; d < D; d++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[a][b][d][r] = 0;
+    // the digit pairs (i, j) with i + j < D are numbered in row order; a slice issues those numbered LO..HI-1
+    constexpr int MFMAS = WM * WN * kept_pairs_before(NA, NB, D, NA, 0);
+    auto mfma_slice = [&](auto lo_tag, auto hi_tag, const v4i (&fa)[WM][NA], const v4i (&fb)[WN][NB]) {
+        constexpr int LO = decltype(lo_tag)::value, HI = decltype(hi_tag)::value;
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+#pragma unroll
+                for (int a = 0; a < WM; a++)
+#pragma unroll
+                    for (int b = 0; b < WN; b++) {
+                        const int idx = (kept_pairs_before(NA, NB, D, i, j) * WM + a) * WN + b;
+                        if (idx >= LO && idx < HI && i + j < D)
+                            acc[a][b][i + j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[a][i], fb[b][j], acc[a][b][i + j], 0, 0, 0);
+                    }
+    };
+    typedef std::integral_constant<int, 0> I0;
+    typedef std::integral_constant<int, MFMAS / 2> IH;
+    typedef std::integral_constant<int, MFMAS> IF;
+    auto compute_all = [&](int buf) {
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++) {
+            v4i fa[WM][NA], fb[WN][NB];
+            load_frags(buf, kk, fa, fb);
+            mfma_slice(I0(), IF(), fa, fb);
         }
     };
 
@@ -818,37 +860,11 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
         __syncthreads();
     };
 
-    // prologue: stage 0 holds the first step, the staging registers hold the second
-    if (ks_begin < full_steps) fetch(ks_begin, std::true_type(), PAll()); else fetch(ks_begin, std::false_type(), PAll());
-    track(PAll());
-    stash(0, PAll());
-    if (ks_begin + 1 < ks_end) {
-        if (ks_begin + 1 < full_steps) fetch(ks_begin + 1, std::true_type(), PAll()); else fetch(ks_begin + 1, std::false_type(), PAll());
-    }
-    __syncthreads();
-    int ks = ks_begin;
-    const int fast_end = full_steps < ks_end ? full_steps : ks_end;
     for (; ks + 2 < fast_end; ks++) step_body(ks, std::true_type());
     for (; ks + 1 < ks_end; ks++) step_body(ks, std::false_type());
     compute_all((ks_end - 1 - ks_begin) & 1);
 
-    // every workgroup leaves the digits of what it saw in its own word; the waves meet in LDS (the stages are free by now)
-    int need_a = 0, need_b = 0;
-    if (verify_a || verify_b) {
-        __syncthreads();
-        int *red = reinterpret_cast<int *>(smem);
-        need_a = wave_max_i32(oa.digits());
-        need_b = wave_max_i32(B32 && !BRS ? digits_i32(rb32_lo, rb32_hi) : ob.digits());
-        if (lane == 0) { red[2 * wave] = need_a; red[2 * wave + 1] = need_b; }
-        __syncthreads();
-        if (tid == 0) {
-            for (int w = 1; w < T / 64; w++) {
-                need_a = red[2 * w] > need_a ? red[2 * w] : need_a;
-                need_b = red[2 * w + 1] > need_b ? red[2 * w + 1] : need_b;
-            }
-        }
-    }
-    if (tid == 0) leave_digits(p.seen ? p.seen + block : nullptr, p.verdict, p.fail_class, NA, NB, need_a, need_b);
+    leave();
 
     // epilogue: diagonals -> 128-bit sum -> shift.  Accumulator register r of lane l holds
     // row 8*(r/4) + 4*(l/32) + r%4, column l%32 of its 32x32 tile.
@@ -1040,6 +1056,7 @@ struct Instance {
     int na, nb, bm, bn, threads, kk;
     bool skinny;                 // 32-row tiles for M <= 32
     int dmax;                    // diagonals from this one up are left out (16: none but the 2^128 one)
+    bool alt;                    // 128x64 tiles for digit counts that also have 128x128 ones: taken by launch size (see smaller_tiles)
     MfmaKernel fn[kVariants];
     PlanesKernel planes[2];      // [b32]: the owned-k pattern follows the element size of B
     FinishKernel finish;         // adds up the partial sums of split tail tiles
@@ -1047,36 +1064,53 @@ struct Instance {
 };
 
 
-// KKSEL: MFMA k-depths (of 32) per pipeline step.  B32ONLY: an instance for int32 B alone.  The 32-row kernels live on
-// the bytes they keep in flight, and a step of int32 weights is half the bytes of a step of int64 weights: with two
-// depths per step they stream as much per step as the int64 kernels do (where the two LDS stages still fit).
-// BPLONLY: an instance for grouped launches on prepared planes of B alone (deeper steps for them: more bytes in flight).
-template <int NA, int NB, bool SKINNY = false, int DMAX = 16, int KKSEL = ZK_KK(0), bool B32ONLY = false, bool BPLONLY = false>
+// Tile shapes by diagonals kept (= int32 accumulator sets): up to 5, eight waves as 2x4 with 64x32 outputs each (128x128);
+// up to 10, 4x2 with 32x32 each (128x64); beyond, four waves as 2x2 (64x64, one wave per SIMD because of the accumulators).
+// kRows32 (few rows): 1x8 waves (32x256).
+enum Tile { kTileAuto = 0, kTileRows32, kTile128x64 };
+// What an instance is for: everything, int32 B alone, grouped launches on prepared planes of B alone, or ungrouped launches
+// with planes on both sides alone.
+enum Use { kUseAll = 0, kUseB32, kUseGroupPlanes, kUsePlanesBoth };
+
+// KK: MFMA k-depths (of 32) per pipeline step.  Two of them halve the barriers and double the bytes under way.  The
+// 32-row kernels live on the latter: a step of int32 weights is half the bytes of a step of int64 weights, and with two
+// depths streams as much.  The 128x64 tiles have the registers for it (at most 256 with (5,5), no more than one spilled)
+// and gain on every shape: 243 rows x [7168,16384] int32, (3,4) digits, 413 -> 353 us; 411 x [18432,7168], (4,4),
+// 908 -> 846; 100 x [18432,7168] 269 -> 248; 131072 x [1024,512] int64, (3,4), 1343 -> 1184.  The 128x128 tiles do not
+// (they spill: 0.74 against 0.67 ms on 512 x 7168 x 18432).
+template <int NA, int NB, int TILE = kTileAuto, int DMAX = 16, int KK = 1, int USE = kUseAll>
 static Instance make_instance()
 {
     constexpr int DD = (NA + NB - 1) > DMAX ? DMAX : (NA + NB - 1);      // diagonals kept = accumulator sets
+    constexpr bool SKINNY = TILE == kTileRows32, B32ONLY = USE == kUseB32;
+    constexpr bool NARROW = !SKINNY && TILE != kTile128x64 && DD <= 5, MID = !SKINNY && !NARROW && DD <= 10;
     static_assert(!SKINNY || DD <= 10, "skinny tiles keep two waves per SIMD");
-    // narrow: 8 waves as 2x4, 64x32 per wave (128x128); mid: 8 waves as 4x2, 32x32 per wave (128x64);
-    // wide: 4 waves as 2x2, 32x32 per wave (64x64, one wave per SIMD because of the accumulator count)
-    // skinny (M <= 32): 8 waves as 1x8, 32x32 per wave (32x256)
-    constexpr int WVM = SKINNY ? 1 : (DD <= 5 ? 2 : (DD <= 10 ? 4 : 2));
-    constexpr int WVN = SKINNY ? 8 : (DD <= 5 ? 4 : 2);
-    constexpr int WM = SKINNY ? 1 : (DD <= 5 ? 2 : 1), WN = 1;
-    constexpr int KK = KKSEL;
+    constexpr int WVM = SKINNY ? 1 : (NARROW ? 2 : (MID ? 4 : 2));
+    constexpr int WVN = SKINNY ? 8 : (NARROW ? 4 : 2);
+    constexpr int WM = NARROW ? 2 : 1, WN = 1;
     static_assert(!B32ONLY || NB <= 5, "int32 values never need more than five digits");
     Instance s;
     s.na = NA; s.nb = NB; s.bm = 32 * WM * WVM; s.bn = 32 * WN * WVN; s.threads = 64 * WVM * WVN; s.kk = KK;
     s.skinny = SKINNY;
     s.dmax = DMAX;
+    s.alt = TILE == kTile128x64;
     for (int v = 0; v < kVariants; v++) s.fn[v] = nullptr;
     s.guarded[0] = s.guarded[1] = nullptr;
     // every operand fits nine digits, every int32 five: these instances can stand behind any speculative launch
-    if constexpr (NA == 9 && !SKINNY && DMAX == 16 && !B32ONLY && !BPLONLY) {
+    if constexpr (NA == 9 && !SKINNY && DMAX == 16 && USE == kUseAll) {
         if constexpr (NB == 9) s.guarded[0] = gemm_mfma_guarded_kernel<NA, NB, WVM, WVN, WM, WN, KK, false, DMAX>;
         if constexpr (NB == 5) s.guarded[1] = gemm_mfma_guarded_kernel<NA, NB, WVM, WVN, WM, WN, KK, true, DMAX>;
     }
-    if constexpr (BPLONLY) {
-        static_assert(SKINNY && !B32ONLY, "grouped launches run on the 32-row tiles");
+    if constexpr (USE == kUsePlanesBoth) {
+        static_assert(!SKINNY && KK == 1, "prepared planes of one matrix are in the order of one depth per step");
+        s.fn[kB64PlanesBoth] = gemm_mfma_kernel<NA, NB, WVM, WVN, WM, WN, KK, false, false, true, false, false, DMAX, true>;
+        s.finish = gemm_split_finish_kernel<WVM, WVN, WM, WN>;
+        s.planes[0] = a_planes_kernel<NA, 2, KK>;
+        s.planes[1] = a_planes_kernel<NA, 4, KK>;
+        return s;
+    }
+    if constexpr (USE == kUseGroupPlanes) {
+        static_assert(SKINNY, "grouped launches run on the 32-row tiles");
         s.fn[kB64GroupBPlanes] = gemm_mfma_kernel<NA, NB, WVM, WVN, WM, WN, KK, false, false, false, true, false, DMAX, true>;
         s.finish = gemm_split_finish_kernel<WVM, WVN, WM, WN>;
         s.planes[0] = a_planes_kernel<NA, 2, KK>;
@@ -1116,6 +1150,7 @@ static Instance make_instance()
 void mfma_instances_narrow(std::vector<Instance> &out);
 void mfma_instances_mid(std::vector<Instance> &out);
 void mfma_instances_wide(std::vector<Instance> &out);
+void mfma_instances_both(std::vector<Instance> &out);
 void mfma_instances_pruned(std::vector<Instance> &out);
 void mfma_instances_rows32(std::vector<Instance> &out);
 void mfma_instances_rows32b(std::vector<Instance> &out);
