@@ -34,21 +34,32 @@ struct GuardArgs {
     unsigned *next;                  // device word cleared for the next speculative launch (the calls take turns with two)
     const unsigned *seen;            // per-workgroup digit counts of the speculative launch: byte 0 A, byte 1 B
     long seen_count;
-    unsigned long long *host;        // receives seq << 32 | verdict << 16 | digits of B << 8 | digits of A in one store (may be null)
+    unsigned long long *host;        // [parts] words; each receives seq << 32 | verdict << 16 | digits of B << 8 | digits of A in one store (may be null)
     unsigned seq;
+    int parts;                       // the first `parts` workgroups share the words of `seen`, see guard_parts
 };
 
-// by one whole workgroup of at most 1024 threads
-__device__ __forceinline__ void guard_report(const GuardArgs &g)
+// One workgroup for every 1024 words of `seen` (a load or four per thread), at most 32: a product of 131072 rows leaves
+// 50000 words, for which one workgroup took 44 us.
+constexpr int kGuardParts = 32;
+inline int guard_parts(long seen_count, long grid)
+{
+    const long n = (seen_count + 1023) / 1024, most = grid < kGuardParts ? grid : kGuardParts;
+    return (int)(n < 1 ? 1 : (n > most ? most : n));
+}
+
+// by whole workgroups of at most 1024 threads, number `part` of g.parts
+__device__ __forceinline__ void guard_report(const GuardArgs &g, int part)
 {
     __shared__ int report_red[16];
     unsigned a = 0, b = 0;
     // (four loads under way per thread: the launch waits for this workgroup)
-    for (long i0 = threadIdx.x; i0 < g.seen_count; i0 += 4L * blockDim.x) {
+    const long stride = (long)g.parts * blockDim.x;
+    for (long i0 = (long)part * blockDim.x + threadIdx.x; i0 < g.seen_count; i0 += 4 * stride) {
         unsigned w[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const long i = i0 + (long)j * blockDim.x;
+            const long i = i0 + j * stride;
             w[j] = i < g.seen_count ? g.seen[i] : 0;
         }
 #pragma unroll
@@ -75,12 +86,13 @@ __device__ __forceinline__ void guard_report(const GuardArgs &g)
         b = (o & 0xFFFFu) > b ? (o & 0xFFFFu) : b;
     }
     const unsigned v = __atomic_load_n(g.verdict, __ATOMIC_RELAXED);
-    if (g.host) __hip_atomic_store(g.host, (unsigned long long)g.seq << 32 | v << 16 | b << 8 | a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    if (g.next) __atomic_store_n(g.next, 0u, __ATOMIC_RELAXED);
+    if (g.host) __hip_atomic_store(g.host + part, (unsigned long long)g.seq << 32 | v << 16 | b << 8 | a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (g.next && part == 0) __atomic_store_n(g.next, 0u, __ATOMIC_RELAXED);
 }
 
 // Native 64-bit multiply-add chains on the vector ALU; handles every descriptor.
-void gemm_valu_launch(const GemmDesc &d, const GuardArgs &guard = GuardArgs());
+// (A guarded launcher settles guard->parts by its grid.)
+void gemm_valu_launch(const GemmDesc &d, GuardArgs *guard = nullptr);
 
 // Matrix-vector kernel of the same family for one or two rows of A against k-contiguous B: one launch, nothing
 // guessed.  Returns false (nothing launched) for any other descriptor.
@@ -139,7 +151,7 @@ bool gemm_gemv_grouped_launch(const GroupedDesc &d);
 
 // The grouped product on the 16-row MFMA tiles (see gemm_rows16_launch): one launch, no wait.  0 / 1 / -1 as there.
 // `guard`: see GuardArgs (the fallback behind a speculative launch of the 32-row kernels).
-int gemm_rows16_grouped(const GroupedDesc &d, const GuardArgs &guard = GuardArgs());
+int gemm_rows16_grouped(const GroupedDesc &d, GuardArgs *guard = nullptr);
 
 // One launch of the 32-row-tile MFMA kernels over all groups.  Returns 0 when done, 1 when the operands need
 // more digits than those kernels are built for (nothing valid was written: the caller takes another route),

@@ -20,7 +20,7 @@
 // The digit counts are speculated from a cached or sampled range.  The kernels track the digits that everything they
 // load needs.  A workgroup that meets an element its digit counts do not hold raises the verdict, a word on the device
 // that nobody writes otherwise; a guarded launch follows on the stream, which recomputes everything if the verdict is
-// raised and returns at once otherwise.  Its first workgroup also folds what every workgroup saw into one 8-byte store
+// raised and returns at once otherwise.  Its first workgroups also fold what every workgroup saw into 8-byte stores
 // to pinned host memory, marked with the call's number: that refreshes the cache at a later call.  (A fold kernel
 // between the two and an event behind them cost 10 us per call: 5 for the kernel, 5.5 of idle device at the event.)
 // Results never depend on the guess, and a call whose operands were seen before never blocks the host.
@@ -113,7 +113,8 @@ typedef std::tuple<const void *, long, long, int> OperandKey;     // (pointer, r
 struct PendingRange {
     OperandKey key_a, key_b;
     int nb_fixed = 0;                        // B came from prepared planes with this many digits (nothing of it was tracked)
-    unsigned seq = 0;                        // the call's number: its report has arrived when the slot's pinned word carries it
+    unsigned seq = 0;                        // the call's number: its report has arrived when all its pinned words carry it
+    int parts = 1;
 };
 
 constexpr unsigned kPendingSlots = 256;      // (a host this many calls ahead of the device skips the report, not the check)
@@ -135,7 +136,7 @@ struct RangeCache {
     size_t b_rows_count = 0;
     int cus = 0;                             // compute units of the device
     PendingRange pending[kPendingSlots];
-    volatile unsigned long long *pinned = nullptr;      // one word per slot
+    volatile unsigned long long *pinned = nullptr;      // kGuardParts words per slot
     unsigned pending_head = 0, pending_tail = 0;        // slots used and drained so far, in ring order; head - tail are on their way
     unsigned seq = 0;
     long guard_hits = 0;                     // calls whose speculation failed after they had returned
@@ -233,13 +234,19 @@ static void drain_pending()
 {
     while (g_cache.pending_tail != g_cache.pending_head) {
         const PendingRange &s = g_cache.pending[g_cache.pending_tail % kPendingSlots];
-        const unsigned long long w = g_cache.pinned[g_cache.pending_tail % kPendingSlots];
-        if ((unsigned)(w >> 32) != s.seq) return;
-        const int na = (int)(w & 0xFF), nb = (int)(w >> 8 & 0xFF);
+        const volatile unsigned long long *words = g_cache.pinned + (size_t)(g_cache.pending_tail % kPendingSlots) * kGuardParts;
+        int na = 0, nb = 0, verdict = 0;
+        for (int i = 0; i < s.parts; i++) {
+            const unsigned long long w = words[i];
+            if ((unsigned)(w >> 32) != s.seq) return;
+            na = (int)(w & 0xFF) > na ? (int)(w & 0xFF) : na;
+            nb = (int)(w >> 8 & 0xFF) > nb ? (int)(w >> 8 & 0xFF) : nb;
+            verdict |= (int)(w >> 16 & 0xFF);
+        }
         if (nb) g_cache.store_pair(s.key_a, na ? na : 1, s.key_b, nb);
         else if (s.nb_fixed) g_cache.store_pair(s.key_a, na ? na : 1, s.key_b, s.nb_fixed);      // (a grouped launch on prepared planes)
         else g_cache.store(s.key_a, na ? na : 1);        // B came from prepared planes: nothing of it was tracked
-        if (w >> 16 & 0xFF) g_cache.guard_hits++;
+        if (verdict) g_cache.guard_hits++;
         g_cache.pending_tail++;
     }
 }
@@ -255,7 +262,7 @@ static GuardArgs make_guard(long seen_count)
     g.seen = g_cache.seen;
     g.seen_count = seen_count;
     if (g_cache.pending_head - g_cache.pending_tail < kPendingSlots) {
-        g.host = const_cast<unsigned long long *>(g_cache.pinned) + g_cache.pending_head % kPendingSlots;
+        g.host = const_cast<unsigned long long *>(g_cache.pinned) + (size_t)(g_cache.pending_head % kPendingSlots) * kGuardParts;
         if (++g_cache.seq == 0) g_cache.seq = 1;
         g.seq = g_cache.seq;
     }
@@ -271,6 +278,7 @@ static void guard_taken(const GuardArgs &g, const OperandKey &key_a, const Opera
     s.key_b = key_b;
     s.nb_fixed = nb_fixed;
     s.seq = g.seq;
+    s.parts = g.parts;
     g_cache.pending_head++;
 }
 
@@ -281,6 +289,7 @@ static bool wait_digits(long seen_count, int *need_a, int *need_b)
     unsigned *word = reinterpret_cast<unsigned *>(g_cache.dev + 5) + g_cache.turn;
     g.verdict = word; g.next = word; g.seen = g_cache.seen; g.seen_count = seen_count;
     g.host = g_cache.dev + 4;
+    g.parts = 1;
     digits_report_kernel<<<1, 256, 0, 0>>>(g);
     unsigned long long w;
     if (hipMemcpy(&w, g_cache.dev + 4, sizeof(w), hipMemcpyDeviceToHost) != hipSuccess) return false;
@@ -319,9 +328,9 @@ static bool init_cache()
     g_cache.cus = n;
     // without the pinned words every call simply waits for its own verdict
     void *pinned = nullptr;
-    if (hipHostMalloc(&pinned, kPendingSlots * sizeof(unsigned long long), hipHostMallocDefault) == hipSuccess) {
+    if (hipHostMalloc(&pinned, kPendingSlots * kGuardParts * sizeof(unsigned long long), hipHostMallocDefault) == hipSuccess) {
         g_cache.pinned = reinterpret_cast<volatile unsigned long long *>(pinned);
-        for (unsigned i = 0; i < kPendingSlots; i++) g_cache.pinned[i] = 0;
+        for (unsigned i = 0; i < kPendingSlots * kGuardParts; i++) g_cache.pinned[i] = 0;
     } else {
         (void)hipGetLastError();
         g_cache.pinned = nullptr;
@@ -546,7 +555,7 @@ constexpr long kBRowsMaxElements = 8L << 20;         // 64 MB
 // digits hold every int64, five every int32; config 4 with stale three-digit guesses: 4 ms where the vector-ALU tiles
 // take 35), one workgroup per compute unit walking the tiles.  Everything else, and a K beyond what its int32
 // accumulators take in one piece: the vector-ALU tiles.
-static Outcome launch_guarded_fallback(const GemmDesc &d, const MfmaParams &spec, int b_shift, const GuardArgs &guard)
+static Outcome launch_guarded_fallback(const GemmDesc &d, const MfmaParams &spec, int b_shift, GuardArgs *guard)
 {
     // (an n-contiguous B that the speculative launch read through its row-major copy is read through that copy here too)
     const bool b_copied = spec.B == (const void *)g_cache.b_rows && g_cache.b_rows != nullptr;
@@ -570,7 +579,6 @@ static Outcome launch_guarded_fallback(const GemmDesc &d, const MfmaParams &spec
         if (total > 0x7FFFFFFFL / 8) fn = nullptr;
         else {
             q.main_tiles = (int)total; q.split = 1; q.tail_xcd = 0; q.partials = nullptr; q.part64 = 0; q.n_fastest = 0;
-            q.guard = guard;
             q.seen = nullptr;                  // (its digit counts hold whatever raised the verdict)
             q.walk_blocks = (int)total;
         }
@@ -589,6 +597,8 @@ static Outcome launch_guarded_fallback(const GemmDesc &d, const MfmaParams &spec
         lds_raised.insert((const void *)fn);
     }
     const long grid = q.walk_blocks < g_cache.cus ? q.walk_blocks : g_cache.cus;
+    guard->parts = guard_parts(guard->seen_count, grid);
+    q.guard = *guard;
     fn<<<dim3((unsigned)grid), dim3((unsigned)wide->threads), lds, 0>>>(q);
     if (hipGetLastError() != hipSuccess) { set_error(kLaunchFailure, "gemm: guarded MFMA launch failed"); return kFailed; }
     return kDone;
@@ -839,8 +849,8 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         *limbs_b = inst->nb;
         if (speculate) {
             // no waiting: a guarded launch redoes the product if the verdict is raised, the digits seen follow later
-            const GuardArgs guard = make_guard(blocks + plane_wgs);
-            if (const Outcome got = launch_guarded_fallback(d, p, b_shift, guard)) return got;
+            GuardArgs guard = make_guard(blocks + plane_wgs);
+            if (const Outcome got = launch_guarded_fallback(d, p, b_shift, &guard)) return got;
             guard_taken(guard, key_a, key_b, prep ? prep->nb : 0);       // (the slots are shared with the grouped launches, which set it too)
             return kDone;
         }
@@ -958,8 +968,8 @@ int gemm_mfma_grouped(const GroupedDesc &d, int *limbs_a, int *limbs_b)
             }
         }
         if (speculate) {
-            const GuardArgs guard = make_guard(blocks);
-            const int rc = gemm_rows16_grouped(d, guard);
+            GuardArgs guard = make_guard(blocks);
+            const int rc = gemm_rows16_grouped(d, &guard);
             if (rc < 0) return -1;
             if (rc == 0) {
                 *limbs_a = inst->na;

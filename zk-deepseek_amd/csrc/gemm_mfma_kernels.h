@@ -359,7 +359,7 @@ __global__ __launch_bounds__(256) void a_planes_kernel(MfmaParams p, unsigned ch
 }
 
 // The report of a launch that has no guarded launch behind it (its caller waits for the digits instead).
-static __global__ __launch_bounds__(256) void digits_report_kernel(GuardArgs g) { guard_report(g); }
+static __global__ __launch_bounds__(256) void digits_report_kernel(GuardArgs g) { guard_report(g, 0); }
 
 // Number of digit pairs (i', j') with i' + j' < d that come before (i, j) in row order (i' < i, or i' == i and j' < j).
 __host__ __device__ constexpr int kept_pairs_before(int na, int nb, int d, int i, int j)
@@ -946,7 +946,7 @@ template <int NA, int NB, int WVM, int WVN, int WM, int WN, int KK, bool B32, in
 __global__ __launch_bounds__(64 * WVM * WVN) void gemm_mfma_guarded_kernel(MfmaParams p)
 {
     const unsigned verdict = __atomic_load_n(p.guard.verdict, __ATOMIC_RELAXED);            // (the same for every thread of the launch)
-    if (blockIdx.x == 0) guard_report(p.guard);
+    if ((int)blockIdx.x < p.guard.parts) guard_report(p.guard, (int)blockIdx.x);
     if (verdict == 0) return;
     if (verdict == 1 && (NA > 5 || NB > 5)) {
         // five digits cover both operands (the fold kernel has seen every element): a third of the digit pairs of (9,9)

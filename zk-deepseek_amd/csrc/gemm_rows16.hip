@@ -434,7 +434,7 @@ __global__ __launch_bounds__(64 * kR16Waves) void gemm_rows16_kernel(Rows16Param
 {
     if (p.guard.verdict) {
         const unsigned verdict = __atomic_load_n(p.guard.verdict, __ATOMIC_RELAXED);       // (the same for every thread of the launch)
-        if (blockIdx.x == 0) guard_report(p.guard);
+        if ((int)blockIdx.x < p.guard.parts) guard_report(p.guard, (int)blockIdx.x);
         if (verdict == 0) return;
     }
     for (unsigned item = blockIdx.x; item < p.items; item += gridDim.x) {
@@ -658,7 +658,7 @@ int gemm_rows16_launch(const GemmDesc &d, unsigned long long *acc, size_t max_sl
     return 0;
 }
 
-int gemm_rows16_grouped(const GroupedDesc &d, const GuardArgs &guard)
+int gemm_rows16_grouped(const GroupedDesc &d, GuardArgs *guard)
 {
     if (d.K < 0 || d.N < 1 || d.rows < 1 || d.groups < 1) return 1;
     std::lock_guard<std::mutex> lock(g_r16_mu);
@@ -671,10 +671,13 @@ int gemm_rows16_grouped(const GroupedDesc &d, const GuardArgs &guard)
     p.col_groups = (d.N + cols - 1) / cols;
     p.nslices = 1;
     p.grp_seg = d.seg; p.grp_tiles = d.tiles; p.grp_ntiles = d.ntiles; p.grp_b = d.B;
-    p.guard = guard;
     // the grid covers the worst case of the tile table (the host never learns the segment sizes): rows / 32 + groups
     // tiles of 32 rows, two halves each
     const long blocks = ((long)d.rows / 32 + d.groups) * 2 * ((p.col_groups + kR16Waves - 1) / kR16Waves);
+    if (guard) {
+        guard->parts = guard_parts(guard->seen_count, blocks < r16_cus() ? blocks : r16_cus());
+        p.guard = *guard;
+    }
     return r16_run(d.b32 ? gemm_rows16_kernel<true, true> : gemm_rows16_kernel<false, true>, p, blocks);
 }
 

@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256) void gemm_valu_kernel(ValuParams p)
     const int tid = threadIdx.x;
     if (p.guard.verdict) {
         const unsigned verdict = __atomic_load_n(p.guard.verdict, __ATOMIC_RELAXED);
-        if (blockIdx.x == 0) guard_report(p.guard);
+        if ((int)blockIdx.x < p.guard.parts) guard_report(p.guard, (int)blockIdx.x);
         if (verdict == 0) return;
     }
     for (long tile = blockIdx.x; tile < p.tiles; tile += gridDim.x) {
@@ -151,7 +151,7 @@ static void launch2(const ValuParams &p, dim3 grid, bool rescale)
     else gemm_valu_kernel<B32, KMAJOR, false><<<grid, dim3(256), 0, 0>>>(p);
 }
 
-void gemm_valu_launch(const GemmDesc &d, const GuardArgs &guard)
+void gemm_valu_launch(const GemmDesc &d, GuardArgs *guard)
 {
     ValuParams p;
     p.A = d.A; p.B = d.B; p.C = d.C; p.R = d.R;
@@ -169,12 +169,13 @@ void gemm_valu_launch(const GemmDesc &d, const GuardArgs &guard)
     p.tiles_m = (d.M + kVT - 1) / kVT;
     p.tiles_n = (d.N + kVT - 1) / kVT;
     p.tiles = (long)p.tiles_m * p.tiles_n * d.G;
-    p.guard = guard;
     const bool rescale = d.a_rs != 1 || d.b_rs != 1;
     const bool kmajor = d.ldbn == 1 && d.ldbk != 1;
     // a guarded launch normally finds nothing to do, so it is kept small; either way workgroups stride over the tiles
-    const long cap = guard.verdict ? 2048 : (1L << 22);
+    const long cap = guard ? 2048 : (1L << 22);
     dim3 grid((unsigned)(p.tiles < cap ? p.tiles : cap));
+    if (guard) guard->parts = guard_parts(guard->seen_count, grid.x);
+    p.guard = guard ? *guard : GuardArgs();
     if (d.b32) { if (kmajor) launch2<true, true>(p, grid, rescale); else launch2<true, false>(p, grid, rescale); }
     else { if (kmajor) launch2<false, true>(p, grid, rescale); else launch2<false, false>(p, grid, rescale); }
 }
