@@ -103,7 +103,7 @@ const char *zk_last_error_string(void);
 void zk_clear_error(void);
 
 /* The reference's library allocates nothing and keeps no state; this one keeps scratch buffers on the device between
- * calls (digit planes of A, partial sums of split tiles, range slots, a row-major copy of a small B, the quotient
+ * calls (digit planes of A and of a small B, partial sums of split tiles, digit counts, the quotient
  * tables of the activations), allocated on demand and grown inside a call when a larger problem arrives.
  * zk_workspace_bytes: device bytes held as scratch right now.  zk_prepared_weights_bytes: device bytes held as digit
  * planes made by zk_gemm_prepare_weights.  zk_release_workspace: waits for the device and frees the scratch (not the
@@ -245,8 +245,8 @@ long zk_gemm_grouped_mfma_calls(void);
 /* How many of those launches ran on the kernel that streams int32 weights through LDS rings (K a multiple of 32,
  * sixteen digit pairs or more; ZK_STREAM32_MIN_PAIRS and ZK_NO_STREAM32 move or remove that choice). */
 long zk_gemm_grouped_streamed_calls(void);
-/* How many GEMM launches so far ran on the software-pipelined 128 x 128 kernel that reads digit planes on both sides
- * (weights prepared with zk_gemm_prepare_weights, three digits a side; ZK_NO_PIPE=1 switches it off). */
+/* How many GEMM launches so far ran on the software-pipelined kernel that reads digit planes on both sides (weights
+ * prepared with zk_gemm_prepare_weights, and a B that is small next to the product; ZK_NO_PIPE=1 switches it off). */
 long zk_gemm_pipe_calls(void);
 /* No reference counterpart: model weights do not change between calls, so a weight matrix W[N,K] (int64, or int32 with
  * b32 != 0; groups == 0, B = the device pointer later passed as B) or all the matrices of a device table of pointers

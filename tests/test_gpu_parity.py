@@ -686,6 +686,48 @@ def test_einsum_values_rewritten_with_contiguous_rows(K, oracle, monkeypatch):
         K.lib.zk_reload_env()
 
 
+@pytest.mark.parametrize("bits_a,bits_b,digits", [(19, 22, (3, 3)), (19, 27, (3, 4)), (27, 19, (4, 3)), (27, 27, (4, 4)), (36, 27, (5, 4)),
+                                                  (27, 35, (4, 5)), (36, 36, (5, 5)), (19, 35, (3, 5)), (43, 19, (6, 3))])
+def test_einsums_with_planes_of_both_operands(K, oracle, monkeypatch, bits_a, bits_b, digits):
+    """a B that is small next to the product is split like A and the pipelined kernel walks several tiles per workgroup:
+    values (n-contiguous) with rows of A that end in zeros at every length, hold nothing at all or are full; scores
+    (k-contiguous) of one step and of many; per-head int32 weights; ragged rows and columns, two batches, row tiles that
+    do not come in eights"""
+    monkeypatch.setenv("ZK_B_ROWS_MIN_MACS", "1")
+    K.lib.zk_reload_env()
+    oracle.set_threads(oracle.max_threads())
+    rng = np.random.default_rng(bits_a * 64 + bits_b)
+    K.lib.zk_gemm_set_path(2)
+
+    def check(name, a, b, shift, pipe=True):
+        da, db = dev(a), dev(b)
+        for _ in range(2):          # (a first call may run on digits remembered for other operands at these addresses)
+            before = K.lib.zk_gemm_pipe_calls()
+            out = getattr(K, name)(da, db, shift)
+            assert np.array_equal(host(out), getattr(oracle, name)(a, b, shift)), (name, a.shape, b.shape)
+        assert K.lib.zk_gemm_pipe_calls() == before + pipe and K.gemm_last_plan()[1:] == digits
+    try:
+        p = rand_i64(rng, (2, 17, 128, 257), bits_a)
+        for s in range(17):
+            p[:, s, :, 15 * s + (s % 3):] = 0       # (the first position's rows hold nothing)
+        p[1, 3, 127, 256], p[0, 16] = (1 << bits_a) - 1, (1 << bits_a) - 2
+        v = rand_i64(rng, (2, 257, 1000), bits_b)
+        v[1, 256, 999] = (1 << bits_b) - 1
+        check("einsum_bsht_btc_bshc", p, v, 23)
+        q, kv = rand_i64(rng, (1, 129, 128, 40), bits_a), rand_i64(rng, (1, 250, 40), bits_b)
+        q[0, 128, 127, 39], kv[0, 249, 39] = -(1 << bits_a), (1 << bits_b) - 1
+        check("einsum_bshc_btc_bsht", q, kv, 21)
+        if digits[1] <= 4:
+            qh, w = rand_i64(rng, (1, 390, 16, 70), bits_a), rand_i32(rng, (16, 70, 520), bits_b)
+            qh[0, 389, 15, 69], w[15, 69, 519] = (1 << bits_a) - 1, (1 << bits_b) - 1
+            check("einsum_bshd_hdc_bshc", qh, w, 30)
+    finally:
+        oracle.set_threads(1)
+        K.lib.zk_gemm_set_path(0)
+        monkeypatch.delenv("ZK_B_ROWS_MIN_MACS")
+        K.lib.zk_reload_env()
+
+
 def _scores(rng, shape, Q, masked=True):
     x = rng.integers(-(12 << Q), 12 << Q, size=shape, dtype=np.int64)
     if masked and shape[-1] > 1:

@@ -25,6 +25,7 @@
 // between the two and an event behind them cost 10 us per call: 5 for the kernel, 5.5 of idle device at the event.)
 // Results never depend on the guess, and a call whose operands were seen before never blocks the host.
 #include "gemm_mfma_kernels.h"
+#include "gemm_mfma_pipe.h"
 
 #include <map>
 #include <mutex>
@@ -32,10 +33,6 @@
 #include <tuple>
 
 namespace zk {
-
-// the 128 x 128 kernel for digit planes on both sides (gemm_mfma_pipe.h), by digit counts (or null), and its dynamic LDS
-MfmaKernel pipe_kernel(int na, int nb);
-size_t pipe_lds_size(int na, int nb);
 
 // the streamed form of the grouped launch for int32 weights (gemm_stream32.h), by digit counts; null: none
 MfmaKernel stream32_grouped_kernel(int na, int nb, size_t *lds);
@@ -132,8 +129,10 @@ struct RangeCache {
     size_t seen_count = 0;
     unsigned long long *partials = nullptr;  // partial sums of split tiles
     size_t partials_bytes = 0;
-    int64_t *b_rows = nullptr;               // a small n-contiguous B rewritten with contiguous rows
-    size_t b_rows_count = 0;
+    unsigned char *b_planes = nullptr;       // digit planes of a small B
+    size_t b_planes_bytes = 0;
+    int *row_steps = nullptr;                // per row tile of A: its steps up to the last one that is not all zeros
+    size_t row_steps_count = 0;
     int cus = 0;                             // compute units of the device
     PendingRange pending[kPendingSlots];
     volatile unsigned long long *pinned = nullptr;      // kGuardParts words per slot
@@ -174,10 +173,10 @@ static RangeCache g_cache;
 // ZK_GEMM_SYNC: every call waits for its own digit verdict; ZK_NO_TAIL_SPLIT: no split-K; ZK_VALU_FALLBACK: the guarded launch
 // behind a speculative one is always the vector-ALU kernel; ZK_NO_STREAM32: grouped launches on int32 weights keep the general
 // 32-row kernel; ZK_B_ROWS_MIN_MACS: product
-// size from which a small n-contiguous int64 B is rewritten with contiguous rows first; ZK_SKINNY_MAX_M: rows up to
+// size from which a B that is small next to it is split into digit planes first; ZK_SKINNY_MAX_M: rows up to
 // which the 32-row tiles are used.
 struct Switches { bool sync_verdict, no_tail_split, valu_fallback, no_stream32, no_pipe; double b_rows_min_macs; int skinny_max_m, planes_min_tiles_n, stream32_min_pairs; };
-constexpr long kBRowsMinMacs = 1L << 32;
+constexpr long kBRowsMinMacs = 1L << 30;
 constexpr double kShapeGuessMaxMacs = 17179869184.0;        // 2^34: about 0.15 ms on the matrix pipe
 // Rows up to which a product runs on the 32-row tiles (two of them from 33 rows on): measured against the 128-row tiles,
 // 48 rows x [1536,7168] int32 34.1 against 38.1 us, 64 x [2048,7168] int64 37.6-39.4 against 41.2, 128 rows 56.8 against 45.1.
@@ -283,11 +282,11 @@ static void guard_taken(const GuardArgs &g, const OperandKey &key_a, const Opera
 }
 
 // Waits for the digits the launch just issued has seen, and clears its verdict word (its caller launches again).
-static bool wait_digits(long seen_count, int *need_a, int *need_b)
+static bool wait_digits(long first, long seen_count, int *need_a, int *need_b)
 {
     GuardArgs g = {};
     unsigned *word = reinterpret_cast<unsigned *>(g_cache.dev + 5) + g_cache.turn;
-    g.verdict = word; g.next = word; g.seen = g_cache.seen; g.seen_count = seen_count;
+    g.verdict = word; g.next = word; g.seen = g_cache.seen + first; g.seen_count = seen_count;
     g.host = g_cache.dev + 4;
     g.parts = 1;
     digits_report_kernel<<<1, 256, 0, 0>>>(g);
@@ -496,7 +495,7 @@ size_t gemm_mfma_workspace_bytes(size_t *prepared_bytes)
     std::lock_guard<std::mutex> lock(g_cache.mu);
     size_t scratch = g_cache.dev ? 8 * sizeof(unsigned long long) : 0;
     scratch += g_cache.planes_bytes + g_cache.seen_count * sizeof(unsigned) + g_cache.partials_bytes * sizeof(unsigned long long) +
-               g_cache.b_rows_count * sizeof(int64_t);
+               g_cache.b_planes_bytes + g_cache.row_steps_count * sizeof(int);
     size_t prepared = 0;
     for (const auto &kv : g_prepared) {
         const PreparedB &pb = kv.second;
@@ -517,62 +516,52 @@ void gemm_mfma_release_workspace()
     if (g_cache.planes) (void)hipFree(g_cache.planes);
     if (g_cache.seen) (void)hipFree(g_cache.seen);
     if (g_cache.partials) (void)hipFree(g_cache.partials);
-    if (g_cache.b_rows) (void)hipFree(g_cache.b_rows);
+    if (g_cache.b_planes) (void)hipFree(g_cache.b_planes);
+    if (g_cache.row_steps) (void)hipFree(g_cache.row_steps);
     g_cache.planes = nullptr; g_cache.planes_bytes = 0;
     g_cache.seen = nullptr; g_cache.seen_count = 0;
     g_cache.partials = nullptr; g_cache.partials_bytes = 0;
-    g_cache.b_rows = nullptr; g_cache.b_rows_count = 0;
+    g_cache.b_planes = nullptr; g_cache.b_planes_bytes = 0;
+    g_cache.row_steps = nullptr; g_cache.row_steps_count = 0;
 }
 
-// B[g][k][n] (n contiguous) -> out[g][n][k]: 32x32 tiles through LDS, both sides coalesced
-__global__ __launch_bounds__(256) void b_rows_kernel(const int64_t *__restrict__ B, long ldbk, long sB, int64_t *__restrict__ out, int N, int K)
+// A B that is small next to the product (a KV cache against the queries of a whole prompt, one head's weights) is split
+// into digit planes like A, and the product runs on the pipelined kernel for planes on both sides (gemm_mfma_pipe.h).
+// One more launch in front and the general kernel's time, against its own split of B in every tile.  Whole calls, (3,4)
+// digits, general against this: k-contiguous int64 B, 131072 rows x [1024,512] 1124 / 864 us, x [1024,64] 379 / 268, 31104 x
+// [243,512] 95.8 / 84.0, 8192 x [512,512] (3,3) 35.2 / 36.7, (4,4) 49.8 / 49.0; the heads' int32 weights (128 heads, 1024
+// rows each) 248 / 310.  n-contiguous B, which the general kernel reads element by element: 512 values of 1024 tokens 1250 /
+// 630 (860 without the causal zeros), of 243 tokens 109 / 68, of 100 tokens 37.7 / 32.5, the heads' int32 weights at 400
+// rows 134 / 132, at 500 169 / 149.
+constexpr long kPipeBMaxElements = 8L << 20;         // 40 MB of planes at most
+constexpr int kPipeMinRows = 16384, kPipeMinRowsKmajor = 385;
+static bool pipe_b_planes(const GemmDesc &d, bool kmajor, long b_batches)
 {
-    __shared__ int64_t tile[32][33];
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    const int n0 = blockIdx.x * 32, k0 = blockIdx.y * 32;
-    const int64_t *src = B + (long)blockIdx.z * sB;
-    int64_t *dst = out + (long)blockIdx.z * N * K;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int k = k0 + ty + 8 * i, n = n0 + tx;
-        tile[ty + 8 * i][tx] = (k < K && n < N) ? src[(long)k * ldbk + n] : 0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int n = n0 + ty + 8 * i, k = k0 + tx;
-        if (n < N && k < K) dst[(long)n * K + k] = tile[tx][ty + 8 * i];
-    }
+    if (g_switches.no_pipe || b_batches * d.N * d.K > kPipeBMaxElements) return false;
+    return d.M >= (kmajor ? kPipeMinRowsKmajor : kPipeMinRows) && (double)d.G * d.M * d.N * d.K >= g_switches.b_rows_min_macs;
 }
-
-// An n-contiguous int64 B that is small next to the product (the values of an attention step against all the
-// probabilities, `bsht,btc->bshc`) is worth rewriting with contiguous rows first: the row-major kernels read it with
-// 16-byte loads and take A from digit planes (measured at S = T = 1024, 128 heads: 1.67 -> 1.45 ms, the rewrite 9 us).
-constexpr long kBRowsMaxElements = 8L << 20;         // 64 MB
 
 // The launch behind a speculative one: it does nothing unless the verdict word says that the digit counts did not cover
-// the operands, and then computes every output again.  Row-major B without a divisor: the widest MFMA instance (nine
+// the operands, and then computes every output again.  B without a divisor: the widest MFMA instance (nine
 // digits hold every int64, five every int32; config 4 with stale three-digit guesses: 4 ms where the vector-ALU tiles
 // take 35), one workgroup per compute unit walking the tiles.  Everything else, and a K beyond what its int32
 // accumulators take in one piece: the vector-ALU tiles.
 static Outcome launch_guarded_fallback(const GemmDesc &d, const MfmaParams &spec, int b_shift, GuardArgs *guard)
 {
-    // (an n-contiguous B that the speculative launch read through its row-major copy is read through that copy here too)
-    const bool b_copied = spec.B == (const void *)g_cache.b_rows && g_cache.b_rows != nullptr;
-    const bool row_major = b_copied || !(d.ldbn == 1 && d.ldbk != 1);
-    const Instance *wide = (row_major && b_shift == 0 && !g_switches.valu_fallback) ? pick_instance(9, d.b32 ? 5 : 9, d.b32 != 0, false, 16) : nullptr;
-    MfmaKernel fn = wide ? wide->guarded[d.b32 ? 1 : 0] : nullptr;
+    const bool kmajor = d.ldbn == 1 && d.ldbk != 1;
+    const Instance *wide = (b_shift == 0 && !g_switches.valu_fallback) ? pick_instance(9, d.b32 ? 5 : 9, d.b32 != 0, false, 16) : nullptr;
+    MfmaKernel fn = wide ? wide->guarded[d.b32 ? 1 : 0][kmajor ? 1 : 0] : nullptr;
     if (fn) {
         const long pairs = wide->na < wide->nb ? wide->na : wide->nb;
         const int ksteps = ((d.K + 32 * wide->kk - 1) / (32 * wide->kk)) * wide->kk;
-        if (pairs * ksteps * 32 * 16384 > 0x7FFFFFFFL) fn = nullptr;
+        if (pairs * ksteps * 32 * 16384 > kMaxDiagonal) fn = nullptr;
     }
     MfmaParams q = spec;
     if (fn) {
         // the caller's operands, not digit planes
         q.A = d.A; q.lda = d.lda; q.sA = d.sA;
-        if (!b_copied) { q.B = d.B; q.ldbn = d.ldbn; q.ldbk = d.ldbk; q.sB = d.sB; }
-        q.a_planes = nullptr; q.a_msub = 0; q.a_ksteps = 0; q.b_nsub = 0; q.b_ksteps = 0;
+        q.B = d.B; q.ldbn = d.ldbn; q.ldbk = d.ldbk; q.sB = d.sB;
+        q.a_planes = nullptr; q.a_msub = 0; q.a_ksteps = 0; q.b_nsub = 0; q.b_ksteps = 0; q.b_gstride = 0; q.row_steps = nullptr;
         q.tiles_m = (d.M + wide->bm - 1) / wide->bm;
         q.tiles_n = (d.N + wide->bn - 1) / wide->bn;
         const long total = (long)q.tiles_m * q.tiles_n * d.G;
@@ -616,7 +605,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
     }
     if (d.K <= 0 || d.M <= 0 || d.N <= 0 || d.G <= 0) return kDeclined;
     if (d.G > 65535) return kDeclined;
-    bool kmajor = d.ldbn == 1 && d.ldbk != 1;
+    const bool kmajor = d.ldbn == 1 && d.ldbk != 1;
     std::lock_guard<std::mutex> lock(g_cache.mu);
     if (!init_cache()) return kFailed;
     drain_pending();
@@ -633,19 +622,6 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             prep = &it->second;
     }
     const long b_batches = d.sB != 0 ? d.G : 1;
-    if (kmajor && !d.b32 && d.M > 32 && b_batches * d.N * d.K <= kBRowsMaxElements &&
-        (double)d.G * d.M * d.N * d.K >= g_switches.b_rows_min_macs) {
-        // (without memory for the copy the n-contiguous kernels run as before)
-        const Outcome got = grow(g_cache.b_rows, g_cache.b_rows_count, (size_t)(b_batches * d.N * d.K), "row-major copy of B");
-        if (got == kDone) {
-            const dim3 grid((unsigned)((d.N + 31) / 32), (unsigned)((d.K + 31) / 32), (unsigned)b_batches);
-            b_rows_kernel<<<grid, dim3(256), 0, 0>>>(reinterpret_cast<const int64_t *>(d.B), d.ldbk, d.sB, g_cache.b_rows, d.N, d.K);
-            p.B = g_cache.b_rows; p.ldbn = d.K; p.ldbk = 1; p.sB = d.sB != 0 ? (long)d.N * d.K : 0;
-            kmajor = false;
-        } else if (got == kFailed) {
-            return kFailed;
-        }
-    }
     p.M = d.M; p.N = d.N; p.K = d.K; p.shift = d.shift; p.init = d.init;
     p.range = g_cache.dev;
     p.verify_b_all_batches = d.sB != 0;
@@ -699,12 +675,29 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         }
         if (!inst) return kDeclined;
         if (!prep && !inst->skinny) inst = smaller_tiles(inst, d, g_cache.cus);
+        if (!prep) { p.B = d.B; p.b_gstride = 0; }
+        p.row_steps = nullptr;
+        // planes on both sides: the pipelined kernel, where there is one for the digit counts
+        PipeForm pipe = {};
+        if (prep && !inst->skinny && inst->kk == 1 && !g_switches.no_pipe) pipe = pipe_form(inst->na, inst->nb);
+        bool pre_b = false;
+        if (!prep && b_shift == 0 && pipe_b_planes(d, kmajor, b_batches)) {
+            const Instance *both = pick_instance(na, nb, false, false, need_diag, 0, kB64PlanesBoth);
+            const PipeForm f = both ? pipe_form(both->na, both->nb) : PipeForm{};
+            const long fewer = both && both->na < both->nb ? both->na : (both ? both->nb : 0);
+            if (f.fn && fewer * ((d.K + 31) / 32) * 32 * 16384 <= kMaxDiagonal &&
+                (long)((d.M + 127) / 128) * ((d.N + f.bn - 1) / f.bn) * d.G >= g_cache.cus) {
+                inst = both;
+                pipe = f;
+                pre_b = true;
+            }
+        }
         // int32 accumulators: at most min(NA,NB) digit pairs per diagonal, each product at most 2^14 in magnitude
         const long pairs = inst->na < inst->nb ? inst->na : inst->nb;
         const int ksteps = ((d.K + 32 * inst->kk - 1) / (32 * inst->kk)) * inst->kk;     // 32-k steps, padded
         // (a K beyond that bound is cut into slices that respect it: every tile is then split, see below)
-        const bool k_over = pairs * ksteps * 32 * 16384 > 0x7FFFFFFFL;
-        const int BM = inst->bm, BN = inst->bn;
+        const bool k_over = pairs * ksteps * 32 * 16384 > kMaxDiagonal;
+        const int BM = inst->bm, BN = pipe.fn ? pipe.bn : inst->bn;
         p.tiles_m = (d.M + BM - 1) / BM;
         p.tiles_n = (d.N + BN - 1) / BN;
         // A B operand that stays in L2 whatever the order (the MLA einsums: a KV cache or one head's weights against
@@ -727,20 +720,15 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         // us, 448 (243 x [512,7168]) 35.6 / 39.4, 896 (128 x [2048,7168]) 46.7 / 46.2, 1024 (128 x [7168,2048]) 49.5 /
         // 47.1, 1434 (243 x [1536,7168]) 54.7 / 52.2, 16384 (243 x [7168,16384]) 449 / 353.)
         const bool long_slices = (long)steps * 32 * inst->kk >= 800L * (small_split > 1 ? small_split : 1);
-        const bool use_planes = !kmajor && !inst->skinny && (prep || (p.tiles_n >= g_switches.planes_min_tiles_n && (total >= g_cache.cus || long_slices)));
+        const bool use_planes = pre_b || (!kmajor && !inst->skinny && (prep || (p.tiles_n >= g_switches.planes_min_tiles_n && (total >= g_cache.cus || long_slices))));
         if (b_shift && (kmajor || !inst->skinny)) return kDeclined;
-        const int variant = prep ? (inst->skinny ? kB64FlyBPlanes : kB64PlanesBoth)
+        const int variant = pre_b ? kB64PlanesBoth : prep ? (inst->skinny ? kB64FlyBPlanes : kB64PlanesBoth)
                           : b_shift ? (d.b32 ? kB32FlyRs : kB64FlyRs)
                           : kmajor ? (d.b32 ? kB32KmajorFly : kB64KmajorFly)
                                    : (d.b32 ? (use_planes ? kB32Planes : kB32Fly) : (use_planes ? kB64Planes : kB64Fly));
         MfmaKernel fn = inst->fn[variant];
         if (!fn) return kDeclined;
-        // planes on both sides and the 128 x 128 tile: the software-pipelined form (gemm_mfma_pipe.h; same tiles, planes,
-        // partial sums and outputs)
-        size_t pipe_lds = 0;
-        if (variant == kB64PlanesBoth && !g_switches.no_pipe && BM == 128 && BN == 128 && inst->kk == 1) {
-            if (MfmaKernel pfn = pipe_kernel(inst->na, inst->nb)) { fn = pfn; pipe_lds = pipe_lds_size(inst->na, inst->nb); }
-        }
+        if (pipe.fn) fn = pipe.fn;
 
         // Split-K: a launch smaller than the device is cut into `split` slices of K per tile, each a workgroup of
         // its own; with more tiles than compute units the same is done for the tiles of the last, partial round
@@ -752,7 +740,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         p.partials = nullptr;
         p.part64 = 0;
         p.finish_rq = 4;
-        if (!g_switches.no_tail_split) {
+        if (!g_switches.no_tail_split && !pre_b) {
             if (total < g_cache.cus) {
                 tail = (int)total;
                 split = small_split;
@@ -775,7 +763,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             // every tile in slices short enough for the int32 accumulators; without room for the partial sums (or with
             // the split switched off) the vector-ALU path takes the product
             int min_split = 2;
-            while (pairs * ((steps + min_split - 1) / min_split) * 32 * inst->kk * 16384 > 0x7FFFFFFFL) min_split++;
+            while (pairs * ((steps + min_split - 1) / min_split) * 32 * inst->kk * 16384 > kMaxDiagonal) min_split++;
             if (g_switches.no_tail_split || min_split > steps) return kDeclined;
             if (tail != (int)total || split < min_split) {
                 tail = (int)total;
@@ -802,7 +790,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             else if (k_over) return kDeclined;
         }
         const long blocks = (long)p.main_tiles + (total - p.main_tiles) * p.split;
-        long plane_wgs = 0;
+        long plane_wgs = 0, b_plane_wgs = 0;
         p.fail_class = inst->na > 5 || inst->nb > 5 ? 2 : 1;
         p.verdict = reinterpret_cast<unsigned *>(g_cache.dev + 5) + g_cache.turn;
         p.a_planes = nullptr; p.a_msub = 0; p.a_ksteps = 0;
@@ -815,12 +803,35 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             const int rows_per_wg = 256 / (4 * inst->kk);
             const dim3 pgrid((unsigned)(ksteps / inst->kk), (unsigned)((msub * 32 + rows_per_wg - 1) / rows_per_wg), (unsigned)d.G);
             plane_wgs = (long)pgrid.x * pgrid.y * pgrid.z;
-            if (const Outcome got = grow(g_cache.seen, g_cache.seen_count, (size_t)(blocks + plane_wgs), "digit counts")) return got;
-            // (the owned-k pattern of the planes of A follows the kernel that reads them: prepared planes of B go with the int64 forms)
-            inst->planes[(d.b32 && !prep) ? 1 : 0]<<<pgrid, dim3(256), 0, 0>>>(p, g_cache.planes, msub, ksteps, g_cache.seen + blocks);
+            const dim3 bgrid((unsigned)ksteps, (unsigned)((d.N + 63) / 64), (unsigned)b_batches);
+            b_plane_wgs = pre_b ? (long)bgrid.x * bgrid.y * bgrid.z : 0;
+            if (const Outcome got = grow(g_cache.seen, g_cache.seen_count, (size_t)(blocks + plane_wgs + b_plane_wgs), "digit counts")) return got;
+            // (the owned-k pattern of the planes of A follows the kernel that reads them: planes of B go with the int64 forms)
+            inst->planes[(d.b32 && !prep && !pre_b) ? 1 : 0]<<<pgrid, dim3(256), 0, 0>>>(p, g_cache.planes, msub, ksteps, g_cache.seen + blocks);
+            if (pre_b) {
+                BPlanesParams b = {};
+                b.B = d.B; b.ldn = d.ldbn; b.ldk = d.ldbk; b.sB = d.sB; b.N = d.N; b.K = d.K;
+                b.nsub = (d.N + 31) / 32; b.ksteps = ksteps;
+                b.gstride = (long)b.nsub * ksteps * inst->nb * 1024;
+                if (const Outcome got = grow(g_cache.b_planes, g_cache.b_planes_bytes, (size_t)(b.gstride * b_batches), "digit planes of B")) return got;
+                if (kmajor && !d.b32) {
+                    // (the one product of the model with zeros in A worth finding: a causal prompt's probabilities times the values)
+                    b.row_tiles = (long)p.tiles_m * d.G;
+                    if (const Outcome got = grow(g_cache.row_steps, g_cache.row_steps_count, (size_t)b.row_tiles, "step counts")) return got;
+                    b.row_steps = g_cache.row_steps;
+                    b.a_seen = g_cache.seen + blocks;
+                }
+                b.planes = g_cache.b_planes; b.seen = g_cache.seen + blocks + plane_wgs; b.verdict = p.verdict; b.fail_class = p.fail_class;
+#define ZK_BPL(NB_) do { if (d.b32) { if (kmajor) b_planes_kernel<NB_, true, true><<<bgrid, 256, 0, 0>>>(b); else b_planes_kernel<NB_, false, true><<<bgrid, 256, 0, 0>>>(b); } \
+                         else { if (kmajor) b_planes_kernel<NB_, true, false><<<bgrid, 256, 0, 0>>>(b); else b_planes_kernel<NB_, false, false><<<bgrid, 256, 0, 0>>>(b); } } while (0)
+                if (inst->nb == 3) ZK_BPL(3); else if (inst->nb == 4) ZK_BPL(4); else ZK_BPL(5);
+#undef ZK_BPL
+                p.B = b.planes; p.b_nsub = b.nsub; p.b_ksteps = ksteps; p.b_gstride = d.sB != 0 ? b.gstride : 0;
+                p.row_steps = b.row_steps;
+            }
         } else if (const Outcome got = grow(g_cache.seen, g_cache.seen_count, (size_t)blocks, "digit counts")) return got;
-        p.seen = g_cache.seen;
-        const size_t lds = pipe_lds ? pipe_lds : 2 * (size_t)inst->kk * ((BM / 32) * inst->na + (BN / 32) * inst->nb) * 1024 + 9 * 1024 + 16;
+        p.seen = pipe.fn ? nullptr : g_cache.seen;
+        const size_t lds = pipe.fn ? pipe.lds : 2 * (size_t)inst->kk * ((BM / 32) * inst->na + (BN / 32) * inst->nb) * 1024 + 9 * 1024 + 16;
         static std::set<const void *> lds_raised;
         if (lds > 64 * 1024 && !lds_raised.count((const void *)fn)) {
             if (hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
@@ -829,10 +840,18 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             }
             lds_raised.insert((const void *)fn);
         }
-        fn<<<dim3((unsigned)blocks), dim3((unsigned)inst->threads), lds, 0>>>(p);
+        unsigned grid = (unsigned)blocks;
+        if (pipe.fn) {
+            // one workgroup per compute unit walks the items; without split tiles they go row tile by row tile
+            p.batches = d.G;
+            p.row_order = pre_b ? 1 : 0;
+            p.items = pre_b ? (int)(((long)p.tiles_m * d.G + 7) / 8 * 8 * p.tiles_n) : (int)blocks;
+            grid = (unsigned)(p.items < g_cache.cus ? p.items : g_cache.cus);
+        }
+        fn<<<dim3(grid), dim3((unsigned)inst->threads), lds, 0>>>(p);
         g_last_pairs = kept_pairs_before(inst->na, inst->nb, inst->dmax, inst->na, 0);
         g_last_prepared = prep ? 1 : 0;
-        if (pipe_lds) g_pipe_calls++;
+        if (pipe.fn) g_pipe_calls++;
         {
             const hipError_t err = hipGetLastError();
             if (err != hipSuccess) {
@@ -842,20 +861,21 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             }
         }
         if (p.split > 1) {
-            inst->finish<<<dim3((unsigned)((total - p.main_tiles) * p.finish_rq)), dim3((unsigned)inst->threads), 0, 0>>>(p);
+            (pipe.fn ? pipe.finish : inst->finish)<<<dim3((unsigned)((total - p.main_tiles) * p.finish_rq)), dim3((unsigned)inst->threads), 0, 0>>>(p);
             if (hipGetLastError() != hipSuccess) { set_error(kLaunchFailure, "gemm: split finish launch failed"); return kFailed; }
         }
         *limbs_a = inst->na;
         *limbs_b = inst->nb;
         if (speculate) {
             // no waiting: a guarded launch redoes the product if the verdict is raised, the digits seen follow later
-            GuardArgs guard = make_guard(blocks + plane_wgs);
+            GuardArgs guard = make_guard(p.seen ? blocks + plane_wgs : plane_wgs + b_plane_wgs);
+            if (!p.seen) guard.seen += blocks;
             if (const Outcome got = launch_guarded_fallback(d, p, b_shift, &guard)) return got;
             guard_taken(guard, key_a, key_b, prep ? prep->nb : 0);       // (the slots are shared with the grouped launches, which set it too)
             return kDone;
         }
         int need_a, need_b;
-        if (!wait_digits(blocks + plane_wgs, &need_a, &need_b)) { set_error(kLaunchFailure, "gemm: digit readback failed"); return kFailed; }
+        if (!wait_digits(p.seen ? 0 : blocks, p.seen ? blocks + plane_wgs : plane_wgs + b_plane_wgs, &need_a, &need_b)) { set_error(kLaunchFailure, "gemm: digit readback failed"); return kFailed; }
         if (prep) need_b = prep->nb;
         g_cache.store_pair(key_a, need_a, key_b, need_b);
         if (need_a <= inst->na && need_b <= inst->nb) return kDone;
@@ -937,7 +957,7 @@ int gemm_mfma_grouped(const GroupedDesc &d, int *limbs_a, int *limbs_b)
         }
         const long pairs = inst->na < inst->nb ? inst->na : inst->nb;
         const int ksteps = (d.K + 31) / 32;
-        if (pairs * ksteps * 32 * 16384 > 0x7FFFFFFFL) return 1;
+        if (pairs * ksteps * 32 * 16384 > kMaxDiagonal) return 1;
         p.tiles_n = (d.N + inst->bn - 1) / inst->bn;
         const long max_mtiles = (long)d.rows / 32 + d.groups;
         const long blocks = (max_mtiles + 7) / 8 * 8 * p.tiles_n;       // (whole rounds of the 8 XCDs: see the kernels' tile order)
@@ -980,7 +1000,7 @@ int gemm_mfma_grouped(const GroupedDesc &d, int *limbs_a, int *limbs_b)
             speculate = false;      // the 16-row kernels do not take this product: wait for the verdict after all
         }
         int need_a, need_b;
-        if (!wait_digits(blocks, &need_a, &need_b)) { set_error(kLaunchFailure, "grouped gemm: digit readback failed"); return -1; }
+        if (!wait_digits(0, blocks, &need_a, &need_b)) { set_error(kLaunchFailure, "grouped gemm: digit readback failed"); return -1; }
         if (prep) need_b = prep->nb;
         g_cache.store_pair(key_a, need_a, key_b, need_b);
         *limbs_a = inst->na;

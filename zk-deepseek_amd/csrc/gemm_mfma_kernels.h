@@ -37,7 +37,10 @@ struct MfmaParams {
     int verify_b_all_batches;       // B differs per batch: every batch's first tile row tracks its range
     const unsigned char *a_planes;  // pre-split digits of A (planes variants only)
     int a_msub, a_ksteps;           // 32-row groups and 32-k steps the planes were written for
-    int b_nsub, b_ksteps;           // BPL kernels: B (or every group's B) is digit planes of that geometry, prepared beforehand
+    int b_nsub, b_ksteps;           // BPL kernels: B (or every group's B) is digit planes of that geometry
+    long b_gstride;                 // ... and this many bytes from one batch's planes to the next one's (0: shared)
+    const int *row_steps;           // 32-k steps of a row tile (128 rows) of A up to its last non-zero one (null: all of them; pipelined kernel only)
+    int row_order, items, batches;  // pipelined kernel: items walked row tile by row tile, how many there are, and batches
     // split-K tail: workgroup ids below main_tiles are whole tiles; the rest are `split` workgroups per tile that
     // each cover a slice of K and leave raw 128-bit partial sums in `partials`
     int main_tiles, split;
@@ -317,7 +320,7 @@ __device__ __forceinline__ int frag_offset(int row, int j, int n_limbs, int subs
 // When A is reused by many column tiles it is split once, into digit planes stored in MFMA fragment order:
 // block (g, sub, ks32, i) of 1 KB holds digit i of rows [32*sub, 32*sub+32) for the 32 owned-k slots of MFMA
 // depth ks32, lane-major.  Rows >= M and k >= K are written as zero digits.  Each workgroup also leaves the
-// digits of what it read needs in seen[block] (when that is given).
+// digits of what it read needs in seen[block] (when that is given; 0: it was all zeros).
 // IN32: the matrix holds int32 elements (weights prepared once; lda and sA count elements as they do for int64).
 template <int NA, int RUN, int KK, bool IN32 = false>
 __global__ __launch_bounds__(256) void a_planes_kernel(MfmaParams p, unsigned char *planes, int msub, int ksteps32, unsigned *seen)
@@ -346,7 +349,7 @@ __global__ __launch_bounds__(256) void a_planes_kernel(MfmaParams p, unsigned ch
         for (int i = 0; i < NA; i++) *reinterpret_cast<uint2 *>(dst + i * 1024) = dg[i];
     }
     if (!seen) return;
-    const int need = wave_max_i32(bound.digits());
+    const int need = wave_max_i32((bound.lo | bound.hi) == 0 ? 0 : bound.digits());
     if ((tid & 63) == 0) red[tid >> 6] = need;
     __syncthreads();
     if (tid == 0) {
@@ -358,8 +361,122 @@ __global__ __launch_bounds__(256) void a_planes_kernel(MfmaParams p, unsigned ch
     }
 }
 
+// The same for a B that is small next to the product (pipe_b_planes in gemm_mfma.hip): its rows (columns of the output) for
+// A's, either layout, both element types, one depth per step.  It runs behind the pass over A and, with `row_steps`,
+// finds the last step of every 128 rows of A that is not all zeros from the words that pass has left.
+struct BPlanesParams {
+    const void *B;
+    long ldn, ldk, sB;              // B[g * sB + n * ldn + k * ldk]
+    int N, K, nsub, ksteps;
+    long gstride;                   // bytes of planes per batch
+    unsigned char *planes;
+    unsigned *seen, *verdict;
+    int fail_class;
+    int *row_steps;                 // may be null
+    const unsigned *a_seen;         // [row tiles][2][ksteps]
+    long row_tiles;
+};
+
+template <int NB, bool KMAJOR, bool IN32>
+__global__ __launch_bounds__(256) void b_planes_kernel(BPlanesParams p)
+{
+    __shared__ int red[4];
+    const int tid = threadIdx.x, g = blockIdx.z, ks = blockIdx.x;
+    // adjacent lanes read adjacent elements: of k where k is contiguous, of n where n is
+    const int row = blockIdx.y * 64 + (KMAJOR ? (tid & 63) : tid >> 2), j = KMAJOR ? tid >> 6 : tid & 3;
+    int64_t x[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const int k = ks * 32 + owned_k<2, 4>(j, e);
+        const long at = (long)g * p.sB + (long)row * p.ldn + (long)k * p.ldk;
+        x[e] = row < p.N && k < p.K ? (IN32 ? (int64_t)reinterpret_cast<const int32_t *>(p.B)[at] : reinterpret_cast<const int64_t *>(p.B)[at]) : 0;
+    }
+    DigitsSeen bound;
+#pragma unroll
+    for (int e = 0; e < 8; e++) bound.add(x[e]);
+    bound.seen = true;
+    uint2 dg[NB];
+    limb_split8<NB>(x, dg);
+    if ((row >> 5) < p.nsub) {
+        unsigned char *dst = p.planes + (long)g * p.gstride + ((long)(row >> 5) * p.ksteps + ks) * (NB * 1024) + ((row & 31) + 32 * (j >> 1)) * 16 + (j & 1) * 8;
+#pragma unroll
+        for (int i = 0; i < NB; i++) *reinterpret_cast<uint2 *>(dst + i * 1024) = dg[i];
+    }
+    const int need = wave_max_i32(bound.digits());
+    if ((tid & 63) == 0) red[tid >> 6] = need;
+    __syncthreads();
+    const long block = ((long)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    if (tid == 0) {
+        int n = red[0];
+#pragma unroll
+        for (int w = 1; w < 4; w++) n = red[w] > n ? red[w] : n;
+        leave_digits(p.seen + block, p.verdict, p.fail_class, NB, NB, 0, n);
+    }
+    if (!p.row_steps) return;
+    // a wavefront per row tile
+    const long waves = 4L * gridDim.x * gridDim.y * gridDim.z;
+    for (long t = block * 4 + (tid >> 6); t < p.row_tiles; t += waves) {
+        const unsigned *w = p.a_seen + t * 2 * p.ksteps;
+        int last = 0;
+        for (int i = tid & 63; i < p.ksteps; i += 64)
+            if ((w[i] | w[p.ksteps + i]) & 0xFFu) last = i + 1;
+        last = wave_max_i32(last);
+        if ((tid & 63) == 0) p.row_steps[t] = last;
+    }
+}
+
 // The report of a launch that has no guarded launch behind it (its caller waits for the digits instead).
 static __global__ __launch_bounds__(256) void digits_report_kernel(GuardArgs g) { guard_report(g, 0); }
+
+// One output from its D int32 diagonals: init + sum_d dg(d) * 2^(8d) as the words of a 128-bit sum.  A diagonal keeps its
+// low byte and hands the rest to the next one, so everything is 32-bit: two instructions per diagonal and a byte permute
+// per byte, where adding the diagonals up in 64 and 128 bits took some forty per output with wait states between the
+// carries (a 128x128 tile of six diagonals: 13k cycles, as long as eight steps of its MFMAs).
+// kMaxDiagonal: what a diagonal may reach for that; 0 <= init < 2^20.
+constexpr long kMaxDiagonal = 0x7F000000L;
+struct Words { uint32_t w[4]; };
+template <int D, class F>
+__device__ __forceinline__ Words sum_diagonals(F &&dg, int init)
+{
+    int c[D];
+    c[0] = dg(0) + init;
+#pragma unroll
+    for (int d = 1; d < D; d++) c[d] = dg(d) + (c[d - 1] >> 8);
+    // bytes 0 .. D-2 are the low bytes of c; from byte D-1 on the sum is c[D-1], sign-extended
+    Words s;
+    constexpr int TOP = D - 1;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        if (4 * q + 3 < TOP) {
+            const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)c[4 * q + 1], (uint32_t)c[4 * q], 0x0c0c0400u);
+            const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)c[4 * q + 3], (uint32_t)c[4 * q + 2], 0x04000c0cu);
+            s.w[q] = p01 | p23;
+        } else if (4 * q <= TOP) {
+            constexpr int n = TOP & 3;                       // whole bytes below c[TOP] in this word
+            uint32_t v = (uint32_t)c[TOP] << (8 * n);
+            if (n == 1) v = __builtin_amdgcn_perm(v, (uint32_t)c[TOP - 1], 0x07060500u);
+            if (n >= 2) v = __builtin_amdgcn_perm(v, __builtin_amdgcn_perm((uint32_t)c[TOP - n + 1], (uint32_t)c[TOP - n], 0x0c0c0400u), 0x07060100u);
+            if (n == 3) v = __builtin_amdgcn_perm(v, __builtin_amdgcn_perm((uint32_t)c[TOP - 1], v, 0x0c040100u), 0x07020100u);
+            s.w[q] = v;
+        } else {
+            s.w[q] = 4 * (q - 1) <= TOP ? (uint32_t)((TOP & 3) ? c[TOP] >> (32 - 8 * (TOP & 3)) : c[TOP] >> 31) : (uint32_t)((int)s.w[q - 1] >> 31);
+        }
+    }
+    return s;
+}
+
+// bits [sh, sh + 64) of the sum, and the bits below sh; sh (0..63) is the same in every lane
+__device__ __forceinline__ int64_t shifted_sum(const Words &s, int sh)
+{
+    const bool upper = sh >= 32;
+    const uint32_t a = upper ? s.w[1] : s.w[0], b = upper ? s.w[2] : s.w[1], c = upper ? s.w[3] : s.w[2];
+    const uint32_t lo = __builtin_amdgcn_alignbit(b, a, (uint32_t)sh & 31), hi = __builtin_amdgcn_alignbit(c, b, (uint32_t)sh & 31);
+    return (int64_t)((uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ int64_t sum_below(const Words &s, uint64_t mask)
+{
+    return (int64_t)((uint64_t)(s.w[1] & (uint32_t)(mask >> 32)) << 32 | (s.w[0] & (uint32_t)mask));
+}
 
 // Number of digit pairs (i', j') with i' + j' < d that come before (i, j) in row order (i' < i, or i' == i and j' < j).
 __host__ __device__ constexpr int kept_pairs_before(int na, int nb, int d, int i, int j)
@@ -533,7 +650,7 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
             const int sub_i = cc / (NB * 64), within = cc - sub_i * (NB * 64);
             int sub = (n0 >> 5) + sub_i;
             sub = sub < p.b_nsub ? sub : p.b_nsub - 1;          // column groups past N: any valid data, never stored
-            b_pl[it] = reinterpret_cast<const unsigned char *>(b_base) + ((long)sub * p.b_ksteps + kk) * (NB * 1024) + within * 16;
+            b_pl[it] = reinterpret_cast<const unsigned char *>(b_base) + (GRP ? 0 : (long)g * p.b_gstride) + ((long)sub * p.b_ksteps + kk) * (NB * 1024) + within * 16;
             plb_dst[it] = live ? A_BLOCKS * 1024 + kk * SUBSTAGE + cc * 16 : DUMMY;
             plb_stride[it] = live ? STAGE : 0;
         }
@@ -868,19 +985,7 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
 
     // epilogue: diagonals -> 128-bit sum -> shift.  Accumulator register r of lane l holds
     // row 8*(r/4) + 4*(l/32) + r%4, column l%32 of its 32x32 tile.
-    // Diagonals are added in groups of four: a group's sum of v[4g+j] * 2^(8j) stays below 2^57, so it is plain 64-bit
-    // arithmetic; the groups (weights 2^0, 2^32, 2^64, 2^96) then meet in one 128-bit sum.
-    auto combine = [&](int a, int b, int r, u128 sum) {
-#pragma unroll
-        for (int gq = 0; gq < (D + 3) / 4; gq++) {
-            uint64_t s = (uint64_t)(int64_t)acc[a][b][4 * gq][r];
-#pragma unroll
-            for (int j = 1; j < 4; j++)
-                if (4 * gq + j < D) s += (uint64_t)(int64_t)acc[a][b][4 * gq + j][r] << (8 * j);
-            sum += (u128)(i128)(int64_t)s << (32 * gq);
-        }
-        return sum;
-    };
+    auto combine = [&](int a, int b, int r, int init) { return sum_diagonals<D>([&](int d) { return acc[a][b][d][r]; }, init); };
     if (nsplit > 1) {
         // raw partial sums (without the rounding term), finished by gemm_split_finish_kernel: 64 lanes' low words, then
         // (unless 64 bits hold the sums) their high words, per (slice, wave, tile, register)
@@ -892,17 +997,18 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
                 for (int r = 0; r < 16; r++) {
                     // rows of this register that all lie past M (uniform over the wave): nothing to keep
                     if (m0 + (wm * WM + a) * 32 + 8 * (r >> 2) + (r & 3) >= m_lim) continue;
-                    const u128 sum = combine(a, b, r, 0);
+                    const Words sum = combine(a, b, r, 0);
                     const long q = (((long)tail_tile * p.split + sidx) * (T / 64) + wave) * (WM * WN * 16) + (a * WN + b) * 16 + r;
-                    if (p.part64) p.partials[q * 64 + lane] = (uint64_t)sum;
-                    else { p.partials[q * 128 + lane] = (uint64_t)sum; p.partials[q * 128 + 64 + lane] = (uint64_t)(sum >> 64); }
+                    const uint64_t lo = (uint64_t)sum.w[1] << 32 | sum.w[0];
+                    if (p.part64) p.partials[q * 64 + lane] = lo;
+                    else { p.partials[q * 128 + lane] = lo; p.partials[q * 128 + 64 + lane] = (uint64_t)sum.w[3] << 32 | sum.w[2]; }
                 }
         return;
     }
     // Whole tiles: the loops carry no uniform branches (tiles that reach past M or N, and calls that want the remainder,
     // have their own copy), and a row's address is the tile's plus a scalar multiple of the row stride.
     const uint64_t rmask = p.shift ? ((1ull << p.shift) - 1) : 0;
-    const u128 sum0 = (u128)(i128)p.init;
+    const int sum0 = (int)p.init;
     const int sh = p.shift;
     auto store_tile = [&](auto edge_tag, auto rem_tag) {
         constexpr bool EDGE = decltype(edge_tag)::value, REM = decltype(rem_tag)::value;
@@ -916,13 +1022,11 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     const int dr = 8 * (r >> 2) + (r & 3);
-                    const u128 sum = combine(a, b, r, sum0);
-                    const uint64_t lo = (uint64_t)sum, hi = (uint64_t)(sum >> 64);
+                    const Words sum = combine(a, b, r, sum0);
                     if (EDGE && !(mrow + dr < m_lim && n < p.N)) continue;
                     const long o = o0 + (long)dr * p.ldc;
-                    // bits [sh, sh + 64): the upper word comes in through two shifts so that sh == 0 needs no case of its own
-                    p.C[o] = (int64_t)((lo >> sh) | ((hi << 1) << (63 - sh)));
-                    if (REM) p.R[o] = (int64_t)(lo & rmask);
+                    p.C[o] = shifted_sum(sum, sh);
+                    if (REM) p.R[o] = sum_below(sum, rmask);
                 }
             }
     };
@@ -942,7 +1046,7 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_mfma_kernel(MfmaParams p)
 // in front of it: its digit counts did not cover the operands), and then the grid, one workgroup per compute unit, walks
 // the workgroup ids of an ordinary launch.  A guarded launch almost always finds nothing to do, and thousands of
 // workgroups with 80 KB of LDS each would take tens of microseconds to find that out.
-template <int NA, int NB, int WVM, int WVN, int WM, int WN, int KK, bool B32, int DMAX = 16>
+template <int NA, int NB, int WVM, int WVN, int WM, int WN, int KK, bool B32, bool BKM, int DMAX = 16>
 __global__ __launch_bounds__(64 * WVM * WVN) void gemm_mfma_guarded_kernel(MfmaParams p)
 {
     const unsigned verdict = __atomic_load_n(p.guard.verdict, __ATOMIC_RELAXED);            // (the same for every thread of the launch)
@@ -952,13 +1056,13 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_mfma_guarded_kernel(MfmaP
         // five digits cover both operands (the fold kernel has seen every element): a third of the digit pairs of (9,9)
         constexpr int NA5 = NA > 5 ? 5 : NA, NB5 = NB > 5 ? 5 : NB;
         for (int block = (int)blockIdx.x; block < p.walk_blocks; block += (int)gridDim.x) {
-            gemm_mfma_block<NA5, NB5, WVM, WVN, WM, WN, KK, B32, false, false, false, false, 16, false>(p, block);
+            gemm_mfma_block<NA5, NB5, WVM, WVN, WM, WN, KK, B32, BKM, false, false, false, 16, false>(p, block);
             __syncthreads();
         }
         return;
     }
     for (int block = (int)blockIdx.x; block < p.walk_blocks; block += (int)gridDim.x) {
-        gemm_mfma_block<NA, NB, WVM, WVN, WM, WN, KK, B32, false, false, false, false, DMAX, false>(p, block);
+        gemm_mfma_block<NA, NB, WVM, WVN, WM, WN, KK, B32, BKM, false, false, false, DMAX, false>(p, block);
         __syncthreads();            // (the LDS stages and the range words in them are used again)
     }
 }
@@ -1060,7 +1164,7 @@ struct Instance {
     MfmaKernel fn[kVariants];
     PlanesKernel planes[2];      // [b32]: the owned-k pattern follows the element size of B
     FinishKernel finish;         // adds up the partial sums of split tail tiles
-    MfmaKernel guarded[2];       // [b32]: the guarded form for row-major B, A split on the fly (the widest instances only)
+    MfmaKernel guarded[2][2];    // [b32][n-contiguous B]: the guarded form, A split on the fly (the widest instances only)
 };
 
 
@@ -1095,11 +1199,17 @@ static Instance make_instance()
     s.dmax = DMAX;
     s.alt = TILE == kTile128x64;
     for (int v = 0; v < kVariants; v++) s.fn[v] = nullptr;
-    s.guarded[0] = s.guarded[1] = nullptr;
+    s.guarded[0][0] = s.guarded[0][1] = s.guarded[1][0] = s.guarded[1][1] = nullptr;
     // every operand fits nine digits, every int32 five: these instances can stand behind any speculative launch
     if constexpr (NA == 9 && !SKINNY && DMAX == 16 && USE == kUseAll) {
-        if constexpr (NB == 9) s.guarded[0] = gemm_mfma_guarded_kernel<NA, NB, WVM, WVN, WM, WN, KK, false, DMAX>;
-        if constexpr (NB == 5) s.guarded[1] = gemm_mfma_guarded_kernel<NA, NB, WVM, WVN, WM, WN, KK, true, DMAX>;
+        if constexpr (NB == 9) {
+            s.guarded[0][0] = gemm_mfma_guarded_kernel<NA, NB, WVM, WVN, WM, WN, KK, false, false, DMAX>;
+            s.guarded[0][1] = gemm_mfma_guarded_kernel<NA, NB, WVM, WVN, WM, WN, KK, false, true, DMAX>;
+        }
+        if constexpr (NB == 5) {
+            s.guarded[1][0] = gemm_mfma_guarded_kernel<NA, NB, WVM, WVN, WM, WN, KK, true, false, DMAX>;
+            s.guarded[1][1] = gemm_mfma_guarded_kernel<NA, NB, WVM, WVN, WM, WN, KK, true, true, DMAX>;
+        }
     }
     if constexpr (USE == kUsePlanesBoth) {
         static_assert(!SKINNY && KK == 1, "prepared planes of one matrix are in the order of one depth per step");

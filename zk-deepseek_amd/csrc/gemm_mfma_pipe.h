@@ -1,16 +1,23 @@
-// 128 x 128 tiles with BOTH operands from digit planes (A pre-split by the pass in front, B prepared once): nothing is
-// split, tracked or staged in registers, so the step is loads, fragment reads and MFMAs only, and it is written as a
-// software pipeline instead of the fenced phases of gemm_mfma_block:
-//   * the planes of a step are 4 (NA + NB) blocks of 1 KB, already in fragment order; every wavefront sends its share of
-//     them from global memory straight into a ring of LDS stages (global_load_lds_dwordx4), kPipeStages - 1 steps before
-//     they are multiplied, one load at a time between MFMAs;
-//   * the fragments of step s+1 are read into registers while the MFMAs of step s run: B's into a second set of
-//     registers at the start of the step, A's digit by digit into the registers whose last use has just been issued
-//     (the MFMAs go through A's digits in order), so that the matrix pipe has its operands the moment the step's one
-//     barrier opens.
-// Eight wavefronts as 2 x 4, 64 x 32 outputs each, as in the general kernel; tiles, split tail tiles, partial sums, digit
-// words and outputs are the general kernel's (gemm_mfma_block with APL and BPL), which this one replaces for three digits
-// a side.
+// Products whose operands are BOTH digit planes (A pre-split by the pass in front; B prepared once, or pre-split like A where
+// it is small next to the product): nothing is split, tracked or staged in registers, so a step is loads, fragment reads
+// and MFMAs only, and it is written as a software pipeline instead of the fenced phases of gemm_mfma_block:
+//   * the planes of a step are blocks of 1 KB, already in fragment order; every wavefront sends its share of them from
+//     global memory straight into a ring of LDS stages (global_load_lds_dwordx4), kPipeStages - 1 steps before they are
+//     multiplied, one load at a time between MFMAs;
+//   * the fragments of step s+1 are read into registers while the MFMAs of step s run, each into the registers whose last
+//     use has just been issued (the MFMAs go through A's digits in order and through B's within each), so that the
+//     matrix pipe has its operands when the step's one barrier opens;
+//   * a workgroup walks several tiles (one workgroup per compute unit), and the ring runs on across them: the first steps
+//     of the next tile are loaded while this one is multiplied and stored.  With a short K (512: sixteen steps) a tile's
+//     first loads and its epilogue are a third of its time.
+// What bounds it: the matrix pipe at the clock the device grants it.  A step takes 0.81 / 1.11 us on 128x128 tiles with
+// (3,3) / (3,4) digits and 0.79 / 1.04 on 128x64 with (4,4) / (5,5): 2.7-3.2 POP/s of i8 products, where the probe that
+// multiplies random bytes out of LDS and loads nothing does 2.9.  Then LDS (108 KB per 1536 cycles of (3,4) MFMAs).  128x128 tiles need 16 (NA + NB - 1) x 2
+// accumulator registers per lane: up to six diagonals fit beside two wavefronts per SIMD, more take 128x64 tiles.
+// Against gemm_mfma_block on planes of A alone: see pipe_b_planes in gemm_mfma.hip.
+//
+// All of a row tile's later steps may hold nothing but zeros in A (the probabilities of a causal prompt: a token's rows
+// end at its own position): p.row_steps then says how many steps of a row tile there are to multiply.
 #pragma once
 #include "lds_dma.h"
 
@@ -18,7 +25,9 @@ namespace zk {
 
 constexpr int kPipeStages = 5;
 
-constexpr size_t pipe_lds_bytes(int na, int nb) { return (size_t)kPipeStages * 4 * (size_t)(na + nb) * 1024; }
+// tile shape by diagonals: 128x128 as 2x4 wavefronts of 64x32, or 128x64 as 4x2 of 32x32
+constexpr bool pipe_wide(int na, int nb) { return na + nb - 1 <= 6; }
+constexpr size_t pipe_lds_bytes(int na, int nb) { return (size_t)kPipeStages * (4 * na + (pipe_wide(na, nb) ? 4 : 2) * nb) * 1024; }
 
 template <int I, int N, class F>
 __device__ __forceinline__ void static_for(F &&f)
@@ -29,98 +38,181 @@ __device__ __forceinline__ void static_for(F &&f)
     }
 }
 
-template <int NA, int NB>
-__global__ __launch_bounds__(512) void gemm_mfma_pipe_kernel(MfmaParams p)
+// 1 KB from a base that is the same in every lane (lane l: 16 bytes at base + off, off = 16 l) to LDS byte address `lds`
+__device__ __forceinline__ void lds_dma16_uniform(uint64_t base, unsigned off, unsigned lds)
 {
+    unsigned saved_m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved_m0) : "s"(lds), "v"(off), "s"(base) : "memory");
+}
+
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ uint64_t uniform64(uint64_t v)
+{
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32;
+}
+
+// one tile, or one slice of K of a split tile
+struct PipeItem {
+    int g, tm, tn, ks_begin, nsteps, tail_tile, sidx, i;      // i: its number
+};
+
+// The launch's arguments, read again wherever a tile begins or ends.  (Kept in scalar registers through the steps, they and
+// what the compiler derives from them took 110 more than there are; the spills' reloads were then waited for inside the
+// steps, and every such wait drained the ring: 1.30 us per step of (3,4) digits where 1.11 is what the matrix pipe takes
+// at the clock it is given.)
+typedef const __attribute__((address_space(4))) MfmaParams ConstParams;
+__device__ __forceinline__ ConstParams &launch_args()
+{
+    ConstParams *q = (ConstParams *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(q));
+    return *q;
+}
+
+template <int NA, int NB>
+__global__ __launch_bounds__(512) void gemm_mfma_pipe_kernel(MfmaParams)
+{
+    constexpr bool WIDE = pipe_wide(NA, NB);
     constexpr int D = NA + NB - 1, STG = kPipeStages, AHEAD = STG - 1, T = 512;
-    constexpr int BLOCKS = 4 * (NA + NB), STAGE = BLOCKS * 1024;
-    constexpr int LOADS = BLOCKS / 8;                       // per wavefront and step
-    static_assert(D <= 5, "160 accumulator registers: two wavefronts share a SIMD");
-    static_assert(BLOCKS % 8 == 0, "every wavefront loads the same number of blocks");
-    static_assert(LOADS * (AHEAD - 1) < 64, "vmcnt is a 6-bit counter");
+    constexpr int WVN = WIDE ? 4 : 2, WM = WIDE ? 2 : 1, BN = 32 * WVN;
+    constexpr int A_BLOCKS = 4 * NA, BLOCKS = A_BLOCKS + WVN * NB, STAGE = BLOCKS * 1024;
+    constexpr int LOADS = (BLOCKS + 7) / 8;                 // per wavefront and step (the last wavefront's may repeat the last block)
+    static_assert(WM * D * 16 + WM * NA * 4 + NB * 4 <= 240, "two wavefronts share a SIMD");
+    static_assert(LOADS * AHEAD < 64, "vmcnt is a 6-bit counter");
+    static_assert(NA * NB >= LOADS, "the loads ride behind the MFMAs");
     extern __shared__ __attribute__((aligned(16))) unsigned char pipe_smem[];
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);            // (the same in every lane)
-    const int wm = wave >> 2, wn = wave & 3;
-    const unsigned ring_lds = (unsigned)(uintptr_t)pipe_smem;
+    const int wave = uniform(tid >> 6);
+    const int wm = wave / WVN, wn = wave % WVN;
+    const unsigned ring_lds = (unsigned)(uintptr_t)pipe_smem, lane16 = (unsigned)lane * 16;
 
-    // workgroup -> tile or slice of a split tile, as in gemm_mfma_block
-    const int per_batch = p.tiles_m * p.tiles_n;
-    int lin = (int)blockIdx.x, sidx = 0, nsplit = 1;
-    if (lin < p.main_tiles) {
-        if ((p.main_tiles & 7) == 0) lin = (lin & 7) * (p.main_tiles >> 3) + (lin >> 3);
-    } else {
-        const int t = lin - p.main_tiles;
-        if (p.tail_xcd) {
-            const int x = t & 7, q = t >> 3;
-            const int pair = (q / p.tiles_m) * 8 + x;
-            lin = p.main_tiles + (pair / p.split) * p.tiles_m + q % p.tiles_m;
-            sidx = pair % p.split;
+    // ---- work items: number i of this workgroup's walk, i = blockIdx.x + n * gridDim.x; false: no such item ----
+    auto decode = [](int i) {
+        ConstParams &p = launch_args();
+        const int per_batch = p.tiles_m * p.tiles_n, tiles_m = p.tiles_m, tiles_n = p.tiles_n;
+        const int ksteps = (p.K + 31) / 32;                 // (the planes are padded with zeros to whole steps)
+        int g, tm, tn, tail_tile = 0, sidx = 0, nsplit = 1;
+        if (p.row_order) {
+            // Consecutive ids go round the 8 XCDs: an XCD takes every eighth row tile and all its tile columns, so that its
+            // planes of A come from memory once and row tiles of different lengths are dealt evenly.
+            const int q = i >> 3, r = q / tiles_n * 8 + (i & 7);
+            tn = q % tiles_n;
+            g = r / tiles_m;
+            tm = r - g * tiles_m;
+            if (g >= p.batches) g = -1;
         } else {
-            lin = p.main_tiles + t / p.split;
-            sidx = t % p.split;
+            int lin = i;
+            if (lin < p.main_tiles) {
+                if ((p.main_tiles & 7) == 0) lin = (lin & 7) * (p.main_tiles >> 3) + (lin >> 3);
+            } else {
+                const int t = lin - p.main_tiles;
+                if (p.tail_xcd) {
+                    const int x = t & 7, q = t >> 3;
+                    const int pair = (q / tiles_m) * 8 + x;
+                    lin = p.main_tiles + (pair / p.split) * tiles_m + q % tiles_m;
+                    sidx = pair % p.split;
+                } else {
+                    lin = p.main_tiles + t / p.split;
+                    sidx = t % p.split;
+                }
+                nsplit = p.split;
+            }
+            tail_tile = lin - p.main_tiles;
+            g = lin / per_batch;
+            const int rem = lin - g * per_batch;
+            if (p.n_fastest) { tm = rem / tiles_n; tn = rem % tiles_n; }
+            else { tn = rem / tiles_m; tm = rem % tiles_m; }
         }
-        nsplit = p.split;
-    }
-    const int tail_tile = lin - p.main_tiles;
-    const int g = lin / per_batch, rem = lin - g * per_batch;
-    int tm, tn;
-    if (p.n_fastest) { tm = rem / p.tiles_n; tn = rem - tm * p.tiles_n; }
-    else { tn = rem / p.tiles_m; tm = rem - tn * p.tiles_m; }
-    const int m0 = tm * 128, n0 = tn * 128, m_lim = p.M;
-    const int ksteps = (p.K + 31) / 32;                     // (the planes are padded with zeros to whole steps)
-    const int ks_begin = (int)((long)sidx * ksteps / nsplit), ks_end = (int)((long)(sidx + 1) * ksteps / nsplit);
-    const int nsteps = ks_end - ks_begin;
-
-    // ---- this wavefront's blocks of a step: numbers wave * LOADS + l of [A: 32-row group 0..3][digit], [B: 32-column group 0..3][digit] ----
-    const unsigned char *src[LOADS];
-    long stride[LOADS];
-#pragma unroll
-    for (int l = 0; l < LOADS; l++) {
-        const int b = wave * LOADS + l;
-        if (b < 4 * NA) {
-            const int grp = b / NA, dig = b - grp * NA;
-            src[l] = p.a_planes + ((((long)g * p.a_msub + (m0 >> 5) + grp) * p.a_ksteps + ks_begin) * NA + dig) * 1024 + lane * 16;
-            stride[l] = NA * 1024;
-        } else {
-            const int bb = b - 4 * NA, grp = bb / NB, dig = bb - grp * NB;
-            int sub = (n0 >> 5) + grp;
-            sub = sub < p.b_nsub ? sub : p.b_nsub - 1;      // column groups past N: any valid data, never stored
-            src[l] = reinterpret_cast<const unsigned char *>(p.B) + (((long)sub * p.b_ksteps + ks_begin) * NB + dig) * 1024 + lane * 16;
-            stride[l] = NB * 1024;
+        const int ks_begin = (int)((long)sidx * ksteps / nsplit);
+        int ks_end = (int)((long)(sidx + 1) * ksteps / nsplit);
+        if (p.row_steps && g >= 0) {
+            // (a scalar load: were it a vector load, the compiler would keep waiting for it, and with it for the whole ring)
+            const int live = *(const __attribute__((address_space(4))) int *)(p.row_steps + uniform64((uint64_t)((long)g * tiles_m + tm)));
+            ks_end = live < ks_end ? live : ks_end;
         }
-    }
-    auto issue_one = [&](int t, auto l_tag) {               // load l of local step t
-        constexpr int L = decltype(l_tag)::value;
-        const int tc = t < nsteps ? t : nsteps - 1;         // (past the end: the last step again, into a stage nobody reads any more)
-        lds_dma16(src[L] + (long)tc * stride[L], ring_lds + (unsigned)(t % STG) * STAGE + (wave * LOADS + L) * 1024);
+        // (at least one step, of zeros if need be: the accumulators are set by it)
+        return PipeItem{ uniform(g), uniform(tm), uniform(tn), uniform(ks_begin), uniform(ks_end > ks_begin ? ks_end - ks_begin : 1),
+                         uniform(tail_tile), uniform(sidx), i };
     };
-    auto issue = [&](int t) { static_for<0, LOADS>([&](auto l) { issue_one(t, l); }); };
+    auto next_item = [&](int i) {                           // the first item from i on; its g is negative if there is none
+        const int items = launch_args().items;
+        PipeItem it{ -1, 0, 0, 0, 1, 0, 0, i };
+        while (it.i < items && (it = decode(it.i)).g < 0) it.i += gridDim.x;
+        return it;
+    };
 
-    v16i acc[2][D];
+    // ---- loading: this wavefront's blocks of a step, numbers wave * LOADS + l of [A: 32-row group 0..3][digit], [B: 32-column group][digit] ----
+    PipeItem li;
+    int l_left;
+    uint64_t l_src[LOADS];
+    auto aim = [&]() {
+        ConstParams &p = launch_args();
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+        for (int l = 0; l < LOADS; l++) {
+            int b = wave * LOADS + l;
+            b = b < BLOCKS ? b : BLOCKS - 1;
+            if (b < A_BLOCKS) {
+                const int grp = b / NA, dig = b - grp * NA;
+                l_src[l] = uniform64((uint64_t)p.a_planes + ((((long)li.g * p.a_msub + li.tm * 4 + grp) * p.a_ksteps + li.ks_begin) * NA + dig) * 1024);
+            } else {
+                const int bb = b - A_BLOCKS, grp = bb / NB, dig = bb - grp * NB;
+                int sub = li.tn * WVN + grp;
+                sub = sub < p.b_nsub ? sub : p.b_nsub - 1;  // column groups past N: any valid data, never stored
+                l_src[l] = uniform64((uint64_t)p.B + (uint64_t)li.g * p.b_gstride + (((long)sub * p.b_ksteps + li.ks_begin) * NB + dig) * 1024);
+            }
+        }
+    };
+    auto issue_one = [&](unsigned stage, auto l_tag) {
+        constexpr int L = decltype(l_tag)::value;
+        int b = wave * LOADS + L;
+        b = b < BLOCKS ? b : BLOCKS - 1;
+        lds_dma16_uniform(l_src[L], lane16, ring_lds + stage * STAGE + b * 1024);
+    };
+    // the loads move on to the next step (past the last one they repeat it, into stages nobody reads any more)
+    auto advance = [&]() {
+        if (--l_left > 0) {
 #pragma unroll
-        for (int d = 0; d < D; d++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[a][d][r] = 0;
+            for (int l = 0; l < LOADS; l++) {
+                const int b = wave * LOADS + l;
+                l_src[l] += (b < A_BLOCKS ? NA : NB) * 1024;
+            }
+            return;
+        }
+        l_left = 1;
+        if (li.g >= 0) {
+            li = next_item(li.i + gridDim.x);
+            if (li.g >= 0) { l_left = li.nsteps; aim(); }
+        }
+    };
 
+    PipeItem it = next_item((int)blockIdx.x);
+    if (it.g < 0) return;
+    li = it;
+    l_left = li.nsteps;
+    aim();
+
+    v16i acc[WM][D];
+    v4i fa[WM][NA], fb[NB];
     auto read_a = [&](unsigned st, int a, int i) {
-        return *reinterpret_cast<const v4i *>(pipe_smem + st * STAGE + ((wm * 2 + a) * NA + i) * 1024 + lane * 16);
+        return *reinterpret_cast<const v4i *>(pipe_smem + st * STAGE + ((wm * WM + a) * NA + i) * 1024 + lane16);
     };
     auto read_b = [&](unsigned st, int j) {
-        return *reinterpret_cast<const v4i *>(pipe_smem + st * STAGE + (4 * NA + wn * NB + j) * 1024 + lane * 16);
+        return *reinterpret_cast<const v4i *>(pipe_smem + st * STAGE + (A_BLOCKS + wn * NB + j) * 1024 + lane16);
     };
 
     // prologue: AHEAD steps under way, the first one's fragments in registers
-#pragma unroll
-    for (int t = 0; t < AHEAD; t++) issue(t);
+#pragma unroll 1
+    for (unsigned t = 0; t < AHEAD; t++) {
+        static_for<0, LOADS>([&](auto l) { issue_one(t, l); });
+        advance();
+    }
     wait_vmcnt<LOADS * (AHEAD - 1)>();                     // step 0 has landed (my share)
     asm volatile("" ::: "memory");
-    __syncthreads();
-    v4i fa[2][NA], fb[NB];
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    unsigned st_next = 1, st_load = AHEAD;                  // stages of step s+1 and of step s+AHEAD
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int a = 0; a < WM; a++)
 #pragma unroll
         for (int i = 0; i < NA; i++) fa[a][i] = read_a(0, a, i);
 #pragma unroll
@@ -128,100 +220,125 @@ __global__ __launch_bounds__(512) void gemm_mfma_pipe_kernel(MfmaParams p)
 
     // Step s: the MFMAs of step s on the fragments in registers; beside them the fragment reads of step s+1 (landed and
     // fenced by the barrier at the top) and the loads of step s+AHEAD into the stage step s-1 was read from (those reads
-    // were waited for by the MFMAs of step s-1).
-    static_assert((NA - 1) * NB >= LOADS, "the loads ride behind the MFMAs of A's digits from the second on");
-    for (int s = 0; s < nsteps; s++) {
-        wait_vmcnt<LOADS * (AHEAD - 2)>();                  // step s+1 has landed (my share): steps s+2 .. s+AHEAD-1 may be under way
+    // were waited for by the MFMAs of step s-1, so the barrier need not wait for LDS).
+    auto step = [&](auto first_tag) {
+        constexpr bool FIRST = decltype(first_tag)::value;
         asm volatile("" ::: "memory");
-        __syncthreads();
-        const unsigned sn = (unsigned)((s + 1) % STG);
-        v4i fbn[NB];
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         static_for<0, NA>([&](auto i_tag) {
             constexpr int I = decltype(i_tag)::value;
             static_for<0, NB>([&](auto j_tag) {
                 constexpr int J = decltype(j_tag)::value;
+                constexpr bool ZERO = FIRST && (I == 0 || J == NB - 1);      // the first pair of diagonal I + J
+                const v16i zero = {};
 #pragma unroll
-                for (int a = 0; a < 2; a++) acc[a][I + J] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[a][I], fb[J], acc[a][I + J], 0, 0, 0);
-                // behind the first digit's MFMAs: the next step's fragments of B; behind the others': the loads, one at a time
-                if constexpr (I == 0) fbn[J] = read_b(sn, J);
-                constexpr int L = (I - 1) * NB + J;
-                if constexpr (I >= 1 && L < LOADS) {
+                for (int a = 0; a < WM; a++)
+                    acc[a][I + J] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[a][I], fb[J], ZERO ? zero : acc[a][I + J], 0, 0, 0);
+                constexpr int L = I * NB + J;
+                if constexpr (L < LOADS) {
                     __builtin_amdgcn_sched_barrier(0);
-                    issue_one(s + AHEAD, std::integral_constant<int, (I >= 1 && L < LOADS) ? L : 0>());
+                    issue_one(st_load, std::integral_constant<int, (L < LOADS ? L : 0)>());
                 }
                 __builtin_amdgcn_sched_barrier(0);
+                if constexpr (I == NA - 1) {                // digit J of B has been issued for the last time this step
+                    fb[J] = read_b(st_next, J);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             });
-            // digit I of A has been issued for the last time this step: its registers take the next step's
-            fa[0][I] = read_a(sn, 0, I);
-            fa[1][I] = read_a(sn, 1, I);
+#pragma unroll
+            for (int a = 0; a < WM; a++) fa[a][I] = read_a(st_next, a, I);   // and so has digit I of A
             __builtin_amdgcn_sched_barrier(0);
         });
+    };
+    auto move_on = [&]() {
+        advance();
+        st_next = st_next + 1 == STG ? 0 : st_next + 1;
+        st_load = st_load + 1 == STG ? 0 : st_load + 1;
+    };
+
+    int landed = 0;                                         // steps whose loads are known to have landed beyond what a step needs
+    for (;;) {
+        // before a step: the one behind it has landed (my share), the AHEAD - 2 after that may be under way
+        if (landed > 0) landed--; else wait_vmcnt<LOADS * (AHEAD - 2)>();
+        step(std::true_type());
+        for (int s = it.nsteps; s > 1; s--) {
+            move_on();
+            if (landed > 0) landed--; else wait_vmcnt<LOADS * (AHEAD - 2)>();
+            step(std::false_type());
+        }
+        move_on();
+        // The stores below count like loads and may complete out of turn with them: everything issued so far is waited for
+        // here, and the next tile's first steps, which that covers, wait for nothing (by the time a later one does, the
+        // stores are through).
+        wait_vmcnt<0>();
+        landed = AHEAD - 1;
+
+        // epilogue: diagonals -> 128-bit sum -> shift, as in gemm_mfma_block (accumulator register r of lane l holds
+        // row 8*(r/4) + 4*(l/32) + r%4, column l%32 of its 32 x 32 tile)
+        ConstParams &p = launch_args();
+        const int m0 = it.tm * 128, n0 = it.tn * BN, sh = p.shift, sum0 = (int)p.init;
+        const uint64_t rmask = sh ? ((1ull << sh) - 1) : 0;
+        auto combine = [&](int a, int r, int init) { return sum_diagonals<D>([&](int d) { return acc[a][d][r]; }, init); };
+        if (!p.row_order && it.tail_tile >= 0 && p.split > 1) {
+            // raw partial sums in the layout gemm_split_finish_kernel<8 / WVN, WVN, WM, 1> adds up
 #pragma unroll
-        for (int j = 0; j < NB; j++) fb[j] = fbn[j];
+            for (int a = 0; a < WM; a++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    if (m0 + (wm * WM + a) * 32 + 8 * (r >> 2) + (r & 3) >= p.M) continue;
+                    const Words sum = combine(a, r, 0);
+                    const long q = (((long)it.tail_tile * p.split + it.sidx) * (T / 64) + wave) * (WM * 16) + a * 16 + r;
+                    const uint64_t lo = (uint64_t)sum.w[1] << 32 | sum.w[0];
+                    if (p.part64) p.partials[q * 64 + lane] = lo;
+                    else { p.partials[q * 128 + lane] = lo; p.partials[q * 128 + 64 + lane] = (uint64_t)sum.w[3] << 32 | sum.w[2]; }
+                }
+        } else {
+            auto store_tile = [&](auto edge_tag, auto rem_tag) {
+                constexpr bool EDGE = decltype(edge_tag)::value, REM = decltype(rem_tag)::value;
+                const int n = n0 + wn * 32 + (lane & 31);
+#pragma unroll
+                for (int a = 0; a < WM; a++) {
+                    const int mrow = m0 + (wm * WM + a) * 32 + 4 * (lane >> 5);
+                    const long o0 = (long)it.g * p.sC + (long)mrow * p.ldc + n;
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const int dr = 8 * (r >> 2) + (r & 3);
+                        const Words sum = combine(a, r, sum0);
+                        if (EDGE && !(mrow + dr < p.M && n < p.N)) continue;
+                        const long o = o0 + (long)dr * p.ldc;
+                        p.C[o] = shifted_sum(sum, sh);
+                        if (REM) p.R[o] = sum_below(sum, rmask);
+                    }
+                }
+            };
+            const bool edge = m0 + 128 > p.M || n0 + BN > p.N;
+            if (p.R) { if (edge) store_tile(std::true_type(), std::true_type()); else store_tile(std::false_type(), std::true_type()); }
+            else { if (edge) store_tile(std::true_type(), std::false_type()); else store_tile(std::false_type(), std::false_type()); }
+        }
+        it = next_item(it.i + gridDim.x);
+        if (it.g < 0) break;
+        // the fragments of its first step once more (read beside the last step's MFMAs already, but no register keeps them
+        // through the epilogue)
+        const unsigned st = st_next == 0 ? STG - 1 : st_next - 1;
+#pragma unroll
+        for (int a = 0; a < WM; a++)
+#pragma unroll
+            for (int i = 0; i < NA; i++) fa[a][i] = read_a(st, a, i);
+#pragma unroll
+        for (int j = 0; j < NB; j++) fb[j] = read_b(st, j);
     }
     wait_vmcnt<0>();                                       // (the loads past the end)
-    asm volatile("" ::: "memory");
-
-    // both operands' digits were counted when their planes were written: nothing seen here
-    if (tid == 0 && p.seen) p.seen[blockIdx.x] = 0;
-
-    // epilogue: diagonals -> 128-bit sum -> shift, as in gemm_mfma_block (accumulator register r of lane l holds
-    // row 8*(r/4) + 4*(l/32) + r%4, column l%32 of its 32 x 32 tile)
-    auto combine = [&](int a, int r, u128 sum) {
-#pragma unroll
-        for (int gq = 0; gq < (D + 3) / 4; gq++) {
-            uint64_t sg = (uint64_t)(int64_t)acc[a][4 * gq][r];
-#pragma unroll
-            for (int j = 1; j < 4; j++)
-                if (4 * gq + j < D) sg += (uint64_t)(int64_t)acc[a][4 * gq + j][r] << (8 * j);
-            sum += (u128)(i128)(int64_t)sg << (32 * gq);
-        }
-        return sum;
-    };
-    if (nsplit > 1) {
-        // raw partial sums in the layout gemm_split_finish_kernel<2, 4, 2, 1> adds up
-#pragma unroll
-        for (int a = 0; a < 2; a++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                if (m0 + (wm * 2 + a) * 32 + 8 * (r >> 2) + (r & 3) >= m_lim) continue;
-                const u128 sum = combine(a, r, 0);
-                const long q = (((long)tail_tile * p.split + sidx) * (T / 64) + wave) * 32 + a * 16 + r;
-                if (p.part64) p.partials[q * 64 + lane] = (uint64_t)sum;
-                else { p.partials[q * 128 + lane] = (uint64_t)sum; p.partials[q * 128 + 64 + lane] = (uint64_t)(sum >> 64); }
-            }
-        return;
-    }
-    const uint64_t rmask = p.shift ? ((1ull << p.shift) - 1) : 0;
-    const u128 sum0 = (u128)(i128)p.init;
-    const int sh = p.shift;
-    auto store_tile = [&](auto edge_tag, auto rem_tag) {
-        constexpr bool EDGE = decltype(edge_tag)::value, REM = decltype(rem_tag)::value;
-        const int n = n0 + wn * 32 + (lane & 31);
-#pragma unroll
-        for (int a = 0; a < 2; a++) {
-            const int mrow = m0 + (wm * 2 + a) * 32 + 4 * (lane >> 5);
-            const long o0 = (long)g * p.sC + (long)mrow * p.ldc + n;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int dr = 8 * (r >> 2) + (r & 3);
-                const u128 sum = combine(a, r, sum0);
-                const uint64_t lo = (uint64_t)sum, hi = (uint64_t)(sum >> 64);
-                if (EDGE && !(mrow + dr < m_lim && n < p.N)) continue;
-                const long o = o0 + (long)dr * p.ldc;
-                p.C[o] = (int64_t)((lo >> sh) | ((hi << 1) << (63 - sh)));
-                if (REM) p.R[o] = (int64_t)(lo & rmask);
-            }
-        }
-    };
-    const bool edge = m0 + 128 > m_lim || n0 + 128 > p.N;
-    if (p.R) { if (edge) store_tile(std::true_type(), std::true_type()); else store_tile(std::false_type(), std::true_type()); }
-    else { if (edge) store_tile(std::true_type(), std::false_type()); else store_tile(std::false_type(), std::false_type()); }
 }
 
-// the kernel for digit counts (na, nb), or null, and its dynamic LDS
-MfmaKernel pipe_kernel(int na, int nb);
-size_t pipe_lds_size(int na, int nb);
+// the kernel for digit counts (na, nb) or null, its dynamic LDS, its tile columns and its finishing kernel
+struct PipeForm {
+    MfmaKernel fn;
+    FinishKernel finish;
+    int bn;
+    size_t lds;
+};
+PipeForm pipe_form(int na, int nb);
 
 }  // namespace zk

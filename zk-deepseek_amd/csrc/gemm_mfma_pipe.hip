@@ -1,15 +1,35 @@
-// Instances of the 128 x 128 kernel for digit planes on both sides (gemm_mfma_pipe.h): three digits a side.
+// Instances of the software-pipelined kernel for digit planes on both sides (gemm_mfma_pipe.h).
 #include "gemm_mfma_kernels.h"
 #include "gemm_mfma_pipe.h"
 
 namespace zk {
 
-MfmaKernel pipe_kernel(int na, int nb)
+template <int NA, int NB>
+static PipeForm form()
 {
-    if (na == 3 && nb == 3) return gemm_mfma_pipe_kernel<3, 3>;
-    return nullptr;
+    PipeForm f;
+    f.fn = gemm_mfma_pipe_kernel<NA, NB>;
+    if constexpr (pipe_wide(NA, NB)) f.finish = gemm_split_finish_kernel<2, 4, 2, 1>;
+    else f.finish = gemm_split_finish_kernel<4, 2, 1, 1>;
+    f.bn = pipe_wide(NA, NB) ? 128 : 64;
+    f.lds = pipe_lds_bytes(NA, NB);
+    return f;
 }
 
-size_t pipe_lds_size(int na, int nb) { return pipe_lds_bytes(na, nb); }
+PipeForm pipe_form(int na, int nb)
+{
+#define ZK_PIPE(NA_, NB_) if (na == NA_ && nb == NB_) return form<NA_, NB_>()
+    ZK_PIPE(3, 3);
+    ZK_PIPE(3, 4);
+    ZK_PIPE(4, 3);
+    ZK_PIPE(4, 4);
+    ZK_PIPE(3, 5);
+    ZK_PIPE(6, 3);
+    ZK_PIPE(5, 4);
+    ZK_PIPE(4, 5);
+    ZK_PIPE(5, 5);
+#undef ZK_PIPE
+    return PipeForm{ nullptr, nullptr, 0, 0 };
+}
 
 }  // namespace zk
