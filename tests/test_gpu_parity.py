@@ -365,6 +365,32 @@ def test_gemm_rows_staged_in_lds(K, oracle, M):
     assert K.gemm_last_plan()[0] == 1
 
 
+@pytest.mark.parametrize("Kd", [128, 132, 256, 260, 1028, 2052, 4100, 7168, 8196, 10244, 12292, 14340, 18432, 18436])
+def test_gemm_one_row_held_in_registers(K, oracle, Kd):
+    """one row against int32 weights: every count of 16-byte units per lane (one to nine, and the first K beyond), whole and
+    partial ones, one column, fewer columns than wavefronts and several rounds of them, batches, per-head weights; values
+    over the whole of both types"""
+    rng = np.random.default_rng(Kd)
+    for Bd, N in ((1, 1), (1, 37), (2, 700)) + (((1, 20000),) if Kd <= 260 else ()):
+        A = rand_i64(rng, (Bd, 1, Kd), 63)
+        W = rand_i32(rng, (N, Kd), 31)
+        A[0, 0, :3], W[N - 1, :3], W[0, Kd - 1] = [-(1 << 63), (1 << 63) - 1, 1 << 42], -(1 << 31), (1 << 31) - 1
+        for c in (0, 37):
+            _gemm_case(K, oracle, 0, A, W, 1, 1, c)
+            assert K.gemm_last_plan()[0] == 1
+    if Kd <= 2052:
+        o, w = rand_i64(rng, (1, 1, 19, Kd), 63), rand_i32(rng, (19, 35, Kd), 31)
+        assert np.array_equal(host(K.einsum_bshc_hdc_bshd(dev(o), dev(w), 29)), oracle.einsum_bshc_hdc_bshd(o, w, 29))
+        idx = np.array([[3, 0, 7], [3, 7, 5]], dtype=np.int64)
+        d = K.moe_dispatch(dev(idx), 9)
+        seg, tok, _ = oracle.moe_dispatch(idx, 9)
+        x, ws = rand_i64(rng, (2, Kd), 63), [rand_i32(rng, (261, Kd), 31) for _ in range(9)]
+        dw = [dev(t) for t in ws]
+        C, R = K.int64_grouped_bmm(K.moe_gather_rows(dev(x), d), K.pointer_table(dw), True, 261, 21, d, want_remainder=True)
+        Ce, Re = oracle.grouped_bmm(x[tok], ws, seg, 21)
+        assert np.array_equal(host(C), Ce) and np.array_equal(host(R), Re)
+
+
 @pytest.mark.parametrize("bits_w", [16, 28, 36, 63, -16, -30, -31])
 def test_gemm_prepared_weights(K, oracle, bits_w):
     """int64 weights split into digit planes once (zk_gemm_prepare_weights): the same bits as the unprepared call on

@@ -355,7 +355,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(ValuParams p)
     }
 }
 
-// One row of A against int32 weights with the row staged in LDS.  Every wave of a workgroup needs the whole row, and
+// Two rows of A (or one longer than the kernel below takes) against int32 weights with the rows staged in LDS.  Every wave of a workgroup needs the whole row, and
 // read from memory it costs twice the bytes of the weights it meets; staged once per workgroup it is split on the way in,
 //     a = a2 * 2^42 + a1 * 2^21 + a0,   a0, a1 in [0, 2^21),   a2 in [-2^21, 2^21),
 // so that a piece times an int32 weight stays below 2^52 in magnitude and a lane can add 1024 of them in a plain 64-bit
@@ -464,6 +464,134 @@ __global__ __launch_bounds__(64 * kStagedWaves) void gemv32_staged_kernel(ValuPa
         }
 }
 
+// One row of A against int32 weights with the row in REGISTERS.  Eight wavefronts, WK of them along K and 8 / WK on
+// different columns: a wavefront's lanes hold their elements of A (4 U of them, in the three pieces of the kernel above)
+// for the whole launch and meet one column after the other, whose loads of the next columns are under way meanwhile.
+// Nothing is staged, so the weights start to flow with the first instruction and no barrier interrupts them: the LDS form
+// waited for its staging, once per 4096 elements, with nothing under way.  What bounds it is the stream of weights:
+// [7168,16384] 85.5 -> 74.7 us (6.3 TB/s), [18432,7168] 95.6 -> 81, [1536,7168] 14.0 -> 8.8, [2048,7168] 12.6 -> 10.3,
+// [16384,1536] 20.2 -> 17.3, a token's eight experts [2048,7168] each 76.5 -> 74.2, 128 heads [128,512] each 13.3 -> 7.9.
+// (More columns under way than 12 units' worth: the registers leave room for one workgroup per compute unit where two
+// do better, the experts 80 us.)
+constexpr int kRegsWaves = 8;
+constexpr int kRegsMaxUnits = 9;         // 16-byte units of a column per lane: 12 registers of A each
+
+// Sum over a wavefront, in lane 63 (row shifts and row broadcasts: no LDS).
+__device__ __forceinline__ u128 wave_sum_last(u128 v)
+{
+    uint32_t w0 = (uint32_t)v, w1 = (uint32_t)(v >> 32), w2 = (uint32_t)(v >> 64), w3 = (uint32_t)(v >> 96);
+#define ZK_DPP_STEP(CTRL, ROWS) do {                                                                                       \
+        const uint32_t t0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w0, CTRL, ROWS, 0xf, false);                   \
+        const uint32_t t1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w1, CTRL, ROWS, 0xf, false);                   \
+        const uint32_t t2 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w2, CTRL, ROWS, 0xf, false);                   \
+        const uint32_t t3 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w3, CTRL, ROWS, 0xf, false);                   \
+        const u128 a = (u128)((uint64_t)w1 << 32 | w0) | (u128)((uint64_t)w3 << 32 | w2) << 64;                          \
+        const u128 b = (u128)((uint64_t)t1 << 32 | t0) | (u128)((uint64_t)t3 << 32 | t2) << 64;                          \
+        const u128 c = a + b;                                                                                               \
+        w0 = (uint32_t)c; w1 = (uint32_t)(c >> 32); w2 = (uint32_t)(c >> 64); w3 = (uint32_t)(c >> 96);                  \
+    } while (0)
+    ZK_DPP_STEP(0x111, 0xf);     // row_shr 1, 2, 4, 8: the sum of a row of 16 in its last lane
+    ZK_DPP_STEP(0x112, 0xf);
+    ZK_DPP_STEP(0x114, 0xf);
+    ZK_DPP_STEP(0x118, 0xf);
+    ZK_DPP_STEP(0x142, 0xa);     // row_bcast 15 into rows 1 and 3
+    ZK_DPP_STEP(0x143, 0xc);     // row_bcast 31 into rows 2 and 3
+#undef ZK_DPP_STEP
+    return (u128)((uint64_t)w1 << 32 | w0) | (u128)((uint64_t)w3 << 32 | w2) << 64;
+}
+
+// acc += x * b.  (Written out: the compiler would keep every piece of A in the 64 bits it is multiplied in, twice the
+// registers, and multiplies the ones it knows to be short in several instructions.)
+__device__ __forceinline__ void mad_i64(int64_t &acc, int x, int b)
+{
+    asm("v_mad_i64_i32 %0, vcc, %1, %2, %0" : "+v"(acc) : "v"(x), "v"(b) : "vcc");
+}
+
+template <int U, bool GRP>
+__global__ __launch_bounds__(64 * kRegsWaves) void gemv32_regs_kernel(ValuParams p, int wk_log2, int cols)
+{
+    constexpr int PF = U == 1 ? 8 : (U <= 4 ? 12 / U : (U == 5 ? 2 : (U <= 8 ? 24 / U : 2)));    // columns whose loads are under way
+    extern __shared__ __align__(16) u128 regs_part[];          // [cols][WK]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int WK = 1 << wk_log2, CG = kRegsWaves >> wk_log2, wk = wave & (WK - 1), cg = wave >> wk_log2;
+    const int g = blockIdx.y;
+    const int64_t *Ag = p.A + (long)g * p.sA;
+    const int32_t *Bbase = reinterpret_cast<const int32_t *>(p.B) + (long)g * p.sB;
+    if (GRP) {
+        // the segment that holds row g: the last one that starts at or before it
+        int lo = 0, hi = p.groups - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (p.grp_seg[mid] <= g) lo = mid; else hi = mid - 1;
+        }
+        Bbase = reinterpret_cast<const int32_t *>(p.grp_b[lo]);
+    }
+    const int n0 = blockIdx.x * cols;
+    const int ncols = p.N - n0 < cols ? p.N - n0 : cols;
+    const int units = p.K >> 2;
+
+    int q[U];
+    bool in[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        q[u] = (u * WK + wk) * 64 + lane;
+        in[u] = q[u] < units;
+    }
+    v4i_s b[PF][U];
+    auto load = [&](int c, v4i_s (&dst)[U]) {                 // column n0 + c
+        const ZK_GLOBAL_MEM v4i_s *row = (const ZK_GLOBAL_MEM v4i_s *)(Bbase + (long)(n0 + c) * p.ldbn);
+#pragma unroll
+        for (int u = 0; u < U; u++) dst[u] = in[u] ? __builtin_nontemporal_load(row + q[u]) : v4i_s{ 0, 0, 0, 0 };
+    };
+#pragma unroll
+    for (int s = 0; s < PF; s++)
+        if (cg + s * CG < ncols) load(cg + s * CG, b[s]);
+
+    int x[U][3][4];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        int64_t a[4] = { 0, 0, 0, 0 };
+        if (in[u]) {
+            const longlong2 t0 = *reinterpret_cast<const longlong2 *>(Ag + 4 * (long)q[u]), t1 = *reinterpret_cast<const longlong2 *>(Ag + 4 * (long)q[u] + 2);
+            a[0] = t0.x; a[1] = t0.y; a[2] = t1.x; a[3] = t1.y;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            x[u][0][e] = (int)((uint32_t)a[e] & 0x1FFFFFu);
+            x[u][1][e] = (int)((uint32_t)(a[e] >> 21) & 0x1FFFFFu);
+            x[u][2][e] = (int)(a[e] >> 42);
+        }
+    }
+
+    for (int c0 = cg; c0 < ncols; c0 += PF * CG) {
+#pragma unroll
+        for (int s = 0; s < PF; s++) {
+            const int c = c0 + s * CG;
+            if (c < ncols) {
+                int64_t acc[3] = { 0, 0, 0 };
+#pragma unroll
+                for (int u = 0; u < U; u++)
+#pragma unroll
+                    for (int i = 0; i < 3; i++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) mad_i64(acc[i], x[u][i][e], b[s][u][e]);
+                if (c + PF * CG < ncols) load(c + PF * CG, b[s]);
+                const u128 sum = wave_sum_last((u128)((i128)acc[0] + ((i128)acc[1] << 21) + ((i128)acc[2] << 42)));
+                if (lane == 63) regs_part[c * WK + wk] = sum;
+            }
+        }
+    }
+    __syncthreads();
+    const uint64_t rmask = p.shift ? ((1ull << p.shift) - 1) : 0;
+    for (int c = threadIdx.x; c < ncols; c += 64 * kRegsWaves) {
+        u128 sum = (u128)(i128)p.init;
+        for (int w = 0; w < WK; w++) sum += regs_part[c * WK + w];
+        const long o = (long)g * p.sC + n0 + c;
+        p.C[o] = (int64_t)(uint64_t)((i128)sum >> p.shift);
+        if (p.R) p.R[o] = (int64_t)((uint64_t)sum & rmask);
+    }
+}
+
 static int device_cus()
 {
     static int cus = 0;
@@ -475,19 +603,55 @@ static int device_cus()
     return cus;
 }
 
-// Launches the staged kernel if the product is one it takes: one or two rows (per batch or segment row), int32 weights,
+// Launches the register or the staged kernel if the product is one they take: one or two rows (per batch or segment row), int32 weights,
 // no divisors, K a multiple of four up to kStagedMaxK, 16-byte aligned rows, and enough columns for a workgroup per
 // compute unit (a narrower output is better served by waves that share a column along K).
+// One row (per batch or segment row), int32 weights, no divisors, K a multiple of four up to 18432, 16-byte aligned rows.
+template <bool GRP>
+static bool gemv32_regs_launch(const ValuParams &p, long rows, int cus)
+{
+    const int units = p.K / 4;
+    if (p.K % 4 != 0 || p.K < 128 || p.M != 1 || rows > 65535 || units > 64 * kRegsWaves * kRegsMaxUnits) return false;
+    int wk = 0;
+    while (wk < 3 && units > (256 << wk)) wk++;                       // at most four units per lane while wavefronts are left
+    const long total = (long)p.N * rows;
+    while (wk < 3 && units > (64 << wk) && total < (long)cus * (kRegsWaves >> wk)) wk++;      // (few columns: more wavefronts on each)
+    const int cg = kRegsWaves >> wk;
+    // columns per workgroup: whole rounds of the device, at most 64 columns each.  Two workgroups per compute unit once
+    // each has 24 columns left (128 heads [128,512]: 9.1 -> 7.8 us), one below that (1536 columns of 7168: 9.3 -> 8.6).
+    const long wgs = total >= 48L * cus ? 2L * cus : cus;
+    const long rounds = (total + 64L * wgs - 1) / (64L * wgs);
+    long cols = (total + wgs * rounds - 1) / (wgs * rounds);
+    cols = (cols + cg - 1) / cg * cg;
+    const dim3 grid((unsigned)((p.N + cols - 1) / cols), (unsigned)rows);
+    const size_t lds = (size_t)cols << (wk + 4);
+    const int u = (units + (64 << wk) - 1) / (64 << wk);
+#define ZK_REGS(U_) case U_: gemv32_regs_kernel<U_, GRP><<<grid, dim3(64 * kRegsWaves), lds, 0>>>(p, wk, (int)cols); return true
+    switch (u) {
+    ZK_REGS(1);
+    ZK_REGS(2);
+    ZK_REGS(3);
+    ZK_REGS(4);
+    ZK_REGS(5);
+    ZK_REGS(6);
+    ZK_REGS(7);
+    ZK_REGS(8);
+    ZK_REGS(9);
+    }
+#undef ZK_REGS
+    return false;
+}
+
 template <bool GRP>
 static bool gemv32_staged_launch(ValuParams p, long rows, int cus)
 {
+    if (gemv32_regs_launch<GRP>(p, rows, cus)) return true;
     if (p.K % 4 != 0 || p.K > kStagedMaxK || p.K < 256 || rows > 65535 || p.M < 1 || p.M > 2) return false;
     const long wg1 = ((p.N + kStagedWaves - 1) / kStagedWaves) * rows;
     if (wg1 < cus) return false;
     p.chunk = p.K < kStagedChunk / p.M ? p.K : kStagedChunk / p.M;      // 48 KB of LDS: three workgroups per compute unit
     const size_t lds = (size_t)3 * p.M * p.chunk * sizeof(int32_t);
-    // more columns per wave (the staging is shared by more of them) while that leaves two workgroups per compute unit
-    const long wg4 = ((p.N + 4 * kStagedWaves - 1) / (4 * kStagedWaves)) * rows;
+    // two columns per wave (the staging is shared by more of them) while that leaves two workgroups per compute unit
     const long wg2 = ((p.N + 2 * kStagedWaves - 1) / (2 * kStagedWaves)) * rows;
     auto launch = [&](auto mr_tag, auto cpw_tag) {
         constexpr int MR = decltype(mr_tag)::value, CPW = decltype(cpw_tag)::value;
@@ -499,10 +663,7 @@ static bool gemv32_staged_launch(ValuParams p, long rows, int cus)
     };
     typedef std::integral_constant<int, 1> I1;
     typedef std::integral_constant<int, 2> I2;
-    typedef std::integral_constant<int, 4> I4;
     if (p.M == 2) return wg2 >= 2L * cus ? launch(I2(), I2()) : launch(I2(), I1());
-    if (wg4 >= 2L * cus) return launch(I1(), I4());
-    if (wg2 >= 2L * cus) return launch(I1(), I2());
     return launch(I1(), I1());
 }
 
