@@ -454,6 +454,25 @@ def test_gemm_prepared_weights_pipelined_kernel(K, oracle):
             K.release_weights(Wd)
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("D,C", [(1, 4), (7, 256), (8, 260), (128, 512), (129, 252), (1000, 300), (1024, 12), (24, 42)])
+def test_per_head_weights_read_along_their_columns(K, oracle, M, D, C):
+    """a decoding step's products with n-contiguous int32 weights: fewer rows of B than wavefronts, whole and broken
+    rounds of sixteen rows, column counts around a workgroup's 256 (42: no multiple of four, the element-wise kernel),
+    weights off the 16-byte grid, extreme elements"""
+    rng = np.random.default_rng(D * 1024 + C)
+    H = 3
+    q, w = rand_i64(rng, (1, M, H, D), 62), rng.integers(-(1 << 31), 1 << 31, size=(H, D, C), dtype=np.int64).astype(np.int32)
+    q[0, M - 1, H - 1], w[H - 1, :, C - 1], w[0, :, 0] = -(1 << 63), -(1 << 31), (1 << 31) - 1
+    off = torch.zeros(w.size + 1, dtype=torch.int32, device="cuda")
+    off[1:] = dev(w).flatten()
+    for shift in (0, 30):
+        expected = oracle.einsum_bshd_hdc_bshc(q, w, shift)
+        assert np.array_equal(host(K.einsum_bshd_hdc_bshc(dev(q), dev(w), shift)), expected)
+        assert K.gemm_last_plan()[0] == 1
+        assert np.array_equal(host(K.einsum_bshd_hdc_bshc(dev(q), off[1:].view(H, D, C), shift)), expected)
+
+
 @pytest.mark.parametrize("w32", [False, True])
 @pytest.mark.parametrize("T,Kr", [(1, 8), (40, 3), (300, 4)])
 def test_grouped_bmm_prepared_weights(K, oracle, T, Kr, w32):
