@@ -473,6 +473,27 @@ def test_per_head_weights_read_along_their_columns(K, oracle, M, D, C):
         assert np.array_equal(host(K.einsum_bshd_hdc_bshc(dev(q), off[1:].view(H, D, C), shift)), expected)
 
 
+@pytest.mark.parametrize("E", [1, 9, 256, 257, 1024, 1025])
+@pytest.mark.parametrize("T,Kr", [(1, 1), (1, 8), (51, 5), (32, 8), (257, 1), (70, 4)])
+def test_moe_dispatch_in_one_workgroup_and_in_three_launches(K, oracle, T, Kr, E):
+    """entries and experts around what one workgroup takes: segments, the stable order, positions and the tile table"""
+    idx = np.random.default_rng(T * 8 + Kr + E).integers(0, E, size=(T, Kr), dtype=np.int64)
+    d = K.moe_dispatch(dev(idx), E)
+    seg, tok, pos = oracle.moe_dispatch(idx, E)
+    assert np.array_equal(host(d["seg"]), seg) and np.array_equal(host(d["token"]), tok) and np.array_equal(host(d["pos"]).ravel(), np.asarray(pos).ravel())
+    tiles = [(e, r) for e in range(E) for r in range(int(seg[e]), int(seg[e + 1]), 32)]
+    assert int(d["ntiles"].item()) == len(tiles) and np.array_equal(host(d["tiles"])[:2 * len(tiles)].reshape(-1, 2), np.array(tiles).reshape(-1, 2))
+
+
+@pytest.mark.parametrize("w32", [False, True])
+@pytest.mark.parametrize("M,N,Kd", [(128, 512, 512), (65, 64, 256), (100, 200, 779), (128, 64, 127), (200, 257, 1000), (128, 577, 385)])
+def test_gemm_short_slices_of_small_launches(K, oracle, M, N, Kd, w32):
+    """a launch of a few tiles, cut along K down to 128 k a slice: whole and broken last steps, one slice alone"""
+    rng = np.random.default_rng(M + N + Kd)
+    for bits_a, bits_w in ((20, 16), (20, 28), (27, 28), (36, 30)):
+        _gemm_case(K, oracle, 0, rand_i64(rng, (1, M, Kd), bits_a), (rand_i32 if w32 else rand_i64)(rng, (N, Kd), bits_w), 1, 1, 21)
+
+
 @pytest.mark.parametrize("w32", [False, True])
 @pytest.mark.parametrize("T,Kr", [(1, 8), (40, 3), (300, 4)])
 def test_grouped_bmm_prepared_weights(K, oracle, T, Kr, w32):

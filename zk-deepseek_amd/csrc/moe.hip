@@ -102,6 +102,66 @@ __global__ __launch_bounds__(256) void moe_place_kernel(const int64_t *__restric
     }
 }
 
+// All three steps in one workgroup, for a decoding step's handful of entries (an entry per thread) and experts that fit
+// LDS: what the three launches cost is their launches.  256 experts, 8 or 256
+// entries: 20.6 -> 15.8 us a call.
+constexpr int kMoeSmallEntries = 256, kMoeSmallExperts = 1024;
+__global__ __launch_bounds__(256) void moe_dispatch_small_kernel(const int64_t *__restrict__ indices, int entries, int K, int E, int *__restrict__ counts,
+                                                                 int *__restrict__ seg, int *__restrict__ tiles, int *__restrict__ ntiles,
+                                                                 int *__restrict__ sorted_token, int *__restrict__ sorted_pos, int *bad_host)
+{
+    __shared__ int count[kMoeSmallExperts], first[kMoeSmallExperts], expert[kMoeSmallEntries], wave_sum[2][4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int e = tid; e < E; e += 256) count[e] = 0;
+    const int64_t idx = tid < entries ? indices[tid] : -1;
+    const bool valid = idx >= 0 && idx < (int64_t)E;
+    const int mine = valid ? (int)idx : -1;
+    expert[tid] = mine;
+    __syncthreads();
+    if (valid) atomicAdd(&count[mine], 1);
+    __syncthreads();
+    int rows = 0, tile_count = 0;                  // of the rounds before this one
+    for (int e0 = 0; e0 < E; e0 += 256) {
+        const int e = e0 + tid;
+        const int c = e < E ? count[e] : 0, t = (c + 31) >> 5;
+        int pc = c, pt = t;                        // inclusive prefix sums over the wave
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int vc = __shfl_up(pc, off, 64), vt = __shfl_up(pt, off, 64);
+            if (lane >= off) { pc += vc; pt += vt; }
+        }
+        if (lane == 63) { wave_sum[0][wave] = pc; wave_sum[1][wave] = pt; }
+        __syncthreads();
+        int row = rows + pc - c, tile = tile_count + pt - t;
+        for (int w = 0; w < 4; w++) {
+            if (w < wave) { row += wave_sum[0][w]; tile += wave_sum[1][w]; }
+            rows += wave_sum[0][w];
+            tile_count += wave_sum[1][w];
+        }
+        if (e < E) {
+            counts[e] = c;
+            seg[e] = first[e] = row;
+            for (int i = 0; i < t; i++) { tiles[2 * (tile + i)] = e; tiles[2 * (tile + i) + 1] = row + 32 * i; }
+        }
+        __syncthreads();
+    }
+    if (tid == 0) {
+        seg[E] = rows;
+        ntiles[0] = tile_count;
+        if (rows != entries && bad_host) *bad_host = 1;
+    }
+    // entries outside [0, E): as in the kernels above
+    if (tid >= rows && tid < entries) sorted_token[tid] = 0;
+    if (tid >= entries) return;
+    int r = 0;
+    if (valid) {
+        r = first[mine];
+        for (int i = 0; i < tid; i++) r += expert[i] == mine ? 1 : 0;      // (earlier entries first: a stable partition)
+        sorted_token[r] = tid / K;
+    }
+    sorted_pos[tid] = r;
+}
+
 struct __attribute__((aligned(16))) i64x2m { int64_t x, y; };
 
 // out[r][:] = x[token[r]][:]
@@ -150,6 +210,12 @@ void moe_dispatch(const int64_t *indices, int T, int K, int E, int *counts_scrat
     }
     if (E > 65535) { zk::set_error(zk::kUnsupportedSize, "%s: more than 65535 experts", name); return; }
     const long entries = (long)T * K;
+    if (entries <= zk::kMoeSmallEntries && E <= zk::kMoeSmallExperts) {
+        zk::moe_dispatch_small_kernel<<<dim3(1), dim3(256), 0, 0>>>(indices, (int)entries, K, E, counts_scratch, seg, tiles, ntiles, sorted_token, sorted_pos,
+                                                                    zk::deferred_error_flag(zk::kDeferredMoeIndex));
+        zk::check_launch(name);
+        return;
+    }
     zk::moe_count_kernel<<<dim3((unsigned)E), dim3(256), 0, 0>>>(indices, entries, counts_scratch);
     zk::moe_scan_kernel<<<dim3(1), dim3(256), 0, 0>>>(counts_scratch, E, seg, tiles, ntiles, entries, sorted_token,
                                                       zk::deferred_error_flag(zk::kDeferredMoeIndex));
