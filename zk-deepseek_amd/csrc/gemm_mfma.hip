@@ -27,6 +27,7 @@
 #include "gemm_mfma_kernels.h"
 #include "gemm_mfma_pipe.h"
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <set>
@@ -712,7 +713,14 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         // slices of K per tile of a launch smaller than the device
         int small_split = total < g_cache.cus ? (int)(g_cache.cus / total) : 1;
         if (small_split > 64) small_split = 64;
-        if (small_split > steps / 4) small_split = steps / 4;
+        // At least four steps a slice: every one more leaves a tile of partial sums to write and to read (100 rows x
+        // [1000,2048] int32: eight slices of 16 tiles 25.7 us, sixteen 33.5; 300 x [600,1536] six of 30 24.2, eight 29.0).
+        // While all of that stays small (64 workgroups), down to 128 k: the launch is then as long as one slice.  128 rows
+        // against a cache of 779: scores 19.5 -> 18.4 us, values 23.9 -> 19.7; of 64: 18.4 -> 15.3; 128 x [512,512] int64
+        // 18.6 -> 17.1.
+        int most_slices = steps / 4;
+        if (total * most_slices < 64) most_slices = (int)std::max<long>(most_slices, std::min<long>(steps * inst->kk / 4, 64 / total));
+        if (small_split > most_slices) small_split = most_slices;
         // A is pre-split into digit planes when enough column tiles reuse it to pay for the extra pass (never for the
         // 32-row tiles: splitting a handful of rows on the fly is cheaper than another kernel in front; nor where the
         // slices of a small launch are so short that the launch in front costs more than three bytes instead of eight per
