@@ -931,9 +931,9 @@ int gemm_mfma_grouped(const GroupedDesc &d, int *limbs_a, int *limbs_b)
     if (!nb) nb = 5;
     // Both digit counts come from what these weights met before: speculate, do not wait.  A guarded launch of the
     // 16-row kernels follows on the stream (they guess nothing and take every operand); its workgroups return at once
-    // unless the verdict is bad, in which case they compute every output again.  What the kernels saw travels to pinned
-    // host memory behind an event and reaches the cache at a later call.  Otherwise (first sight of the weights, no
-    // free slot) the verdict is read back before the call returns, as it used to be for every grouped launch.
+    // unless the verdict is bad, in which case they compute every output again.  What the kernels saw is
+    // stored to pinned host memory by the guarded launch and reaches the cache at a later call.  Otherwise (first sight
+    // of the weights) the verdict is read back before the call returns.
     bool speculate = informed && g_cache.pinned && !g_switches.sync_verdict;
 
     for (int attempt = 0; attempt < 3; attempt++) {
