@@ -391,6 +391,21 @@ def test_gemm_one_row_held_in_registers(K, oracle, Kd):
         assert np.array_equal(host(C), Ce) and np.array_equal(host(R), Re)
 
 
+@pytest.mark.parametrize("Kd", [128, 130, 258, 386, 1022, 2050, 4098, 5122, 7168, 8190, 8192, 8194])
+def test_gemm_one_row_against_int64_weights(K, oracle, Kd):
+    """one row held in registers, int64 weights: every count of 16-byte units per lane (one to eight, and the first K beyond),
+    the fewest columns it takes and one fewer, batches, divisors of B; the whole range of both types"""
+    rng = np.random.default_rng(Kd)
+    least = min(16384, (1 << 24) // Kd + ((1 << 24) % Kd != 0))
+    for Bd, N in ((1, least - 1), (1, least), (2, least // 2 + 3)):
+        A = rand_i64(rng, (Bd, 1, Kd), 63)
+        W = rand_i64(rng, (N, Kd), 63)
+        A[0, 0, :3], W[N - 1, :3], W[0, Kd - 1] = [-(1 << 63), (1 << 63) - 1, 1 << 42], -(1 << 63), (1 << 63) - 1
+        for b_rs, c in ((1, 0), (256, 43)):
+            _gemm_case(K, oracle, 0, A, W, 1, b_rs, c)
+            assert K.gemm_last_plan()[0] == 1
+
+
 @pytest.mark.parametrize("bits_w", [16, 28, 36, 63, -16, -30, -31])
 def test_gemm_prepared_weights(K, oracle, bits_w):
     """int64 weights split into digit planes once (zk_gemm_prepare_weights): the same bits as the unprepared call on

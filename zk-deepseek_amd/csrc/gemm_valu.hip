@@ -592,6 +592,88 @@ __global__ __launch_bounds__(64 * kRegsWaves) void gemv32_regs_kernel(ValuParams
     }
 }
 
+// The same against int64 weights, whose power-of-two divisor (the head's 256) is applied to what has been loaded: units of
+// two elements, full 128-bit multiply-adds.  A unit's register is loaded again as soon as it has been multiplied, so the
+// stream never pauses; what bounds it is that stream.  gemv_kernel's eight loads per wavefront all drain before the next
+// column begins: [129280,7168] 1233 -> 1092 us (6.8 TB/s; with the divisor 1276 -> 1115), [18432,7168] 182 -> 165, [8192,8192]
+// 98.8 -> 83.9, [16384,1536] 38.5 -> 36.3, [24576,512] 26.4 -> 20.8.  Eight units of A per lane at most (K = 8192), which take
+// the 128 registers of two workgroups per compute unit; with a whole column loaded at a time 104 of them were spilled.
+constexpr int kRegs64MaxUnits = 8;
+
+template <int U, bool RESCALE>
+__global__ __launch_bounds__(64 * kRegsWaves, 4) void gemv64_regs_kernel(ValuParams p, int wk_log2, int cols)
+{
+    constexpr int PF = U == 1 ? 8 : (U <= 3 ? 8 / U : (U == 4 ? 2 : 1));     // columns whose loads are under way
+    extern __shared__ __align__(16) u128 regs_part[];          // [cols][WK]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int WK = 1 << wk_log2, CG = kRegsWaves >> wk_log2, wk = wave & (WK - 1), cg = wave >> wk_log2;
+    const int g = blockIdx.y;
+    const int64_t *Ag = p.A + (long)g * p.sA;
+    const int64_t *Bbase = reinterpret_cast<const int64_t *>(p.B) + (long)g * p.sB;
+    const int n0 = blockIdx.x * cols;
+    const int ncols = p.N - n0 < cols ? p.N - n0 : cols;
+    const int units = p.K >> 1;
+
+    int q[U];
+    bool in[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        q[u] = (u * WK + wk) * 64 + lane;
+        in[u] = q[u] < units;
+    }
+    v2l_g b[PF][U];
+    auto load = [&](int c, int u, bool more) {                 // column n0 + c
+        const ZK_GLOBAL_MEM v2l_g *row = (const ZK_GLOBAL_MEM v2l_g *)(Bbase + (long)(n0 + c) * p.ldbn);
+        return more && in[u] ? __builtin_nontemporal_load(row + q[u]) : v2l_g{ 0, 0 };
+    };
+#pragma unroll
+    for (int s = 0; s < PF; s++)
+        if (cg + s * CG < ncols)
+#pragma unroll
+            for (int u = 0; u < U; u++) b[s][u] = load(cg + s * CG, u, true);
+
+    int64_t a[U][2];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        a[u][0] = a[u][1] = 0;
+        if (in[u]) {
+            const longlong2 t = *reinterpret_cast<const longlong2 *>(Ag + 2 * (long)q[u]);
+            a[u][0] = t.x; a[u][1] = t.y;
+        }
+    }
+
+    for (int c0 = cg; c0 < ncols; c0 += PF * CG) {
+#pragma unroll
+        for (int s = 0; s < PF; s++) {
+            const int c = c0 + s * CG;
+            if (c < ncols) {
+                u128 acc = 0;
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        int64_t w = b[s][u][e];
+                        if (RESCALE) w = rescale_operand(w, p.b_rs, p.b_shift);
+                        acc += (u128)((i128)a[u][e] * (i128)w);
+                    }
+                    b[s][u] = load(c + PF * CG, u, c + PF * CG < ncols);
+                }
+                const u128 sum = wave_sum_last(acc);
+                if (lane == 63) regs_part[c * WK + wk] = sum;
+            }
+        }
+    }
+    __syncthreads();
+    const uint64_t rmask = p.shift ? ((1ull << p.shift) - 1) : 0;
+    for (int c = threadIdx.x; c < ncols; c += 64 * kRegsWaves) {
+        u128 sum = (u128)(i128)p.init;
+        for (int w = 0; w < WK; w++) sum += regs_part[c * WK + w];
+        const long o = (long)g * p.sC + n0 + c;
+        p.C[o] = (int64_t)(uint64_t)((i128)sum >> p.shift);
+        if (p.R) p.R[o] = (int64_t)((uint64_t)sum & rmask);
+    }
+}
+
 static int device_cus()
 {
     static int cus = 0;
@@ -607,11 +689,9 @@ static int device_cus()
 // no divisors, K a multiple of four up to kStagedMaxK, 16-byte aligned rows, and enough columns for a workgroup per
 // compute unit (a narrower output is better served by waves that share a column along K).
 // One row (per batch or segment row), int32 weights, no divisors, K a multiple of four up to 18432, 16-byte aligned rows.
-template <bool GRP>
-static bool gemv32_regs_launch(const ValuParams &p, long rows, int cus)
+struct RegsPlan { int wk, u; long cols; dim3 grid; size_t lds; };
+static RegsPlan regs_plan(const ValuParams &p, int units, long rows, int cus)
 {
-    const int units = p.K / 4;
-    if (p.K % 4 != 0 || p.K < 128 || p.M != 1 || rows > 65535 || units > 64 * kRegsWaves * kRegsMaxUnits) return false;
     int wk = 0;
     while (wk < 3 && units > (256 << wk)) wk++;                       // at most four units per lane while wavefronts are left
     const long total = (long)p.N * rows;
@@ -623,11 +703,17 @@ static bool gemv32_regs_launch(const ValuParams &p, long rows, int cus)
     const long rounds = (total + 64L * wgs - 1) / (64L * wgs);
     long cols = (total + wgs * rounds - 1) / (wgs * rounds);
     cols = (cols + cg - 1) / cg * cg;
-    const dim3 grid((unsigned)((p.N + cols - 1) / cols), (unsigned)rows);
-    const size_t lds = (size_t)cols << (wk + 4);
-    const int u = (units + (64 << wk) - 1) / (64 << wk);
-#define ZK_REGS(U_) case U_: gemv32_regs_kernel<U_, GRP><<<grid, dim3(64 * kRegsWaves), lds, 0>>>(p, wk, (int)cols); return true
-    switch (u) {
+    return RegsPlan{ wk, (units + (64 << wk) - 1) / (64 << wk), cols, dim3((unsigned)((p.N + cols - 1) / cols), (unsigned)rows), (size_t)cols << (wk + 4) };
+}
+
+template <bool GRP>
+static bool gemv32_regs_launch(const ValuParams &p, long rows, int cus)
+{
+    const int units = p.K / 4;
+    if (p.K % 4 != 0 || p.K < 128 || p.M != 1 || rows > 65535 || units > 64 * kRegsWaves * kRegsMaxUnits) return false;
+    const RegsPlan r = regs_plan(p, units, rows, cus);
+#define ZK_REGS(U_) case U_: gemv32_regs_kernel<U_, GRP><<<r.grid, dim3(64 * kRegsWaves), r.lds, 0>>>(p, r.wk, (int)r.cols); return true
+    switch (r.u) {
     ZK_REGS(1);
     ZK_REGS(2);
     ZK_REGS(3);
@@ -637,6 +723,35 @@ static bool gemv32_regs_launch(const ValuParams &p, long rows, int cus)
     ZK_REGS(7);
     ZK_REGS(8);
     ZK_REGS(9);
+    }
+#undef ZK_REGS
+    return false;
+}
+
+// One row against int64 weights, B's divisor a power of two (or 1), K even up to 8192, 16-byte aligned rows; a matrix of 2^24
+// weights or 16384 columns and more.  Below that a workgroup has too few columns for the stream to make up for the load of
+// A in front and the meeting of the wavefronts behind: gemv_kernel against this, [576,7168] 10.0 / 10.9 us, [7168,2048] 22.3 /
+// 24.0, [8192,1536] 22.1 / 22.3, [2048,7168] 24.7 / 24.0, [4096,4096] 26.1 / 26.0.
+constexpr long kRegs64MinWeights = 1L << 24, kRegs64MinColumns = 16384;
+static bool gemv64_regs_launch(const ValuParams &p, long rows, int cus)
+{
+    const int units = p.K / 2;
+    if (p.K % 2 != 0 || p.K < 128 || p.M != 1 || rows > 65535 || units > 64 * kRegsWaves * kRegs64MaxUnits) return false;
+    if (p.a_rs != 1 || p.b_shift < 0) return false;
+    if ((long)p.N * rows < kRegs64MinColumns && (long)p.N * p.K * rows < kRegs64MinWeights) return false;
+    const RegsPlan r = regs_plan(p, units, rows, cus);
+#define ZK_REGS(U_) case U_: if (p.b_shift) gemv64_regs_kernel<U_, true><<<r.grid, dim3(64 * kRegsWaves), r.lds, 0>>>(p, r.wk, (int)r.cols); \
+                             else gemv64_regs_kernel<U_, false><<<r.grid, dim3(64 * kRegsWaves), r.lds, 0>>>(p, r.wk, (int)r.cols);          \
+                             return true
+    switch (r.u) {
+    ZK_REGS(1);
+    ZK_REGS(2);
+    ZK_REGS(3);
+    ZK_REGS(4);
+    ZK_REGS(5);
+    ZK_REGS(6);
+    ZK_REGS(7);
+    ZK_REGS(8);
     }
 #undef ZK_REGS
     return false;
@@ -846,6 +961,7 @@ bool gemm_gemv_launch(const GemmDesc &d)
         return true;
     }
     if (d.b32 && !rescale && p.tiles_m && gemv32_staged_launch<false>(p, d.G, device_cus())) return true;
+    if (!d.b32 && p.tiles_m && gemv64_regs_launch(p, d.G, device_cus())) return true;
 #define ZK_GEMV(B32, RS) do { if (d.M == 1) gemv_launch3<B32, RS, 1>(p, d.G); else gemv_launch3<B32, RS, 2>(p, d.G); } while (0)
     if (d.b32) { if (rescale) ZK_GEMV(true, true); else ZK_GEMV(true, false); }
     else { if (rescale) ZK_GEMV(false, true); else ZK_GEMV(false, false); }
