@@ -38,14 +38,6 @@ __device__ __forceinline__ void static_for(F &&f)
     }
 }
 
-// 1 KB from a base that is the same in every lane (lane l: 16 bytes at base + off, off = 16 l) to LDS byte address `lds`
-__device__ __forceinline__ void lds_dma16_uniform(uint64_t base, unsigned off, unsigned lds)
-{
-    unsigned saved_m0;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved_m0) : "s"(lds), "v"(off), "s"(base) : "memory");
-}
-
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ uint64_t uniform64(uint64_t v)
 {

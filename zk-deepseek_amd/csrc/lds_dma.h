@@ -15,9 +15,21 @@ __device__ __forceinline__ void lds_dma16(const void *gptr, unsigned lds_base)
     // (the base is the same in every lane, but derived from the wavefront's number, which the compiler holds in a vector register)
     // M0 is put back as it was: the compiler does not see the statement write it (the register cannot be named as
     // clobbered) and may be keeping a value of its own there across the statement.
+    // s_nop: a load into LDS may read M0 one wait state after a scalar instruction wrote it at the earliest, and the
+    // hardware does not check (the compiler adds this wait to its own code, not inside a statement like this one).
     unsigned saved_m0;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
                  : "=&s"(saved_m0) : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(gptr) : "memory");
+}
+
+// 1 KB from a base that is the same in every lane (lane l: 16 bytes at base + off, off = 16 l) to LDS byte address `lds`.
+// s_nop: as above, and `base` may come from a vector instruction (v_readfirstlane) directly in front of the statement: a
+// load may read such a scalar register five wait states later, two of which the moves are.
+__device__ __forceinline__ void lds_dma16_uniform(uint64_t base, unsigned off, unsigned lds)
+{
+    unsigned saved_m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 2\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved_m0) : "s"(lds), "v"(off), "s"(base) : "memory");
 }
 
 template <int N>
