@@ -469,10 +469,19 @@ def test_gemm_prepared_weights_pipelined_kernel(K, oracle):
             K.release_weights(Wd)
 
 
+@pytest.mark.parametrize("S,D", [(1, 1), (1, 63), (1, 64), (1, 65), (2, 64), (2, 95), (2, 96), (2, 97)])
+def test_per_head_weights_around_the_shortest_k_of_the_wide_loads(K, oracle, S, D):
+    """one and two rows against n-contiguous int32 weights on either side of the K from which the wide loads are taken, more
+    column blocks than compute units"""
+    rng = np.random.default_rng(100 * S + D)
+    q, w = rand_i64(rng, (1, S, 75, D), 63), rand_i32(rng, (75, D, 928), 31)
+    assert np.array_equal(host(K.einsum_bshd_hdc_bshc(dev(q), dev(w), 30)), oracle.einsum_bshd_hdc_bshc(q, w, 30))
+
+
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
 @pytest.mark.parametrize("D,C", [(1, 4), (7, 256), (8, 260), (128, 512), (129, 252), (1000, 300), (1024, 12), (24, 42)])
 def test_per_head_weights_read_along_their_columns(K, oracle, M, D, C):
-    """a decoding step's products with n-contiguous int32 weights: fewer rows of B than wavefronts, whole and broken
+    """a decoding step's products with n-contiguous int32 weights: a short K (the element-wise kernel), whole and broken
     rounds of sixteen rows, column counts around a workgroup's 256 (42: no multiple of four, the element-wise kernel),
     weights off the 16-byte grid, extreme elements"""
     rng = np.random.default_rng(D * 1024 + C)
