@@ -406,6 +406,24 @@ def test_gemm_one_row_against_int64_weights(K, oracle, Kd):
             assert K.gemm_last_plan()[0] == 1
 
 
+@pytest.mark.parametrize("w32", [False, True])
+@pytest.mark.parametrize("Bd,N", [(2, 8200), (3, 1536), (20, 63), (20, 64), (20, 900), (64, 2), (64, 257), (257, 70), (1000, 65)])
+def test_gemm_one_row_per_batch_against_shared_weights(K, oracle, Bd, N, w32):
+    """batches of one row against the same weights, held in registers: the workgroups of a row dealt out over the device
+    (fewer and more rows than compute units, rounds that do not come out even, workgroups without columns)"""
+    rng = np.random.default_rng(Bd * 10000 + N)
+    oracle.set_threads(oracle.max_threads())
+    try:
+        for Kd in (130, 2052) if Bd < 257 else (132,):
+            A = rand_i64(rng, (Bd, 1, Kd), 63)
+            W = rand_i32(rng, (N, Kd), 31) if w32 else rand_i64(rng, (N, Kd), 63)
+            for b_rs in (1,) if w32 else (1, 256):
+                _gemm_case(K, oracle, 0, A, W, 1, b_rs, 30)
+                assert K.gemm_last_plan()[0] == 1
+    finally:
+        oracle.set_threads(1)
+
+
 @pytest.mark.parametrize("bits_w", [16, 28, 36, 63, -16, -30, -31])
 def test_gemm_prepared_weights(K, oracle, bits_w):
     """int64 weights split into digit planes once (zk_gemm_prepare_weights): the same bits as the unprepared call on

@@ -528,6 +528,7 @@ __global__ __launch_bounds__(64 * kRegsWaves) void gemv32_regs_kernel(ValuParams
     }
     const int n0 = blockIdx.x * cols;
     const int ncols = p.N - n0 < cols ? p.N - n0 : cols;
+    if (ncols <= 0) return;
     const int units = p.K >> 2;
 
     int q[U];
@@ -612,6 +613,7 @@ __global__ __launch_bounds__(64 * kRegsWaves, 4) void gemv64_regs_kernel(ValuPar
     const int64_t *Bbase = reinterpret_cast<const int64_t *>(p.B) + (long)g * p.sB;
     const int n0 = blockIdx.x * cols;
     const int ncols = p.N - n0 < cols ? p.N - n0 : cols;
+    if (ncols <= 0) return;
     const int units = p.K >> 1;
 
     int q[U];
@@ -685,33 +687,44 @@ static int device_cus()
     return cus;
 }
 
-// Launches the register or the staged kernel if the product is one they take: one or two rows (per batch or segment row), int32 weights,
-// no divisors, K a multiple of four up to kStagedMaxK, 16-byte aligned rows, and enough columns for a workgroup per
-// compute unit (a narrower output is better served by waves that share a column along K).
-// One row (per batch or segment row), int32 weights, no divisors, K a multiple of four up to 18432, 16-byte aligned rows.
+// How a launch of the register kernels is cut: WK = 2^wk wavefronts along K, u units of K per lane, `cols` columns per workgroup.
 struct RegsPlan { int wk, u; long cols; dim3 grid; size_t lds; };
-static RegsPlan regs_plan(const ValuParams &p, int units, long rows, int cus)
+static RegsPlan regs_plan(const ValuParams &p, int units, long rows, bool shared_b, int two_fit, int cus)
 {
     int wk = 0;
     while (wk < 3 && units > (256 << wk)) wk++;                       // at most four units per lane while wavefronts are left
     const long total = (long)p.N * rows;
     while (wk < 3 && units > (64 << wk) && total < (long)cus * (kRegsWaves >> wk)) wk++;      // (few columns: more wavefronts on each)
     const int cg = kRegsWaves >> wk;
-    // columns per workgroup: whole rounds of the device, at most 64 columns each.  Two workgroups per compute unit once
+    // Columns per workgroup: whole rounds of the device, at most 64 columns each.  Two workgroups per compute unit once
     // each has 24 columns left (128 heads [128,512]: 9.1 -> 7.8 us), one below that (1536 columns of 7168: 9.3 -> 8.6).
-    const long wgs = total >= 48L * cus ? 2L * cus : cus;
-    const long rounds = (total + 64L * wgs - 1) / (64L * wgs);
-    long cols = (total + wgs * rounds - 1) / (wgs * rounds);
+    // A workgroup has columns of one row only (of its own B), so the rounds are filled row by row: with the columns of
+    // all rows dealt out together, three rows of 1536 columns became 3 x 86 workgroups, two more than there are compute
+    // units, and a second round (int32 [1536,7168] 34.2 -> 23.7 us, int64 63.2 -> 46.1).
+    // Rows that share their B have a multiple of eight workgroups each: consecutive workgroups go round the XCDs, so the
+    // same columns of every row then meet in the same L2 (20 batches x [1536,7168] int32 122 -> 78 us,
+    // [2048,7168] 159 -> 105), with two workgroups per compute unit where two fit (`two_fit`: up to that many units per lane).
+    const int u = (units + (64 << wk) - 1) / (64 << wk);
+    const long wgs = (shared_b && rows > 2 && u <= two_fit) || total >= 48L * cus ? 2L * cus : cus;
+    const long eight = shared_b && p.N >= 64 ? 8 : 1;
+    const long least = ((p.N + 63) / 64 + eight - 1) / eight * eight;
+    long rounds = (rows * least + wgs - 1) / wgs;
+    long per_row = wgs * rounds / rows / eight * eight;               // workgroups of a row, at least one per 64 columns
+    if (rows * per_row * 5 < wgs * rounds * 4) { rounds++; per_row = wgs * rounds / rows / eight * eight; }
+    long cols = (p.N + per_row - 1) / per_row;
     cols = (cols + cg - 1) / cg * cg;
-    return RegsPlan{ wk, (units + (64 << wk) - 1) / (64 << wk), cols, dim3((unsigned)((p.N + cols - 1) / cols), (unsigned)rows), (size_t)cols << (wk + 4) };
+    const long groups = ((p.N + cols - 1) / cols + eight - 1) / eight * eight;             // (the last ones may have no columns)
+    return RegsPlan{ wk, u, cols, dim3((unsigned)groups, (unsigned)rows), (size_t)cols << (wk + 4) };
 }
 
+// One row (per batch or segment row), int32 weights, no divisors, K a multiple of four up to 18432, 16-byte
+// aligned rows.
 template <bool GRP>
 static bool gemv32_regs_launch(const ValuParams &p, long rows, int cus)
 {
     const int units = p.K / 4;
     if (p.K % 4 != 0 || p.K < 128 || p.M != 1 || rows > 65535 || units > 64 * kRegsWaves * kRegsMaxUnits) return false;
-    const RegsPlan r = regs_plan(p, units, rows, cus);
+    const RegsPlan r = regs_plan(p, units, rows, GRP ? rows >= 2L * p.groups : rows > 1 && p.sB == 0, 5, cus);
 #define ZK_REGS(U_) case U_: gemv32_regs_kernel<U_, GRP><<<r.grid, dim3(64 * kRegsWaves), r.lds, 0>>>(p, r.wk, (int)r.cols); return true
     switch (r.u) {
     ZK_REGS(1);
@@ -739,7 +752,7 @@ static bool gemv64_regs_launch(const ValuParams &p, long rows, int cus)
     if (p.K % 2 != 0 || p.K < 128 || p.M != 1 || rows > 65535 || units > 64 * kRegsWaves * kRegs64MaxUnits) return false;
     if (p.a_rs != 1 || p.b_shift < 0) return false;
     if ((long)p.N * rows < kRegs64MinColumns && (long)p.N * p.K * rows < kRegs64MinWeights) return false;
-    const RegsPlan r = regs_plan(p, units, rows, cus);
+    const RegsPlan r = regs_plan(p, units, rows, rows > 1 && p.sB == 0, kRegs64MaxUnits, cus);
 #define ZK_REGS(U_) case U_: if (p.b_shift) gemv64_regs_kernel<U_, true><<<r.grid, dim3(64 * kRegsWaves), r.lds, 0>>>(p, r.wk, (int)r.cols); \
                              else gemv64_regs_kernel<U_, false><<<r.grid, dim3(64 * kRegsWaves), r.lds, 0>>>(p, r.wk, (int)r.cols);          \
                              return true
@@ -757,6 +770,9 @@ static bool gemv64_regs_launch(const ValuParams &p, long rows, int cus)
     return false;
 }
 
+// Launches the register or the staged kernel if the product is one they take: one or two rows (per batch or segment row), int32 weights,
+// no divisors, K a multiple of four up to kStagedMaxK, 16-byte aligned rows, and for the staged kernel enough columns for a
+// workgroup per compute unit (a narrower output is better served by waves that share a column along K).
 template <bool GRP>
 static bool gemv32_staged_launch(ValuParams p, long rows, int cus)
 {
@@ -766,7 +782,8 @@ static bool gemv32_staged_launch(ValuParams p, long rows, int cus)
     if (wg1 < cus) return false;
     p.chunk = p.K < kStagedChunk / p.M ? p.K : kStagedChunk / p.M;      // 48 KB of LDS: three workgroups per compute unit
     const size_t lds = (size_t)3 * p.M * p.chunk * sizeof(int32_t);
-    // two columns per wave (the staging is shared by more of them) while that leaves two workgroups per compute unit
+    // two columns per wave (the staging is shared by both) while that leaves two workgroups per compute unit; for one row,
+    // which comes here only beyond the register kernel's K, it makes no difference ([7168,32768] 156 us with one, two or four)
     const long wg2 = ((p.N + 2 * kStagedWaves - 1) / (2 * kStagedWaves)) * rows;
     auto launch = [&](auto mr_tag, auto cpw_tag) {
         constexpr int MR = decltype(mr_tag)::value, CPW = decltype(cpw_tag)::value;
