@@ -26,6 +26,7 @@
 // Results never depend on the guess, and a call whose operands were seen before never blocks the host.
 #include "gemm_mfma_kernels.h"
 #include "gemm_mfma_pipe.h"
+#include "report_ring.h"
 
 #include <algorithm>
 #include <map>
@@ -107,12 +108,10 @@ static const Instance *smaller_tiles(const Instance *inst, const GemmDesc &d, in
 
 typedef std::tuple<const void *, long, long, int> OperandKey;     // (pointer, rows, K, element size)
 
-// Digit counts on their way from the device to the host behind the stream (calls that do not wait for their verdict).
+// Whose digit counts are on their way from the device to the host behind the stream (calls that do not wait for their verdict).
 struct PendingRange {
     OperandKey key_a, key_b;
     int nb_fixed = 0;                        // B came from prepared planes with this many digits (nothing of it was tracked)
-    unsigned seq = 0;                        // the call's number: its report has arrived when all its pinned words carry it
-    int parts = 1;
 };
 
 constexpr unsigned kPendingSlots = 256;      // (a host this many calls ahead of the device skips the report, not the check)
@@ -135,10 +134,7 @@ struct RangeCache {
     int *row_steps = nullptr;                // per row tile of A: its steps up to the last one that is not all zeros
     size_t row_steps_count = 0;
     int cus = 0;                             // compute units of the device
-    PendingRange pending[kPendingSlots];
-    volatile unsigned long long *pinned = nullptr;      // kGuardParts words per slot
-    unsigned pending_head = 0, pending_tail = 0;        // slots used and drained so far, in ring order; head - tail are on their way
-    unsigned seq = 0;
+    ReportRing<PendingRange, kPendingSlots, kGuardParts> reports;       // its words are pinned memory; without any, calls wait
     long guard_hits = 0;                     // calls whose speculation failed after they had returned
     int lookup(const OperandKey &k)
     {
@@ -229,16 +225,13 @@ static bool read_range(unsigned long long *dev, int64_t (&out)[4])
     return true;
 }
 
-// Takes in the reports that have arrived since the last call, oldest first (the stream delivers them in that order).
+// Takes in the reports that have arrived since the last call.
 static void drain_pending()
 {
-    while (g_cache.pending_tail != g_cache.pending_head) {
-        const PendingRange &s = g_cache.pending[g_cache.pending_tail % kPendingSlots];
-        const volatile unsigned long long *words = g_cache.pinned + (size_t)(g_cache.pending_tail % kPendingSlots) * kGuardParts;
+    g_cache.reports.drain([](const PendingRange &s, const volatile unsigned long long *words, int parts) {
         int na = 0, nb = 0, verdict = 0;
-        for (int i = 0; i < s.parts; i++) {
+        for (int i = 0; i < parts; i++) {
             const unsigned long long w = words[i];
-            if ((unsigned)(w >> 32) != s.seq) return;
             na = (int)(w & 0xFF) > na ? (int)(w & 0xFF) : na;
             nb = (int)(w >> 8 & 0xFF) > nb ? (int)(w >> 8 & 0xFF) : nb;
             verdict |= (int)(w >> 16 & 0xFF);
@@ -247,8 +240,7 @@ static void drain_pending()
         else if (s.nb_fixed) g_cache.store_pair(s.key_a, na ? na : 1, s.key_b, s.nb_fixed);      // (a grouped launch on prepared planes)
         else g_cache.store(s.key_a, na ? na : 1);        // B came from prepared planes: nothing of it was tracked
         if (verdict) g_cache.guard_hits++;
-        g_cache.pending_tail++;
-    }
+    });
 }
 
 // The guard of the call being launched: its verdict word, the word cleared for the next call, and, while a slot is free,
@@ -261,11 +253,7 @@ static GuardArgs make_guard(long seen_count)
     g.next = words + (g_cache.turn ^ 1);
     g.seen = g_cache.seen;
     g.seen_count = seen_count;
-    if (g_cache.pending_head - g_cache.pending_tail < kPendingSlots) {
-        g.host = const_cast<unsigned long long *>(g_cache.pinned) + (size_t)(g_cache.pending_head % kPendingSlots) * kGuardParts;
-        if (++g_cache.seq == 0) g_cache.seq = 1;
-        g.seq = g_cache.seq;
-    }
+    g.host = g_cache.reports.open(&g.seq);
     return g;
 }
 
@@ -273,13 +261,11 @@ static void guard_taken(const GuardArgs &g, const OperandKey &key_a, const Opera
 {
     g_cache.turn ^= 1;
     if (!g.host) return;
-    PendingRange &s = g_cache.pending[g_cache.pending_head % kPendingSlots];
+    PendingRange s;
     s.key_a = key_a;
     s.key_b = key_b;
     s.nb_fixed = nb_fixed;
-    s.seq = g.seq;
-    s.parts = g.parts;
-    g_cache.pending_head++;
+    g_cache.reports.push(s, g.seq, g.parts);
 }
 
 // Waits for the digits the launch just issued has seen, and clears its verdict word (its caller launches again).
@@ -329,11 +315,11 @@ static bool init_cache()
     // without the pinned words every call simply waits for its own verdict
     void *pinned = nullptr;
     if (hipHostMalloc(&pinned, kPendingSlots * kGuardParts * sizeof(unsigned long long), hipHostMallocDefault) == hipSuccess) {
-        g_cache.pinned = reinterpret_cast<volatile unsigned long long *>(pinned);
-        for (unsigned i = 0; i < kPendingSlots * kGuardParts; i++) g_cache.pinned[i] = 0;
+        volatile unsigned long long *words = reinterpret_cast<volatile unsigned long long *>(pinned);
+        for (unsigned i = 0; i < kPendingSlots * kGuardParts; i++) words[i] = 0;
+        g_cache.reports.words = words;
     } else {
         (void)hipGetLastError();
-        g_cache.pinned = nullptr;
     }
     return true;
 }
@@ -575,6 +561,7 @@ static Outcome launch_guarded_fallback(const GemmDesc &d, const MfmaParams &spec
     }
     if (!fn) {
         gemm_valu_launch(d, guard);
+        if (hipGetLastError() != hipSuccess) { set_error(kLaunchFailure, "gemm: guarded vector-ALU launch failed"); return kFailed; }
         return kDone;
     }
     const size_t lds = 2 * (size_t)wide->kk * ((wide->bm / 32) * wide->na + (wide->bn / 32) * wide->nb) * 1024 + 9 * 1024 + 16;
@@ -647,7 +634,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
     }
     // No call waits for its verdict (unless there is no pinned memory, or ZK_GEMM_SYNC asks for it): a guarded launch
     // behind the product redoes it with digits that cover everything if the verdict is raised.
-    const bool speculate = g_cache.pinned && !g_switches.sync_verdict;
+    const bool speculate = g_cache.reports.words && !g_switches.sync_verdict;
     if (!na || !nb) {
         p.tiles_m = p.tiles_n = 1;
         range_reset_kernel<<<1, 64, 0, 0>>>(p.range);
@@ -934,7 +921,7 @@ int gemm_mfma_grouped(const GroupedDesc &d, int *limbs_a, int *limbs_b)
     // unless the verdict is bad, in which case they compute every output again.  What the kernels saw is
     // stored to pinned host memory by the guarded launch and reaches the cache at a later call.  Otherwise (first sight
     // of the weights) the verdict is read back before the call returns.
-    bool speculate = informed && g_cache.pinned && !g_switches.sync_verdict;
+    bool speculate = informed && g_cache.reports.words && !g_switches.sync_verdict;
 
     for (int attempt = 0; attempt < 3; attempt++) {
         const Instance *inst = nullptr;
