@@ -456,3 +456,72 @@ def test_workspace_is_reported_and_released(K, oracle):
     assert K.workspace_bytes()[0] < scratch
     C, R = K.int64_bmm_broadcast(dA, dW, 1, 1, 29)
     assert np.array_equal(host(C), Ce) and np.array_equal(host(R), Re)
+
+
+@pytest.fixture
+def scratch_limit(K, monkeypatch):
+    """sets the size a scratch buffer may grow to, as if the device had no more memory; what is held is released first"""
+    def set_limit(size):
+        if size is None:
+            monkeypatch.delenv("ZK_SCRATCH_LIMIT", raising=False)
+        else:
+            monkeypatch.setenv("ZK_SCRATCH_LIMIT", str(size))
+        K.lib.zk_reload_env()
+        K.release_workspace()
+    yield set_limit
+    monkeypatch.delenv("ZK_SCRATCH_LIMIT", raising=False)
+    monkeypatch.delenv("ZK_B_ROWS_MIN_MACS", raising=False)
+    K.lib.zk_reload_env()
+
+
+@pytest.mark.parametrize("S,T,C,limit", [(12800, 40, 512, 1 << 20),       # no room for the planes of A
+                                         (385, 40, 12416, 1 << 20)])      # room for the planes of A, none for those of B
+def test_values_without_memory_for_digit_planes(K, oracle, monkeypatch, scratch_limit, S, T, C, limit):
+    """a small n-contiguous B whose product would run on planes of both operands: without memory for them it stays on the
+    MFMA kernels that split both themselves, and leaves nothing behind that the next call trips over"""
+    monkeypatch.setenv("ZK_B_ROWS_MIN_MACS", "1")
+    rng = np.random.default_rng(S)
+    p, v = rand_i64(rng, (1, S, 1, T), 19), rand_i64(rng, (1, T, C), 20)
+    expected = oracle.einsum_bsht_btc_bshc(p, v, 23)
+    dp, dv = torch.from_numpy(p).cuda(), torch.from_numpy(v).cuda()
+    # one element of A does not fit the digits remembered for it: its pre-pass would raise the verdict
+    wide = p.copy()
+    wide[0, S - 1, 0, T - 1] = WIDE
+    for size, on_planes in ((None, 1), (limit, 0), (None, 1)):
+        scratch_limit(size)
+        for _ in range(3):
+            before = K.lib.zk_gemm_pipe_calls()
+            assert np.array_equal(host(K.einsum_bsht_btc_bshc(dp, dv, 23)), expected)
+            assert K.gemm_last_plan()[0] == 2
+        assert K.lib.zk_gemm_pipe_calls() == before + on_planes
+        hits = K.lib.zk_gemm_guard_hits()
+        dp.copy_(torch.from_numpy(wide))
+        assert np.array_equal(host(K.einsum_bsht_btc_bshc(dp, dv, 23)), oracle.einsum_bsht_btc_bshc(wide, v, 23))
+        assert K.lib.zk_gemm_guard_hits() == hits + 1
+        dp.copy_(torch.from_numpy(p))
+        for _ in range(3):
+            assert np.array_equal(host(K.einsum_bsht_btc_bshc(dp, dv, 23)), expected)
+        assert K.lib.zk_gemm_guard_hits() == hits + 1
+
+
+@pytest.mark.parametrize("prepared", [False, True])
+def test_product_without_memory_for_the_planes_of_a(K, oracle, scratch_limit, prepared):
+    """a product whose A would be split by a pass in front (and, with prepared weights, has to be): without memory for the
+    planes both operands are split in the kernel"""
+    rng = np.random.default_rng(5)
+    A, W = rand_i64(rng, (1, 128, 16384), 20), rand_i64(rng, (1024, 16384), 16)
+    expected = oracle.int64_bmm_broadcast(A, W, 1, 1, 29)
+    dA, dW = torch.from_numpy(A).cuda(), torch.from_numpy(W).cuda()
+    if prepared:
+        K.prepare_weights(dW)
+    try:
+        for size in (None, 4 << 20, None):
+            scratch_limit(size)
+            for _ in range(3):
+                C, R = K.int64_bmm_broadcast(dA, dW, 1, 1, 29)
+                assert np.array_equal(host(C), expected[0]) and np.array_equal(host(R), expected[1])
+                assert K.gemm_last_plan()[0] == 2
+            assert K.lib.zk_gemm_last_prepared() == (1 if prepared and size is None else 0)
+    finally:
+        if prepared:
+            K.release_weights(dW)

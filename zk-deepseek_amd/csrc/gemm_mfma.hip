@@ -171,8 +171,8 @@ static RangeCache g_cache;
 // behind a speculative one is always the vector-ALU kernel; ZK_NO_STREAM32: grouped launches on int32 weights keep the general
 // 32-row kernel; ZK_B_ROWS_MIN_MACS: product
 // size from which a B that is small next to it is split into digit planes first; ZK_SKINNY_MAX_M: rows up to
-// which the 32-row tiles are used.
-struct Switches { bool sync_verdict, no_tail_split, valu_fallback, no_stream32, no_pipe; double b_rows_min_macs; int skinny_max_m, planes_min_tiles_n, stream32_min_pairs; };
+// which the 32-row tiles are used; ZK_SCRATCH_LIMIT: bytes a scratch buffer may grow to, as if the device had no more.
+struct Switches { bool sync_verdict, no_tail_split, valu_fallback, no_stream32, no_pipe; double b_rows_min_macs, scratch_limit; int skinny_max_m, planes_min_tiles_n, stream32_min_pairs; };
 constexpr long kBRowsMinMacs = 1L << 30;
 constexpr double kShapeGuessMaxMacs = 17179869184.0;        // 2^34: about 0.15 ms on the matrix pipe
 // Rows up to which a product runs on the 32-row tiles (two of them from 33 rows on): measured against the 128-row tiles,
@@ -190,6 +190,8 @@ static Switches read_switches()
     s.stream32_min_pairs = sp ? atoi(sp) : 16;
     const char *m = getenv("ZK_B_ROWS_MIN_MACS");
     s.b_rows_min_macs = m ? atof(m) : (double)kBRowsMinMacs;
+    const char *sl = getenv("ZK_SCRATCH_LIMIT");
+    s.scratch_limit = sl ? atof(sl) : 1e30;
     const char *sk = getenv("ZK_SKINNY_MAX_M");
     s.skinny_max_m = sk ? atoi(sk) : kSkinnyMaxRows;
     const char *pt = getenv("ZK_PLANES_MIN_TILES_N");
@@ -209,6 +211,7 @@ template <typename T>
 static Outcome grow(T *&buf, size_t &have, size_t need, const char *what)
 {
     if (need <= have) return kDone;
+    if ((double)need * sizeof(T) > g_switches.scratch_limit) return kDeclined;
     if (buf && hipFree(buf) != hipSuccess) { set_error(kLaunchFailure, "gemm: cannot release the %s", what); return kFailed; }
     buf = nullptr;
     have = 0;
@@ -647,6 +650,10 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
     }
     if (prep) { p.B = prep->planes; p.b_nsub = prep->nsub; p.b_ksteps = prep->ksteps; }
 
+    // Everything an attempt allocates is allocated before its first launch: memory that is short for digit planes then
+    // sends the call to the kernels that split both operands themselves (which need none), and nothing it has launched
+    // can have raised the verdict that the next call relies on being clear.
+    bool planes_fit = true;
     for (int attempt = 0; attempt < 3; attempt++) {
         // the stored bits are [shift, shift + 64) of the sum (the remainder lies below them)
         const int need_diag = (d.shift + 64 + 7) / 8;
@@ -669,7 +676,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         PipeForm pipe = {};
         if (prep && !inst->skinny && inst->kk == 1 && !g_switches.no_pipe) pipe = pipe_form(inst->na, inst->nb);
         bool pre_b = false;
-        if (!prep && b_shift == 0 && pipe_b_planes(d, kmajor, b_batches)) {
+        if (planes_fit && !prep && b_shift == 0 && pipe_b_planes(d, kmajor, b_batches)) {
             const Instance *both = pick_instance(na, nb, false, false, need_diag, 0, kB64PlanesBoth);
             const PipeForm f = both ? pipe_form(both->na, both->nb) : PipeForm{};
             const long fewer = both && both->na < both->nb ? both->na : (both ? both->nb : 0);
@@ -715,7 +722,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         // us, 448 (243 x [512,7168]) 35.6 / 39.4, 896 (128 x [2048,7168]) 46.7 / 46.2, 1024 (128 x [7168,2048]) 49.5 /
         // 47.1, 1434 (243 x [1536,7168]) 54.7 / 52.2, 16384 (243 x [7168,16384]) 449 / 353.)
         const bool long_slices = (long)steps * 32 * inst->kk >= 800L * (small_split > 1 ? small_split : 1);
-        const bool use_planes = pre_b || (!kmajor && !inst->skinny && (prep || (p.tiles_n >= g_switches.planes_min_tiles_n && (total >= g_cache.cus || long_slices))));
+        const bool use_planes = pre_b || (planes_fit && !kmajor && !inst->skinny && (prep || (p.tiles_n >= g_switches.planes_min_tiles_n && (total >= g_cache.cus || long_slices))));
         if (b_shift && (kmajor || !inst->skinny)) return kDeclined;
         const int variant = pre_b ? kB64PlanesBoth : prep ? (inst->skinny ? kB64FlyBPlanes : kB64PlanesBoth)
                           : b_shift ? (d.b32 ? kB32FlyRs : kB64FlyRs)
@@ -789,42 +796,54 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         p.fail_class = inst->na > 5 || inst->nb > 5 ? 2 : 1;
         p.verdict = reinterpret_cast<unsigned *>(g_cache.dev + 5) + g_cache.turn;
         p.a_planes = nullptr; p.a_msub = 0; p.a_ksteps = 0;
-        if (use_planes) {
-            const int msub = p.tiles_m * (BM / 32);
-            const size_t need = (size_t)d.G * msub * ksteps * inst->na * 1024;
-            // not enough memory for planes: the caller uses the VALU path
-            if (const Outcome got = grow(g_cache.planes, g_cache.planes_bytes, need, "digit-plane buffer")) return got;
-            p.a_planes = g_cache.planes; p.a_msub = msub; p.a_ksteps = ksteps;
-            const int rows_per_wg = 256 / (4 * inst->kk);
-            const dim3 pgrid((unsigned)(ksteps / inst->kk), (unsigned)((msub * 32 + rows_per_wg - 1) / rows_per_wg), (unsigned)d.G);
-            plane_wgs = (long)pgrid.x * pgrid.y * pgrid.z;
-            const dim3 bgrid((unsigned)ksteps, (unsigned)((d.N + 63) / 64), (unsigned)b_batches);
-            b_plane_wgs = pre_b ? (long)bgrid.x * bgrid.y * bgrid.z : 0;
-            if (const Outcome got = grow(g_cache.seen, g_cache.seen_count, (size_t)(blocks + plane_wgs + b_plane_wgs), "digit counts")) return got;
-            // (the owned-k pattern of the planes of A follows the kernel that reads them: planes of B go with the int64 forms)
-            inst->planes[(d.b32 && !prep && !pre_b) ? 1 : 0]<<<pgrid, dim3(256), 0, 0>>>(p, g_cache.planes, msub, ksteps, g_cache.seen + blocks);
-            if (pre_b) {
-                BPlanesParams b = {};
+        const int msub = p.tiles_m * (BM / 32), rows_per_wg = 256 / (4 * inst->kk);
+        const dim3 pgrid((unsigned)(ksteps / inst->kk), (unsigned)((msub * 32 + rows_per_wg - 1) / rows_per_wg), (unsigned)d.G);
+        const dim3 bgrid((unsigned)ksteps, (unsigned)((d.N + 63) / 64), (unsigned)b_batches);
+        BPlanesParams b = {};
+        {
+            Outcome got = kDone;
+            if (use_planes) {
+                plane_wgs = (long)pgrid.x * pgrid.y * pgrid.z;
+                got = grow(g_cache.planes, g_cache.planes_bytes, (size_t)d.G * msub * ksteps * inst->na * 1024, "digit-plane buffer");
+            }
+            if (pre_b && got == kDone) {
+                b_plane_wgs = (long)bgrid.x * bgrid.y * bgrid.z;
                 b.B = d.B; b.ldn = d.ldbn; b.ldk = d.ldbk; b.sB = d.sB; b.N = d.N; b.K = d.K;
                 b.nsub = (d.N + 31) / 32; b.ksteps = ksteps;
                 b.gstride = (long)b.nsub * ksteps * inst->nb * 1024;
-                if (const Outcome got = grow(g_cache.b_planes, g_cache.b_planes_bytes, (size_t)(b.gstride * b_batches), "digit planes of B")) return got;
-                if (kmajor && !d.b32) {
-                    // (the one product of the model with zeros in A worth finding: a causal prompt's probabilities times the values)
-                    b.row_tiles = (long)p.tiles_m * d.G;
-                    if (const Outcome got = grow(g_cache.row_steps, g_cache.row_steps_count, (size_t)b.row_tiles, "step counts")) return got;
-                    b.row_steps = g_cache.row_steps;
-                    b.a_seen = g_cache.seen + blocks;
-                }
-                b.planes = g_cache.b_planes; b.seen = g_cache.seen + blocks + plane_wgs; b.verdict = p.verdict; b.fail_class = p.fail_class;
+                // (the one product of the model with zeros in A worth finding: a causal prompt's probabilities times the values)
+                b.row_tiles = kmajor && !d.b32 ? (long)p.tiles_m * d.G : 0;
+                got = grow(g_cache.b_planes, g_cache.b_planes_bytes, (size_t)(b.gstride * b_batches), "digit planes of B");
+                if (got == kDone && b.row_tiles) got = grow(g_cache.row_steps, g_cache.row_steps_count, (size_t)b.row_tiles, "step counts");
+            }
+            if (got == kDone) got = grow(g_cache.seen, g_cache.seen_count, (size_t)(blocks + plane_wgs + b_plane_wgs), "digit counts");
+            if (got == kFailed) return kFailed;
+            if (got == kDeclined) {
+                if (!use_planes) return kDeclined;
+                planes_fit = false;
+                prep = nullptr;
+                attempt--;
+                continue;
+            }
+        }
+        if (use_planes) {
+            p.a_planes = g_cache.planes; p.a_msub = msub; p.a_ksteps = ksteps;
+            // (the owned-k pattern of the planes of A follows the kernel that reads them: planes of B go with the int64 forms)
+            inst->planes[(d.b32 && !prep && !pre_b) ? 1 : 0]<<<pgrid, dim3(256), 0, 0>>>(p, g_cache.planes, msub, ksteps, g_cache.seen + blocks);
+        }
+        if (pre_b) {
+            if (b.row_tiles) {
+                b.row_steps = g_cache.row_steps;
+                b.a_seen = g_cache.seen + blocks;
+            }
+            b.planes = g_cache.b_planes; b.seen = g_cache.seen + blocks + plane_wgs; b.verdict = p.verdict; b.fail_class = p.fail_class;
 #define ZK_BPL(NB_) do { if (d.b32) { if (kmajor) b_planes_kernel<NB_, true, true><<<bgrid, 256, 0, 0>>>(b); else b_planes_kernel<NB_, false, true><<<bgrid, 256, 0, 0>>>(b); } \
                          else { if (kmajor) b_planes_kernel<NB_, true, false><<<bgrid, 256, 0, 0>>>(b); else b_planes_kernel<NB_, false, false><<<bgrid, 256, 0, 0>>>(b); } } while (0)
-                if (inst->nb == 3) ZK_BPL(3); else if (inst->nb == 4) ZK_BPL(4); else ZK_BPL(5);
+            if (inst->nb == 3) ZK_BPL(3); else if (inst->nb == 4) ZK_BPL(4); else ZK_BPL(5);
 #undef ZK_BPL
-                p.B = b.planes; p.b_nsub = b.nsub; p.b_ksteps = ksteps; p.b_gstride = d.sB != 0 ? b.gstride : 0;
-                p.row_steps = b.row_steps;
-            }
-        } else if (const Outcome got = grow(g_cache.seen, g_cache.seen_count, (size_t)blocks, "digit counts")) return got;
+            p.B = b.planes; p.b_nsub = b.nsub; p.b_ksteps = ksteps; p.b_gstride = d.sB != 0 ? b.gstride : 0;
+            p.row_steps = b.row_steps;
+        }
         p.seen = pipe.fn ? nullptr : g_cache.seen;
         const size_t lds = pipe.fn ? pipe.lds : 2 * (size_t)inst->kk * ((BM / 32) * inst->na + (BN / 32) * inst->nb) * 1024 + 9 * 1024 + 16;
         static std::set<const void *> lds_raised;
