@@ -523,12 +523,27 @@ void gemm_mfma_release_workspace()
 // rows each) 248 / 310.  n-contiguous B, which the general kernel reads element by element: 512 values of 1024 tokens 1250 /
 // 630 (860 without the causal zeros), of 243 tokens 109 / 68, of 100 tokens 37.7 / 32.5, the heads' int32 weights at 400
 // rows 134 / 132, at 500 169 / 149.
+// Few columns do not pay for the pass over A: 131072 rows x [64,512], (3,3) 167 / 230 us, (4,4) 148 / 236, x [192,512] 243 /
+// 305 and 304 / 345, x [256,512] (3,3) 259 / 308, from 384 columns equal; 64000 x [64,1024] n-contiguous (3,4) 116 / 227,
+// [256,1024] (3,3) 243 / 275; int32 n-contiguous, 500 rows of 128 heads [512,64] 72 / 144, [512,128] 130 / 158, [256,256]
+// 126 / 134 (675 rows of 128 heads [70,300] 121 / 107).  Nor do launches of hardly more than one tile per compute unit, where the ring has no next tile to run on to:
+// 8192 x [256,512] n-contiguous (4,4) 28 / 37, 16384 x [192,512] (3,3) 31 / 46 (with the 128x128 tiles of six diagonals a
+// long K makes up for it: 8192 x [512,1024] (3,4) 76 / 66).
 constexpr long kPipeBMaxElements = 8L << 20;         // 40 MB of planes at most
 constexpr int kPipeMinRows = 16384, kPipeMinRowsKmajor = 385;
+constexpr int kPipeMinCols = 256, kPipeMinCols33 = 320, kPipeMinCols32 = 257;      // ((3,3) digits; int32 weights)
 static bool pipe_b_planes(const GemmDesc &d, bool kmajor, long b_batches)
 {
     if (g_switches.no_pipe || b_batches * d.N * d.K > kPipeBMaxElements) return false;
     return d.M >= (kmajor ? kPipeMinRowsKmajor : kPipeMinRows) && (double)d.G * d.M * d.N * d.K >= g_switches.b_rows_min_macs;
+}
+
+// ... by digit counts, with `tiles` tiles of its kernel.  (With the product size lowered by its switch, whatever fills the device.)
+static bool pipe_b_pays(const GemmDesc &d, int na, int nb, long tiles, int cus)
+{
+    if (g_switches.b_rows_min_macs < kBRowsMinMacs) return tiles >= cus;
+    if (d.N < (na + nb <= 6 ? kPipeMinCols33 : d.b32 ? kPipeMinCols32 : kPipeMinCols)) return false;
+    return 2 * tiles >= 3L * cus || (tiles >= cus && na + nb == 7 && d.K >= 512);
 }
 
 // The launch behind a speculative one: it does nothing unless the verdict word says that the digit counts did not cover
@@ -681,7 +696,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             const PipeForm f = both ? pipe_form(both->na, both->nb) : PipeForm{};
             const long fewer = both && both->na < both->nb ? both->na : (both ? both->nb : 0);
             if (f.fn && fewer * ((d.K + 31) / 32) * 32 * 16384 <= kMaxDiagonal &&
-                (long)((d.M + 127) / 128) * ((d.N + f.bn - 1) / f.bn) * d.G >= g_cache.cus) {
+                pipe_b_pays(d, both->na, both->nb, (long)((d.M + 127) / 128) * ((d.N + f.bn - 1) / f.bn) * d.G, g_cache.cus)) {
                 inst = both;
                 pipe = f;
                 pre_b = true;
