@@ -964,10 +964,12 @@ bool gemm_gemv_launch(const GemmDesc &d)
     const bool rescale = d.a_rs != 1 || d.b_rs != 1;
     if (kmajor) {
         const dim3 grid((unsigned)((d.N + 255) / 256), (unsigned)d.G);
-        // 16-byte loads of B along n, sixteen rows of B at a time in each of eight wavefronts: from K = 64 on, with two rows
-        // from 96.  (Below, most of those loads repeat a wavefront's last row: 75 heads [32,928], one row 7.3 us with the
-        // kernel below and 8.5 with this one, two rows 7.0 / 16.7; [96,928] 13.3 / 8.8 and 18.9 / 17.1.)
-        if (d.K >= (d.M == 1 ? 64 : 96) && d.b32 && !rescale && d.N % 4 == 0 && (((uintptr_t)d.B | (uintptr_t)(d.ldbk * 4) | (uintptr_t)(d.sB * 4)) & 15) == 0) {
+        // 16-byte loads of B along n, sixteen rows of B at a time in each of eight wavefronts: from K = 64 on, with two rows and
+        // more workgroups than compute units from 96 (one of them fits a unit).  Below, most of those loads repeat a
+        // wavefront's last row: 75 heads [32,928], one row 7.3 us with the kernel below and 8.5 with this one, two rows 7.0 /
+        // 16.7; [64,928] two rows 12.2 / 16.8, 128 heads [64,512] 12.9 / 9.3, [70,300] 11.8 / 9.7; 75 heads [96,928] 18.9 / 17.1.
+        const bool long_k = d.K >= 96 || (d.K >= 64 && (d.M == 1 || (long)grid.x * grid.y <= device_cus()));
+        if (long_k && d.b32 && !rescale && d.N % 4 == 0 && (((uintptr_t)d.B | (uintptr_t)(d.ldbk * 4) | (uintptr_t)(d.sB * 4)) & 15) == 0) {
             if (d.M == 1) gemv32_kmajor_kernel<1><<<grid, dim3(512), 0, 0>>>(p);
             else gemv32_kmajor_kernel<2><<<grid, dim3(512), 0, 0>>>(p);
             return true;
