@@ -103,7 +103,7 @@ const char *zk_last_error_string(void);
 void zk_clear_error(void);
 
 /* The reference's library allocates nothing and keeps no state; this one keeps scratch buffers on the device between
- * calls (digit planes of A and of a small B, partial sums of split tiles, digit counts, the quotient
+ * calls (digit planes of A and of a small B, a row-major copy of a small B, partial sums of split tiles, digit counts, the quotient
  * tables of the activations), allocated on demand and grown inside a call when a larger problem arrives.
  * zk_workspace_bytes: device bytes held as scratch right now.  zk_prepared_weights_bytes: device bytes held as digit
  * planes made by zk_gemm_prepare_weights.  zk_release_workspace: waits for the device and frees the scratch (not the

@@ -774,20 +774,27 @@ def test_empty_operands(K, oracle):
 
 # ---------------------------------------------------------------------------------- softmax -----
 def test_einsum_values_rewritten_with_contiguous_rows(K, oracle, monkeypatch):
-    """`bsht,btc->bshc` on the MFMA path copies a small n-contiguous int64 B into row-major scratch first (products of
-    2^32 MACs and more; the threshold is lowered here): ragged T and C, two batches, and a second call with another B
-    through the same scratch"""
+    """`bsht,btc->bshc` on the MFMA path copies a small n-contiguous int64 B of more than five digits into row-major scratch
+    first (products of 2^32 MACs and more; the threshold is lowered here): ragged T and C, two batches, A split in the
+    kernel and from planes, and a second call with another B through the same scratch"""
     monkeypatch.setenv("ZK_B_ROWS_MIN_MACS", "1")
     K.lib.zk_reload_env()           # the switches are read when the library is loaded, not per call
     rng = np.random.default_rng(77)
     K.lib.zk_gemm_set_path(2)
+    K.release_workspace()
     try:
-        for Bq, S, H, T, Cc in ((2, 9, 5, 70, 45), (1, 40, 3, 33, 130), (1, 3, 16, 257, 64)):
-            for rep in range(2):
+        for Bq, S, H, T, Cc in ((2, 9, 5, 70, 45), (1, 40, 3, 33, 130), (1, 3, 16, 257, 64), (1, 300, 16, 65, 300)):
+            for bits in (44, 62):
                 pr = rng.integers(0, 1 << 19, size=(Bq, S, H, T), dtype=np.int64)
-                kv = rand_i64(rng, (Bq, T, Cc), 36 if rep else 24)
-                assert np.array_equal(host(K.einsum_bsht_btc_bshc(dev(pr), dev(kv), 23)), oracle.einsum_bsht_btc_bshc(pr, kv, 23)), (Bq, S, H, T, Cc, rep)
-                assert K.gemm_last_plan()[0] == 2
+                kv = rand_i64(rng, (Bq, T, Cc), bits)
+                expected = oracle.einsum_bsht_btc_bshc(pr, kv, 23)
+                held = K.workspace_bytes()[0]
+                for _ in range(2):          # (a first call may run on digits remembered for other operands at these addresses)
+                    assert np.array_equal(host(K.einsum_bsht_btc_bshc(dev(pr), dev(kv), 23)), expected), (Bq, S, H, T, Cc, bits)
+                    torch.cuda.synchronize()
+                assert K.gemm_last_plan()[0] == 2 and K.gemm_last_plan()[2] > 5
+                if (Bq, S) == (2, 9) and bits == 44:
+                    assert K.workspace_bytes()[0] >= held + Bq * T * Cc * 8, "the copy's buffer"
     finally:
         K.lib.zk_gemm_set_path(0)
         monkeypatch.delenv("ZK_B_ROWS_MIN_MACS")

@@ -271,28 +271,40 @@ def test_stale_guess_fresh_activations_known_weights(K, oracle):
         assert K.lib.zk_gemm_guard_hits() == hits + 1
 
 
-@pytest.mark.parametrize("rewrite", [False, True])
-def test_stale_guess_values_einsum(K, oracle, rewrite):
-    """bsht,btc->bshc: an n-contiguous int64 B per batch, read as it lies or through the row-major rewrite"""
-    import os
-    rng = np.random.default_rng(21 + rewrite)
+@pytest.fixture
+def small_b_first(K, monkeypatch):
+    """a B that is small next to the product is split (or rewritten) in front of it, however small the product"""
+    monkeypatch.setenv("ZK_B_ROWS_MIN_MACS", "1")
+    K.lib.zk_reload_env()
+    yield
+    monkeypatch.delenv("ZK_B_ROWS_MIN_MACS")
+    K.lib.zk_reload_env()
+
+
+def _values_rounds(K, oracle, P, V, pokes):
+    _stale_guess_rounds(K, lambda: (K.einsum_bsht_btc_bshc(P.d, V.d, 23),),
+                        lambda: (oracle.einsum_bsht_btc_bshc(P.h, V.h, 23),), [P, V], pokes)
+
+
+def test_stale_guess_values_einsum(K, oracle):
+    """bsht,btc->bshc: an n-contiguous int64 B per batch, read as it lies"""
+    rng = np.random.default_rng(21)
     Bq, S, H, T, Cc = 2, 9, 8, 200, 300
     P = Operand(rng.integers(0, 1 << 19, size=(Bq, S, H, T), dtype=np.int64))
     V = Operand(rand_i64(rng, (Bq, T, Cc), 20))
-    old = os.environ.get("ZK_B_ROWS_MIN_MACS")
-    os.environ["ZK_B_ROWS_MIN_MACS"] = "1" if rewrite else "1e30"
-    K.lib.zk_reload_env()
-    try:
-        pokes = [lambda: V.poke((1, T - 1, Cc - 1), WIDE), lambda: V.poke((0, 0, 0), -WIDE), lambda: V.poke((1, 77, 131), WIDE),
-                 lambda: P.poke((1, S - 1, H - 1, T - 1), WIDE), lambda: P.poke((0, 2, 3, 5), WIDE)]
-        _stale_guess_rounds(K, lambda: (K.einsum_bsht_btc_bshc(P.d, V.d, 23),),
-                            lambda: (oracle.einsum_bsht_btc_bshc(P.h, V.h, 23),), [P, V], pokes)
-    finally:
-        if old is None:
-            del os.environ["ZK_B_ROWS_MIN_MACS"]
-        else:
-            os.environ["ZK_B_ROWS_MIN_MACS"] = old
-        K.lib.zk_reload_env()
+    pokes = [lambda: V.poke((1, T - 1, Cc - 1), WIDE), lambda: V.poke((0, 0, 0), -WIDE), lambda: V.poke((1, 77, 131), WIDE),
+             lambda: P.poke((1, S - 1, H - 1, T - 1), WIDE), lambda: P.poke((0, 2, 3, 5), WIDE)]
+    _values_rounds(K, oracle, P, V, pokes)
+
+
+def test_stale_guess_values_einsum_rewritten(K, oracle, small_b_first):
+    """the same through the row-major copy, which a B of more than five digits takes"""
+    rng = np.random.default_rng(22)
+    Bq, S, H, T, Cc = 2, 9, 8, 200, 300
+    P = Operand(rng.integers(0, 1 << 19, size=(Bq, S, H, T), dtype=np.int64))
+    V = Operand(rand_i64(rng, (Bq, T, Cc), 44))
+    pokes = [lambda: P.poke((1, S - 1, H - 1, T - 1), 1 << 62), lambda: P.poke((0, 2, 3, 5), 1 << 62), lambda: P.poke((0, 0, 0, 0), -(1 << 62))]
+    _values_rounds(K, oracle, P, V, pokes)
 
 
 def test_stale_guess_scores_einsum(K, oracle):

@@ -131,6 +131,8 @@ struct RangeCache {
     size_t partials_bytes = 0;
     unsigned char *b_planes = nullptr;       // digit planes of a small B
     size_t b_planes_bytes = 0;
+    int64_t *b_rows = nullptr;               // a small n-contiguous B of many digits rewritten with contiguous rows
+    size_t b_rows_count = 0;
     int *row_steps = nullptr;                // per row tile of A: its steps up to the last one that is not all zeros
     size_t row_steps_count = 0;
     int cus = 0;                             // compute units of the device
@@ -170,7 +172,7 @@ static RangeCache g_cache;
 // ZK_GEMM_SYNC: every call waits for its own digit verdict; ZK_NO_TAIL_SPLIT: no split-K; ZK_VALU_FALLBACK: the guarded launch
 // behind a speculative one is always the vector-ALU kernel; ZK_NO_STREAM32: grouped launches on int32 weights keep the general
 // 32-row kernel; ZK_B_ROWS_MIN_MACS: product
-// size from which a B that is small next to it is split into digit planes first; ZK_SKINNY_MAX_M: rows up to
+// size from which a B that is small next to it is split into digit planes or rewritten first; ZK_SKINNY_MAX_M: rows up to
 // which the 32-row tiles are used; ZK_SCRATCH_LIMIT: bytes a scratch buffer may grow to, as if the device had no more.
 struct Switches { bool sync_verdict, no_tail_split, valu_fallback, no_stream32, no_pipe; double b_rows_min_macs, scratch_limit; int skinny_max_m, planes_min_tiles_n, stream32_min_pairs; };
 constexpr long kBRowsMinMacs = 1L << 30;
@@ -485,7 +487,7 @@ size_t gemm_mfma_workspace_bytes(size_t *prepared_bytes)
     std::lock_guard<std::mutex> lock(g_cache.mu);
     size_t scratch = g_cache.dev ? 8 * sizeof(unsigned long long) : 0;
     scratch += g_cache.planes_bytes + g_cache.seen_count * sizeof(unsigned) + g_cache.partials_bytes * sizeof(unsigned long long) +
-               g_cache.b_planes_bytes + g_cache.row_steps_count * sizeof(int);
+               g_cache.b_planes_bytes + g_cache.b_rows_count * sizeof(int64_t) + g_cache.row_steps_count * sizeof(int);
     size_t prepared = 0;
     for (const auto &kv : g_prepared) {
         const PreparedB &pb = kv.second;
@@ -507,11 +509,13 @@ void gemm_mfma_release_workspace()
     if (g_cache.seen) (void)hipFree(g_cache.seen);
     if (g_cache.partials) (void)hipFree(g_cache.partials);
     if (g_cache.b_planes) (void)hipFree(g_cache.b_planes);
+    if (g_cache.b_rows) (void)hipFree(g_cache.b_rows);
     if (g_cache.row_steps) (void)hipFree(g_cache.row_steps);
     g_cache.planes = nullptr; g_cache.planes_bytes = 0;
     g_cache.seen = nullptr; g_cache.seen_count = 0;
     g_cache.partials = nullptr; g_cache.partials_bytes = 0;
     g_cache.b_planes = nullptr; g_cache.b_planes_bytes = 0;
+    g_cache.b_rows = nullptr; g_cache.b_rows_count = 0;
     g_cache.row_steps = nullptr; g_cache.row_steps_count = 0;
 }
 
@@ -544,6 +548,39 @@ static bool pipe_b_pays(const GemmDesc &d, int na, int nb, long tiles, int cus)
     if (g_switches.b_rows_min_macs < kBRowsMinMacs) return tiles >= cus;
     if (d.N < (na + nb <= 6 ? kPipeMinCols33 : d.b32 ? kPipeMinCols32 : kPipeMinCols)) return false;
     return 2 * tiles >= 3L * cus || (tiles >= cus && na + nb == 7 && d.K >= 512);
+}
+
+// B[g][k][n] (n contiguous) -> out[g][n][k]: 32x32 tiles through LDS, both sides coalesced
+__global__ __launch_bounds__(256) void b_rows_kernel(const int64_t *__restrict__ B, long ldbk, long sB, int64_t *__restrict__ out, int N, int K)
+{
+    __shared__ int64_t tile[32][33];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const int n0 = blockIdx.x * 32, k0 = blockIdx.y * 32;
+    const int64_t *src = B + (long)blockIdx.z * sB;
+    int64_t *dst = out + (long)blockIdx.z * N * K;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int k = k0 + ty + 8 * i, n = n0 + tx;
+        tile[ty + 8 * i][tx] = (k < K && n < N) ? src[(long)k * ldbk + n] : 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int n = n0 + ty + 8 * i, k = k0 + tx;
+        if (n < N && k < K) dst[(long)n * K + k] = tile[tx][ty + 8 * i];
+    }
+}
+
+// An n-contiguous int64 B that is small next to the product and needs more digits than the pipelined kernel has instances
+// for is rewritten with contiguous rows: the kernels of many digits then read it with 16-byte loads and take A from digit
+// planes.  As it lies / rewritten, (5,9) digits, the values of 128 heads: 16 tokens x [4096,512] 169 / 161 us, 32 x [4096,512]
+// 332 / 309, 63 x [8192,512] 1307 / 1220, 200 x [779,512] 539 / 475, 100 x [2048,1000] 1062 / 927.  (Of up to five digits the
+// kernels with two depths per step read it as it lies in the same time: 32 x [4096,512], (3,4), 161 rewritten, 159.)
+constexpr double kBCopyMinMacs = 4294967296.0;       // 2^32
+static bool b_copy_pays(const GemmDesc &d, int nb, long b_batches)
+{
+    if (d.b32 || nb <= 5 || d.M <= 32 || b_batches * d.N * d.K > kPipeBMaxElements) return false;
+    return (double)d.G * d.M * d.N * d.K >= (g_switches.b_rows_min_macs < kBRowsMinMacs ? g_switches.b_rows_min_macs : kBCopyMinMacs);
 }
 
 // The launch behind a speculative one: it does nothing unless the verdict word says that the digit counts did not cover
@@ -686,6 +723,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         if (!inst) return kDeclined;
         if (!prep && !inst->skinny) inst = smaller_tiles(inst, d, g_cache.cus);
         if (!prep) { p.B = d.B; p.b_gstride = 0; }
+        p.ldbn = d.ldbn; p.ldbk = d.ldbk; p.sB = d.sB;
         p.row_steps = nullptr;
         // planes on both sides: the pipelined kernel, where there is one for the digit counts
         PipeForm pipe = {};
@@ -702,6 +740,14 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
                 pre_b = true;
             }
         }
+        bool b_copied = false;
+        if (kmajor && !pre_b && b_copy_pays(d, inst->nb, b_batches)) {
+            // (without memory for the copy the n-contiguous kernels run as they are)
+            const Outcome got = grow(g_cache.b_rows, g_cache.b_rows_count, (size_t)(b_batches * d.N * d.K), "row-major copy of B");
+            if (got == kFailed) return kFailed;
+            b_copied = got == kDone;
+        }
+        const bool by_columns = kmajor && !b_copied;         // the kernels read B along n
         // int32 accumulators: at most min(NA,NB) digit pairs per diagonal, each product at most 2^14 in magnitude
         const long pairs = inst->na < inst->nb ? inst->na : inst->nb;
         const int ksteps = ((d.K + 32 * inst->kk - 1) / (32 * inst->kk)) * inst->kk;     // 32-k steps, padded
@@ -737,11 +783,11 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         // us, 448 (243 x [512,7168]) 35.6 / 39.4, 896 (128 x [2048,7168]) 46.7 / 46.2, 1024 (128 x [7168,2048]) 49.5 /
         // 47.1, 1434 (243 x [1536,7168]) 54.7 / 52.2, 16384 (243 x [7168,16384]) 449 / 353.)
         const bool long_slices = (long)steps * 32 * inst->kk >= 800L * (small_split > 1 ? small_split : 1);
-        const bool use_planes = pre_b || (planes_fit && !kmajor && !inst->skinny && (prep || (p.tiles_n >= g_switches.planes_min_tiles_n && (total >= g_cache.cus || long_slices))));
-        if (b_shift && (kmajor || !inst->skinny)) return kDeclined;
+        const bool use_planes = pre_b || (planes_fit && !by_columns && !inst->skinny && (prep || (p.tiles_n >= g_switches.planes_min_tiles_n && (total >= g_cache.cus || long_slices))));
+        if (b_shift && (by_columns || !inst->skinny)) return kDeclined;
         const int variant = pre_b ? kB64PlanesBoth : prep ? (inst->skinny ? kB64FlyBPlanes : kB64PlanesBoth)
                           : b_shift ? (d.b32 ? kB32FlyRs : kB64FlyRs)
-                          : kmajor ? (d.b32 ? kB32KmajorFly : kB64KmajorFly)
+                          : by_columns ? (d.b32 ? kB32KmajorFly : kB64KmajorFly)
                                    : (d.b32 ? (use_planes ? kB32Planes : kB32Fly) : (use_planes ? kB64Planes : kB64Fly));
         MfmaKernel fn = inst->fn[variant];
         if (!fn) return kDeclined;
@@ -840,6 +886,11 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
                 attempt--;
                 continue;
             }
+        }
+        if (b_copied) {
+            const dim3 grid((unsigned)((d.N + 31) / 32), (unsigned)((d.K + 31) / 32), (unsigned)b_batches);
+            b_rows_kernel<<<grid, dim3(256), 0, 0>>>(reinterpret_cast<const int64_t *>(d.B), d.ldbk, d.sB, g_cache.b_rows, d.N, d.K);
+            p.B = g_cache.b_rows; p.ldbn = d.K; p.ldbk = 1; p.sB = d.sB != 0 ? (long)d.N * d.K : 0;
         }
         if (use_planes) {
             p.a_planes = g_cache.planes; p.a_msub = msub; p.a_ksteps = ksteps;
