@@ -307,6 +307,84 @@ def test_stale_guess_values_einsum_rewritten(K, oracle, small_b_first):
     _values_rounds(K, oracle, P, V, pokes)
 
 
+@pytest.fixture
+def oracle_threads(oracle):
+    oracle.set_threads(oracle.max_threads())
+    yield
+    oracle.set_threads(1)
+
+
+def _on_planes_of_both(K, fn):
+    """the call, which has to run on the kernel that reads planes of both operands while the digits are the narrow ones"""
+    def call():
+        before = K.lib.zk_gemm_pipe_calls()
+        out = fn()
+        call.on_planes = K.lib.zk_gemm_pipe_calls() == before + 1
+        return (out,)
+    return call
+
+
+def _planes_rounds(K, call, expect, operands, pokes):
+    """as _stale_guess_rounds, and the call on the stale guess ran on the planes of both operands: their two pre-passes are
+    all that can raise the verdict there"""
+    def poked(poke):
+        def f():
+            assert call.on_planes, "the narrow call is expected on planes of both operands"
+            poke()
+        return f
+    _stale_guess_rounds(K, call, expect, operands, [poked(p) for p in pokes])
+
+
+def test_stale_guess_values_on_planes_of_both_operands(K, oracle, oracle_threads, small_b_first):
+    """values of a causal prompt (n-contiguous, a batch each): wide elements of B at its ends and in its last batch, of A in
+    its rows' ends, and in what had been all zeros and cut off"""
+    rng = np.random.default_rng(23)
+    Bq, S, T, Cc = 2, 3300, 70, 520
+    p = rand_i64(rng, (Bq, S, 1, T), 19)
+    p[:, :1024, :, 33:] = 0             # whole row tiles that end after two steps of three
+    p[:, 1024:1152] = 0                 # ... and one that holds nothing
+    P, V = Operand(p), Operand(rand_i64(rng, (Bq, T, Cc), 20))
+    pokes = [lambda: V.poke((1, T - 1, Cc - 1), WIDE), lambda: V.poke((0, 0, 0), -WIDE), lambda: V.poke((0, 63, 64), WIDE),
+             lambda: P.poke((1, S - 1, 0, T - 1), WIDE), lambda: P.poke((0, 5, 0, T - 1), WIDE), lambda: P.poke((1, 1100, 0, 0), -WIDE)]
+    call = _on_planes_of_both(K, lambda: K.einsum_bsht_btc_bshc(P.d, V.d, 23))
+    _planes_rounds(K, call, lambda: (oracle.einsum_bsht_btc_bshc(P.h, V.h, 23),), [P, V], pokes)
+    # an element where A was cut off that fits the digits: the next call must see that the rows end later
+    for op in (P, V):
+        op.restore()
+    for _ in range(3):
+        call()
+        torch.cuda.synchronize()
+    assert call.on_planes
+    hits = K.lib.zk_gemm_guard_hits()
+    P.poke((0, 1023, 0, T - 1), 77)
+    P.poke((1, 1151, 0, 40), -5)
+    out, = call()
+    assert call.on_planes and np.array_equal(host(out), oracle.einsum_bsht_btc_bshc(P.h, V.h, 23))
+    assert K.lib.zk_gemm_guard_hits() == hits
+
+
+def test_stale_guess_scores_on_planes_of_both_operands(K, oracle, oracle_threads, small_b_first):
+    """scores (k-contiguous, one cache for all rows) from 16384 rows on"""
+    rng = np.random.default_rng(24)
+    Bq, S, T, Cc = 1, 16400, 270, 40
+    Q, Kc = Operand(rand_i64(rng, (Bq, S, 1, Cc), 20)), Operand(rand_i64(rng, (Bq, T, Cc), 20))
+    pokes = [lambda: Kc.poke((0, T - 1, Cc - 1), WIDE), lambda: Kc.poke((0, 0, 0), -WIDE), lambda: Kc.poke((0, 130, 31), WIDE),
+             lambda: Q.poke((0, S - 1, 0, Cc - 1), WIDE), lambda: Q.poke((0, 0, 0, 0), -WIDE)]
+    call = _on_planes_of_both(K, lambda: K.einsum_bshc_btc_bsht(Q.d, Kc.d, 21))
+    _planes_rounds(K, call, lambda: (oracle.einsum_bshc_btc_bsht(Q.h, Kc.h, 21),), [Q, Kc], pokes)
+
+
+def test_stale_guess_per_head_weights_on_planes_of_both_operands(K, oracle, oracle_threads, small_b_first):
+    """one int32 matrix per head, n-contiguous, from 385 rows on; the widest weight belongs to the last head"""
+    rng = np.random.default_rng(25)
+    S, H, D, Cc = 390, 16, 70, 520
+    q, w = Operand(rand_i64(rng, (1, S, H, D), 20)), Operand(rand_i32(rng, (H, D, Cc), 16))
+    pokes = [lambda: w.poke((H - 1, D - 1, Cc - 1), 1 << 30), lambda: w.poke((0, 0, 0), -(1 << 30)), lambda: w.poke((7, 33, 300), 1 << 30),
+             lambda: q.poke((0, S - 1, H - 1, D - 1), WIDE), lambda: q.poke((0, 200, 3, 64), -WIDE)]
+    call = _on_planes_of_both(K, lambda: K.einsum_bshd_hdc_bshc(q.d, w.d, 30))
+    _planes_rounds(K, call, lambda: (oracle.einsum_bshd_hdc_bshc(q.h, w.h, 30),), [q, w], pokes)
+
+
 def test_stale_guess_scores_einsum(K, oracle):
     """bshc,btc->bsht: a k-contiguous B per batch; the wide element sits in the second batch's B"""
     rng = np.random.default_rng(31)
