@@ -119,10 +119,10 @@ def test_gemm_two_depths_per_step(K, oracle, bits_a, bits_w, digits, w32):
     K.lib.zk_gemm_set_path(0)
 
 
-@pytest.mark.parametrize("Kd", [14560, 14600, 16384, 18432])
+@pytest.mark.parametrize("Kd", [14432, 14464, 16384, 18432])
 def test_gemm_long_k_with_nine_digit_operands(K, oracle, Kd):
-    """the int32 accumulators of the MFMA path hold min(NA, NB) * K * 2^14: with nine digits that ends at K = 14563.
-    Beyond it every tile is split along K (partial sums, then the finishing kernel) instead of falling back to the
+    """the int32 accumulators of the MFMA path hold min(NA, NB) * K * 2^14 up to 0x7F000000 (the epilogue hands carries from
+    diagonal to diagonal in 32 bits): with nine digits that ends at K = 14432.  Beyond it every tile is split along K (partial sums, then the finishing kernel) instead of falling back to the
     vector ALU; operands whose digits all sit at their extremes, on both sides of the bound and at the model's 16384 /
     18432"""
     rng = np.random.default_rng(Kd)
@@ -136,6 +136,45 @@ def test_gemm_long_k_with_nine_digit_operands(K, oracle, Kd):
         _gemm_case(K, oracle, 2, A, W, 1, 1, c)
         assert K.gemm_last_plan() == (2, 9, 9), "the long K must stay on the MFMA path"
     K.lib.zk_gemm_set_path(0)
+
+
+@pytest.mark.parametrize("digits,longest,prepared", [(9, 14432, False), (5, 25984, False), (3, 43328, False), (3, 43328, True)])
+def test_gemm_longest_k_in_one_piece(K, oracle, monkeypatch, digits, longest, prepared):
+    """no tile cut along K: the accumulators at the longest K that they take in one piece, every digit at its extreme (the
+    largest diagonals that the epilogue's 32-bit carries see), on the general and on the pipelined kernel; one step more
+    and the product goes to the vector ALU"""
+    monkeypatch.setenv("ZK_NO_TAIL_SPLIT", "1")
+    K.lib.zk_reload_env()
+    n = min(digits, 8)
+    low, high = -int("80" * n, 16), int("7F" * n, 16)          # all digits -128, all 127
+    low = low if digits < 9 else -0x7F7F7F7F7F7F7F80 - 1
+    try:
+        for Kd, path in ((longest, 2), (longest + 32 * (2 if digits == 5 else 1), 1)):
+            rng = np.random.default_rng(Kd)
+            A, W = rand_i64(rng, (1, 70, Kd), 63) >> (64 - 8 * n), rand_i64(rng, (150, Kd), 63) >> (64 - 8 * n)
+            A, W = np.clip(A, low, high), np.clip(W, low, high)
+            A[0, 0], A[0, 1], W[0], W[1] = low, high, low, high
+            dA, dW = dev(A), dev(W)
+            if prepared:
+                K.prepare_weights(dW)
+            try:
+                K.lib.zk_gemm_set_path(2)
+                for c in (29, 63):
+                    expected = oracle.int64_bmm_broadcast(A, W, 1, 1, c)
+                    for _ in range(2):
+                        before = K.lib.zk_gemm_pipe_calls()
+                        C, R = K.int64_bmm_broadcast(dA, dW, 1, 1, c)
+                        assert np.array_equal(host(C), expected[0]) and np.array_equal(host(R), expected[1]), (Kd, c)
+                    assert K.gemm_last_plan()[0] == path
+                    assert path == 1 or K.gemm_last_plan()[1:] == (digits, digits)
+                    assert K.lib.zk_gemm_pipe_calls() == before + (prepared and path == 2)
+            finally:
+                if prepared:
+                    K.release_weights(dW)
+    finally:
+        K.lib.zk_gemm_set_path(0)
+        monkeypatch.delenv("ZK_NO_TAIL_SPLIT")
+        K.lib.zk_reload_env()
 
 
 @pytest.mark.parametrize("path", PATHS)
