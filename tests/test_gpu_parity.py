@@ -526,6 +526,36 @@ def test_gemm_prepared_weights_pipelined_kernel(K, oracle):
             K.release_weights(Wd)
 
 
+@pytest.mark.parametrize("bits_a,bits_w,digits", [(20, 16, (3, 3)), (28, 20, (4, 3)), (44, 20, (6, 3)), (20, 28, (3, 4)), (28, 28, (4, 4)),
+                                                  (36, 28, (5, 4)), (20, 36, (3, 5)), (28, 36, (4, 5)), (36, 36, (5, 5))])
+def test_gemm_prepared_weights_without_the_pipelined_kernel(K, oracle, monkeypatch, bits_a, bits_w, digits):
+    """planes on both sides in the general kernel, which ZK_NO_PIPE leaves to every digit pair: the pipelined kernel and it
+    give the oracle's bits from the same planes"""
+    rng = np.random.default_rng(bits_a * 64 + bits_w)
+    A, W = rand_i64(rng, (1, 300, 530), bits_a), rand_i64(rng, (390, 530), bits_w)
+    A[0, 299, 529], W[389, 529] = (1 << bits_a) - 1, (1 << bits_w) - 1
+    expected = oracle.int64_bmm_broadcast(A, W, 1, 1, 29)
+    dA, dW = dev(A), dev(W)
+    K.prepare_weights(dW)
+    try:
+        for no_pipe in (True, False):
+            if no_pipe:
+                monkeypatch.setenv("ZK_NO_PIPE", "1")
+            else:
+                monkeypatch.delenv("ZK_NO_PIPE")
+            K.lib.zk_reload_env()
+            for _ in range(2):      # (a first call may run on digits remembered for other operands at these addresses)
+                before = K.lib.zk_gemm_pipe_calls()
+                C, R = K.int64_bmm_broadcast(dA, dW, 1, 1, 29)
+                assert np.array_equal(host(C), expected[0]) and np.array_equal(host(R), expected[1])
+            assert K.gemm_last_plan()[1:] == digits and K.lib.zk_gemm_last_prepared() == 1
+            assert K.lib.zk_gemm_pipe_calls() == before + (not no_pipe)
+    finally:
+        monkeypatch.delenv("ZK_NO_PIPE", raising=False)
+        K.lib.zk_reload_env()
+        K.release_weights(dW)
+
+
 @pytest.mark.parametrize("S,D", [(1, 1), (1, 63), (1, 64), (1, 65), (2, 64), (2, 95), (2, 96), (2, 97)])
 def test_per_head_weights_around_the_shortest_k_of_the_wide_loads(K, oracle, S, D):
     """one and two rows against n-contiguous int32 weights on either side of the K from which the wide loads are taken, more
