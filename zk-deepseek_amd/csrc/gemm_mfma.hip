@@ -93,12 +93,16 @@ static const Instance *pick_instance(int na, int nb, bool b32, bool skinny, int 
 // weights, 128x128 against 128x64 tiles, both on planes of A: 128 rows x [2048,7168] (16 tiles) 39.0 / 36.9 us, 128 x
 // [7168,2048] (56) 41.7 / 38.0, 200 x [7168,7168] (112) 159 / 147, 300 x [7168,7168] (168) 217 / 202.  Not where the
 // halves fill a round and three quarters (their last round is then not split): 500 x [7168,2048] (224) 69.5 / 80; nor for
-// launches larger than the device, which are bound by operand traffic: 512 x [18432,7168] 607 / 666.
+// launches larger than the device, which are bound by operand traffic: 512 x [18432,7168] 607 / 666.  Halves that take a
+// second round need a long K, too (300 x [7168,1024] 39 / 45, 700 x [4096,2048] 68 / 77), and tall products of a long K and
+// one or two tile columns stay as they are, where the slices of the halves no longer fall into step with the XCDs (1100 x [256,7168] 45 /
+// 58, 2400 x [256,16384] 150 / 196).
 static const Instance *smaller_tiles(const Instance *inst, const GemmDesc &d, int cus)
 {
     const long tiles = (long)((d.M + inst->bm - 1) / inst->bm) * ((d.N + inst->bn - 1) / inst->bn) * d.G;
     if (inst->bm != 128 || inst->bn != 128 || tiles >= cus) return inst;
-    if (2 * tiles > cus && 2 * tiles - cus > cus / 2) return inst;
+    if (2 * tiles > cus && (2 * tiles - cus > cus / 2 || d.K < 4096)) return inst;
+    if (d.N <= 256 && d.M > 1024 && d.K >= 4096) return inst;
     int count;
     const Instance *t = instances(&count);
     for (int i = 0; i < count; i++)
@@ -782,7 +786,12 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         // element of A save.  On the fly against planes, by K per workgroup: 256 (512 rows x [1024,1024] int32) 34.6 / 36.6
         // us, 448 (243 x [512,7168]) 35.6 / 39.4, 896 (128 x [2048,7168]) 46.7 / 46.2, 1024 (128 x [7168,2048]) 49.5 /
         // 47.1, 1434 (243 x [1536,7168]) 54.7 / 52.2, 16384 (243 x [7168,16384]) 449 / 353.)
-        const bool long_slices = (long)steps * 32 * inst->kk >= 800L * (small_split > 1 ? small_split : 1);
+        // Four tile columns of a small launch are too few: 909 x [256,7168] 37 on the fly, 42 on planes, (5,4) digits 50 / 59,
+        // 500 x [256,16384] (4,4) 47 / 55; but for three digits of A and slices that do not fall into step with the eight
+        // XCDs, so that each of them reads every slice: 1100 x [256,16384] (3,4), seven slices, 117 / 99.
+        const bool in_step = small_split > 1 && (small_split % 8 == 0 || 8 % small_split == 0);
+        const bool few_columns = p.tiles_n <= 4 && (inst->na > 3 || in_step);
+        const bool long_slices = !few_columns && (long)steps * 32 * inst->kk >= 800L * (small_split > 1 ? small_split : 1);
         const bool use_planes = pre_b || (planes_fit && !by_columns && !inst->skinny && (prep || (p.tiles_n >= g_switches.planes_min_tiles_n && (total >= g_cache.cus || long_slices))));
         if (b_shift && (by_columns || !inst->skinny)) return kDeclined;
         const int variant = pre_b ? kB64PlanesBoth : prep ? (inst->skinny ? kB64FlyBPlanes : kB64PlanesBoth)
