@@ -539,7 +539,7 @@ void gemm_mfma_release_workspace()
 // long K makes up for it: 8192 x [512,1024] (3,4) 76 / 66).
 constexpr long kPipeBMaxElements = 8L << 20;         // 40 MB of planes at most
 constexpr int kPipeMinRows = 16384, kPipeMinRowsKmajor = 385;
-constexpr int kPipeMinCols = 256, kPipeMinCols33 = 320, kPipeMinCols32 = 257;      // ((3,3) digits; int32 weights)
+constexpr int kPipeMinCols = 193, kPipeMinColsWide = 257;        // (a fourth column of 64; wide: (3,3) digits, a third of 128, and int32 weights)
 static bool pipe_b_planes(const GemmDesc &d, bool kmajor, long b_batches)
 {
     if (g_switches.no_pipe || b_batches * d.N * d.K > kPipeBMaxElements) return false;
@@ -550,7 +550,7 @@ static bool pipe_b_planes(const GemmDesc &d, bool kmajor, long b_batches)
 static bool pipe_b_pays(const GemmDesc &d, int na, int nb, long tiles, int cus)
 {
     if (g_switches.b_rows_min_macs < kBRowsMinMacs) return tiles >= cus;
-    if (d.N < (na + nb <= 6 ? kPipeMinCols33 : d.b32 ? kPipeMinCols32 : kPipeMinCols)) return false;
+    if (d.N < (na + nb <= 6 || d.b32 ? kPipeMinColsWide : kPipeMinCols)) return false;
     return 2 * tiles >= 3L * cus || (tiles >= cus && na + nb == 7 && d.K >= 512);
 }
 

@@ -114,13 +114,14 @@ __device__ __forceinline__ int64_t smx_prepare(int64_t v, const SmxPre &pre, lon
 // One row per wavefront; EPL = elements per lane (even).  VEC: T is even and the pointers are 16-byte aligned, a lane
 // owns pairs of adjacent elements; otherwise lanes own every 64th element, so that 8-byte accesses are contiguous over
 // the wavefront.  Score preparation: the operands of eight elements (sixteen where a row is short enough for the registers
-// and accesses are narrow, without VEC) are loaded at a time, and the prepared scores are stored once the whole row has
-// been loaded.  Loads and stores taken in turn wait for each other, the compiler having to assume that they overlap and the
-// count of what is under way covering both: one round trip to memory per element, or per batch.  Bound by memory on many
-// rows, by a row's chain of loads, reductions and divisions on few.  Element by element / stores behind each batch / behind the
-// row, inputs that change from call to call: 128 rows of 779 13.3 / 10.5 / 9.3 us, 31104 of 243 67 / 53 / 48, 2304 of 1142 22.6 /
-// 25.8 / 20.8, of 2047 58 / 62 / 49, 131072 of 1024 761 / 765 / 746 (5.8 TB/s).  Without preparation 4224 of
-// 1999 41.3 -> 30.9.
+// and accesses are narrow, without VEC) are loaded before the first of their scores is stored.  Loads and stores taken in
+// turn wait for each other, the compiler having to assume that they overlap and the count of what is under way covering
+// both: one round trip to memory per element, or per batch.  The scores are stored once the whole row has been loaded, but
+// for the two batches of 16-byte accesses of a row of 513 to 1024, where that costs more than it gives (131072 causal rows of
+// 1024 734 -> 755 us).  Bound by memory on many rows, by a row's chain of loads, reductions and divisions on few.  Element by
+// element / stores behind each batch / as it is, inputs that change from call to call: 128 rows of 779 13.3 / 10.5 / 9.3 us, 31104
+// of 243 67 / 53 / 48, 2304 of 1142 22.6 / 25.8 / 20.8, of 2047 58 / 62 / 49, 131072 of 1024 761 / 765 / 765 (5.6 TB/s; 780 with
+// sixteen at a time, which takes wavefronts).  Without preparation 4224 of 1999 41.3 -> 30.9.
 template <int Q, int EPL, bool VEC, bool PRE>
 __global__ __launch_bounds__(kSmxThreads) void softmax_wave_kernel(int64_t *__restrict__ R, int64_t *__restrict__ C,
                                                                    const int64_t *__restrict__ lut_g, long rows, int T,
@@ -138,6 +139,12 @@ __global__ __launch_bounds__(kSmxThreads) void softmax_wave_kernel(int64_t *__re
     auto at = [&](int j) { return VEC ? ((j >> 1) * 64 + lane) * 2 + (j & 1) : j * 64 + lane; };     // element j of this lane
     int64_t v[EPL];
     int64_t rmax = INT64_MIN;
+    constexpr bool LATE = !VEC || EPL != 16;
+    auto store_score = [&](int idx, int j) {
+        int64_t *dst = pre.scores + row * T + idx;
+        if (VEC) st_stream(reinterpret_cast<i64x2s *>(dst), i64x2s{ v[j], v[j + 1] });
+        else *dst = v[j];
+    };
     constexpr int MOST = VEC || EPL > 16 ? 8 : 16, BATCH = PRE && EPL > MOST ? MOST : EPL;
 #pragma unroll
     for (int j0 = 0; j0 < EPL; j0 += BATCH) {
@@ -170,17 +177,13 @@ __global__ __launch_bounds__(kSmxThreads) void softmax_wave_kernel(int64_t *__re
                 if (PRE) e = smx_prepare_value(e, b[q + h], m[q + h], pre);
                 rmax = e > rmax ? e : rmax;
             }
+            if (PRE && !LATE && pre.scores) store_score(idx, j0 + q);
         }
     }
-    if (PRE && pre.scores) {
-        int64_t *dst = pre.scores + row * T;
+    if (PRE && LATE && pre.scores) {
 #pragma unroll
-        for (int j = 0; j < EPL; j += VEC ? 2 : 1) {
-            const int idx = at(j);
-            if (idx >= T) continue;
-            if (VEC) st_stream(reinterpret_cast<i64x2s *>(dst + idx), i64x2s{ v[j], v[j + 1] });
-            else dst[idx] = v[j];
-        }
+        for (int j = 0; j < EPL; j += VEC ? 2 : 1)
+            if (at(j) < T) store_score(at(j), j);
     }
     rmax = wave_max_i64(rmax);
 
