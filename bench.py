@@ -3,13 +3,12 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu]
 
-Prints ONE JSON line.  `value` is the int64 GEMM throughput (Gmac/s) of benchmark config 4
+Prints ONE JSON line on stdout.  `value` is the int64 GEMM throughput (Gmac/s) of benchmark config 4
 (512 x 7168 against W[18432,7168], config-1 operand ranges, shift 29) through the C ABI with operands
-resident in HBM; one step = one call of int64_64_bmm_broadcast_launcher.  The same line carries the
-other shapes the metric names (config-1 GEMM, full-range config 4, softmax / SiLU / sigmoid / RMSNorm
-HBM GB/s) under "extra", the roofline of the dominant kernel (with the figures of config 1 and of the HBM-bound
-shapes the metric names as flat keys inside it, and once more at the end of the line under "summary"), the calls on
-operands never seen (--only cold), and a CPU baseline timed on this host.
+resident in HBM; one step = one call of int64_64_bmm_broadcast_launcher.  The line carries the roofline of the dominant
+kernel, a CPU baseline timed on this host, and under "summary" the other shapes the metric names (config-1 GEMM, softmax /
+SiLU / RMSNorm HBM fractions) and the calls on operands never seen (--only cold).  Everything that was measured and
+checked goes to stderr as a second JSON object, behind "details: ".
 
 Nothing is timed before it has been checked: the headline product is compared with torch's int64 matmul on the CPU
 (same input bytes) on a block of columns before the timed loop starts, and the run aborts on a mismatch; the other
@@ -904,7 +903,10 @@ def run():
         out["summary"]["child_processes_at_exit"] = len(psutil.Process().children(recursive=True))
     except Exception:
         out["summary"]["child_processes_at_exit"] = None
-    print(json.dumps(out))
+    # everything that was measured goes to stderr; the one line on stdout stays short enough for a record that keeps only the
+    # last 2000 characters of it
+    print("details: " + json.dumps(out), file=sys.stderr)
+    print(json.dumps(short_line(out)))
     sys.stdout.flush()
     sys.stderr.flush()
     # Nothing is left to do: leave without the interpreter's teardown of a process that held 90 GB of tensors.  A
@@ -912,6 +914,21 @@ def run():
     # the ordinary way, so under one the ordinary way it is.
     if not any(k.startswith("ROCPROF") for k in os.environ):
         os._exit(0)
+
+
+def short_line(out):
+    """the benchmark's line: the workload, its figures and the summary of the other legs, these to four digits"""
+    def four(v):
+        return float("%.4g" % v) if isinstance(v, float) else v
+    line = {k: out[k] for k in ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+                                "vs_baseline", "dtype", "data")}
+    line["config"] = {k: out["config"][k] for k in ("workload", "path", "limbs_a", "limbs_b", "verified")}
+    line["roofline"] = {k: four(out["roofline"].get(k)) for k in ("bound", "achieved", "peak", "unit", "frac")}
+    cpu = out["cpu_baseline"]
+    line["cpu_baseline"] = {k: four(cpu.get(k)) for k in ("value", "unit", "cores", "kind")} if cpu else None
+    skip = ("value_gmacs", "ms_per_step", "roofline_frac", "verified", "cpu_baseline_gmacs")
+    line["summary"] = {k: four(v) for k, v in out["summary"].items() if k not in skip and not k.startswith("sigmoid")}
+    return line
 
 
 def measured_traffic(key="gemm_config4_bytes_per_launch"):

@@ -2,6 +2,7 @@
 include/int64gemm.h declares, and its host-only table initialisers reproduce the tables the reference's
 circuits hold.  Nothing here launches a kernel."""
 import ctypes
+import json
 import os
 import re
 import subprocess
@@ -165,3 +166,30 @@ def test_bench_refuses_more_than_one_gpu_and_defaults_to_one():
     assert m and int(m.group(1)) == 1
     m = re.search(r'add_argument\("--steps",[^)]*default=(\d+)', src)
     assert m and 1 <= int(m.group(1)) <= 1000
+
+
+def test_bench_line_fits_a_record_of_two_thousand_characters():
+    """the line on stdout, built from a full run's record (every figure as long as a float gets), parses and stays short"""
+    src = open(os.path.join(ROOT, "bench.py")).read()
+    scope = {}
+    exec(src[src.index("def short_line"):src.index("def measured_traffic")], scope)
+    legs = re.findall(r'"((?:softmax|silu|sigmoid|rmsnorm)_[a-z0-9_]*x[0-9x]+)"', src)
+    long = 0.12345678901234567
+    summary = {n + "_frac_hbm": long for n in set(legs)}
+    summary.update({n: long for n in ("value_gmacs", "gemm_config1_us", "gemm_config1_frac_hbm", "gemm_config1_two_launch_floor_us", "gemm_config2_w1_us",
+                                      "gemm_config2_w2_us", "gemm_config4_prepared_us", "gemm_config4_prepared_frac_mfma_peak",
+                                      "gemm_1token_wkv_a_7168x576_int32_us", "moe_experts_int32_256tok_top8_of_256_frac_hbm",
+                                      "moe_experts_config5_256tok_top8_of_256_frac_hbm")})
+    summary.update({"%s_%s_ms" % (c, k): long for c in ("config4", "config2_w1", "config1") for k in ("first_call", "warm_call", "recycled_wider")})
+    out = {"metric": "m" * 76, "value": 107816.39734350423, "unit": "Gmac/s", "n_gpus": 1, "steps": 200, "warmup": 20, "ms_per_step": 0.6274160200000001,
+           "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "int64", "data": "synthetic",
+           "config": {"workload": "w" * 144, "path": "mfma_i8", "limbs_a": 3, "limbs_b": 3, "verified": True, "kernel_ms_hip_events": long},
+           "roofline": {"bound": "mfma", "achieved": 1947.2220094238935, "peak": 5000.0, "unit": "TOP/s", "frac": long, "others": {}},
+           "cpu_baseline": {"value": 17.41878290103771, "unit": "Gmac/s", "cores": 16, "kind": "reference", "sample": "s" * 147},
+           "verified": {"gemm_config4": "v" * 3000}, "extra": {"gemm": "e" * 10000}, "summary": summary}
+    line = json.dumps(scope["short_line"](out))
+    assert len(line) < 2000 and "\n" not in line
+    back = json.loads(line)
+    assert back["value"] == out["value"] and back["ms_per_step"] == out["ms_per_step"]
+    for k in ("metric", "unit", "n_gpus", "steps", "warmup", "higher_is_better", "scaling", "vs_baseline", "dtype", "data", "config"):
+        assert k in back
