@@ -1,5 +1,6 @@
 // Instances of the i8 MFMA GEMM kernels: planes on both sides (weights prepared once), one depth per step: the digit counts of
-// which the unprepared kernels have two depths per step.
+// which the unprepared kernels have two depths per step.  (The pipelined kernel has every one of these pairs and is what runs;
+// these are its dimensions and plane layouts, and the kernels that ZK_NO_PIPE puts in its place.)
 #include "gemm_mfma_kernels.h"
 
 namespace zk {

@@ -1053,7 +1053,8 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_mfma_guarded_kernel(MfmaP
     if ((int)blockIdx.x < p.guard.parts) guard_report(p.guard, (int)blockIdx.x);
     if (verdict == 0) return;
     if (verdict == 1 && (NA > 5 || NB > 5)) {
-        // five digits cover both operands (the fold kernel has seen every element): a third of the digit pairs of (9,9)
+        // five digits cover both operands (every workgroup that met a wider element would have raised the verdict to 2): a
+        // third of the digit pairs of (9,9)
         constexpr int NA5 = NA > 5 ? 5 : NA, NB5 = NB > 5 ? 5 : NB;
         for (int block = (int)blockIdx.x; block < p.walk_blocks; block += (int)gridDim.x) {
             gemm_mfma_block<NA5, NB5, WVM, WVN, WM, WN, KK, B32, BKM, false, false, false, 16, false>(p, block);

@@ -11,8 +11,10 @@
 //     of the next tile are loaded while this one is multiplied and stored.  With a short K (512: sixteen steps) a tile's
 //     first loads and its epilogue are a third of its time.
 // What bounds it: the matrix pipe at the clock the device grants it.  A step takes 0.81 / 1.11 us on 128x128 tiles with
-// (3,3) / (3,4) digits and 0.79 / 1.04 on 128x64 with (4,4) / (5,5): 2.7-3.2 POP/s of i8 products, where the probe that
-// multiplies random bytes out of LDS and loads nothing does 2.9.  Then LDS (108 KB per 1536 cycles of (3,4) MFMAs).  128x128 tiles need 16 (NA + NB - 1) x 2
+// (3,3) / (3,4) digits and 0.79 / 1.04 on 128x64 with (4,4) / (5,5): 2.7-3.2 POP/s of i8 products while steps run, where the
+// probe that multiplies random bytes out of LDS and loads nothing does 2.9.  A tile's epilogue, in which all eight wavefronts of
+// a compute unit's only workgroup combine and store, comes on top and leaves the matrix pipe idle: 8-9 us against 18 of steps at
+// K = 512, so that 131072 rows x [1024,512] take 800-850 us, 2.0 POP/s.  Then LDS (108 KB per 1536 cycles of (3,4) MFMAs).  128x128 tiles need 16 (NA + NB - 1) x 2
 // accumulator registers per lane: up to six diagonals fit beside two wavefronts per SIMD, more take 128x64 tiles.
 // Against gemm_mfma_block on planes of A alone: see pipe_b_planes in gemm_mfma.hip.
 //
