@@ -101,7 +101,8 @@ static const Instance *smaller_tiles(const Instance *inst, const GemmDesc &d, in
 {
     const long tiles = (long)((d.M + inst->bm - 1) / inst->bm) * ((d.N + inst->bn - 1) / inst->bn) * d.G;
     if (inst->bm != 128 || inst->bn != 128 || tiles >= cus) return inst;
-    if (2 * tiles > cus && (2 * tiles - cus > cus / 2 || d.K < 4096)) return inst;
+    const long halves = (long)((d.M + inst->bm - 1) / inst->bm) * ((d.N + 63) / 64) * d.G;        // (fewer than twice as many where the last column is)
+    if (2 * tiles - cus > cus / 2 || (halves > cus && d.K < 4096)) return inst;
     if (d.N <= 256 && d.M > 1024 && d.K >= 4096) return inst;
     int count;
     const Instance *t = instances(&count);
