@@ -912,6 +912,46 @@ def test_einsums_with_planes_of_both_operands(K, oracle, monkeypatch, bits_a, bi
         K.lib.zk_reload_env()
 
 
+@pytest.mark.parametrize("bits_a,bits_b,digits", [(19, 22, (3, 3)), (19, 27, (3, 4)), (27, 19, (4, 3)), (27, 27, (4, 4)), (36, 27, (5, 4)),
+                                                  (27, 35, (4, 5)), (36, 36, (5, 5)), (19, 35, (3, 5)), (43, 19, (6, 3))])
+def test_row_tiles_split_by_the_product(K, oracle, monkeypatch, bits_a, bits_b, digits):
+    """products whose row tiles fill whole rounds of two workgroups per compute unit: the product splits A itself.  One and
+    two rounds with a ragged last row tile and last columns, tile columns dealt in two parts, rows of C in whole lines and
+    not, K of less than a step, of whole ones, and odd (rows of A off the 16-byte grid), rows that end in zeros at every length,
+    a remainder"""
+    monkeypatch.setenv("ZK_B_ROWS_MIN_MACS", "1")
+    K.lib.zk_reload_env()
+    oracle.set_threads(oracle.max_threads())
+    rng = np.random.default_rng(bits_a * 64 + bits_b + 1)
+    K.lib.zk_gemm_set_path(2)
+    top_a, top_b = (1 << bits_a) - 1, (1 << bits_b) - 1
+    try:
+        for rows, N, Kd in ((65500, 130, 131), (32700, 256, 128), (16300, 520, 160), (32768, 200, 31)):
+            p, v = rand_i64(rng, (1, 4, rows // 4, Kd), bits_a), rand_i64(rng, (1, Kd, N), bits_b)
+            for r in range(0, rows // 4, 64):
+                p[0, :, r:r + 64, (r // 64) % Kd:] = 0
+            p[0, 3, -1, -1], v[0, -1, -1] = top_a, top_b
+            expected = oracle.einsum_bsht_btc_bshc(p, v, 23)
+            dp, dv = dev(p), dev(v)
+            for _ in range(2):          # (a first call may run on digits remembered for other operands at these addresses)
+                before = K.lib.zk_gemm_pipe_calls()
+                out = K.einsum_bsht_btc_bshc(dp, dv, 23)
+                assert np.array_equal(host(out), expected), (rows, N, Kd)
+            assert K.lib.zk_gemm_pipe_calls() == before + 1 and K.gemm_last_plan()[1:] == digits
+        a, w = rand_i64(rng, (1, 32700, 66), bits_a), rand_i64(rng, (257, 66), bits_b)
+        a[0, -1, -1], w[-1, -1] = top_a, -top_b
+        expected = oracle.int64_bmm_broadcast(a, w, 1, 1, 29)
+        da, dw = dev(a), dev(w)
+        for _ in range(2):
+            C, R = K.int64_bmm_broadcast(da, dw, 1, 1, 29)
+            assert np.array_equal(host(C), expected[0]) and np.array_equal(host(R), expected[1])
+    finally:
+        oracle.set_threads(1)
+        K.lib.zk_gemm_set_path(0)
+        monkeypatch.delenv("ZK_B_ROWS_MIN_MACS")
+        K.lib.zk_reload_env()
+
+
 def _scores(rng, shape, Q, masked=True):
     x = rng.integers(-(12 << Q), 12 << Q, size=shape, dtype=np.int64)
     if masked and shape[-1] > 1:

@@ -26,6 +26,7 @@
 // Results never depend on the guess, and a call whose operands were seen before never blocks the host.
 #include "gemm_mfma_kernels.h"
 #include "gemm_mfma_pipe.h"
+#include "gemm_mfma_rowtile.h"
 #include "report_ring.h"
 
 #include <algorithm>
@@ -555,6 +556,27 @@ static bool pipe_b_pays(const GemmDesc &d, int na, int nb, long tiles, int cus)
     return 2 * tiles >= 3L * cus || (tiles >= cus && na + nb == 7 && d.K >= 512);
 }
 
+// How the row-tile kernel (gemm_mfma_rowtile.h) would run a product that b_planes_kernel serves: the parts that a row tile's
+// columns are dealt in, or 0 where the pass over A in front of the pipelined kernel is expected to be as fast.  In us: a tile
+// of the row-tile kernel's two workgroups, or of the pipelined kernel's one twice as tall, has its steps and 3 for the sums and
+// stores; 64 rows of A are split at 11.7 KB per us when every workgroup does it; the pass over A moves 5.5 TB/s behind a
+// launch of 5.  What decides is how well the items fill whole rounds: pass and pipelined kernel / row tiles in one part, 17024 rows x
+// [1746,512] 209 / 265 us, 622 rows of 64 heads [457,128] 82 / 100, 61184 x [512,209] 151 / 115.
+static int rowtile_parts(const GemmDesc &d, int na, int nb, int bn, int cus)
+{
+    const long row_tiles = (long)((d.M + kRowtileRows - 1) / kRowtileRows) * d.G, tiles_n = (d.N + bn - 1) / bn, slots = 2L * cus;
+    const double steps = (d.K + 31) / 32, tile = steps * na * nb * (bn == 128 ? 0.104 : 0.052) + 3, split = d.K * (8.0 * kRowtileRows / 11700);
+    const long old_tiles = (long)((d.M + 127) / 128) * d.G * tiles_n;
+    double best = (double)((old_tiles + cus - 1) / cus) * tile + (double)d.G * d.M * d.K * (8 + na) / 5.5e6 + 5;
+    int parts = 0;
+    if (bn != 128 && d.K < 128) return 0;               // (584 rows of 128 heads [350,80], (4,4): 126 / 147)
+    for (long n = 1; n <= tiles_n && n <= 8; n++) {
+        const double t = (double)((row_tiles * n + slots - 1) / slots) * (split + (double)((tiles_n + n - 1) / n) * tile);
+        if (t < best) { best = t; parts = (int)n; }
+    }
+    return parts;
+}
+
 // B[g][k][n] (n contiguous) -> out[g][n][k]: 32x32 tiles through LDS, both sides coalesced
 __global__ __launch_bounds__(256) void b_rows_kernel(const int64_t *__restrict__ B, long ldbk, long sB, int64_t *__restrict__ out, int N, int K)
 {
@@ -733,6 +755,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         // planes on both sides: the pipelined kernel, where there is one for the digit counts
         PipeForm pipe = {};
         if (prep && !inst->skinny && inst->kk == 1 && !g_switches.no_pipe) pipe = pipe_form(inst->na, inst->nb);
+        RowtileForm rowtile = {};
         bool pre_b = false;
         if (planes_fit && !prep && b_shift == 0 && pipe_b_planes(d, kmajor, b_batches)) {
             const Instance *both = pick_instance(na, nb, false, false, need_diag, 0, kB64PlanesBoth);
@@ -743,6 +766,8 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
                 inst = both;
                 pipe = f;
                 pre_b = true;
+                p.col_parts = rowtile_parts(d, inst->na, inst->nb, f.bn, g_cache.cus);
+                if (p.col_parts) { rowtile = rowtile_form(inst->na, inst->nb); pipe = PipeForm{}; }
             }
         }
         bool b_copied = false;
@@ -758,7 +783,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         const int ksteps = ((d.K + 32 * inst->kk - 1) / (32 * inst->kk)) * inst->kk;     // 32-k steps, padded
         // (a K beyond that bound is cut into slices that respect it: every tile is then split, see below)
         const bool k_over = pairs * ksteps * 32 * 16384 > kMaxDiagonal;
-        const int BM = inst->bm, BN = pipe.fn ? pipe.bn : inst->bn;
+        const int BM = rowtile.fn ? kRowtileRows : inst->bm, BN = rowtile.fn ? rowtile.bn : pipe.fn ? pipe.bn : inst->bn;
         p.tiles_m = (d.M + BM - 1) / BM;
         p.tiles_n = (d.N + BN - 1) / BN;
         // A B operand that stays in L2 whatever the order (the MLA einsums: a KV cache or one head's weights against
@@ -793,7 +818,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         const bool in_step = small_split > 1 && (small_split % 8 == 0 || 8 % small_split == 0);
         const bool few_columns = p.tiles_n <= 4 && (inst->na > 3 || in_step);
         const bool long_slices = !few_columns && (long)steps * 32 * inst->kk >= 800L * (small_split > 1 ? small_split : 1);
-        const bool use_planes = pre_b || (planes_fit && !by_columns && !inst->skinny && (prep || (p.tiles_n >= g_switches.planes_min_tiles_n && (total >= g_cache.cus || long_slices))));
+        const bool use_planes = !rowtile.fn && (pre_b || (planes_fit && !by_columns && !inst->skinny && (prep || (p.tiles_n >= g_switches.planes_min_tiles_n && (total >= g_cache.cus || long_slices)))));
         if (b_shift && (by_columns || !inst->skinny)) return kDeclined;
         const int variant = pre_b ? kB64PlanesBoth : prep ? (inst->skinny ? kB64FlyBPlanes : kB64PlanesBoth)
                           : b_shift ? (d.b32 ? kB32FlyRs : kB64FlyRs)
@@ -802,6 +827,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         MfmaKernel fn = inst->fn[variant];
         if (!fn) return kDeclined;
         if (pipe.fn) fn = pipe.fn;
+        if (rowtile.fn) fn = rowtile.fn;
 
         // Split-K: a launch smaller than the device is cut into `split` slices of K per tile, each a workgroup of
         // its own; with more tiles than compute units the same is done for the tiles of the last, partial round
@@ -862,7 +888,8 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             } else if (got == kFailed) return kFailed;
             else if (k_over) return kDeclined;
         }
-        const long blocks = (long)p.main_tiles + (total - p.main_tiles) * p.split;
+        const long row_items = rowtile.fn ? (long)p.tiles_m * d.G * p.col_parts : 0;
+        const long blocks = rowtile.fn ? std::min<long>(row_items, 2L * g_cache.cus) : (long)p.main_tiles + (total - p.main_tiles) * p.split;
         long plane_wgs = 0, b_plane_wgs = 0;
         p.fail_class = inst->na > 5 || inst->nb > 5 ? 2 : 1;
         p.verdict = reinterpret_cast<unsigned *>(g_cache.dev + 5) + g_cache.turn;
@@ -883,14 +910,16 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
                 b.nsub = (d.N + 31) / 32; b.ksteps = ksteps;
                 b.gstride = (long)b.nsub * ksteps * inst->nb * 1024;
                 // (the one product of the model with zeros in A worth finding: a causal prompt's probabilities times the values)
-                b.row_tiles = kmajor && !d.b32 ? (long)p.tiles_m * d.G : 0;
+                b.row_tiles = kmajor && !d.b32 && !rowtile.fn ? (long)p.tiles_m * d.G : 0;
                 got = grow(g_cache.b_planes, g_cache.b_planes_bytes, (size_t)(b.gstride * b_batches), "digit planes of B");
+                // (two slots per workgroup for the digit planes of its row tiles)
+                if (got == kDone && rowtile.fn) got = grow(g_cache.planes, g_cache.planes_bytes, (size_t)blocks * 2 * (kRowtileRows / 32) * ksteps * inst->na * 1024, "digit-plane buffer");
                 if (got == kDone && b.row_tiles) got = grow(g_cache.row_steps, g_cache.row_steps_count, (size_t)b.row_tiles, "step counts");
             }
             if (got == kDone) got = grow(g_cache.seen, g_cache.seen_count, (size_t)(blocks + plane_wgs + b_plane_wgs), "digit counts");
             if (got == kFailed) return kFailed;
             if (got == kDeclined) {
-                if (!use_planes) return kDeclined;
+                if (!use_planes && !pre_b) return kDeclined;
                 planes_fit = false;
                 prep = nullptr;
                 attempt--;
@@ -919,9 +948,10 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
 #undef ZK_BPL
             p.B = b.planes; p.b_nsub = b.nsub; p.b_ksteps = ksteps; p.b_gstride = d.sB != 0 ? b.gstride : 0;
             p.row_steps = b.row_steps;
+            if (rowtile.fn) { p.a_planes = g_cache.planes; p.a_ksteps = ksteps; p.items = (int)row_items; }
         }
         p.seen = pipe.fn ? nullptr : g_cache.seen;
-        const size_t lds = pipe.fn ? pipe.lds : 2 * (size_t)inst->kk * ((BM / 32) * inst->na + (BN / 32) * inst->nb) * 1024 + 9 * 1024 + 16;
+        const size_t lds = rowtile.fn ? rowtile.lds : pipe.fn ? pipe.lds : 2 * (size_t)inst->kk * ((BM / 32) * inst->na + (BN / 32) * inst->nb) * 1024 + 9 * 1024 + 16;
         static std::set<const void *> lds_raised;
         if (lds > 64 * 1024 && !lds_raised.count((const void *)fn)) {
             if (hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
@@ -938,15 +968,16 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             p.items = pre_b ? (int)(((long)p.tiles_m * d.G + 7) / 8 * 8 * p.tiles_n) : (int)blocks;
             grid = (unsigned)(p.items < g_cache.cus ? p.items : g_cache.cus);
         }
-        fn<<<dim3(grid), dim3((unsigned)inst->threads), lds, 0>>>(p);
+        const unsigned threads = rowtile.fn ? 256 : (unsigned)inst->threads;
+        fn<<<dim3(grid), dim3(threads), lds, 0>>>(p);
         g_last_pairs = kept_pairs_before(inst->na, inst->nb, inst->dmax, inst->na, 0);
         g_last_prepared = prep ? 1 : 0;
-        if (pipe.fn) g_pipe_calls++;
+        if (pipe.fn || rowtile.fn) g_pipe_calls++;
         {
             const hipError_t err = hipGetLastError();
             if (err != hipSuccess) {
                 set_error(kLaunchFailure, "gemm: MFMA kernel launch failed (%s; digits %d,%d, %ld workgroups of %d threads, %zu bytes of LDS)",
-                          hipGetErrorString(err), inst->na, inst->nb, blocks, inst->threads, lds);
+                          hipGetErrorString(err), inst->na, inst->nb, blocks, (int)threads, lds);
                 return kFailed;
             }
         }
@@ -958,14 +989,14 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         *limbs_b = inst->nb;
         if (speculate) {
             // no waiting: a guarded launch redoes the product if the verdict is raised, the digits seen follow later
-            GuardArgs guard = make_guard(p.seen ? blocks + plane_wgs : plane_wgs + b_plane_wgs);
+            GuardArgs guard = make_guard((p.seen ? blocks : 0) + plane_wgs + b_plane_wgs);
             if (!p.seen) guard.seen += blocks;
             if (const Outcome got = launch_guarded_fallback(d, p, b_shift, &guard)) return got;
             guard_taken(guard, key_a, key_b, prep ? prep->nb : 0);       // (the slots are shared with the grouped launches, which set it too)
             return kDone;
         }
         int need_a, need_b;
-        if (!wait_digits(p.seen ? 0 : blocks, p.seen ? blocks + plane_wgs : plane_wgs + b_plane_wgs, &need_a, &need_b)) { set_error(kLaunchFailure, "gemm: digit readback failed"); return kFailed; }
+        if (!wait_digits(p.seen ? 0 : blocks, (p.seen ? blocks : 0) + plane_wgs + b_plane_wgs, &need_a, &need_b)) { set_error(kLaunchFailure, "gemm: digit readback failed"); return kFailed; }
         if (prep) need_b = prep->nb;
         g_cache.store_pair(key_a, need_a, key_b, need_b);
         if (need_a <= inst->na && need_b <= inst->nb) return kDone;

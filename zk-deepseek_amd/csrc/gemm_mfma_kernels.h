@@ -41,6 +41,7 @@ struct MfmaParams {
     long b_gstride;                 // ... and this many bytes from one batch's planes to the next one's (0: shared)
     const int *row_steps;           // 32-k steps of a row tile (128 rows) of A up to its last non-zero one (null: all of them; pipelined kernel only)
     int row_order, items, batches;  // pipelined kernel: items walked row tile by row tile, how many there are, and batches
+    int col_parts;                  // row-tile kernel: an item is a row tile and one of this many parts of its tile columns
     // split-K tail: workgroup ids below main_tiles are whole tiles; the rest are `split` workgroups per tile that
     // each cover a slice of K and leave raw 128-bit partial sums in `partials`
     int main_tiles, split;
