@@ -952,6 +952,25 @@ def test_row_tiles_split_by_the_product(K, oracle, monkeypatch, bits_a, bits_b, 
         K.lib.zk_reload_env()
 
 
+@pytest.mark.parametrize("heads,cols,k", [(5, 1, 1), (16, 16, 63), (17, 15, 64), (33, 70, 65), (128, 779, 512), (128, 512, 779), (128, 512, 1024),
+                                          (256, 256, 2048), (31, 1200, 2047)])
+def test_attention_of_few_positions_in_one_launch(K, oracle, heads, cols, k):
+    """scores and values of at most two rounds of 16 x 16 tiles: edges of tiles, of steps of 64 k and of the eight wavefronts
+    that share K, rows off the 16-byte grid, batches, every digit count from 3 to 9 with single elements that need more than
+    the rest, the largest magnitudes"""
+    rng = np.random.default_rng(heads * 4096 + cols + k)
+    for bits_a, bits_b in ((19, 21), (27, 28), (36, 35), (36, 60), (62, 22), (63, 63)):
+        B, S = (2, 3) if heads * cols < 3000 else (1, 1)
+        a, b = rand_i64(rng, (B, S, heads, k), bits_a), rand_i64(rng, (B, cols, k), bits_b)
+        a[-1, -1, -1, -1], b[-1, -1, -1] = -(1 << bits_a), (1 << bits_b) - 1
+        if bits_a == 27:
+            a[0, 0, 0, 0], b[0, 0, k // 2] = (1 << 45) + 1, -(1 << 37)
+        assert np.array_equal(host(K.einsum_bshc_btc_bsht(dev(a), dev(b), 23)), oracle.einsum_bshc_btc_bsht(a, b, 23)), (bits_a, bits_b)
+        assert K.gemm_last_plan() == (2, 0, 0)
+        v = np.ascontiguousarray(b.transpose(0, 2, 1))
+        assert np.array_equal(host(K.einsum_bsht_btc_bshc(dev(a), dev(v), 41)), oracle.einsum_bsht_btc_bshc(a, v, 41)), (bits_a, bits_b)
+
+
 def _scores(rng, shape, Q, masked=True):
     x = rng.integers(-(12 << Q), 12 << Q, size=shape, dtype=np.int64)
     if masked and shape[-1] > 1:

@@ -22,6 +22,7 @@ struct GemmDesc {
     int shift;                // 0..63
     int64_t init;             // added to the sum before the shift
     int64_t a_rs, b_rs;       // operand divisors (truncating), 1 = none
+    bool few_positions = false;       // the attention of a decoding step or a handful of positions (gemm_small_launch)
 };
 
 enum GemmPath { kPathAuto = 0, kPathValu = 1, kPathMfma = 2 };
@@ -97,6 +98,9 @@ void gemm_valu_launch(const GemmDesc &d, GuardArgs *guard = nullptr);
 // Matrix-vector kernel of the same family for one or two rows of A against k-contiguous B: one launch, nothing
 // guessed.  Returns false (nothing launched) for any other descriptor.
 bool gemm_gemv_launch(const GemmDesc &d);
+
+// Small products in one launch, nothing guessed (gemm_small.hip).  Returns false (nothing launched) for any other descriptor.
+bool gemm_small_launch(const GemmDesc &d);
 
 // Limb-decomposed i8 MFMA.  Returns 0 when the product was launched, 1 when the descriptor is outside what it
 // supports or memory for its buffers is short (nothing was launched; the caller falls back to the VALU path), -1 on an

@@ -48,6 +48,11 @@ bool gemm_dispatch(const char *name, const GemmDesc &d)
         g_last_path = kPathValu; g_last_la = 0; g_last_lb = 0; g_last_digits = false;
         return check_launch(name);
     }
+    // small products (a decoding step's attention): one launch of tiles that nothing is guessed for
+    if (d.few_positions && g_gemm_path == kPathAuto && !gemm_mfma_is_prepared(d.B) && gemm_small_launch(d)) {
+        g_last_path = kPathMfma; g_last_la = 0; g_last_lb = 0; g_last_digits = false;
+        return check_launch(name);
+    }
     // up to 16 rows against k-contiguous weights: the 16-row MFMA tiles, digit counts taken from the data on the device
     // (prepared weights keep the kernels that read their planes: fewer bytes per weight)
     if (g_gemm_path != kPathValu && !gemm_mfma_is_prepared(d.B)) {
@@ -208,6 +213,8 @@ void einsum_bshd_hdc_bshc(const int64_t *q_nope, const int32_t *wkv_b_1, int64_t
     zk::gemm_dispatch(name, d);
 }
 
+constexpr int kFewPositions = 8;
+
 // out[b,s,h,t] = (rescale/2 + sum_c A[b,s,h,c] * Bm[b,t,c]) >> rescale: one GEMM per batch, rows (s,h).
 void einsum_bshc_btc_bsht(const int64_t *A, const int64_t *B, int64_t *C, int64_t rescale,
                           int Bsz, int S, int H, int T, int Cdim)
@@ -221,6 +228,7 @@ void einsum_bshc_btc_bsht(const int64_t *A, const int64_t *B, int64_t *C, int64_
     d.B = B; d.b32 = 0; d.ldbn = Cdim; d.ldbk = 1; d.sB = (long)T * Cdim;
     d.C = C; d.R = nullptr; d.ldc = T; d.sC = (long)S * H * T;
     d.G = Bsz; d.M = S * H; d.N = T; d.K = Cdim;
+    d.few_positions = S <= kFewPositions;
     d.shift = (int)rescale; d.init = rescale / 2; d.a_rs = 1; d.b_rs = 1;
     zk::gemm_dispatch(name, d);
 }
@@ -238,6 +246,7 @@ void einsum_bsht_btc_bshc(const int64_t *A, const int64_t *B, int64_t *C, int64_
     d.B = B; d.b32 = 0; d.ldbn = 1; d.ldbk = Cdim; d.sB = (long)T * Cdim;
     d.C = C; d.R = nullptr; d.ldc = Cdim; d.sC = (long)S * H * Cdim;
     d.G = Bsz; d.M = S * H; d.N = Cdim; d.K = T;
+    d.few_positions = S <= kFewPositions;
     d.shift = (int)rescale; d.init = rescale / 2; d.a_rs = 1; d.b_rs = 1;
     zk::gemm_dispatch(name, d);
 }

@@ -1,0 +1,190 @@
+// Products so small that launches and latencies are all they cost (the attention of a decoding step: 128 heads against
+// the cache): one launch, nothing guessed.  What bounds them is one round trip to memory per step of a wavefront.
+//
+// On the general kernel such a product is three dependent launches (tiles cut along K, the sum of the slices, the guarded
+// launch behind a guess of digit counts) of 4 to 11 us each.  Here a workgroup owns a tile of 16 x 16 outputs and all of K: its
+// eight wavefronts take every eighth step of 64 k, load their fragments straight into registers (the four lanes of a
+// row read 64 contiguous bytes per load), take the digit counts that those need (3, 4 or 5 per operand, gemm_frag16.h),
+// split, multiply, and meet in LDS with their 128-bit sums.  A wavefront that meets values beyond five digits (2^38 and up)
+// multiplies its share again with nine digits.
+#include "gemm_frag16.h"
+
+namespace zk {
+
+struct SmallParams {
+    const int64_t *A, *B;
+    int64_t *C;
+    long lda, sA, ldbn, ldbk, sB, ldc, sC;
+    int M, N, K, shift, tiles_m, tiles_n;
+    int64_t init;
+};
+
+constexpr int kSmallWaves = 8, kSmallTile = 16, kSmallDiagonals = 9;
+// Where it pays, against the general and the 16-row kernels over 250 shapes of 5 to 600 rows and 16 to 2048 columns (those / this, us):
+// one round of tiles 0.3-0.8 of their time up to K = 2048 (128 rows x [512,779] n-contiguous 20.0 / 8.9, 50 x [94,321] (5,5)
+// 24.9 / 7.1, 32 x [1513,759] 23.2 / 8.7, 274 x [161,2145] 22.6 / 16.2) and level at 4000; two rounds up to K = 1024 (128 x
+// [779,512] 18.8 / 13.3, 128 x [1024,512] 19.4 / 13.9; 66 x [1398,1454] 26.5 / 30.4); three rounds no longer (256 x [779,512]
+// 21.6 / 24.3).  Offered to it are scores and values of up to eight positions; other products keep the kernels that guess
+// digit counts and check them.
+constexpr int kSmallMaxK = 2048, kSmallMaxKTwoRounds = 1024;
+
+template <int NA, int NB>
+__device__ __forceinline__ void small_step(const RawFrag<false> &fa_raw, const RawFrag<false> &fb_raw, v4i (&acc)[kSmallDiagonals])
+{
+    v4i fa[NA], fb[NB];
+    split_frag<NA, false>(fa_raw, fa);
+    split_frag<NB, false>(fb_raw, fb);
+#pragma unroll
+    for (int i = 0; i < NA; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+            acc[i + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[i], fb[j], acc[i + j], 0, 0, 0);
+}
+
+// A fragment element by element: byte b of the fragment is k = frag_k(q, b) of the step, `lane_at` the lane's offset with its
+// first k, `step_at` the step's first element, `ldk` elements from one k to the next; k of `k_left` and up are zeros.  (Offsets
+// that all lanes share stay in scalar registers.)
+__device__ __forceinline__ void load_elements(RawFrag<false> &f, const int64_t *base, long lane_at, long step_at, long ldk, int k_left)
+{
+#pragma unroll
+    for (int b = 0; b < 16; b++) {
+        const int k = frag_k<false>(0, b);
+        const int64_t *at = base + (step_at + k * ldk);
+        const int64_t x = k < k_left ? ((const ZK_GLOBAL_MEM int64_t *)at)[lane_at] : 0;
+        f.v[b >> 1][2 * (b & 1)] = (int)(uint32_t)x;
+        f.v[b >> 1][2 * (b & 1) + 1] = (int)(uint32_t)((uint64_t)x >> 32);
+    }
+}
+
+// BKM: B is contiguous along n
+template <bool BKM>
+__global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(SmallParams p)
+{
+    __shared__ Words red[kSmallWaves][4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, q = lane >> 4;
+    const int per_batch = p.tiles_m * p.tiles_n;
+    const int g = blockIdx.x / per_batch, rem = blockIdx.x - g * per_batch;
+    const int m0 = rem % p.tiles_m * kSmallTile, n0 = rem / p.tiles_m * kSmallTile;
+
+    // this lane's rows (clamped: what lies past the end lands in outputs that are never stored)
+    const long a_at = (long)g * p.sA + (long)(m0 + li < p.M ? m0 + li : p.M - 1) * p.lda;
+    const long ldbk = BKM ? p.ldbk : 1;
+    const int nc = n0 + li < p.N ? n0 + li : p.N - 1;
+    const long b_at = (long)g * p.sB + (long)nc * p.ldbn;
+    const bool a_vec = (((uintptr_t)p.A | (uintptr_t)(p.lda * 8) | (uintptr_t)(p.sA * 8)) & 15) == 0;
+    const bool b_vec = !BKM && (((uintptr_t)p.B | (uintptr_t)(p.ldbn * 8) | (uintptr_t)(p.sB * 8)) & 15) == 0;
+
+    const int steps = (p.K + 63) / 64;
+    auto load = [&](int ks, RawFrag<false> &fa, RawFrag<false> &fb) {
+        const int k0 = ks * 64, k_left = p.K - k0, kq = frag_k<false>(q, 0);
+        const bool whole = k_left >= 64;
+        if (whole && b_vec) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) fb.v[j] = *(const ZK_GLOBAL_MEM v4i *)(p.B + b_at + k0 + frag_k<false>(q, 2 * j));
+        } else if (whole) {
+            load_elements(fb, p.B, b_at + kq * ldbk, k0 * ldbk, ldbk, 64);
+        } else {
+            load_elements(fb, p.B, b_at + kq * ldbk, k0 * ldbk, ldbk, k_left - kq);
+        }
+        if (whole && a_vec) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) fa.v[j] = *(const ZK_GLOBAL_MEM v4i *)(p.A + a_at + k0 + frag_k<false>(q, 2 * j));
+        } else if (whole) {
+            load_elements(fa, p.A, a_at + kq, k0, 1, 64);
+        } else {
+            load_elements(fa, p.A, a_at + kq, k0, 1, k_left - kq);
+        }
+    };
+    // accumulator register r of lane (li, q) holds row 4*q + r, column li of the tile
+    bool wide = false;
+    {
+        v4i acc[kSmallDiagonals];
+#pragma unroll
+        for (int d = 0; d < kSmallDiagonals; d++) acc[d] = v4i{ 0, 0, 0, 0 };
+        for (int ks = wave; ks < steps; ks += kSmallWaves) {
+            RawFrag<false> fa;
+            RawFrag<false> fb;
+            load(ks, fa, fb);
+            const int na = wave_digits(magnitude_or<false>(fa));
+            const int nb = wave_digits(magnitude_or<false>(fb));
+            if (na > 5 || nb > 5) { wide = true; break; }
+            switch ((na - 3) * 3 + (nb - 3)) {
+            case 0: small_step<3, 3>(fa, fb, acc); break;
+            case 1: small_step<3, 4>(fa, fb, acc); break;
+            case 2: small_step<3, 5>(fa, fb, acc); break;
+            case 3: small_step<4, 3>(fa, fb, acc); break;
+            case 4: small_step<4, 4>(fa, fb, acc); break;
+            case 5: small_step<4, 5>(fa, fb, acc); break;
+            case 6: small_step<5, 3>(fa, fb, acc); break;
+            case 7: small_step<5, 4>(fa, fb, acc); break;
+            default: small_step<5, 5>(fa, fb, acc); break;
+            }
+        }
+        // (5 pairs x 64 products of 2^14 a step)
+        static_assert((kSmallMaxK / 64 + kSmallWaves - 1) / kSmallWaves * 5L * 64 * 16384 <= kMaxDiagonal, "the int32 accumulators hold a wavefront's share");
+#pragma unroll
+        for (int o = 0; o < 4; o++) red[wave][o][lane] = sum_diagonals<kSmallDiagonals>([&](int d) { return acc[d][o]; }, 0);
+    }
+    if (wide) {
+        // wider than five digits: this wavefront's steps once more with nine (what lies at 2^128 and above does not matter)
+        constexpr int D = 16;
+        v4i acc[D];
+#pragma unroll
+        for (int d = 0; d < D; d++) acc[d] = v4i{ 0, 0, 0, 0 };
+        for (int ks = wave; ks < steps; ks += kSmallWaves) {
+            RawFrag<false> fa_raw;
+            RawFrag<false> fb_raw;
+            load(ks, fa_raw, fb_raw);
+            v4i fa[9], fb[9];
+            split_frag<9, false>(fa_raw, fa);
+            split_frag<9, false>(fb_raw, fb);
+#pragma unroll
+            for (int i = 0; i < 9; i++)
+#pragma unroll
+                for (int j = 0; j < 9; j++)
+                    if (i + j < D) acc[i + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[i], fb[j], acc[i + j], 0, 0, 0);
+        }
+        static_assert((kSmallMaxK / 64 + kSmallWaves - 1) / kSmallWaves * 9L * 64 * 16384 <= kMaxDiagonal, "and of nine digits");
+#pragma unroll
+        for (int o = 0; o < 4; o++) red[wave][o][lane] = sum_diagonals<D>([&](int d) { return acc[d][o]; }, 0);
+    }
+    __syncthreads();
+    const int m = m0 + 4 * q + (wave & 3), n = n0 + li;
+    if (wave >= 4 || m >= p.M || n >= p.N) return;
+    u128 s = (u128)(i128)p.init;
+#pragma unroll
+    for (int w = 0; w < kSmallWaves; w++) {
+        const Words t = red[w][wave][lane];
+        s += (u128)((uint64_t)t.w[3] << 32 | t.w[2]) << 64 | ((uint64_t)t.w[1] << 32 | t.w[0]);
+    }
+    const uint64_t lo = (uint64_t)s, hi = (uint64_t)(s >> 64);
+    p.C[(long)g * p.sC + (long)m * p.ldc + n] = (int64_t)((lo >> p.shift) | ((hi << 1) << (63 - p.shift)));
+}
+
+static int device_cus()
+{
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        return n;
+    }();
+    return cus;
+}
+
+bool gemm_small_launch(const GemmDesc &d)
+{
+    const long tiles_m = (d.M + kSmallTile - 1) / kSmallTile, tiles_n = (d.N + kSmallTile - 1) / kSmallTile, tiles = tiles_m * tiles_n * d.G;
+    if (d.b32 || d.R || d.a_rs != 1 || d.b_rs != 1 || d.K < 1 || d.K > kSmallMaxK || d.M < 1 || d.N < 1 || d.G < 1) return false;
+    if (tiles > (d.K <= kSmallMaxKTwoRounds ? 2 : 1) * (long)device_cus()) return false;
+    SmallParams p = {};
+    p.A = d.A; p.B = reinterpret_cast<const int64_t *>(d.B); p.C = d.C;
+    p.lda = d.lda; p.sA = d.sA; p.ldbn = d.ldbn; p.ldbk = d.ldbk; p.sB = d.sB; p.ldc = d.ldc; p.sC = d.sC;
+    p.M = d.M; p.N = d.N; p.K = d.K; p.shift = d.shift; p.init = d.init;
+    p.tiles_m = (int)tiles_m; p.tiles_n = (int)tiles_n;
+    const dim3 grid((unsigned)tiles), block(64 * kSmallWaves);
+    if (d.ldbk != 1) gemm_small_kernel<true><<<grid, block, 0, 0>>>(p);
+    else gemm_small_kernel<false><<<grid, block, 0, 0>>>(p);
+    return true;
+}
+
+}  // namespace zk
