@@ -993,6 +993,26 @@ def test_softmax_lengths(K, oracle, fn, Q, T):
     assert np.array_equal(host(R), x), "input must stay intact by default"
 
 
+@pytest.mark.parametrize("rows", [1, 1024, 1025])
+@pytest.mark.parametrize("T", [256, 257, 511, 512, 514, 1023, 1026, 2048])
+def test_softmax_rows_shared_by_wavefronts(K, oracle, rows, T):
+    """up to 1024 rows of more than 256 elements are shared by four wavefronts each, longer lists by none: both sides of the
+    line, maxima and sums in any of the four, with and without score preparation, both roundings"""
+    rng = np.random.default_rng(rows + T)
+    x = _scores(rng, (1, rows, 1, T), 19)
+    x[0, :, 0, rng.integers(0, T)] += 1 << 20
+    C = torch.empty_like(dev(x))
+    for fn in ("softmax_q19", "softmax_q21"):
+        getattr(K, fn)(dev(x), C)
+        assert np.array_equal(host(C), getattr(oracle, fn)(x)[0])
+    s1, s2 = rand_i64(rng, (1, rows, 1, T), 23), rand_i64(rng, (1, rows, 1, T), 23)
+    mask = np.where(np.arange(T)[None, :] <= rng.integers(0, T, size=(rows, 1)), 0, -(64 << 36)).astype(np.int64)
+    prepared = (s1 + s2) * 94 // 695 + mask[None, :, None, :]
+    kept = torch.empty_like(C)
+    K.softmax_q19_scores(dev(s1), dev(s2), dev(mask), C, kept)
+    assert np.array_equal(host(kept), prepared) and np.array_equal(host(C), oracle.softmax_q19(prepared)[0])
+
+
 @pytest.mark.parametrize("fn", ["softmax_q19", "softmax_q21"])
 @pytest.mark.parametrize("T", [96, 1024, 3001])
 def test_softmax_reference_clobber_mode(K, oracle, fn, T):

@@ -1,6 +1,6 @@
 // Fixed-point row softmax over the last dimension of [Bsz,S,H,T] int64 (Q19 truncating, Q21 rounding).
 //
-// Rows of up to 2048 elements are handled one row per wavefront: the row is read once with 16-byte loads
+// Rows of up to 2048 elements are handled one row per wavefront (or, few rows, per four of them): the row is read once with 16-byte loads
 // into registers, the maximum and the weight sum are 64-lane butterfly reductions, and the per-row divide
 // is a reciprocal multiply made exact by a remainder test.  HBM traffic is the algorithmic 16 bytes per
 // element (24 when the reference's write-back of the weights into the input is switched on).
@@ -69,6 +69,7 @@ __device__ __forceinline__ int64_t smx_norm(int64_t w, int64_t s, double inv, bo
 }
 
 constexpr int kSmxThreads = 256;
+constexpr long kSmxFewRows = 1024;          // see softmax_wave_kernel
 
 // Optional score preparation fused into the row load (inference/model.py:896-906 does it with three tensor ops):
 //   x = floor((s1 + s2) * mul / div) + mask[s][t]
@@ -122,7 +123,11 @@ __device__ __forceinline__ int64_t smx_prepare(int64_t v, const SmxPre &pre, lon
 // element / stores behind each batch / as it is, inputs that change from call to call: 128 rows of 779 13.3 / 10.5 / 9.3 us, 31104
 // of 243 67 / 53 / 48, 2304 of 1142 22.6 / 25.8 / 20.8, of 2047 58 / 62 / 49, 131072 of 1024 761 / 765 / 765 (5.6 TB/s; 780 with
 // sixteen at a time, which takes wavefronts).  Without preparation 4224 of 1999 41.3 -> 30.9.
-template <int Q, int EPL, bool VEC, bool PRE>
+// RW: wavefronts that share a row.  Few rows (a decoding step has one per head) leave most of the device idle and live on the chain of
+// loads, divisions and reductions of one wavefront: four of them per row, meeting twice in LDS, have a quarter of it each.
+// One / four wavefronts per row, with preparation: 128 rows of 300 6.3 / 6.0 us, of 779 9.6 / 6.0, of 2047 23.4 / 8.0, 1024 rows of 512 8.1 /
+// 6.1, of 1142 15.0 / 10.3; of 243 elements equal; 2048 rows of 512 9.0 / 8.8, of 1500 20.9 / 22.3, 4096 of 1024 25.4 / 27.2.
+template <int Q, int EPL, bool VEC, bool PRE, int RW = 1>
 __global__ __launch_bounds__(kSmxThreads) void softmax_wave_kernel(int64_t *__restrict__ R, int64_t *__restrict__ C,
                                                                    const int64_t *__restrict__ lut_g, long rows, int T,
                                                                    int clobber, SmxPre pre)
@@ -130,13 +135,15 @@ __global__ __launch_bounds__(kSmxThreads) void softmax_wave_kernel(int64_t *__re
     __shared__ int64_t lut[256];
     lut[threadIdx.x] = lut_g[threadIdx.x];
     __syncthreads();
-    const int lane = threadIdx.x & 63;
-    const long row = (long)blockIdx.x * (kSmxThreads / 64) + (threadIdx.x >> 6);
+    static_assert(RW == 1 || RW == kSmxThreads / 64, "a row belongs to a wavefront or to the workgroup");
+    constexpr int LANES = 64 * RW;
+    const int lane = threadIdx.x & (LANES - 1);
+    const long row = (long)blockIdx.x * (kSmxThreads / LANES) + threadIdx.x / LANES;
     if (row >= rows) return;
     int64_t *x = R + row * T;
     int64_t *c = C + row * T;
 
-    auto at = [&](int j) { return VEC ? ((j >> 1) * 64 + lane) * 2 + (j & 1) : j * 64 + lane; };     // element j of this lane
+    auto at = [&](int j) { return VEC ? ((j >> 1) * LANES + lane) * 2 + (j & 1) : j * LANES + lane; };     // element j of this lane
     int64_t v[EPL];
     int64_t rmax = INT64_MIN;
     constexpr bool LATE = !VEC || EPL != 16;
@@ -186,6 +193,13 @@ __global__ __launch_bounds__(kSmxThreads) void softmax_wave_kernel(int64_t *__re
             if (at(j) < T) store_score(at(j), j);
     }
     rmax = wave_max_i64(rmax);
+    __shared__ int64_t red[2][kSmxThreads / 64];
+    if (RW > 1) {
+        if ((lane & 63) == 0) red[0][lane >> 6] = rmax;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < RW; w++) rmax = red[0][w] > rmax ? red[0][w] : rmax;
+    }
 
     uint64_t sum = 0;
 #pragma unroll
@@ -195,7 +209,15 @@ __global__ __launch_bounds__(kSmxThreads) void softmax_wave_kernel(int64_t *__re
             sum += (uint64_t)v[j];
         }
     }
-    const int64_t s = (int64_t)wave_sum_u64(sum);
+    sum = wave_sum_u64(sum);
+    if (RW > 1) {
+        if ((lane & 63) == 0) red[1][lane >> 6] = (int64_t)sum;
+        __syncthreads();
+        sum = 0;
+#pragma unroll
+        for (int w = 0; w < RW; w++) sum += (uint64_t)red[1][w];
+    }
+    const int64_t s = (int64_t)sum;
     const bool fast = s >= ((int64_t)1 << 12) && s < ((int64_t)1 << 52);
     const double inv = fast ? 1.0 / (double)s : 0.0;
 
@@ -261,18 +283,19 @@ __global__ __launch_bounds__(kSmxThreads) void softmax_block_kernel(int64_t *__r
     for (int i = threadIdx.x; i < T; i += kSmxThreads) c[i] = smx_norm<Q>(c[i], s, inv, fast);
 }
 
-template <int Q, int EPL>
+template <int Q, int EPL, int RW = 1>
 static void launch_wave(int64_t *R, int64_t *C, const int64_t *lut, long rows, int T, bool vec, int clobber, const SmxPre *pre)
 {
-    long blocks = (rows + (kSmxThreads / 64) - 1) / (kSmxThreads / 64);
+    constexpr int PER_BLOCK = kSmxThreads / (64 * RW);
+    long blocks = (rows + PER_BLOCK - 1) / PER_BLOCK;
     const dim3 grid((unsigned)blocks), block(kSmxThreads);
     SmxPre none = {};
     if (pre) {
-        if (vec) softmax_wave_kernel<Q, EPL, true, true><<<grid, block, 0, 0>>>(R, C, lut, rows, T, clobber, *pre);
-        else softmax_wave_kernel<Q, EPL, false, true><<<grid, block, 0, 0>>>(R, C, lut, rows, T, clobber, *pre);
+        if (vec) softmax_wave_kernel<Q, EPL, true, true, RW><<<grid, block, 0, 0>>>(R, C, lut, rows, T, clobber, *pre);
+        else softmax_wave_kernel<Q, EPL, false, true, RW><<<grid, block, 0, 0>>>(R, C, lut, rows, T, clobber, *pre);
     } else {
-        if (vec) softmax_wave_kernel<Q, EPL, true, false><<<grid, block, 0, 0>>>(R, C, lut, rows, T, clobber, none);
-        else softmax_wave_kernel<Q, EPL, false, false><<<grid, block, 0, 0>>>(R, C, lut, rows, T, clobber, none);
+        if (vec) softmax_wave_kernel<Q, EPL, true, false, RW><<<grid, block, 0, 0>>>(R, C, lut, rows, T, clobber, none);
+        else softmax_wave_kernel<Q, EPL, false, false, RW><<<grid, block, 0, 0>>>(R, C, lut, rows, T, clobber, none);
     }
 }
 
@@ -298,7 +321,11 @@ static void launch_softmax(const char *name, int64_t *R, int64_t *C, const int64
     int clobber = g_softmax_clobber && !pre ? 1 : 0;
     bool vec = (T % 2 == 0) && ((((uintptr_t)R | (uintptr_t)C) & 15) == 0);
     if (pre && ((((uintptr_t)pre->s2 | (uintptr_t)pre->mask | (uintptr_t)pre->scores) & 15) != 0)) vec = false;
-    if (T <= 128) launch_wave<Q, 2>(R, C, lut, rows, T, vec, clobber, pre);
+    if (rows <= kSmxFewRows && T > 256 && T <= 2048) {
+        if (T <= 512) launch_wave<Q, 2, 4>(R, C, lut, rows, T, vec, clobber, pre);
+        else if (T <= 1024) launch_wave<Q, 4, 4>(R, C, lut, rows, T, vec, clobber, pre);
+        else launch_wave<Q, 8, 4>(R, C, lut, rows, T, vec, clobber, pre);
+    } else if (T <= 128) launch_wave<Q, 2>(R, C, lut, rows, T, vec, clobber, pre);
     else if (T <= 256) launch_wave<Q, 4>(R, C, lut, rows, T, vec, clobber, pre);
     else if (T <= 512) launch_wave<Q, 8>(R, C, lut, rows, T, vec, clobber, pre);
     else if (T <= 1024) launch_wave<Q, 16>(R, C, lut, rows, T, vec, clobber, pre);
