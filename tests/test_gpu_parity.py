@@ -1281,6 +1281,19 @@ def test_rmsnorm_residual_fusion(K, oracle, N, k, w32, inplace):
     assert np.array_equal(host(C), Ce)
 
 
+@pytest.mark.parametrize("M", [64, 65, 256, 257])
+@pytest.mark.parametrize("N,bits", [(513, 31), (2048, 55), (2049, 31), (5001, 20), (7168, 31), (8192, 62)])
+def test_rmsnorm_row_counts_next_to_the_lines(K, oracle, M, N, bits):
+    """few rows take a thousand threads each: both sides of each line, odd lengths, statistics of one digit to six"""
+    rng = np.random.default_rng(M * N)
+    X, Y, W = rand_i64(rng, (M, N), bits), rand_i64(rng, (M, N), 22), rng.integers(1 << 5, 1 << 20, size=(N,), dtype=np.int32)
+    Xe, Ce, rmse = oracle.RMS_Norm_residual_int64(X, Y, 8, W, 1, N)
+    Xn, C, rms = K.RMS_Norm_residual_int64(dev(X), dev(Y), 8, dev(W), 1, N)
+    assert np.array_equal(host(Xn), Xe) and np.array_equal(rms[:M].numpy(), rmse) and np.array_equal(host(C), Ce)
+    C, rms = K.RMS_Norm_int64(Xn, dev(W), 1, N)
+    assert np.array_equal(rms[:M].numpy(), rmse) and np.array_equal(host(C), Ce)
+
+
 def test_rmsnorm_residual_fusion_unaligned_and_bad_arguments(K, oracle):
     rng = np.random.default_rng(77)
     M, N = 3, 1000
