@@ -1903,6 +1903,16 @@ def test_converters(K, oracle):
     K._check("converters")
 
 
+@pytest.mark.parametrize("rows,cols", [(300, 4), (1, 1024), (129, 12), (257, 2052), (2051, 2052), (513, 8200), (100, 16384)])
+def test_fp8_quantisation_over_ends_of_rows(K, oracle, rows, cols):
+    """workgroups take the pieces of the matrix one after the other, whatever its rows: rows of one piece, ends of rows and of
+    scale blocks inside a workgroup's stretch, a last stretch that is not whole, one and two pieces per thread"""
+    rng = np.random.default_rng(rows + cols)
+    w = rng.integers(0, 256, size=(rows, cols), dtype=np.uint8)
+    sc = rng.uniform(1e-5, 4e-4, size=((rows + 127) // 128, (cols + 127) // 128)).astype(np.float32)
+    assert np.array_equal(host(K.quantize_fp8_weight(dev(w), dev(sc), 28)), oracle.fp8_block_scaled_to_int32(w, sc, 28))
+
+
 @pytest.mark.parametrize("shape", [(256, 256), (300, 520), (1, 129), (129, 1), (7, 2048), (2048, 7168)])
 def test_fp8_checkpoint_quantisation(K, oracle, shape):
     """block-scaled fp8 weights -> int32 fixed point in one pass (convert2.py:144-147): every fp8 code incl. NaN,

@@ -50,42 +50,39 @@ __device__ __forceinline__ int64_t round_to_i64(float z)
 
 typedef int v4i_q __attribute__((ext_vector_type(4)));
 
-// Four consecutive weights of a row per thread and round (cols % 4 == 0, aligned pointers): a 4-byte load and a 16-byte
-// store, adjacent lanes on adjacent pieces so that both are contiguous over the wave; four rounds in flight per thread.
-// A 128-wide scale block covers whole 4-element pieces, so one scale serves a piece.
-__global__ __launch_bounds__(256) void fp8_to_int32_vec_kernel(const uint8_t *__restrict__ w, const float *__restrict__ scale,
-                                                               int32_t *__restrict__ out, int rows, int pieces_per_row,
-                                                               int scale_cols, float mult)
+// Four consecutive weights per thread and round (cols % 4 == 0, aligned pointers): a 4-byte load and a 16-byte store, adjacent
+// lanes on adjacent pieces so that both are contiguous over the wave, and over the launch: workgroup after workgroup takes the next
+// U * 256 pieces of the matrix, whatever the rows.  A 128-wide scale block covers whole 4-element pieces, so one scale serves a
+// piece.  Bound by its stores, four fifths of the bytes.  A workgroup per row, four rounds of 1024 pieces one after the other /
+// as it is: [18432,7168] 148.6 / 103.7 us (6.4 TB/s), [2048,7168] 17.9 / 14.3, [7168,2048] 16.0 / 13.8, [576,7168] 7.4 / 5.3,
+// [1536,1536] 3.9 / 3.6, [100,16000] 9.0 / 3.3.
+template <int U>
+__global__ __launch_bounds__(256) void fp8_to_int32_vec_kernel(const uint32_t *__restrict__ w, const float *__restrict__ scale,
+                                                               v4i_q *__restrict__ out, long pieces, int pieces_per_row, int scale_cols, float mult)
 {
-    // blockIdx.y walks the rows, blockIdx.x the 1024-piece stretches of a row: no division anywhere
-    for (int row = blockIdx.y; row < rows; row += gridDim.y) {
-        const float *srow = scale + (long)(row / kScaleBlock) * scale_cols;
-        const uint32_t *wrow = reinterpret_cast<const uint32_t *>(w) + (long)row * pieces_per_row;
-        v4i_q *orow = reinterpret_cast<v4i_q *>(out) + (long)row * pieces_per_row;
-        for (int base = blockIdx.x * 1024; base < pieces_per_row; base += gridDim.x * 1024) {
-            uint32_t in[4];
-            float s[4];
+    const long first = (long)blockIdx.x * (256 * U);
+    const long row0 = first / pieces_per_row;
+    const unsigned col0 = (unsigned)(first - row0 * pieces_per_row) + threadIdx.x;
+    uint32_t in[U];
+    float s[U];
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int pc = base + u * 256 + threadIdx.x;
-                if (pc < pieces_per_row) {
-                    in[u] = __builtin_nontemporal_load(wrow + pc);
-                    s[u] = srow[pc / (kScaleBlock / 4)];
-                }
-            }
+    for (int u = 0; u < U; u++) {
+        if (first + u * 256 + threadIdx.x >= pieces) continue;
+        unsigned col = col0 + u * 256;
+        long row = row0;
+        if (col >= (unsigned)pieces_per_row) { const unsigned n = col / (unsigned)pieces_per_row; row += n; col -= n * (unsigned)pieces_per_row; }
+        in[u] = __builtin_nontemporal_load(w + first + u * 256 + threadIdx.x);
+        s[u] = scale[(row / kScaleBlock) * scale_cols + col / (kScaleBlock / 4)];
+    }
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int pc = base + u * 256 + threadIdx.x;
-                if (pc < pieces_per_row) {
-                    v4i_q o;
-                    o[0] = round_to_i32(round_to_bf16(e4m3fn_to_f32<0>(in[u]) * s[u]) * mult);
-                    o[1] = round_to_i32(round_to_bf16(e4m3fn_to_f32<1>(in[u]) * s[u]) * mult);
-                    o[2] = round_to_i32(round_to_bf16(e4m3fn_to_f32<2>(in[u]) * s[u]) * mult);
-                    o[3] = round_to_i32(round_to_bf16(e4m3fn_to_f32<3>(in[u]) * s[u]) * mult);
-                    __builtin_nontemporal_store(o, orow + pc);
-                }
-            }
-        }
+    for (int u = 0; u < U; u++) {
+        if (first + u * 256 + threadIdx.x >= pieces) continue;
+        v4i_q o;
+        o[0] = round_to_i32(round_to_bf16(e4m3fn_to_f32<0>(in[u]) * s[u]) * mult);
+        o[1] = round_to_i32(round_to_bf16(e4m3fn_to_f32<1>(in[u]) * s[u]) * mult);
+        o[2] = round_to_i32(round_to_bf16(e4m3fn_to_f32<2>(in[u]) * s[u]) * mult);
+        o[3] = round_to_i32(round_to_bf16(e4m3fn_to_f32<3>(in[u]) * s[u]) * mult);
+        __builtin_nontemporal_store(o, out + first + u * 256 + threadIdx.x);
     }
 }
 
@@ -150,8 +147,16 @@ void fp8_block_scaled_to_int32(const uint8_t *w, const float *scale, int32_t *ou
     const long n = (long)rows * cols;
     if (cols % 4 == 0 && ((uintptr_t)w & 3) == 0 && ((uintptr_t)out & 15) == 0) {
         const int ppr = cols / 4;
-        const dim3 grid((unsigned)((ppr + 4095) / 4096), (unsigned)(rows < 65535 ? rows : 65535));     // a workgroup walks up to 4 stretches
-        zk::fp8_to_int32_vec_kernel<<<grid, dim3(256), 0, 0>>>(w, scale, out, rows, ppr, scale_cols, mult);
+        const long pieces = (long)rows * ppr;
+        // two pieces per thread once the launch is long enough to be bound by memory (one / two, us: 1536 x 1536 3.6 / 4.4, 576 x 7168
+        // 5.3 / 5.1, 2048 x 7168 15.7 / 14.3, 18432 x 7168 122.7 / 103.7; four: 110.9)
+        const bool two = pieces > (1L << 20);
+        const long blocks = (pieces + (two ? 511 : 255)) / (two ? 512 : 256);
+        if (blocks > 0x7FFFFFFFL) { zk::set_error(zk::kUnsupportedSize, "%s: matrix too large", name); return; }
+        const uint32_t *wp = reinterpret_cast<const uint32_t *>(w);
+        zk::v4i_q *op = reinterpret_cast<zk::v4i_q *>(out);
+        if (two) zk::fp8_to_int32_vec_kernel<2><<<dim3((unsigned)blocks), dim3(256), 0, 0>>>(wp, scale, op, pieces, ppr, scale_cols, mult);
+        else zk::fp8_to_int32_vec_kernel<1><<<dim3((unsigned)blocks), dim3(256), 0, 0>>>(wp, scale, op, pieces, ppr, scale_cols, mult);
     } else {
         zk::fp8_to_int32_kernel<<<dim3(zk::grid_for(n)), dim3(256), 0, 0>>>(w, scale, out, n, cols, scale_cols, mult);
     }
