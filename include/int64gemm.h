@@ -245,8 +245,9 @@ long zk_gemm_grouped_mfma_calls(void);
 /* How many of those launches ran on the kernel that streams int32 weights through LDS rings (K a multiple of 32,
  * sixteen digit pairs or more; ZK_STREAM32_MIN_PAIRS and ZK_NO_STREAM32 move or remove that choice). */
 long zk_gemm_grouped_streamed_calls(void);
-/* How many GEMM launches so far ran on the software-pipelined kernel that reads digit planes on both sides (weights
- * prepared with zk_gemm_prepare_weights, and a B that is small next to the product; ZK_NO_PIPE=1 switches it off). */
+/* How many GEMM launches so far ran on the software-pipelined kernels that read digit planes on both sides (weights
+ * prepared with zk_gemm_prepare_weights, and a B that is small next to the product, with A split by a pass in front or by the
+ * kernel itself; ZK_NO_PIPE=1 switches them off). */
 long zk_gemm_pipe_calls(void);
 /* No reference counterpart: model weights do not change between calls, so a weight matrix W[N,K] (int64, or int32 with
  * b32 != 0; groups == 0, B = the device pointer later passed as B) or all the matrices of a device table of pointers

@@ -526,7 +526,8 @@ void gemm_mfma_release_workspace()
 }
 
 // A B that is small next to the product (a KV cache against the queries of a whole prompt, one head's weights) is split
-// into digit planes like A, and the product runs on the pipelined kernel for planes on both sides (gemm_mfma_pipe.h).
+// into digit planes like A, and the product runs on the pipelined kernel for planes on both sides (gemm_mfma_pipe.h),
+// or on the one that splits A itself (gemm_mfma_rowtile.h, see rowtile_parts).
 // One more launch in front and the general kernel's time, against its own split of B in every tile.  Whole calls, (3,4)
 // digits, general against this: k-contiguous int64 B, 131072 rows x [1024,512] 1124 / 864 us, x [1024,64] 379 / 268, 31104 x
 // [243,512] 95.8 / 84.0, 8192 x [512,512] (3,3) 35.2 / 36.7, (4,4) 49.8 / 49.0; the heads' int32 weights (128 heads, 1024
@@ -569,7 +570,12 @@ static int rowtile_parts(const GemmDesc &d, int na, int nb, int bn, int cus)
     const long old_tiles = (long)((d.M + 127) / 128) * d.G * tiles_n;
     double best = (double)((old_tiles + cus - 1) / cus) * tile + (double)d.G * d.M * d.K * (8 + na) / 5.5e6 + 5;
     int parts = 0;
-    if (bn != 128 && d.K < 128) return 0;               // (584 rows of 128 heads [350,80], (4,4): 126 / 147)
+    // It has to be expected to win by more than the estimate is off.  Tiles of 64x64 read twice the planes per product of the pipelined
+    // kernel's 128x64 ((6,3) digits 20096 x [1760,542] 352 / 374, (5,4) 46464 x [512,214] 158 / 166, 79104 x [512,1081] 984 / 906, (4,4) 584
+    // rows of 128 heads [350,80] 126 / 147), and nine products a step leave less to hide the splits behind ((3,3) 94976 x [1903,512] 958 /
+    // 1022, 54144 x [588,98] 97 / 111, 29568 x [512,244] 72 / 61).
+    if (bn != 128 && d.K < 128) return 0;
+    best *= bn != 128 ? 0.93 : (na * nb <= 9 ? 0.88 : 0.97);
     for (long n = 1; n <= tiles_n && n <= 8; n++) {
         const double t = (double)((row_tiles * n + slots - 1) / slots) * (split + (double)((tiles_n + n - 1) / n) * tile);
         if (t < best) { best = t; parts = (int)n; }
@@ -889,6 +895,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             else if (k_over) return kDeclined;
         }
         const long row_items = rowtile.fn ? (long)p.tiles_m * d.G * p.col_parts : 0;
+        const int row_slots = row_items > 2L * g_cache.cus ? 2 : 1;
         const long blocks = rowtile.fn ? std::min<long>(row_items, 2L * g_cache.cus) : (long)p.main_tiles + (total - p.main_tiles) * p.split;
         long plane_wgs = 0, b_plane_wgs = 0;
         p.fail_class = inst->na > 5 || inst->nb > 5 ? 2 : 1;
@@ -912,8 +919,8 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
                 // (the one product of the model with zeros in A worth finding: a causal prompt's probabilities times the values)
                 b.row_tiles = kmajor && !d.b32 && !rowtile.fn ? (long)p.tiles_m * d.G : 0;
                 got = grow(g_cache.b_planes, g_cache.b_planes_bytes, (size_t)(b.gstride * b_batches), "digit planes of B");
-                // (two slots per workgroup for the digit planes of its row tiles)
-                if (got == kDone && rowtile.fn) got = grow(g_cache.planes, g_cache.planes_bytes, (size_t)blocks * 2 * (kRowtileRows / 32) * ksteps * inst->na * 1024, "digit-plane buffer");
+                // (slots for the digit planes of its row tiles, two per workgroup that has more than one)
+                if (got == kDone && rowtile.fn) got = grow(g_cache.planes, g_cache.planes_bytes, (size_t)blocks * row_slots * (kRowtileRows / 32) * ksteps * inst->na * 1024, "digit-plane buffer");
                 if (got == kDone && b.row_tiles) got = grow(g_cache.row_steps, g_cache.row_steps_count, (size_t)b.row_tiles, "step counts");
             }
             if (got == kDone) got = grow(g_cache.seen, g_cache.seen_count, (size_t)(blocks + plane_wgs + b_plane_wgs), "digit counts");
@@ -948,7 +955,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
 #undef ZK_BPL
             p.B = b.planes; p.b_nsub = b.nsub; p.b_ksteps = ksteps; p.b_gstride = d.sB != 0 ? b.gstride : 0;
             p.row_steps = b.row_steps;
-            if (rowtile.fn) { p.a_planes = g_cache.planes; p.a_ksteps = ksteps; p.items = (int)row_items; }
+            if (rowtile.fn) { p.a_planes = g_cache.planes; p.a_msub = row_slots; p.a_ksteps = ksteps; p.items = (int)row_items; }
         }
         p.seen = pipe.fn ? nullptr : g_cache.seen;
         const size_t lds = rowtile.fn ? rowtile.lds : pipe.fn ? pipe.lds : 2 * (size_t)inst->kk * ((BM / 32) * inst->na + (BN / 32) * inst->nb) * 1024 + 9 * 1024 + 16;

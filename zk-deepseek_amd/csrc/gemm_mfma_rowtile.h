@@ -29,7 +29,8 @@ constexpr size_t rowtile_lds_bytes(int na, int nb) { return (size_t)rowtile_stag
 
 constexpr int kRowtileRows = 64;
 
-// One item: row tile `tm` of batch `g`.  p.a_planes: slots of `a_ksteps` steps of planes of 64 rows, one per workgroup.
+// One item: row tile `tm` of batch `g`, or a part of its tile columns.  p.a_planes: slots of `a_ksteps` steps of planes of 64 rows, `a_msub` per
+// workgroup: two, or one where no workgroup has a second item.
 template <int NA, int NB>
 __global__ __launch_bounds__(256, 2) void gemm_mfma_rowtile_kernel(MfmaParams)
 {
@@ -48,10 +49,10 @@ __global__ __launch_bounds__(256, 2) void gemm_mfma_rowtile_kernel(MfmaParams)
     const unsigned ring_lds = (unsigned)(uintptr_t)rowtile_smem, lane16 = (unsigned)lane * 16;
 
     int it_g, it_tm, tn_begin, tn_end, nsteps;
-    uint64_t slot;                                          // the planes of the row tile that is multiplied: one of this workgroup's two
+    uint64_t slot;                                          // the planes of the row tile that is multiplied: one of this workgroup's slots
     auto slot_of = [&](int turn) {
         ConstParams &p = launch_args();
-        return uniform64((uint64_t)p.a_planes + (uint64_t)(blockIdx.x * 2 + (turn & 1)) * (2 * NA * 1024) * p.a_ksteps);
+        return uniform64((uint64_t)p.a_planes + (uint64_t)(blockIdx.x * p.a_msub + (turn & 1)) * (2 * NA * 1024) * p.a_ksteps);
     };
 
     // ---- the split: 64 rows of A -> planes [32-row group][step][digit] of 1 KB; a thread owns 8 elements of a row and step ----
