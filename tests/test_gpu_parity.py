@@ -1903,10 +1903,12 @@ def test_converters(K, oracle):
     K._check("converters")
 
 
-@pytest.mark.parametrize("rows,cols", [(300, 4), (1, 1024), (129, 12), (257, 2052), (2051, 2052), (513, 8200), (100, 16384)])
+@pytest.mark.parametrize("rows,cols", [(300, 4), (1, 1024), (129, 12), (257, 2052), (2051, 2052), (513, 8200), (100, 16384),
+                                       (1, 5), (131, 5), (300, 6), (129, 129), (257, 1027), (2053, 2051), (3, 1), (5, 3)])
 def test_fp8_quantisation_over_ends_of_rows(K, oracle, rows, cols):
     """workgroups take the pieces of the matrix one after the other, whatever its rows: rows of one piece, ends of rows and of
-    scale blocks inside a workgroup's stretch, a last stretch that is not whole, one and two pieces per thread"""
+    scale blocks inside a workgroup's stretch, a last stretch that is not whole, one and two pieces per thread,
+    pieces over two rows and weights behind the last whole piece"""
     rng = np.random.default_rng(rows + cols)
     w = rng.integers(0, 256, size=(rows, cols), dtype=np.uint8)
     sc = rng.uniform(1e-5, 4e-4, size=((rows + 127) // 128, (cols + 127) // 128)).astype(np.float32)

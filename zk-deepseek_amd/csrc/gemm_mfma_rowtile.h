@@ -14,7 +14,7 @@
 // own position) end there; the split sees it.
 // What bounds it: power.  131072 rows x [1024,512], (3,4) digits: 630 us with neither stores nor splits (2.6 POP/s of i8
 // products, at 1.7-2.0 GHz), 595 with every load at one address on top; the stores add 105 and the splits 110-130,
-// overlapped or not.  Whole calls, pass over A and pipelined kernel / this, one box: 131072 x [1024,512] 874 / 818-840 us,
+// overlapped or not.  Whole calls, pass over A and pipelined kernel / this, both on one device: 131072 x [1024,512] 874 / 818-840 us,
 // x [1024,64] 262 / 236, values of 1024 causal tokens 642 / 562-574, 31104 x [243,512] 86 / 81.
 #pragma once
 #include "gemm_mfma_pipe.h"

@@ -86,6 +86,51 @@ __global__ __launch_bounds__(256) void fp8_to_int32_vec_kernel(const uint32_t *_
     }
 }
 
+// The same for rows of any length from four on: a piece's four weights may lie in two rows and in two scale blocks, and what is left
+// behind the last whole piece goes one by one.  Bound by memory where the matrix is large.  Element by element with a division each, as below / this, us:
+// 2048 x 7169 26.5 / 17.2, 18432 x 7171 277 / 125 (5.3 TB/s), 16384 x 513 16.5 / 11.9, 576 x 7166 8.6 / 6.3, 1535 x 1537 5.7 / 4.4;
+// 100 x 101, 5000 x 130 and 100000 x 5 the same.
+template <int U>
+__global__ __launch_bounds__(256) void fp8_to_int32_any_kernel(const uint8_t *__restrict__ w, const float *__restrict__ scale, int32_t *__restrict__ out,
+                                                               long n, int cols, int scale_cols, float mult)
+{
+    const long first = (long)blockIdx.x * (256 * U), pieces = n >> 2;
+    const long row0 = 4 * first / cols;
+    const unsigned col0 = (unsigned)(4 * first - row0 * cols) + 4 * threadIdx.x;
+    uint32_t in[U];
+    float s[U][4];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const long piece = first + u * 256 + threadIdx.x;
+        if (piece >= pieces) continue;
+        unsigned col = col0 + u * 1024;
+        const unsigned over = col / (unsigned)cols;
+        long row = row0 + over;
+        col -= over * (unsigned)cols;
+        in[u] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(w) + piece);
+#pragma unroll
+        for (int z = 0; z < 4; z++) {
+            s[u][z] = scale[(row / kScaleBlock) * scale_cols + col / kScaleBlock];
+            if (++col == (unsigned)cols) { col = 0; row++; }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const long piece = first + u * 256 + threadIdx.x;
+        if (piece >= pieces) continue;
+        v4i_q o;
+        o[0] = round_to_i32(round_to_bf16(e4m3fn_to_f32<0>(in[u]) * s[u][0]) * mult);
+        o[1] = round_to_i32(round_to_bf16(e4m3fn_to_f32<1>(in[u]) * s[u][1]) * mult);
+        o[2] = round_to_i32(round_to_bf16(e4m3fn_to_f32<2>(in[u]) * s[u][2]) * mult);
+        o[3] = round_to_i32(round_to_bf16(e4m3fn_to_f32<3>(in[u]) * s[u][3]) * mult);
+        __builtin_nontemporal_store(o, reinterpret_cast<v4i_q *>(out) + piece);
+    }
+    const long rest = 4 * pieces + threadIdx.x;
+    if (blockIdx.x == 0 && rest < n)
+        out[rest] = round_to_i32(round_to_bf16(e4m3fn_to_f32<0>(w[rest]) * scale[(rest / cols / kScaleBlock) * scale_cols + rest % cols / kScaleBlock]) * mult);
+}
+
+// element by element: rows of one to three weights, and pointers that are not aligned to the vectors
 __global__ __launch_bounds__(256) void fp8_to_int32_kernel(const uint8_t *__restrict__ w, const float *__restrict__ scale,
                                                            int32_t *__restrict__ out, long n, int cols, int scale_cols, float mult)
 {
@@ -157,6 +202,12 @@ void fp8_block_scaled_to_int32(const uint8_t *w, const float *scale, int32_t *ou
         zk::v4i_q *op = reinterpret_cast<zk::v4i_q *>(out);
         if (two) zk::fp8_to_int32_vec_kernel<2><<<dim3((unsigned)blocks), dim3(256), 0, 0>>>(wp, scale, op, pieces, ppr, scale_cols, mult);
         else zk::fp8_to_int32_vec_kernel<1><<<dim3((unsigned)blocks), dim3(256), 0, 0>>>(wp, scale, op, pieces, ppr, scale_cols, mult);
+    } else if (cols >= 4 && ((uintptr_t)w & 3) == 0 && ((uintptr_t)out & 15) == 0) {
+        const bool two = n > (4L << 20);  // as above, in weights
+        const long blocks = (n / 4 + (two ? 511 : 255)) / (two ? 512 : 256);
+        if (blocks > 0x7FFFFFFFL) { zk::set_error(zk::kUnsupportedSize, "%s: matrix too large", name); return; }
+        if (two) zk::fp8_to_int32_any_kernel<2><<<dim3((unsigned)blocks), dim3(256), 0, 0>>>(w, scale, out, n, cols, scale_cols, mult);
+        else zk::fp8_to_int32_any_kernel<1><<<dim3((unsigned)blocks), dim3(256), 0, 0>>>(w, scale, out, n, cols, scale_cols, mult);
     } else {
         zk::fp8_to_int32_kernel<<<dim3(zk::grid_for(n)), dim3(256), 0, 0>>>(w, scale, out, n, cols, scale_cols, mult);
     }
