@@ -1294,6 +1294,32 @@ def test_rmsnorm_row_counts_next_to_the_lines(K, oracle, M, N, bits):
     assert np.array_equal(rms[:M].numpy(), rmse) and np.array_equal(host(C), Ce)
 
 
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("M,N,off", [(300, 513, 0), (300, 1023, 1), (70, 2049, 0), (300, 4097, 0), (300, 8191, 1), (300, 8192, 1), (3, 8193, 0),
+                                     (2, 16383, 0), (2, 16384, 1), (3, 16385, 0), (2, 16386, 0), (2, 24575, 0), (2, 24576, 1), (2, 24577, 0)])
+def test_rmsnorm_rows_in_pairs(K, oracle, M, N, off, wide):
+    """rows that begin at any element and end with half a pair, next to the lines between the kernels, the longest in registers;
+    every buffer `off` elements behind a 16-byte boundary, the one behind the row's last left as it was"""
+    rng = np.random.default_rng(M * N + off)
+    X, Y = rand_i64(rng, (M, N), 31), rand_i64(rng, (M, N), 22)
+    W = rng.integers(-(1 << 20), 1 << 20, size=(N,), dtype=np.int64 if wide else np.int32)
+    Xe, Ce, rmse = oracle.RMS_Norm_residual_int64(X, Y, 8, W, 1, N)
+    buf = [torch.full((off + M * N + 1,), 77, dtype=torch.int64, device="cuda") for _ in range(4)]
+    Xd, Yd, Xo, C = (b[off:-1].view(M, N) for b in buf)
+    Xd.copy_(dev(X)), Yd.copy_(dev(Y))
+    Wd, r = dev(W), torch.empty((M,), dtype=torch.int64, device="cuda")
+    fused, residual = (K.lib.rms_norm_fused_64, K.lib.rms_norm_residual_fused_64) if wide else (K.lib.rms_norm_fused_32, K.lib.rms_norm_residual_fused_32)
+    residual(Xd.data_ptr(), Yd.data_ptr(), 8, Wd.data_ptr(), Xo.data_ptr(), r.data_ptr(), C.data_ptr(), M, N, 1, N)
+    torch.cuda.synchronize()
+    K._check("residual norm")
+    assert np.array_equal(host(Xo), Xe) and np.array_equal(host(C), Ce) and np.array_equal(host(r), rmse)
+    C.zero_(), r.zero_()
+    fused(Xo.data_ptr(), Wd.data_ptr(), r.data_ptr(), C.data_ptr(), M, N, 1, N)
+    torch.cuda.synchronize()
+    assert np.array_equal(host(C), Ce) and np.array_equal(host(r), rmse)
+    assert all(int(b[-1]) == 77 and int(b[:off].sum()) == 77 * off for b in buf)
+
+
 def test_rmsnorm_residual_fusion_unaligned_and_bad_arguments(K, oracle):
     rng = np.random.default_rng(77)
     M, N = 3, 1000

@@ -276,6 +276,7 @@ __device__ __forceinline__ U192 block_sum_u192(U192 acc, U192 *red)
 }
 
 typedef int v4i_r __attribute__((ext_vector_type(4)));
+typedef v4i_r v4i_r8 __attribute__((aligned(8)));   // two elements from any element on
 
 // Statistic only: one workgroup per row, any N.
 __global__ __launch_bounds__(kRmsThreads) void rms_stat_kernel(const int64_t *__restrict__ A, int64_t *__restrict__ rms,
@@ -374,13 +375,37 @@ __global__ __launch_bounds__(kRmsThreads) void rms_apply_kernel(const int64_t *_
     }
 }
 
+// Two elements of a row.  VEC: streaming accesses to whole 16 bytes.  Otherwise the row may begin at any element and end with a pair of
+// which only the first is there: the same 16 bytes from an 8-byte boundary (the hardware asks for four), through the caches, since
+// neighbours share lines (350 rows of 8191, us: 18.6 so, 22.5 with streaming loads, 21.3 with streaming loads and stores; 350 rows
+// of 18431 39.0, 35.8, 36.2, but 64 of them 14.7, 16.3, 15.4).
+template <bool VEC>
+__device__ __forceinline__ v4i_r load_pair(const int64_t *p, bool both)
+{
+    if (VEC) return __builtin_nontemporal_load(reinterpret_cast<const v4i_r *>(p));
+    if (both) return *reinterpret_cast<const v4i_r8 *>(p);
+    const uint2 t = *reinterpret_cast<const uint2 *>(p);
+    return { (int)t.x, (int)t.y, 0, 0 };
+}
+
+template <bool VEC>
+__device__ __forceinline__ void store_pair(int64_t *p, int64_t x, int64_t y, bool both)
+{
+    const v4i_r t = { (int)(uint32_t)x, (int)(uint32_t)((uint64_t)x >> 32), (int)(uint32_t)y, (int)(uint32_t)((uint64_t)y >> 32) };
+    if (VEC) __builtin_nontemporal_store(t, reinterpret_cast<v4i_r *>(p));
+    else if (both) *reinterpret_cast<v4i_r8 *>(p) = t;
+    else *p = x;
+}
+
 // Statistic + normalisation, one workgroup of THREADS per row, the row kept in registers (N <= THREADS * EPT).
 // Long rows get more threads rather than more elements per thread: fewer registers mean more rows in flight per
 // compute unit, which is what hides the serial stretch (reduction, division, square root) in the middle.
-// VEC: N is even and the rows are 16-byte aligned: elements are moved two at a time with streaming accesses.
+// VEC: N is even and the rows are 16-byte aligned.  Other rows went one element at a time, each through the remainder tier, their
+// weights read behind the barrier; in pairs like the rest, before / now, us: 1 row of 7169 10.8 / 7.2, 256 rows 15.7 / 11.1, 500 rows
+// 20.1 / 15.8, 500 of 1537 8.8 / 7.4, 500 of 12001 33.8 / 26.7.
 // WPE: waves per SIMD the register allocation must leave room for.  Rows of 4K-8K elements run three workgroups of
 // eight waves per compute unit (WPE 6, 80 registers): measured, a third row in flight pays; a fourth (64 registers)
-// spills again and does not.
+// spills again and does not.  Rows that are not VEC spill at 80 already and run two (500 rows of 8191 24.1 -> 17.2 us).
 // RES: the row that is normalised is A + Y * 2^k (wrapping int64 arithmetic, as the tensor ops of the reference's
 // residual connection, inference/model.py:1465, 1472), and that sum is also stored to Xout (which may be A itself).
 struct RmsResidual { const int64_t *Y; int64_t *Xout; int k; };
@@ -395,51 +420,39 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) 
     const long row = blockIdx.x;
     const int64_t *a = A + row * N;
     int64_t v[EPT];
-    // The weights travel with the row: no load is left for after the barrier.  Where several rows share a compute unit
+    // The weights travel with the row, up to eight elements a thread: no load is left for after the barrier.  Where several rows share a compute unit
     // through a tight register budget (WPE > 1), int32 weights wait in LDS instead of registers (each thread reads
     // back only what it wrote itself): the registers they held were being spilled to scratch memory, and those
     // stores reached HBM (a tenth more bytes written than the output has).
-    constexpr bool W_LDS = VEC && sizeof(WT) == 4 && WPE > 1;
+    constexpr bool W_LDS = sizeof(WT) == 4 && WPE > 1;
+    constexpr bool W_LATE = EPT >= 16 && !W_LDS;   // they would spill: read behind the barrier (500 rows of 16383 36.9 -> 35.0 us)
     __shared__ WPair<WT> w_s[W_LDS ? (EPT / 2) * THREADS : 1];
-    WPair<WT> wp[W_LDS ? 1 : EPT / 2];
+    WPair<WT> wp[W_LDS || W_LATE ? 1 : EPT / 2];
     const bool w_vec = ((uintptr_t)W & 7) == 0;
     SquareSum sq;
-    if (VEC) {
 #pragma unroll
-        for (int j = 0; j < EPT / 2; j++) {
-            const int i = (j * THREADS + threadIdx.x) * 2;
-            if (i < N) {
-                const v4i_r t = __builtin_nontemporal_load(reinterpret_cast<const v4i_r *>(a + i));
-                if (W_LDS) w_s[j * THREADS + threadIdx.x] = load_w_pair(W, i, w_vec);
-                else wp[j] = load_w_pair(W, i, w_vec);
-                v[2 * j] = (int64_t)(((uint64_t)(uint32_t)t[1] << 32) | (uint32_t)t[0]);
-                v[2 * j + 1] = (int64_t)(((uint64_t)(uint32_t)t[3] << 32) | (uint32_t)t[2]);
-                if (RES) {
-                    const v4i_r u = __builtin_nontemporal_load(reinterpret_cast<const v4i_r *>(res.Y + row * N + i));
-                    const uint64_t y0 = ((uint64_t)(uint32_t)u[1] << 32) | (uint32_t)u[0];
-                    const uint64_t y1 = ((uint64_t)(uint32_t)u[3] << 32) | (uint32_t)u[2];
-                    v[2 * j] = (int64_t)((uint64_t)v[2 * j] + (y0 << res.k));
-                    v[2 * j + 1] = (int64_t)((uint64_t)v[2 * j + 1] + (y1 << res.k));
-                    const v4i_r o = { (int)(uint32_t)v[2 * j], (int)(uint32_t)((uint64_t)v[2 * j] >> 32),
-                                      (int)(uint32_t)v[2 * j + 1], (int)(uint32_t)((uint64_t)v[2 * j + 1] >> 32) };
-                    __builtin_nontemporal_store(o, reinterpret_cast<v4i_r *>(res.Xout + row * N + i));
-                }
-                sq.add(v[2 * j]);
-                sq.add(v[2 * j + 1]);
+    for (int j = 0; j < EPT / 2; j++) {
+        const int i = (j * THREADS + threadIdx.x) * 2;
+        if (i < N) {
+            const bool both = VEC || i + 1 < N;
+            const v4i_r t = load_pair<VEC>(a + i, both);
+            if (!W_LATE) {
+                const WPair<WT> w = both ? load_w_pair(W, i, w_vec) : WPair<WT>{ W[i], 0 };
+                if (W_LDS) w_s[j * THREADS + threadIdx.x] = w;
+                else wp[j] = w;
             }
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < EPT; j++) {
-            const int i = j * THREADS + threadIdx.x;
-            if (i < N) {
-                v[j] = a[i];
-                if (RES) {
-                    v[j] = (int64_t)((uint64_t)v[j] + ((uint64_t)res.Y[row * N + i] << res.k));
-                    res.Xout[row * N + i] = v[j];
-                }
-                sq.add(v[j]);
+            v[2 * j] = (int64_t)(((uint64_t)(uint32_t)t[1] << 32) | (uint32_t)t[0]);
+            v[2 * j + 1] = (int64_t)(((uint64_t)(uint32_t)t[3] << 32) | (uint32_t)t[2]);
+            if (RES) {
+                const v4i_r u = load_pair<VEC>(res.Y + row * N + i, both);
+                const uint64_t y0 = ((uint64_t)(uint32_t)u[1] << 32) | (uint32_t)u[0];
+                const uint64_t y1 = ((uint64_t)(uint32_t)u[3] << 32) | (uint32_t)u[2];
+                v[2 * j] = (int64_t)((uint64_t)v[2 * j] + (y0 << res.k));
+                v[2 * j + 1] = (int64_t)((uint64_t)v[2 * j + 1] + (y1 << res.k));
+                store_pair<VEC>(res.Xout + row * N + i, v[2 * j], v[2 * j + 1], both);
             }
+            sq.add(v[2 * j]);
+            sq.add(v[2 * j + 1]);
         }
     }
     U192 tot = block_sum_u192<THREADS>(sq.total(), red);
@@ -452,37 +465,36 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) 
     const int64_t r = rms_s;
     const bool fast_r = r > 0 && r < ((int64_t)1 << 62);
     const double inv_r = fast_r ? 1.0 / (double)r : 0.0;
-    if (VEC) {
-        unsigned redo = 0;
+    const auto weights = [&](int i, int j, bool both) -> WPair<WT> {
+        if (W_LDS) return w_s[j * THREADS + threadIdx.x];
+        if (!W_LATE) return wp[W_LDS || W_LATE ? 0 : j];
+        return both ? load_w_pair(W, i, w_vec) : WPair<WT>{ W[i], 0 };
+    };
+    unsigned redo = 0;
+#pragma unroll
+    for (int j = 0; j < EPT / 2; j++) {
+        const int i = (j * THREADS + threadIdx.x) * 2;
+        if (i < N) {
+            const bool both = VEC || i + 1 < N;
+            bool ok0, ok1;
+            const WPair<WT> w = weights(i, j, both);
+            const int64_t c0 = rms_apply_quick(v[2 * j], w.x, inv_r, fast_r, ok0);
+            const int64_t c1 = rms_apply_quick(v[2 * j + 1], w.y, inv_r, fast_r, ok1);
+            redo |= (ok0 ? 0u : 1u << (2 * j)) | (ok1 || !both ? 0u : 2u << (2 * j));
+            store_pair<VEC>(C + row * N + i, c0, c1, both);
+        }
+    }
+    // rare: elements the quick tier could not settle go through the other two and are stored again
+    if (__builtin_expect(redo != 0, 0)) {
 #pragma unroll
         for (int j = 0; j < EPT / 2; j++) {
             const int i = (j * THREADS + threadIdx.x) * 2;
-            if (i < N) {
-                bool ok0, ok1;
-                const WPair<WT> w = W_LDS ? w_s[j * THREADS + threadIdx.x] : wp[W_LDS ? 0 : j];
-                const int64_t c0 = rms_apply_quick(v[2 * j], w.x, inv_r, fast_r, ok0);
-                const int64_t c1 = rms_apply_quick(v[2 * j + 1], w.y, inv_r, fast_r, ok1);
-                redo |= (ok0 ? 0u : 1u << (2 * j)) | (ok1 ? 0u : 2u << (2 * j));
-                const v4i_r t = { (int)(uint32_t)c0, (int)(uint32_t)((uint64_t)c0 >> 32), (int)(uint32_t)c1,
-                                  (int)(uint32_t)((uint64_t)c1 >> 32) };
-                __builtin_nontemporal_store(t, reinterpret_cast<v4i_r *>(C + row * N + i));
-            }
-        }
-        // rare: elements the quick tier could not settle go through the other two and are stored again
-        if (__builtin_expect(redo != 0, 0)) {
-#pragma unroll
-            for (int j = 0; j < EPT / 2; j++) {
-                const int i = (j * THREADS + threadIdx.x) * 2;
-                const WPair<WT> w = W_LDS ? w_s[j * THREADS + threadIdx.x] : wp[W_LDS ? 0 : j];
+            if (redo & (3u << (2 * j))) {
+                const bool both = VEC || i + 1 < N;
+                const WPair<WT> w = weights(i, j, both);
                 if (redo & (1u << (2 * j))) C[row * N + i] = rms_apply_one(v[2 * j], w.x, r, inv_r, fast_r);
                 if (redo & (2u << (2 * j))) C[row * N + i + 1] = rms_apply_one(v[2 * j + 1], w.y, r, inv_r, fast_r);
             }
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < EPT; j++) {
-            const int i = j * THREADS + threadIdx.x;
-            if (i < N) C[row * N + i] = rms_apply_one(v[j], W[i], r, inv_r, fast_r);
         }
     }
 }
@@ -539,7 +551,7 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
     const bool vec = N % 2 == 0 && (align & 15) == 0;
     const dim3 grid((unsigned)M);
 #define ZK_RMS_LAUNCH2(THREADS, EPT, WPE, VEC, RES) \
-    rms_fused_kernel<WT, THREADS, EPT, VEC, WPE, RES><<<grid, dim3(THREADS), 0, 0>>>(A, W, rms, C, N, eps, dim, r)
+    rms_fused_kernel<WT, THREADS, EPT, VEC, VEC || WPE < 4 ? WPE : 4, RES><<<grid, dim3(THREADS), 0, 0>>>(A, W, rms, C, N, eps, dim, r)
 #define ZK_RMS_LAUNCH(THREADS, EPT, WPE)                                                   \
     do {                                                                                   \
         if (res) { if (vec) ZK_RMS_LAUNCH2(THREADS, EPT, WPE, true, true); else ZK_RMS_LAUNCH2(THREADS, EPT, WPE, false, true); }    \
@@ -555,6 +567,10 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
     else if (N <= 4096) ZK_RMS_LAUNCH(512, 8, 1);
     else if (N <= 8192) ZK_RMS_LAUNCH(512, 16, 6);
     else if (N <= 16384) ZK_RMS_LAUNCH(1024, 16, 1);
+    // up to what a workgroup's registers hold: 24 elements a thread, 128 registers of which 20 spill; statistic and product as two
+    // kernels, as below / this, us: 1 row of 18432 10.5 / 9.9, 64 rows 17.3 / 13.7, 500 rows 42.6 / 33.1, with residual 74.6 / 56.3;
+    // 500 rows of 24576 54.0 / 42.2, of 18431 71.2 / 45.1
+    else if (N <= 24576 && M <= 65535) ZK_RMS_LAUNCH(1024, 24, 1);
     else {
         const int64_t *src = A;
         if (res) {
