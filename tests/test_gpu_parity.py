@@ -1325,7 +1325,7 @@ def test_rmsnorm_residual_fusion_unaligned_and_bad_arguments(K, oracle):
     M, N = 3, 1000
     X, Y = rand_i64(rng, (M, N), 37), rand_i64(rng, (M, N), 30)
     W = rng.integers(1, 1 << 20, size=(N,), dtype=np.int32)
-    # rows that start 8 bytes off a 16-byte boundary take the element-wise path
+    # rows that start 8 bytes off a 16-byte boundary take the path of unaligned pairs
     buf = torch.zeros((M * N + 1,), dtype=torch.int64, device="cuda")
     Xd = buf[1:].view(M, N)
     Xd.copy_(dev(X))
