@@ -1347,6 +1347,26 @@ def test_rmsnorm_residual_fusion_unaligned_and_bad_arguments(K, oracle):
     K.lib.zk_clear_error()
 
 
+@pytest.mark.parametrize("N", [16385, 24577])
+def test_rmsnorm_refuses_rows_before_it_writes(K, N):
+    """more than 65535 rows of more than 16384 elements are refused, and nothing has been written by then: neither the residual
+    sum, which may go over the input itself, nor the statistic"""
+    M = 65536
+    X = torch.full((M, N), 3, dtype=torch.int64, device="cuda")
+    C = torch.empty((M, N), dtype=torch.int64, device="cuda")
+    r = torch.full((M,), 7, dtype=torch.int64, device="cuda")
+    W = torch.ones((N,), dtype=torch.int64, device="cuda")
+    W32 = W.to(torch.int32)
+    for call in (lambda: K.lib.rms_norm_residual_fused_64(X.data_ptr(), X.data_ptr(), 2, W.data_ptr(), X.data_ptr(), r.data_ptr(), C.data_ptr(), M, N, 1, N),
+                 lambda: K.lib.rms_norm_residual_fused_32(X.data_ptr(), X.data_ptr(), 2, W32.data_ptr(), X.data_ptr(), r.data_ptr(), C.data_ptr(), M, N, 1, N),
+                 lambda: K.lib.rms_norm_fused_32(X.data_ptr(), W32.data_ptr(), r.data_ptr(), C.data_ptr(), M, N, 1, N)):
+        call()
+        torch.cuda.synchronize()
+        assert K.lib.zk_last_error() == 3
+        K.lib.zk_clear_error()
+        assert bool((r == 7).all()) and all(bool((x == 3).all()) for x in X.split(8192))
+
+
 def test_rmsnorm_model_shape(K, oracle):
     """[256,7168] at residual-stream magnitudes (|x| up to ~2^37, Q31) with int32 Q21 weights"""
     g = torch.Generator(device="cpu").manual_seed(600)

@@ -507,11 +507,17 @@ static bool rms_args_ok(const char *name, const void *A, const void *W, const vo
     return true;
 }
 
+// rms_apply_kernel has its rows in the second dimension of the grid
+static bool apply_rows_ok(const char *name, int M)
+{
+    if (M > 65535) set_error(kUnsupportedSize, "%s: more than 65535 rows", name);
+    return M <= 65535;
+}
+
 template <typename WT>
 static void launch_apply(const char *name, const int64_t *A, const WT *W, const int64_t *rms, int64_t *C, int M, int N)
 {
-    if (!rms_args_ok(name, A, W, rms, C, M, N)) return;
-    if (M > 65535) { set_error(kUnsupportedSize, "%s: more than 65535 rows", name); return; }
+    if (!rms_args_ok(name, A, W, rms, C, M, N) || !apply_rows_ok(name, M)) return;
     const int per_wg = kRmsThreads * kApplyEpt;
     dim3 grid((unsigned)((N + per_wg - 1) / per_wg), (unsigned)M);
     const bool vec = N % 2 == 0 && (((uintptr_t)A | (uintptr_t)C) & 15) == 0;
@@ -572,6 +578,7 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
     // 500 rows of 24576 54.0 / 42.2, of 18431 71.2 / 45.1
     else if (N <= 24576 && M <= 65535) ZK_RMS_LAUNCH(1024, 24, 1);
     else {
+        if (!apply_rows_ok(name, M)) return;          // before the residual sum or the statistic is written
         const int64_t *src = A;
         if (res) {
             const long n = (long)M * N;
