@@ -1961,6 +1961,29 @@ def test_fp8_quantisation_over_ends_of_rows(K, oracle, rows, cols):
     assert np.array_equal(host(K.quantize_fp8_weight(dev(w), dev(sc), 28)), oracle.fp8_block_scaled_to_int32(w, sc, 28))
 
 
+@pytest.mark.parametrize("cols", [32768, 32766])
+def test_fp8_quantisation_of_more_than_one_launch(K, oracle, cols):
+    """a launch takes less than 2^32 threads: a matrix of 2^35 weights and some, whose slabs repeat, gives the same slab again
+    and again, up to its last weight"""
+    slab, count = 4096, 257
+    if torch.cuda.mem_get_info()[0] < 220 << 30:
+        pytest.skip("needs 176 GB of free device memory")
+    rows = slab * count - 1
+    rng = np.random.default_rng(cols)
+    w = rng.integers(0, 256, size=(slab, cols), dtype=np.uint8)
+    sc = rng.uniform(1e-5, 4e-4, size=(slab // 128, (cols + 127) // 128)).astype(np.float32)
+    expected = dev(oracle.fp8_block_scaled_to_int32(w, sc, 28))
+    W = dev(w).repeat(count, 1)[:rows]
+    out = K.quantize_fp8_weight(W, dev(sc).repeat(count, 1), 28)
+    try:
+        for i in range(count):
+            part = out[i * slab:(i + 1) * slab]
+            assert torch.equal(part, expected[:part.shape[0]]), i
+    finally:
+        del W, out, part
+        torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("shape", [(256, 256), (300, 520), (1, 129), (129, 1), (7, 2048), (2048, 7168)])
 def test_fp8_checkpoint_quantisation(K, oracle, shape):
     """block-scaled fp8 weights -> int32 fixed point in one pass (convert2.py:144-147): every fp8 code incl. NaN,

@@ -58,9 +58,9 @@ typedef int v4i_q __attribute__((ext_vector_type(4)));
 // [1536,1536] 3.9 / 3.6, [100,16000] 9.0 / 3.3.
 template <int U>
 __global__ __launch_bounds__(256) void fp8_to_int32_vec_kernel(const uint32_t *__restrict__ w, const float *__restrict__ scale,
-                                                               v4i_q *__restrict__ out, long pieces, int pieces_per_row, int scale_cols, float mult)
+                                                               v4i_q *__restrict__ out, long begin, long pieces, int pieces_per_row, int scale_cols, float mult)
 {
-    const long first = (long)blockIdx.x * (256 * U);
+    const long first = begin + (long)blockIdx.x * (256 * U);
     const long row0 = first / pieces_per_row;
     const unsigned col0 = (unsigned)(first - row0 * pieces_per_row) + threadIdx.x;
     uint32_t in[U];
@@ -92,9 +92,9 @@ __global__ __launch_bounds__(256) void fp8_to_int32_vec_kernel(const uint32_t *_
 // 100 x 101, 5000 x 130 and 100000 x 5 the same.
 template <int U>
 __global__ __launch_bounds__(256) void fp8_to_int32_any_kernel(const uint8_t *__restrict__ w, const float *__restrict__ scale, int32_t *__restrict__ out,
-                                                               long n, int cols, int scale_cols, float mult)
+                                                               long begin, long n, int cols, int scale_cols, float mult)
 {
-    const long first = (long)blockIdx.x * (256 * U), pieces = n >> 2;
+    const long first = begin + (long)blockIdx.x * (256 * U), pieces = n >> 2;
     const long row0 = 4 * first / cols;
     const unsigned col0 = (unsigned)(4 * first - row0 * cols) + 4 * threadIdx.x;
     uint32_t in[U];
@@ -126,8 +126,21 @@ __global__ __launch_bounds__(256) void fp8_to_int32_any_kernel(const uint8_t *__
         __builtin_nontemporal_store(o, reinterpret_cast<v4i_q *>(out) + piece);
     }
     const long rest = 4 * pieces + threadIdx.x;
-    if (blockIdx.x == 0 && rest < n)
+    if (first == 0 && rest < n)
         out[rest] = round_to_i32(round_to_bf16(e4m3fn_to_f32<0>(w[rest]) * scale[(rest / cols / kScaleBlock) * scale_cols + rest % cols / kScaleBlock]) * mult);
+}
+
+// Launches of 256 threads over `pieces` pieces: launch(grid, first piece, two pieces a thread).
+// Two pieces per thread once the launch is long enough to be bound by memory (one / two, us: 1536 x 1536 3.6 / 4.4, 576 x 7168
+// 5.3 / 5.1, 2048 x 7168 15.7 / 14.3, 18432 x 7168 122.7 / 103.7; four: 110.9).  A grid of 2^32 threads or more runs only what is
+// left of their number in 32 bits, with no error: a matrix of 2^35 weights and more takes several launches.
+template <typename Launch>
+static void for_stretches(long pieces, Launch launch)
+{
+    constexpr long kMost = 1L << 23;
+    const bool two = pieces > (1L << 20);
+    const long per_block = two ? 512 : 256, blocks = (pieces + per_block - 1) / per_block;
+    for (long b = 0; b < blocks; b += kMost) launch(dim3((unsigned)(blocks - b < kMost ? blocks - b : kMost)), b * per_block, two);
 }
 
 // element by element: rows of one to three weights, and pointers that are not aligned to the vectors
@@ -192,22 +205,17 @@ void fp8_block_scaled_to_int32(const uint8_t *w, const float *scale, int32_t *ou
     const long n = (long)rows * cols;
     if (cols % 4 == 0 && ((uintptr_t)w & 3) == 0 && ((uintptr_t)out & 15) == 0) {
         const int ppr = cols / 4;
-        const long pieces = (long)rows * ppr;
-        // two pieces per thread once the launch is long enough to be bound by memory (one / two, us: 1536 x 1536 3.6 / 4.4, 576 x 7168
-        // 5.3 / 5.1, 2048 x 7168 15.7 / 14.3, 18432 x 7168 122.7 / 103.7; four: 110.9)
-        const bool two = pieces > (1L << 20);
-        const long blocks = (pieces + (two ? 511 : 255)) / (two ? 512 : 256);
-        if (blocks > 0x7FFFFFFFL) { zk::set_error(zk::kUnsupportedSize, "%s: matrix too large", name); return; }
         const uint32_t *wp = reinterpret_cast<const uint32_t *>(w);
         zk::v4i_q *op = reinterpret_cast<zk::v4i_q *>(out);
-        if (two) zk::fp8_to_int32_vec_kernel<2><<<dim3((unsigned)blocks), dim3(256), 0, 0>>>(wp, scale, op, pieces, ppr, scale_cols, mult);
-        else zk::fp8_to_int32_vec_kernel<1><<<dim3((unsigned)blocks), dim3(256), 0, 0>>>(wp, scale, op, pieces, ppr, scale_cols, mult);
+        zk::for_stretches(n / 4, [&](dim3 grid, long begin, bool two) {
+            if (two) zk::fp8_to_int32_vec_kernel<2><<<grid, dim3(256), 0, 0>>>(wp, scale, op, begin, n / 4, ppr, scale_cols, mult);
+            else zk::fp8_to_int32_vec_kernel<1><<<grid, dim3(256), 0, 0>>>(wp, scale, op, begin, n / 4, ppr, scale_cols, mult);
+        });
     } else if (cols >= 4 && ((uintptr_t)w & 3) == 0 && ((uintptr_t)out & 15) == 0) {
-        const bool two = n > (4L << 20);  // as above, in weights
-        const long blocks = (n / 4 + (two ? 511 : 255)) / (two ? 512 : 256);
-        if (blocks > 0x7FFFFFFFL) { zk::set_error(zk::kUnsupportedSize, "%s: matrix too large", name); return; }
-        if (two) zk::fp8_to_int32_any_kernel<2><<<dim3((unsigned)blocks), dim3(256), 0, 0>>>(w, scale, out, n, cols, scale_cols, mult);
-        else zk::fp8_to_int32_any_kernel<1><<<dim3((unsigned)blocks), dim3(256), 0, 0>>>(w, scale, out, n, cols, scale_cols, mult);
+        zk::for_stretches(n / 4, [&](dim3 grid, long begin, bool two) {
+            if (two) zk::fp8_to_int32_any_kernel<2><<<grid, dim3(256), 0, 0>>>(w, scale, out, begin, n, cols, scale_cols, mult);
+            else zk::fp8_to_int32_any_kernel<1><<<grid, dim3(256), 0, 0>>>(w, scale, out, begin, n, cols, scale_cols, mult);
+        });
     } else {
         zk::fp8_to_int32_kernel<<<dim3(zk::grid_for(n)), dim3(256), 0, 0>>>(w, scale, out, n, cols, scale_cols, mult);
     }
