@@ -111,8 +111,8 @@ void zk_clear_error(void);
 size_t zk_workspace_bytes(void);
 size_t zk_prepared_weights_bytes(void);
 void zk_release_workspace(void);
-/* Reads the diagnosis switches ZK_GEMM_SYNC, ZK_NO_TAIL_SPLIT, ZK_B_ROWS_MIN_MACS, ZK_SCRATCH_LIMIT, ZK_ROWS16_MAX_WEIGHTS and ZK_SKINNY_MAX_M from the
- * environment again (they are read once when the library is loaded, not per call). */
+/* Reads the diagnosis switches ZK_GEMM_SYNC, ZK_NO_TAIL_SPLIT, ZK_B_ROWS_MIN_MACS, ZK_SCRATCH_LIMIT, ZK_ROWS16_MAX_WEIGHTS, ZK_SKINNY_MAX_M, ZK_NO_PIPE,
+ * ZK_NO_ROWTILE and their like from the environment again (they are read once when the library is loaded, not per call). */
 void zk_reload_env(void);
 
 /* RMS statistic on the device: rms[m] = isqrt((eps + sum_n A[m,n]^2) / dim), exact (192-bit sum).
@@ -249,6 +249,10 @@ long zk_gemm_grouped_streamed_calls(void);
  * prepared with zk_gemm_prepare_weights, and a B that is small next to the product, with A split by a pass in front or by the
  * kernel itself; ZK_NO_PIPE=1 switches them off). */
 long zk_gemm_pipe_calls(void);
+/* How many of those ran on the kernel that splits A itself (ZK_NO_ROWTILE=1 leaves their A to the pass in front), and how many
+ * launches so far were small products done in one launch (scores and values of up to eight positions). */
+long zk_gemm_rowtile_calls(void);
+long zk_gemm_small_calls(void);
 /* No reference counterpart: model weights do not change between calls, so a weight matrix W[N,K] (int64, or int32 with
  * b32 != 0; groups == 0, B = the device pointer later passed as B) or all the matrices of a device table of pointers
  * (groups > 0, B = the table later passed to int64_grouped_bmm_launcher) can be split into base-256 digit planes ONCE.

@@ -101,6 +101,7 @@ bool gemm_gemv_launch(const GemmDesc &d);
 
 // Small products in one launch, nothing guessed (gemm_small.hip).  Returns false (nothing launched) for any other descriptor.
 bool gemm_small_launch(const GemmDesc &d);
+long gemm_small_calls();                   // launches so far
 
 // Limb-decomposed i8 MFMA.  Returns 0 when the product was launched, 1 when the descriptor is outside what it
 // supports or memory for its buffers is short (nothing was launched; the caller falls back to the VALU path), -1 on an
@@ -129,6 +130,7 @@ int gemm_mfma_last_pairs();       // digit pairs multiplied per element of K by 
 int gemm_mfma_last_prepared();    // 1 when the last MFMA launch read B from prepared planes
 long gemm_mfma_grouped_streamed_calls();   // grouped launches so far that ran on the streamed int32 kernel
 long gemm_mfma_pipe_calls();               // launches so far that ran on the software-pipelined kernels for planes on both sides
+long gemm_mfma_rowtile_calls();            // ... and those of them on the kernel that splits A itself (gemm_mfma_rowtile.h)
 
 // Grouped product: the rows of A and C form one contiguous segment per group and every group has its own
 // k-contiguous B[N,K] (the experts of a MoE layer after the tokens have been sorted by expert):

@@ -177,10 +177,10 @@ static RangeCache g_cache;
 // Diagnosis switches, read from the environment once when the library is loaded (and again on zk_reload_env):
 // ZK_GEMM_SYNC: every call waits for its own digit verdict; ZK_NO_TAIL_SPLIT: no split-K; ZK_VALU_FALLBACK: the guarded launch
 // behind a speculative one is always the vector-ALU kernel; ZK_NO_STREAM32: grouped launches on int32 weights keep the general
-// 32-row kernel; ZK_B_ROWS_MIN_MACS: product
+// 32-row kernel; ZK_NO_PIPE: no pipelined kernel for planes on both sides; ZK_NO_ROWTILE: none that splits A itself; ZK_B_ROWS_MIN_MACS: product
 // size from which a B that is small next to it is split into digit planes or rewritten first; ZK_SKINNY_MAX_M: rows up to
 // which the 32-row tiles are used; ZK_SCRATCH_LIMIT: bytes a scratch buffer may grow to, as if the device had no more.
-struct Switches { bool sync_verdict, no_tail_split, valu_fallback, no_stream32, no_pipe; double b_rows_min_macs, scratch_limit; int skinny_max_m, planes_min_tiles_n, stream32_min_pairs; };
+struct Switches { bool sync_verdict, no_tail_split, valu_fallback, no_stream32, no_pipe, no_rowtile; double b_rows_min_macs, scratch_limit; int skinny_max_m, planes_min_tiles_n, stream32_min_pairs; };
 constexpr long kBRowsMinMacs = 1L << 30;
 constexpr double kShapeGuessMaxMacs = 17179869184.0;        // 2^34: about 0.15 ms on the matrix pipe
 // Rows up to which a product runs on the 32-row tiles (two of them from 33 rows on): measured against the 128-row tiles,
@@ -194,6 +194,7 @@ static Switches read_switches()
     s.valu_fallback = getenv("ZK_VALU_FALLBACK") != nullptr;
     s.no_stream32 = getenv("ZK_NO_STREAM32") != nullptr;
     s.no_pipe = getenv("ZK_NO_PIPE") != nullptr;
+    s.no_rowtile = getenv("ZK_NO_ROWTILE") != nullptr;
     const char *sp = getenv("ZK_STREAM32_MIN_PAIRS");
     s.stream32_min_pairs = sp ? atoi(sp) : 16;
     const char *m = getenv("ZK_B_ROWS_MIN_MACS");
@@ -298,11 +299,12 @@ static bool wait_digits(long first, long seen_count, int *need_a, int *need_b)
 }
 
 static int g_last_pairs = 0, g_last_prepared = 0;
-static long g_streamed_calls = 0, g_pipe_calls = 0;
+static long g_streamed_calls = 0, g_pipe_calls = 0, g_rowtile_calls = 0;
 int gemm_mfma_last_pairs() { return g_last_pairs; }
 int gemm_mfma_last_prepared() { return g_last_prepared; }
 long gemm_mfma_grouped_streamed_calls() { return g_streamed_calls; }
 long gemm_mfma_pipe_calls() { return g_pipe_calls; }
+long gemm_mfma_rowtile_calls() { return g_rowtile_calls; }
 
 long gemm_mfma_guard_hits()
 {
@@ -772,7 +774,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
                 inst = both;
                 pipe = f;
                 pre_b = true;
-                p.col_parts = rowtile_parts(d, inst->na, inst->nb, f.bn, g_cache.cus);
+                p.col_parts = g_switches.no_rowtile ? 0 : rowtile_parts(d, inst->na, inst->nb, f.bn, g_cache.cus);
                 if (p.col_parts) { rowtile = rowtile_form(inst->na, inst->nb); pipe = PipeForm{}; }
             }
         }
@@ -980,6 +982,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         g_last_pairs = kept_pairs_before(inst->na, inst->nb, inst->dmax, inst->na, 0);
         g_last_prepared = prep ? 1 : 0;
         if (pipe.fn || rowtile.fn) g_pipe_calls++;
+        if (rowtile.fn) g_rowtile_calls++;
         {
             const hipError_t err = hipGetLastError();
             if (err != hipSuccess) {

@@ -171,6 +171,9 @@ static int device_cus()
     return cus;
 }
 
+static long g_small_calls = 0;
+long gemm_small_calls() { return g_small_calls; }
+
 bool gemm_small_launch(const GemmDesc &d)
 {
     const long tiles_m = (d.M + kSmallTile - 1) / kSmallTile, tiles_n = (d.N + kSmallTile - 1) / kSmallTile, tiles = tiles_m * tiles_n * d.G;
@@ -184,6 +187,7 @@ bool gemm_small_launch(const GemmDesc &d)
     const dim3 grid((unsigned)tiles), block(64 * kSmallWaves);
     if (d.ldbk != 1) gemm_small_kernel<true><<<grid, block, 0, 0>>>(p);
     else gemm_small_kernel<false><<<grid, block, 0, 0>>>(p);
+    g_small_calls++;
     return true;
 }
 
