@@ -326,6 +326,10 @@ __global__ __launch_bounds__(512) void gemm_mfma_pipe_kernel(MfmaParams)
     wait_vmcnt<0>();                                       // (the loads past the end)
 }
 
+// Digit counts (A, B) that this kernel and the one that splits A itself (gemm_mfma_rowtile.h) exist for: one list, since a product that
+// finds the first may be given to the second.
+#define ZK_PIPE_DIGITS(X) X(3, 3) X(3, 4) X(4, 3) X(4, 4) X(3, 5) X(6, 3) X(5, 4) X(4, 5) X(5, 5)
+
 // the kernel for digit counts (na, nb) or null, its dynamic LDS, its tile columns and its finishing kernel
 struct PipeForm {
     MfmaKernel fn;

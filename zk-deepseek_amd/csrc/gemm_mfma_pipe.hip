@@ -18,16 +18,8 @@ static PipeForm form()
 
 PipeForm pipe_form(int na, int nb)
 {
-#define ZK_PIPE(NA_, NB_) if (na == NA_ && nb == NB_) return form<NA_, NB_>()
-    ZK_PIPE(3, 3);
-    ZK_PIPE(3, 4);
-    ZK_PIPE(4, 3);
-    ZK_PIPE(4, 4);
-    ZK_PIPE(3, 5);
-    ZK_PIPE(6, 3);
-    ZK_PIPE(5, 4);
-    ZK_PIPE(4, 5);
-    ZK_PIPE(5, 5);
+#define ZK_PIPE(NA_, NB_) if (na == NA_ && nb == NB_) return form<NA_, NB_>();
+    ZK_PIPE_DIGITS(ZK_PIPE)
 #undef ZK_PIPE
     return PipeForm{ nullptr, nullptr, 0, 0 };
 }
