@@ -594,6 +594,23 @@ def test_values_without_memory_for_digit_planes(K, oracle, monkeypatch, scratch_
         assert K.lib.zk_gemm_guard_hits() == hits + 1
 
 
+def test_row_tiles_without_memory_for_their_slots(K, oracle, monkeypatch, scratch_limit):
+    """row tiles dealt in parts keep the planes of a tile once per part: where there is room for the planes of A but not for
+    that, the product goes through the pass over A, and through the row tiles again once there is room"""
+    monkeypatch.setenv("ZK_B_ROWS_MIN_MACS", "1")
+    rng = np.random.default_rng(3)
+    S, T, C = 12800, 40, 512                # 2.5 MB of planes of A, 4.9 MB of slots
+    p, v = rand_i64(rng, (1, S, 1, T), 19), rand_i64(rng, (1, T, C), 20)
+    expected = oracle.einsum_bsht_btc_bshc(p, v, 23)
+    dp, dv = torch.from_numpy(p).cuda(), torch.from_numpy(v).cuda()
+    for size, on_row_tiles in ((None, 1), (3 << 20, 0), (None, 1)):
+        scratch_limit(size)
+        for _ in range(3):
+            before = K.lib.zk_gemm_pipe_calls(), K.lib.zk_gemm_rowtile_calls()
+            assert np.array_equal(host(K.einsum_bsht_btc_bshc(dp, dv, 23)), expected)
+        assert K.lib.zk_gemm_pipe_calls() == before[0] + 1 and K.lib.zk_gemm_rowtile_calls() == before[1] + on_row_tiles
+
+
 @pytest.mark.parametrize("prepared", [False, True])
 def test_product_without_memory_for_the_planes_of_a(K, oracle, scratch_limit, prepared):
     """a product whose A would be split by a pass in front (and, with prepared weights, has to be): without memory for the

@@ -740,7 +740,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
     // Everything an attempt allocates is allocated before its first launch: memory that is short for digit planes then
     // sends the call to the kernels that split both operands themselves (which need none), and nothing it has launched
     // can have raised the verdict that the next call relies on being clear.
-    bool planes_fit = true;
+    bool planes_fit = true, slots_fit = true;
     for (int attempt = 0; attempt < 3; attempt++) {
         // the stored bits are [shift, shift + 64) of the sum (the remainder lies below them)
         const int need_diag = (d.shift + 64 + 7) / 8;
@@ -774,7 +774,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
                 inst = both;
                 pipe = f;
                 pre_b = true;
-                p.col_parts = g_switches.no_rowtile ? 0 : rowtile_parts(d, inst->na, inst->nb, f.bn, g_cache.cus);
+                p.col_parts = g_switches.no_rowtile || !slots_fit ? 0 : rowtile_parts(d, inst->na, inst->nb, f.bn, g_cache.cus);
                 if (p.col_parts) { rowtile = rowtile_form(inst->na, inst->nb); pipe = PipeForm{}; }
             }
         }
@@ -929,8 +929,9 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             if (got == kFailed) return kFailed;
             if (got == kDeclined) {
                 if (!use_planes && !pre_b) return kDeclined;
-                planes_fit = false;
-                prep = nullptr;
+                // (row tiles dealt in parts take more room than the planes of A in one piece)
+                if (rowtile.fn) slots_fit = false;
+                else { planes_fit = false; prep = nullptr; }
                 attempt--;
                 continue;
             }
