@@ -952,6 +952,26 @@ def test_row_tiles_split_by_the_product(K, oracle, monkeypatch, bits_a, bits_b, 
         K.lib.zk_reload_env()
 
 
+@pytest.mark.parametrize("rows,N,Kd,bits,rem,on_row_tiles", [(44292, 712, 39, (27, 20), True, 0), (25409, 356, 223, (27, 20), True, 1),
+                                                             (60551, 441, 55, (20, 20), False, 1), (29181, 503, 145, (43, 19), True, 0),
+                                                             (47202, 1225, 55, (20, 27), False, 0)])
+def test_row_tiles_where_their_stores_are_the_slower_ones(K, oracle, rows, N, Kd, bits, rem, on_row_tiles):
+    """outputs beyond the memory-side cache in parts of lines, and remainders there, leave the row tiles to the pass over A"""
+    oracle.set_threads(oracle.max_threads())
+    rng = np.random.default_rng(rows)
+    a, w = rand_i64(rng, (1, rows, Kd), bits[0]), rand_i64(rng, (N, Kd), bits[1])
+    try:
+        expected = oracle.int64_bmm_broadcast(a, w, 1, 1, 29)
+    finally:
+        oracle.set_threads(1)
+    da, dw = dev(a), dev(w)
+    for _ in range(2):          # (a first call may run on digits remembered for other operands at these addresses)
+        before = K.lib.zk_gemm_pipe_calls(), K.lib.zk_gemm_rowtile_calls()
+        C, R = K.int64_bmm_broadcast(da, dw, 1, 1, 29, want_remainder=rem)
+        assert np.array_equal(host(C), expected[0]) and (not rem or np.array_equal(host(R), expected[1]))
+    assert K.lib.zk_gemm_pipe_calls() == before[0] + 1 and K.lib.zk_gemm_rowtile_calls() == before[1] + on_row_tiles
+
+
 @pytest.mark.parametrize("heads,cols,k", [(5, 1, 1), (16, 16, 63), (17, 15, 64), (33, 70, 65), (128, 779, 512), (128, 512, 779), (128, 512, 1024),
                                           (256, 256, 2048), (31, 1200, 2047)])
 def test_attention_of_few_positions_in_one_launch(K, oracle, heads, cols, k):

@@ -577,9 +577,19 @@ static int rowtile_parts(const GemmDesc &d, int na, int nb, int bn, int cus)
     // rows of 128 heads [350,80] 126 / 147), and nine products a step leave less to hide the splits behind ((3,3) 94976 x [1903,512] 958 /
     // 1022, 54144 x [588,98] 97 / 111, 29568 x [512,244] 72 / 61).
     if (bn != 128 && d.K < 128) return 0;
+    // Two workgroups per compute unit store parts of lines, and remainders, at a lower rate than one, once the outputs are more than the
+    // 256 MB of the memory-side cache hold: 3.5 against 4.5 TB/s.  With remainder, pass over A and pipelined kernel / row tiles: 127714
+    // x [743,76] 371 / 519 us, 129713 x [692,334] 592 / 691, 121446 x [492,96] 260 / 317, (6,3) 122597 x [398,246] 363 / 393, but 25409
+    // x [356,223] (145 MB) 76 / 60; without, 126912 x [635,61] 191 / 228, 47202 x [1225,55] 139 / 166, but 60551 x [441,55] 80 / 63.
+    const bool lines = (((uintptr_t)d.C | (uintptr_t)d.R | (uintptr_t)(d.ldc * 8) | (uintptr_t)(d.sC * 8)) & 127) == 0;
+    const double beyond = std::max(0.0, (double)d.G * d.M * d.N * (d.R ? 16 : 8) - 256e6);
+    if (beyond > 0 && d.K < 96 && (d.R || !lines)) return 0;
+    if (d.R && !lines && na == 6) return 0;
+    const double stores = d.R && !lines ? beyond / 3.5e6 : 0;
+    best += stores * (3.5 / 4.5);
     best *= bn != 128 ? 0.93 : (na * nb <= 9 ? 0.88 : 0.97);
     for (long n = 1; n <= tiles_n && n <= 8; n++) {
-        const double t = (double)((row_tiles * n + slots - 1) / slots) * (split + (double)((tiles_n + n - 1) / n) * tile);
+        const double t = (double)((row_tiles * n + slots - 1) / slots) * (split + (double)((tiles_n + n - 1) / n) * tile) + stores;
         if (t < best) { best = t; parts = (int)n; }
     }
     return parts;
