@@ -6,7 +6,9 @@
 // eight wavefronts take every eighth step of 64 k, load their fragments straight into registers (the four lanes of a
 // row read 64 contiguous bytes per load), take the digit counts that those need (3, 4 or 5 per operand, gemm_frag16.h),
 // split, multiply, and meet in LDS with their 128-bit sums.  A wavefront that meets values beyond five digits (2^38 and up)
-// multiplies its share again with nine digits.
+// multiplies its share again with nine digits.  Where a wavefront has one step at most (K up to 512) that step's elements are still in
+// its registers: a cache of 44 bits, share read again / this, kernel alone, 128 rows x [512,7] n-contiguous 7.2 / 5.3 us, x [512,300]
+// 9.6 / 7.0, x [779,512] k-contiguous 21.7 / 15.0 (the first had become slower than on the general kernel, 10.3 -> 11.8 a call).
 #include "gemm_frag16.h"
 
 namespace zk {
@@ -19,7 +21,7 @@ struct SmallParams {
     int64_t init;
 };
 
-constexpr int kSmallWaves = 8, kSmallTile = 16, kSmallDiagonals = 9;
+constexpr int kSmallWaves = 8, kSmallTile = 16, kSmallDiagonals = 9, kSmallWideDiagonals = 16;   // of five digits a side, of nine (what lies at 2^128 and above does not matter)
 // Where it pays, against the general and the 16-row kernels over 250 shapes of 5 to 600 rows and 16 to 2048 columns (those / this, us):
 // one round of tiles 0.3-0.8 of their time up to K = 2048 (128 rows x [512,779] n-contiguous 20.0 / 8.9, 50 x [94,321] (5,5)
 // 24.9 / 7.1, 32 x [1513,759] 23.2 / 8.7, 274 x [161,2145] 22.6 / 16.2) and level at 4000; two rounds up to K = 1024 (128 x
@@ -28,8 +30,8 @@ constexpr int kSmallWaves = 8, kSmallTile = 16, kSmallDiagonals = 9;
 // digit counts and check them.
 constexpr int kSmallMaxK = 2048, kSmallMaxKTwoRounds = 1024;
 
-template <int NA, int NB>
-__device__ __forceinline__ void small_step(const RawFrag<false> &fa_raw, const RawFrag<false> &fb_raw, v4i (&acc)[kSmallDiagonals])
+template <int NA, int NB, int D>
+__device__ __forceinline__ void small_step(const RawFrag<false> &fa_raw, const RawFrag<false> &fb_raw, v4i (&acc)[D])
 {
     v4i fa[NA], fb[NB];
     split_frag<NA, false>(fa_raw, fa);
@@ -38,7 +40,23 @@ __device__ __forceinline__ void small_step(const RawFrag<false> &fa_raw, const R
     for (int i = 0; i < NA; i++)
 #pragma unroll
         for (int j = 0; j < NB; j++)
-            acc[i + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[i], fb[j], acc[i + j], 0, 0, 0);
+            if (i + j < D) acc[i + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[i], fb[j], acc[i + j], 0, 0, 0);
+}
+
+// up to five digits a side
+__device__ __forceinline__ void small_narrow_step(int na, int nb, const RawFrag<false> &fa, const RawFrag<false> &fb, v4i (&acc)[kSmallDiagonals])
+{
+    switch ((na - 3) * 3 + (nb - 3)) {
+    case 0: small_step<3, 3>(fa, fb, acc); break;
+    case 1: small_step<3, 4>(fa, fb, acc); break;
+    case 2: small_step<3, 5>(fa, fb, acc); break;
+    case 3: small_step<4, 3>(fa, fb, acc); break;
+    case 4: small_step<4, 4>(fa, fb, acc); break;
+    case 5: small_step<4, 5>(fa, fb, acc); break;
+    case 6: small_step<5, 3>(fa, fb, acc); break;
+    case 7: small_step<5, 4>(fa, fb, acc); break;
+    default: small_step<5, 5>(fa, fb, acc); break;
+    }
 }
 
 // A fragment element by element: byte b of the fragment is k = frag_k(q, b) of the step, `lane_at` the lane's offset with its
@@ -56,8 +74,8 @@ __device__ __forceinline__ void load_elements(RawFrag<false> &f, const int64_t *
     }
 }
 
-// BKM: B is contiguous along n
-template <bool BKM>
+// BKM: B is contiguous along n.  ONE: no wavefront has more than one step
+template <bool BKM, bool ONE>
 __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(SmallParams p)
 {
     __shared__ Words red[kSmallWaves][4][64];
@@ -97,7 +115,27 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(SmallParam
     };
     // accumulator register r of lane (li, q) holds row 4*q + r, column li of the tile
     bool wide = false;
-    {
+    if (ONE) {
+        v4i acc[kSmallWideDiagonals], narrow[kSmallDiagonals];
+#pragma unroll
+        for (int d = 0; d < kSmallWideDiagonals; d++) acc[d] = v4i{ 0, 0, 0, 0 };
+#pragma unroll
+        for (int d = 0; d < kSmallDiagonals; d++) narrow[d] = v4i{ 0, 0, 0, 0 };
+        if (wave < steps) {
+            RawFrag<false> fa, fb;
+            load(wave, fa, fb);
+            const int na = wave_digits(magnitude_or<false>(fa));
+            const int nb = wave_digits(magnitude_or<false>(fb));
+            wide = na > 5 || nb > 5;
+            if (!wide) small_narrow_step(na, nb, fa, fb, narrow);
+            else if (na <= 5) small_step<5, 9>(fa, fb, acc);
+            else if (nb <= 5) small_step<9, 5>(fa, fb, acc);
+            else small_step<9, 9>(fa, fb, acc);
+        }
+#pragma unroll
+        for (int o = 0; o < 4; o++)
+            red[wave][o][lane] = wide ? sum_diagonals<kSmallWideDiagonals>([&](int d) { return acc[d][o]; }, 0) : sum_diagonals<kSmallDiagonals>([&](int d) { return narrow[d][o]; }, 0);
+    } else {
         v4i acc[kSmallDiagonals];
 #pragma unroll
         for (int d = 0; d < kSmallDiagonals; d++) acc[d] = v4i{ 0, 0, 0, 0 };
@@ -108,26 +146,16 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(SmallParam
             const int na = wave_digits(magnitude_or<false>(fa));
             const int nb = wave_digits(magnitude_or<false>(fb));
             if (na > 5 || nb > 5) { wide = true; break; }
-            switch ((na - 3) * 3 + (nb - 3)) {
-            case 0: small_step<3, 3>(fa, fb, acc); break;
-            case 1: small_step<3, 4>(fa, fb, acc); break;
-            case 2: small_step<3, 5>(fa, fb, acc); break;
-            case 3: small_step<4, 3>(fa, fb, acc); break;
-            case 4: small_step<4, 4>(fa, fb, acc); break;
-            case 5: small_step<4, 5>(fa, fb, acc); break;
-            case 6: small_step<5, 3>(fa, fb, acc); break;
-            case 7: small_step<5, 4>(fa, fb, acc); break;
-            default: small_step<5, 5>(fa, fb, acc); break;
-            }
+            small_narrow_step(na, nb, fa, fb, acc);
         }
         // (5 pairs x 64 products of 2^14 a step)
         static_assert((kSmallMaxK / 64 + kSmallWaves - 1) / kSmallWaves * 5L * 64 * 16384 <= kMaxDiagonal, "the int32 accumulators hold a wavefront's share");
 #pragma unroll
         for (int o = 0; o < 4; o++) red[wave][o][lane] = sum_diagonals<kSmallDiagonals>([&](int d) { return acc[d][o]; }, 0);
     }
-    if (wide) {
-        // wider than five digits: this wavefront's steps once more with nine (what lies at 2^128 and above does not matter)
-        constexpr int D = 16;
+    if (!ONE && wide) {
+        // wider than five digits: this wavefront's steps once more with nine
+        constexpr int D = kSmallWideDiagonals;
         v4i acc[D];
 #pragma unroll
         for (int d = 0; d < D; d++) acc[d] = v4i{ 0, 0, 0, 0 };
@@ -135,14 +163,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(SmallParam
             RawFrag<false> fa_raw;
             RawFrag<false> fb_raw;
             load(ks, fa_raw, fb_raw);
-            v4i fa[9], fb[9];
-            split_frag<9, false>(fa_raw, fa);
-            split_frag<9, false>(fb_raw, fb);
-#pragma unroll
-            for (int i = 0; i < 9; i++)
-#pragma unroll
-                for (int j = 0; j < 9; j++)
-                    if (i + j < D) acc[i + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[i], fb[j], acc[i + j], 0, 0, 0);
+            small_step<9, 9>(fa_raw, fb_raw, acc);
         }
         static_assert((kSmallMaxK / 64 + kSmallWaves - 1) / kSmallWaves * 9L * 64 * 16384 <= kMaxDiagonal, "and of nine digits");
 #pragma unroll
@@ -185,8 +206,12 @@ bool gemm_small_launch(const GemmDesc &d)
     p.M = d.M; p.N = d.N; p.K = d.K; p.shift = d.shift; p.init = d.init;
     p.tiles_m = (int)tiles_m; p.tiles_n = (int)tiles_n;
     const dim3 grid((unsigned)tiles), block(64 * kSmallWaves);
-    if (d.ldbk != 1) gemm_small_kernel<true><<<grid, block, 0, 0>>>(p);
-    else gemm_small_kernel<false><<<grid, block, 0, 0>>>(p);
+    const bool one = d.K <= 64 * kSmallWaves;
+    if (d.ldbk != 1) {
+        if (one) gemm_small_kernel<true, true><<<grid, block, 0, 0>>>(p);
+        else gemm_small_kernel<true, false><<<grid, block, 0, 0>>>(p);
+    } else if (one) gemm_small_kernel<false, true><<<grid, block, 0, 0>>>(p);
+    else gemm_small_kernel<false, false><<<grid, block, 0, 0>>>(p);
     g_small_calls++;
     return true;
 }
