@@ -1314,6 +1314,21 @@ def test_rmsnorm_row_counts_next_to_the_lines(K, oracle, M, N, bits):
     assert np.array_equal(rms[:M].numpy(), rmse) and np.array_equal(host(C), Ce)
 
 
+@pytest.mark.parametrize("M,N", [(1, 24576), (16, 22528), (16, 22530), (17, 22530), (17, 24576)])
+def test_rmsnorm_few_of_the_longest_rows(K, oracle, M, N):
+    """a statistic and a product of their own, or one kernel: both sides of the line, and residual and odd rows beside it"""
+    rng = np.random.default_rng(M * N)
+    for n in (N, N - 1):
+        X, W = rand_i64(rng, (M, n), 31), rand_i64(rng, (n,), 20)
+        for w in (W, W.astype(np.int32)):
+            Ce, rmse = oracle.RMS_Norm_int64(X, w, 1, n)
+            C, rms = K.RMS_Norm_int64(dev(X), dev(w), 1, n)
+            assert np.array_equal(rms[:M].numpy(), rmse) and np.array_equal(host(C), Ce)
+            zero = torch.zeros((M, n), dtype=torch.int64, device="cuda")
+            Xn, C, rms = K.RMS_Norm_residual_int64(dev(X), zero, 8, dev(w), 1, n)
+            assert np.array_equal(host(Xn), X) and np.array_equal(rms[:M].numpy(), rmse) and np.array_equal(host(C), Ce)
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("M,N,off", [(300, 513, 0), (300, 1023, 1), (70, 2049, 0), (300, 4097, 0), (300, 8191, 1), (300, 8192, 1), (3, 8193, 0),
                                      (2, 16383, 0), (2, 16384, 1), (3, 16385, 0), (2, 16386, 0), (2, 24575, 0), (2, 24576, 1), (2, 24577, 0)])

@@ -575,8 +575,10 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
     else if (N <= 16384) ZK_RMS_LAUNCH(1024, 16, 1);
     // up to what a workgroup's registers hold: 24 elements a thread, 128 registers of which 20 spill; statistic and product as two
     // kernels, as below / this, us: 1 row of 18432 10.5 / 9.9, 64 rows 17.3 / 13.7, 500 rows 42.6 / 33.1, with residual 74.6 / 56.3;
-    // 500 rows of 24576 54.0 / 42.2, of 18431 71.2 / 45.1
-    else if (N <= 24576 && M <= 65535) ZK_RMS_LAUNCH(1024, 24, 1);
+    // 500 rows of 24576 54.0 / 42.2, of 18431 71.2 / 45.1.  A few of the longest, where nothing overlaps the spills and the second
+    // kernel's several workgroups per row are worth their launch, keep the two: 1 row of 24576 13.8 / 15.3, 2 rows 13.2 / 14.4, 16 rows
+    // 13.9 / 14.6, 24 rows 16.8 / 16.1 (of 20480 13.7 / 11.5; with residual 16 rows 21.0 / 17.4)
+    else if (N <= 24576 && M <= 65535 && !(M <= 16 && N > 22528 && vec && !res)) ZK_RMS_LAUNCH(1024, 24, 1);
     else {
         if (!apply_rows_ok(name, M)) return;          // before the residual sum or the statistic is written
         const int64_t *src = A;
