@@ -1069,6 +1069,33 @@ def test_softmax_hostile_inputs(K, oracle, fn):
         assert np.array_equal(host(C), Ce)
 
 
+@pytest.mark.parametrize("fn", ["softmax_q19", "softmax_q21"])
+@pytest.mark.parametrize("rows,T", [(3, 255), (3, 130), (5, 300), (1030, 200), (1030, 513), (1030, 1024), (1030, 1025), (1030, 1026), (1030, 2047)])
+def test_softmax_hostile_inputs_in_every_kernel(K, oracle, fn, rows, T):
+    """rows of which some lanes' weights leave the range of the quick division and others' do not, and whole rows that do, with
+    the input kept and overwritten, in place too: the general division of each row length"""
+    rng = np.random.default_rng(rows + T)
+    x = _scores(rng, (1, rows, 1, T), 19)
+    x[0, 0], x[0, 1] = rand_i64(rng, (1, T), 63), 7
+    lut = rng.integers(0, 1 << 20, size=256, dtype=np.int64)
+    lut[::7] = rand_i64(rng, (37,), 63)
+    for table in (lut, rand_i64(rng, (256,), 63)):
+        Ce, We = getattr(oracle, fn)(x, table)
+        t = dev(table)
+        for clobber in (0, 1):
+            K.lib.zk_softmax_clobber_input(clobber)
+            try:
+                R = dev(x)
+                C = torch.empty_like(R)
+                getattr(K.lib, fn)(R.data_ptr(), C.data_ptr(), t.data_ptr(), 1, rows, 1, T)
+                assert np.array_equal(host(C), Ce) and np.array_equal(host(R), We if clobber else x)
+                R = dev(x)
+                getattr(K.lib, fn)(R.data_ptr(), R.data_ptr(), t.data_ptr(), 1, rows, 1, T)
+                assert np.array_equal(host(R), We if clobber else Ce)
+            finally:
+                K.lib.zk_softmax_clobber_input(0)
+
+
 def test_softmax_and_activation_hand_worked_literals(K):
     """the results worked by hand from the reference's source (the steps are written out in test_oracle_pins.py:
     softmax q19 :700-740 and q21 :624-657 of inference/int64_gemm.cu, sigmoid/SiLU q23 :932-946 and q25 :804-818),

@@ -58,13 +58,22 @@ __device__ __forceinline__ int64_t smx_weight(int64_t x, int64_t rmax, const int
     }
 }
 
-// Per-row divide.  fast: 2^12 <= s < 2^52 (true for every row whose maximum has weight LUT[0] = 2^Q).
 template <int Q>
-__device__ __forceinline__ int64_t smx_norm(int64_t w, int64_t s, double inv, bool fast)
+__device__ __forceinline__ int64_t smx_numerator(int64_t w, int64_t s)
 {
     int64_t num = (int64_t)((uint64_t)w << Q);
     if (Q == 21) num = (int64_t)((uint64_t)num + (uint64_t)(s / 2));
-    if (fast && w >= 0 && w < ((int64_t)1 << 30)) return (int64_t)udiv_by_inv((uint64_t)num, (uint64_t)s, inv);
+    return num;
+}
+
+// Per-row divide.  fast: 2^12 <= s < 2^52 (true for every row whose maximum has weight LUT[0] = 2^Q).
+constexpr int64_t kSmxQuickWeights = (int64_t)1 << 30;
+
+template <int Q>
+__device__ __forceinline__ int64_t smx_norm(int64_t w, int64_t s, double inv, bool fast)
+{
+    const int64_t num = smx_numerator<Q>(w, s);
+    if (fast && w >= 0 && w < kSmxQuickWeights) return (int64_t)udiv_by_inv((uint64_t)num, (uint64_t)s, inv);
     return s ? tdiv64(num, s) : 0;
 }
 
@@ -201,12 +210,13 @@ __global__ __launch_bounds__(kSmxThreads) void softmax_wave_kernel(int64_t *__re
         for (int w = 0; w < RW; w++) rmax = red[0][w] > rmax ? red[0][w] : rmax;
     }
 
-    uint64_t sum = 0;
+    uint64_t sum = 0, all = 0;
 #pragma unroll
     for (int j = 0; j < EPL; j++) {
         if (at(j) < T) {
             v[j] = smx_weight<Q>(v[j], rmax, lut);
             sum += (uint64_t)v[j];
+            if (!VEC) all |= (uint64_t)v[j];
         }
     }
     sum = wave_sum_u64(sum);
@@ -221,22 +231,37 @@ __global__ __launch_bounds__(kSmxThreads) void softmax_wave_kernel(int64_t *__re
     const bool fast = s >= ((int64_t)1 << 12) && s < ((int64_t)1 << 52);
     const double inv = fast ? 1.0 / (double)s : 0.0;
 
+    // Without VEC the general division, some 200 instructions of 64-bit arithmetic, is here once, in a loop over weights put where the
+    // results go.  Beside every element of a long row it made 69 KB of code with preparation, more than the instruction cache (64 KB)
+    // holds, and times that hung on where the code came to lie: 5120 rows of 1301 43.9 us in one build and 47.2 in the next, now 43.5,
+    // 12800 of 1999 200, 210, now 207; without preparation 25.9 -> 22.0 and 83.2 -> 81.  The forms with VEC are smaller, and slower
+    // this way (131072 rows of 1024 348 -> 365, with preparation 20352 of 1438 177 -> 186).
+    constexpr bool ONCE = !VEC;
+    const bool quick = fast && all < (uint64_t)kSmxQuickWeights;
+    auto result = [&](int64_t w) {
+        if (!ONCE) return smx_norm<Q>(w, s, inv, fast);
+        return quick ? (int64_t)udiv_by_inv((uint64_t)smx_numerator<Q>(w, s), (uint64_t)s, inv) : w;
+    };
 #pragma unroll
     for (int j = 0; j < EPL; j += VEC ? 2 : 1) {
         const int idx = at(j);
         if (idx >= T) continue;
         if (VEC) {
-            i64x2s w, o;
-            w.x = v[j];
-            w.y = v[j + 1];
-            o.x = smx_norm<Q>(w.x, s, inv, fast);
-            o.y = smx_norm<Q>(w.y, s, inv, fast);
-            st_stream(reinterpret_cast<i64x2s *>(c + idx), o);
-            if (clobber) st_stream(reinterpret_cast<i64x2s *>(x + idx), w);
+            st_stream(reinterpret_cast<i64x2s *>(c + idx), i64x2s{ result(v[j]), result(v[j + 1]) });
+            if (clobber) st_stream(reinterpret_cast<i64x2s *>(x + idx), i64x2s{ v[j], v[j + 1] });
         } else {
-            c[idx] = smx_norm<Q>(v[j], s, inv, fast);
-            if (clobber) x[idx] = v[j];
+            c[idx] = result(v[j]);
         }
+    }
+    if (ONCE && !quick) {
+#pragma unroll 1
+        for (int j = 0; j < EPL; j++)
+            if (at(j) < T) c[at(j)] = smx_norm<Q>(c[at(j)], s, inv, fast);
+    }
+    if (!VEC && clobber) {
+#pragma unroll
+        for (int j = 0; j < EPL; j++)
+            if (at(j) < T) x[at(j)] = v[j];
     }
 }
 
