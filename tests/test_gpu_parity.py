@@ -872,12 +872,15 @@ def test_einsum_values_rewritten_with_contiguous_rows(K, oracle, monkeypatch):
 
 @pytest.mark.parametrize("bits_a,bits_b,digits", [(19, 22, (3, 3)), (19, 27, (3, 4)), (27, 19, (4, 3)), (27, 27, (4, 4)), (36, 27, (5, 4)),
                                                   (27, 35, (4, 5)), (36, 36, (5, 5)), (19, 35, (3, 5)), (43, 19, (6, 3))])
-def test_einsums_with_planes_of_both_operands(K, oracle, monkeypatch, bits_a, bits_b, digits):
-    """a B that is small next to the product is split like A and the pipelined kernel walks several tiles per workgroup:
-    values (n-contiguous) with rows of A that end in zeros at every length, hold nothing at all or are full; scores
+@pytest.mark.parametrize("row_tiles", [False, True])
+def test_einsums_with_planes_of_both_operands(K, oracle, monkeypatch, row_tiles, bits_a, bits_b, digits):
+    """a B that is small next to the product is split like A and the pipelined kernel walks several tiles per workgroup, or,
+    where it is expected to win, the row tiles split A themselves: values (n-contiguous) with rows of A that end in zeros at every length, hold nothing at all or are full; scores
     (k-contiguous) of one step and of many; per-head int32 weights; ragged rows and columns, two batches, row tiles that
     do not come in eights"""
     monkeypatch.setenv("ZK_B_ROWS_MIN_MACS", "1")
+    if not row_tiles:
+        monkeypatch.setenv("ZK_NO_ROWTILE", "1")
     K.lib.zk_reload_env()
     oracle.set_threads(oracle.max_threads())
     rng = np.random.default_rng(bits_a * 64 + bits_b)
@@ -886,10 +889,11 @@ def test_einsums_with_planes_of_both_operands(K, oracle, monkeypatch, bits_a, bi
     def check(name, a, b, shift, pipe=True):
         da, db = dev(a), dev(b)
         for _ in range(2):          # (a first call may run on digits remembered for other operands at these addresses)
-            before = K.lib.zk_gemm_pipe_calls()
+            before = K.lib.zk_gemm_pipe_calls(), K.lib.zk_gemm_rowtile_calls()
             out = getattr(K, name)(da, db, shift)
             assert np.array_equal(host(out), getattr(oracle, name)(a, b, shift)), (name, a.shape, b.shape)
-        assert K.lib.zk_gemm_pipe_calls() == before + pipe and K.gemm_last_plan()[1:] == digits
+        assert K.lib.zk_gemm_pipe_calls() == before[0] + pipe and K.gemm_last_plan()[1:] == digits
+        assert row_tiles or K.lib.zk_gemm_rowtile_calls() == before[1]
     try:
         p = rand_i64(rng, (2, 17, 128, 257), bits_a)
         for s in range(17):
@@ -909,16 +913,18 @@ def test_einsums_with_planes_of_both_operands(K, oracle, monkeypatch, bits_a, bi
         oracle.set_threads(1)
         K.lib.zk_gemm_set_path(0)
         monkeypatch.delenv("ZK_B_ROWS_MIN_MACS")
+        monkeypatch.delenv("ZK_NO_ROWTILE", raising=False)
         K.lib.zk_reload_env()
 
 
 @pytest.mark.parametrize("bits_a,bits_b,digits", [(19, 22, (3, 3)), (19, 27, (3, 4)), (27, 19, (4, 3)), (27, 27, (4, 4)), (36, 27, (5, 4)),
                                                   (27, 35, (4, 5)), (36, 36, (5, 5)), (19, 35, (3, 5)), (43, 19, (6, 3))])
 def test_row_tiles_split_by_the_product(K, oracle, monkeypatch, bits_a, bits_b, digits):
-    """products whose row tiles fill whole rounds of two workgroups per compute unit: the product splits A itself.  One and
-    two rounds with a ragged last row tile and last columns, tile columns dealt in two parts, rows of C in whole lines and
-    not, K of less than a step, of whole ones, and odd (rows of A off the 16-byte grid), rows that end in zeros at every length,
-    a remainder"""
+    """products whose row tiles fill whole rounds of two workgroups per compute unit: the product splits A itself.  One, two and
+    three rounds (the third rewrites what the first has read) with a ragged last row tile and last columns, tile columns dealt in
+    two parts, two batches, rows of C in whole lines and not, K of less than a step (tiles of 128 columns; those of 64 begin at 128
+    k), of whole ones, and odd (rows of A off the 16-byte grid), rows that end in zeros at every length, a remainder (rows in
+    parts of lines not with six digits of A, which keep the pass over A there)"""
     monkeypatch.setenv("ZK_B_ROWS_MIN_MACS", "1")
     K.lib.zk_reload_env()
     oracle.set_threads(oracle.max_threads())
@@ -926,25 +932,31 @@ def test_row_tiles_split_by_the_product(K, oracle, monkeypatch, bits_a, bits_b, 
     K.lib.zk_gemm_set_path(2)
     top_a, top_b = (1 << bits_a) - 1, (1 << bits_b) - 1
     try:
-        for rows, N, Kd in ((65500, 130, 131), (32700, 256, 128), (16300, 520, 160), (32768, 200, 31)):
-            p, v = rand_i64(rng, (1, 4, rows // 4, Kd), bits_a), rand_i64(rng, (1, Kd, N), bits_b)
+        wide = digits[0] + digits[1] <= 7           # tiles of 128 columns
+        for B, rows, N, Kd in ((1, 65500, 130, 131), (1, 32700, 256, 128), (1, 16300, 520, 128 if digits == (3, 3) else 160), (1, 32768, 200, 31),
+                               (1, 98000, 130, 131), (2, 16352, 130, 131)):
+            p, v = rand_i64(rng, (B, 4, rows // 4, Kd), bits_a), rand_i64(rng, (B, Kd, N), bits_b)
             for r in range(0, rows // 4, 64):
-                p[0, :, r:r + 64, (r // 64) % Kd:] = 0
-            p[0, 3, -1, -1], v[0, -1, -1] = top_a, top_b
+                p[:, :, r:r + 64, (r // 64) % Kd:] = 0
+            p[-1, 3, -1, -1], v[-1, -1, -1] = top_a, top_b
             expected = oracle.einsum_bsht_btc_bshc(p, v, 23)
             dp, dv = dev(p), dev(v)
             for _ in range(2):          # (a first call may run on digits remembered for other operands at these addresses)
-                before = K.lib.zk_gemm_pipe_calls()
+                before = K.lib.zk_gemm_pipe_calls(), K.lib.zk_gemm_rowtile_calls()
                 out = K.einsum_bsht_btc_bshc(dp, dv, 23)
-                assert np.array_equal(host(out), expected), (rows, N, Kd)
-            assert K.lib.zk_gemm_pipe_calls() == before + 1 and K.gemm_last_plan()[1:] == digits
-        a, w = rand_i64(rng, (1, 32700, 66), bits_a), rand_i64(rng, (257, 66), bits_b)
-        a[0, -1, -1], w[-1, -1] = top_a, -top_b
-        expected = oracle.int64_bmm_broadcast(a, w, 1, 1, 29)
-        da, dw = dev(a), dev(w)
-        for _ in range(2):
-            C, R = K.int64_bmm_broadcast(da, dw, 1, 1, 29)
-            assert np.array_equal(host(C), expected[0]) and np.array_equal(host(R), expected[1])
+                assert np.array_equal(host(out), expected), (B, rows, N, Kd)
+            assert K.lib.zk_gemm_pipe_calls() == before[0] + 1 and K.gemm_last_plan()[1:] == digits
+            assert K.lib.zk_gemm_rowtile_calls() == before[1] + (wide or Kd >= 128), (B, rows, N, Kd)
+        for N, Kd in ((257, 66), (257, 130), (256, 130)):
+            a, w = rand_i64(rng, (1, 32700, Kd), bits_a), rand_i64(rng, (N, Kd), bits_b)
+            a[0, -1, -1], w[-1, -1] = top_a, -top_b
+            expected = oracle.int64_bmm_broadcast(a, w, 1, 1, 29)
+            da, dw = dev(a), dev(w)
+            for _ in range(2):
+                before = K.lib.zk_gemm_rowtile_calls()
+                C, R = K.int64_bmm_broadcast(da, dw, 1, 1, 29)
+                assert np.array_equal(host(C), expected[0]) and np.array_equal(host(R), expected[1])
+            assert K.lib.zk_gemm_rowtile_calls() == before + (wide or Kd >= 128 and (N == 256 or digits[0] < 6)), (N, Kd)
     finally:
         oracle.set_threads(1)
         K.lib.zk_gemm_set_path(0)
@@ -985,10 +997,12 @@ def test_attention_of_few_positions_in_one_launch(K, oracle, heads, cols, k):
         a[-1, -1, -1, -1], b[-1, -1, -1] = -(1 << bits_a), (1 << bits_b) - 1
         if bits_a == 27:
             a[0, 0, 0, 0], b[0, 0, k // 2] = (1 << 45) + 1, -(1 << 37)
+        before = K.lib.zk_gemm_small_calls()
         assert np.array_equal(host(K.einsum_bshc_btc_bsht(dev(a), dev(b), 23)), oracle.einsum_bshc_btc_bsht(a, b, 23)), (bits_a, bits_b)
-        assert K.gemm_last_plan() == (2, 0, 0)
+        assert K.gemm_last_plan() == (2, 0, 0) and K.lib.zk_gemm_small_calls() == before + 1
         v = np.ascontiguousarray(b.transpose(0, 2, 1))
         assert np.array_equal(host(K.einsum_bsht_btc_bshc(dev(a), dev(v), 41)), oracle.einsum_bsht_btc_bshc(a, v, 41)), (bits_a, bits_b)
+        assert K.gemm_last_plan() == (2, 0, 0) and K.lib.zk_gemm_small_calls() == before + 2
 
 
 def _scores(rng, shape, Q, masked=True):

@@ -307,6 +307,17 @@ def test_stale_guess_values_einsum_rewritten(K, oracle, small_b_first):
     _values_rounds(K, oracle, P, V, pokes)
 
 
+@pytest.fixture(params=[False, True], ids=["pass_over_a", "row_tiles"])
+def row_tiles(request, K, monkeypatch, small_b_first):
+    """A split by a pass in front of the pipelined kernel, or by the product itself"""
+    if not request.param:
+        monkeypatch.setenv("ZK_NO_ROWTILE", "1")
+        K.lib.zk_reload_env()
+    yield request.param
+    monkeypatch.delenv("ZK_NO_ROWTILE", raising=False)
+    K.lib.zk_reload_env()
+
+
 @pytest.fixture
 def oracle_threads(oracle):
     oracle.set_threads(oracle.max_threads())
@@ -314,19 +325,20 @@ def oracle_threads(oracle):
     oracle.set_threads(1)
 
 
-def _on_planes_of_both(K, fn):
-    """the call, which has to run on the kernel that reads planes of both operands while the digits are the narrow ones"""
+def _on_planes_of_both(K, fn, row_tiles):
+    """the call, which has to run on the kernel that reads planes of both operands, with A split as asked, while the digits are
+    the narrow ones"""
     def call():
-        before = K.lib.zk_gemm_pipe_calls()
+        before = K.lib.zk_gemm_pipe_calls(), K.lib.zk_gemm_rowtile_calls()
         out = fn()
-        call.on_planes = K.lib.zk_gemm_pipe_calls() == before + 1
+        call.on_planes = K.lib.zk_gemm_pipe_calls() == before[0] + 1 and K.lib.zk_gemm_rowtile_calls() == before[1] + row_tiles
         return (out,)
     return call
 
 
 def _planes_rounds(K, call, expect, operands, pokes):
-    """as _stale_guess_rounds, and the call on the stale guess ran on the planes of both operands: their two pre-passes are
-    all that can raise the verdict there"""
+    """as _stale_guess_rounds, and the call on the stale guess ran on the planes of both operands: what splits them (the pass
+    over B, and the pass over A or the row tiles) is all that can raise the verdict there"""
     def poked(poke):
         def f():
             assert call.on_planes, "the narrow call is expected on planes of both operands"
@@ -335,7 +347,7 @@ def _planes_rounds(K, call, expect, operands, pokes):
     _stale_guess_rounds(K, call, expect, operands, [poked(p) for p in pokes])
 
 
-def test_stale_guess_values_on_planes_of_both_operands(K, oracle, oracle_threads, small_b_first):
+def test_stale_guess_values_on_planes_of_both_operands(K, oracle, oracle_threads, row_tiles):
     """values of a causal prompt (n-contiguous, a batch each): wide elements of B at its ends and in its last batch, of A in
     its rows' ends, and in what had been all zeros and cut off"""
     rng = np.random.default_rng(23)
@@ -346,7 +358,7 @@ def test_stale_guess_values_on_planes_of_both_operands(K, oracle, oracle_threads
     P, V = Operand(p), Operand(rand_i64(rng, (Bq, T, Cc), 20))
     pokes = [lambda: V.poke((1, T - 1, Cc - 1), WIDE), lambda: V.poke((0, 0, 0), -WIDE), lambda: V.poke((0, 63, 64), WIDE),
              lambda: P.poke((1, S - 1, 0, T - 1), WIDE), lambda: P.poke((0, 5, 0, T - 1), WIDE), lambda: P.poke((1, 1100, 0, 0), -WIDE)]
-    call = _on_planes_of_both(K, lambda: K.einsum_bsht_btc_bshc(P.d, V.d, 23))
+    call = _on_planes_of_both(K, lambda: K.einsum_bsht_btc_bshc(P.d, V.d, 23), row_tiles)
     _planes_rounds(K, call, lambda: (oracle.einsum_bsht_btc_bshc(P.h, V.h, 23),), [P, V], pokes)
     # an element where A was cut off that fits the digits: the next call must see that the rows end later
     for op in (P, V):
@@ -363,25 +375,25 @@ def test_stale_guess_values_on_planes_of_both_operands(K, oracle, oracle_threads
     assert K.lib.zk_gemm_guard_hits() == hits
 
 
-def test_stale_guess_scores_on_planes_of_both_operands(K, oracle, oracle_threads, small_b_first):
+def test_stale_guess_scores_on_planes_of_both_operands(K, oracle, oracle_threads, row_tiles):
     """scores (k-contiguous, one cache for all rows) from 16384 rows on"""
     rng = np.random.default_rng(24)
     Bq, S, T, Cc = 1, 16400, 270, 40
     Q, Kc = Operand(rand_i64(rng, (Bq, S, 1, Cc), 20)), Operand(rand_i64(rng, (Bq, T, Cc), 20))
     pokes = [lambda: Kc.poke((0, T - 1, Cc - 1), WIDE), lambda: Kc.poke((0, 0, 0), -WIDE), lambda: Kc.poke((0, 130, 31), WIDE),
              lambda: Q.poke((0, S - 1, 0, Cc - 1), WIDE), lambda: Q.poke((0, 0, 0, 0), -WIDE)]
-    call = _on_planes_of_both(K, lambda: K.einsum_bshc_btc_bsht(Q.d, Kc.d, 21))
+    call = _on_planes_of_both(K, lambda: K.einsum_bshc_btc_bsht(Q.d, Kc.d, 21), row_tiles)
     _planes_rounds(K, call, lambda: (oracle.einsum_bshc_btc_bsht(Q.h, Kc.h, 21),), [Q, Kc], pokes)
 
 
-def test_stale_guess_per_head_weights_on_planes_of_both_operands(K, oracle, oracle_threads, small_b_first):
+def test_stale_guess_per_head_weights_on_planes_of_both_operands(K, oracle, oracle_threads, row_tiles):
     """one int32 matrix per head, n-contiguous, from 385 rows on; the widest weight belongs to the last head"""
     rng = np.random.default_rng(25)
     S, H, D, Cc = 390, 16, 70, 520
     q, w = Operand(rand_i64(rng, (1, S, H, D), 20)), Operand(rand_i32(rng, (H, D, Cc), 16))
     pokes = [lambda: w.poke((H - 1, D - 1, Cc - 1), 1 << 30), lambda: w.poke((0, 0, 0), -(1 << 30)), lambda: w.poke((7, 33, 300), 1 << 30),
              lambda: q.poke((0, S - 1, H - 1, D - 1), WIDE), lambda: q.poke((0, 200, 3, 64), -WIDE)]
-    call = _on_planes_of_both(K, lambda: K.einsum_bshd_hdc_bshc(q.d, w.d, 30))
+    call = _on_planes_of_both(K, lambda: K.einsum_bshd_hdc_bshc(q.d, w.d, 30), row_tiles)
     _planes_rounds(K, call, lambda: (oracle.einsum_bshd_hdc_bshc(q.h, w.h, 30),), [q, w], pokes)
 
 
@@ -561,15 +573,19 @@ def scratch_limit(K, monkeypatch):
     yield set_limit
     monkeypatch.delenv("ZK_SCRATCH_LIMIT", raising=False)
     monkeypatch.delenv("ZK_B_ROWS_MIN_MACS", raising=False)
+    monkeypatch.delenv("ZK_NO_ROWTILE", raising=False)
     K.lib.zk_reload_env()
 
 
 @pytest.mark.parametrize("S,T,C,limit", [(12800, 40, 512, 1 << 20),       # no room for the planes of A
                                          (385, 40, 12416, 1 << 20)])      # room for the planes of A, none for those of B
-def test_values_without_memory_for_digit_planes(K, oracle, monkeypatch, scratch_limit, S, T, C, limit):
+@pytest.mark.parametrize("row_tiles", [False, True])
+def test_values_without_memory_for_digit_planes(K, oracle, monkeypatch, scratch_limit, row_tiles, S, T, C, limit):
     """a small n-contiguous B whose product would run on planes of both operands: without memory for them it stays on the
     MFMA kernels that split both themselves, and leaves nothing behind that the next call trips over"""
     monkeypatch.setenv("ZK_B_ROWS_MIN_MACS", "1")
+    if not row_tiles:
+        monkeypatch.setenv("ZK_NO_ROWTILE", "1")
     rng = np.random.default_rng(S)
     p, v = rand_i64(rng, (1, S, 1, T), 19), rand_i64(rng, (1, T, C), 20)
     expected = oracle.einsum_bsht_btc_bshc(p, v, 23)
@@ -580,10 +596,11 @@ def test_values_without_memory_for_digit_planes(K, oracle, monkeypatch, scratch_
     for size, on_planes in ((None, 1), (limit, 0), (None, 1)):
         scratch_limit(size)
         for _ in range(3):
-            before = K.lib.zk_gemm_pipe_calls()
+            before = K.lib.zk_gemm_pipe_calls(), K.lib.zk_gemm_rowtile_calls()
             assert np.array_equal(host(K.einsum_bsht_btc_bshc(dp, dv, 23)), expected)
             assert K.gemm_last_plan()[0] == 2
-        assert K.lib.zk_gemm_pipe_calls() == before + on_planes
+        assert K.lib.zk_gemm_pipe_calls() == before[0] + on_planes
+        assert K.lib.zk_gemm_rowtile_calls() == before[1] + (on_planes and row_tiles and S == 12800)
         hits = K.lib.zk_gemm_guard_hits()
         dp.copy_(torch.from_numpy(wide))
         assert np.array_equal(host(K.einsum_bsht_btc_bshc(dp, dv, 23)), oracle.einsum_bsht_btc_bshc(wide, v, 23))

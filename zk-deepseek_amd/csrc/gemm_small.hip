@@ -11,6 +11,8 @@
 // 9.6 / 7.0, x [779,512] k-contiguous 21.7 / 15.0 (the first had become slower than on the general kernel, 10.3 -> 11.8 a call).
 #include "gemm_frag16.h"
 
+#include <atomic>
+
 namespace zk {
 
 struct SmallParams {
@@ -192,7 +194,7 @@ static int device_cus()
     return cus;
 }
 
-static long g_small_calls = 0;
+static std::atomic<long> g_small_calls(0);
 long gemm_small_calls() { return g_small_calls; }
 
 bool gemm_small_launch(const GemmDesc &d)
