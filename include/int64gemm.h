@@ -228,7 +228,8 @@ void int64_bmm_broadcast_noalloc(const int64_t *A, const void *B, int b32, int64
 void zk_gemm_set_path(int path);
 int zk_gemm_get_path(void);
 /* What the last GEMM-like call used: path (1/2) and the limb counts of A and B (0 for the VALU path, and for the
- * MFMA kernels for up to 16 rows, which take their digit counts from the data step by step). */
+ * MFMA kernels for up to 16 rows and for the scores and values of up to eight positions, which take their digit counts from
+ * the data step by step). */
 void zk_gemm_last_plan(int *path, int *limbs_a, int *limbs_b);
 /* i8 digit products per int64 multiply-add in the last GEMM-like call (0 for the VALU path).  At most
  * limbs_a * limbs_b; fewer when the stored bits [shift, shift + 64) of the sum lie below the weight of the top

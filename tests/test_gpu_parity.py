@@ -2042,8 +2042,9 @@ def test_fp8_quantisation_of_more_than_one_launch(K, oracle, cols):
     """a launch takes less than 2^32 threads: a matrix of 2^35 weights and some, whose slabs repeat, gives the same slab again
     and again, up to its last weight"""
     slab, count = 4096, 257
-    if torch.cuda.mem_get_info()[0] < 220 << 30:
-        pytest.skip("needs 176 GB of free device memory")
+    torch.cuda.empty_cache()            # what earlier tests left in torch's cache
+    if torch.cuda.mem_get_info()[0] < 170 << 30:
+        pytest.skip("needs 174 GB of free device memory")
     rows = slab * count - 1
     rng = np.random.default_rng(cols)
     w = rng.integers(0, 256, size=(slab, cols), dtype=np.uint8)

@@ -213,6 +213,10 @@ void einsum_bshd_hdc_bshc(const int64_t *q_nope, const int32_t *wkv_b_1, int64_t
     zk::gemm_dispatch(name, d);
 }
 
+// Positions up to which scores and values are offered to gemm_small_launch: a decoding step, or a few tokens checked together, which it
+// was made for.  Timing draws no line there: 9 to 64 positions whose tiles fit its limits would take 0.44 to 0.52 of the general
+// kernels' time (means of some 25 products each: 1 x 9 x 16 heads x [25,512] n-contiguous 9.8 / 7.2 us, 1 x 64 x 4 x [932,512] 22.3 / 15.8,
+// 1 x 32 x 16 x [170,512] k-contiguous 15.3 / 12.6); they keep the kernels that guess digit counts and check them.
 constexpr int kFewPositions = 8;
 
 // out[b,s,h,t] = (rescale/2 + sum_c A[b,s,h,c] * Bm[b,t,c]) >> rescale: one GEMM per batch, rows (s,h).

@@ -28,8 +28,7 @@ constexpr int kSmallWaves = 8, kSmallTile = 16, kSmallDiagonals = 9, kSmallWideD
 // one round of tiles 0.3-0.8 of their time up to K = 2048 (128 rows x [512,779] n-contiguous 20.0 / 8.9, 50 x [94,321] (5,5)
 // 24.9 / 7.1, 32 x [1513,759] 23.2 / 8.7, 274 x [161,2145] 22.6 / 16.2) and level at 4000; two rounds up to K = 1024 (128 x
 // [779,512] 18.8 / 13.3, 128 x [1024,512] 19.4 / 13.9; 66 x [1398,1454] 26.5 / 30.4); three rounds no longer (256 x [779,512]
-// 21.6 / 24.3).  Offered to it are scores and values of up to eight positions; other products keep the kernels that guess
-// digit counts and check them.
+// 21.6 / 24.3).  Offered to it are scores and values of up to eight positions (kFewPositions).
 constexpr int kSmallMaxK = 2048, kSmallMaxKTwoRounds = 1024;
 
 template <int NA, int NB, int D>
@@ -182,16 +181,6 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(SmallParam
     }
     const uint64_t lo = (uint64_t)s, hi = (uint64_t)(s >> 64);
     p.C[(long)g * p.sC + (long)m * p.ldc + n] = (int64_t)((lo >> p.shift) | ((hi << 1) << (63 - p.shift)));
-}
-
-static int device_cus()
-{
-    static const int cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        return n;
-    }();
-    return cus;
 }
 
 static std::atomic<long> g_small_calls(0);

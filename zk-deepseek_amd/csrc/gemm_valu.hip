@@ -676,14 +676,13 @@ __global__ __launch_bounds__(64 * kRegsWaves, 4) void gemv64_regs_kernel(ValuPar
     }
 }
 
-static int device_cus()
+int device_cus()
 {
-    static int cus = 0;
-    if (!cus) {
+    static const int cus = [] {
         int dev = 0, n = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cus = n;
-    }
+        return n;
+    }();
     return cus;
 }
 
