@@ -7,8 +7,8 @@
 // row read 64 contiguous bytes per load), take the digit counts that those need (3, 4 or 5 per operand, gemm_frag16.h),
 // split, multiply, and meet in LDS with their 128-bit sums.  A wavefront that meets values beyond five digits (2^38 and up)
 // multiplies its share again with nine digits.  Where a wavefront has one step at most (K up to 512) that step's elements are still in
-// its registers: a cache of 44 bits, share read again / this, kernel alone, 128 rows x [512,7] n-contiguous 7.2 / 5.3 us, x [512,300]
-// 9.6 / 7.0, x [779,512] k-contiguous 21.7 / 15.0 (the first had become slower than on the general kernel, 10.3 -> 11.8 a call).
+// its registers: a cache of 44 bits, share read again / this, us a call, 128 rows x [512,7] n-contiguous 8.9 / 6.3, x [512,300]
+// 9.4 / 6.5, x [779,512] k-contiguous 20.9 / 13.2 (the first had become slower than on the general kernel).
 #include "gemm_frag16.h"
 
 #include <atomic>
@@ -27,8 +27,8 @@ constexpr int kSmallWaves = 8, kSmallTile = 16, kSmallDiagonals = 9, kSmallWideD
 // Where it pays, against the general and the 16-row kernels over 250 shapes of 5 to 600 rows and 16 to 2048 columns (those / this, us):
 // one round of tiles 0.3-0.8 of their time up to K = 2048 (128 rows x [512,779] n-contiguous 20.0 / 8.9, 50 x [94,321] (5,5)
 // 24.9 / 7.1, 32 x [1513,759] 23.2 / 8.7, 274 x [161,2145] 22.6 / 16.2) and level at 4000; two rounds up to K = 1024 (128 x
-// [779,512] 18.8 / 13.3, 128 x [1024,512] 19.4 / 13.9; 66 x [1398,1454] 26.5 / 30.4); three rounds no longer (256 x [779,512]
-// 21.6 / 24.3).  Offered to it are scores and values of up to eight positions (kFewPositions).
+// [779,512] 18.8 / 11.7, 128 x [1024,512] 19.4 / 12.1; 66 x [1398,1454] 26.5 / 30.4); three rounds no longer (256 x [779,512]
+// 19.4 / 21.1).  Offered to it are scores and values of up to eight positions (kFewPositions).
 constexpr int kSmallMaxK = 2048, kSmallMaxKTwoRounds = 1024;
 
 template <int NA, int NB, int D>
@@ -117,25 +117,35 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(SmallParam
     // accumulator register r of lane (li, q) holds row 4*q + r, column li of the tile
     bool wide = false;
     if (ONE) {
-        v4i acc[kSmallWideDiagonals], narrow[kSmallDiagonals];
-#pragma unroll
-        for (int d = 0; d < kSmallWideDiagonals; d++) acc[d] = v4i{ 0, 0, 0, 0 };
-#pragma unroll
-        for (int d = 0; d < kSmallDiagonals; d++) narrow[d] = v4i{ 0, 0, 0, 0 };
+        RawFrag<false> fa, fb;
+        int na = 0, nb = 0;
         if (wave < steps) {
-            RawFrag<false> fa, fb;
             load(wave, fa, fb);
-            const int na = wave_digits(magnitude_or<false>(fa));
-            const int nb = wave_digits(magnitude_or<false>(fb));
-            wide = na > 5 || nb > 5;
-            if (!wide) small_narrow_step(na, nb, fa, fb, narrow);
-            else if (na <= 5) small_step<5, 9>(fa, fb, acc);
+            na = wave_digits(magnitude_or<false>(fa));
+            nb = wave_digits(magnitude_or<false>(fb));
+        }
+        // (each width adds up its own sums: with a choice between the two sets of accumulators in front of the sums a call takes 12.6 us
+        // on 128 rows x [779,512], now 11.7, and with 44 bits 14.3, now 13.2)
+        if (na == 0) {
+#pragma unroll
+            for (int o = 0; o < 4; o++) red[wave][o][lane] = Words{};
+        } else if (na <= 5 && nb <= 5) {
+            v4i acc[kSmallDiagonals];
+#pragma unroll
+            for (int d = 0; d < kSmallDiagonals; d++) acc[d] = v4i{ 0, 0, 0, 0 };
+            small_narrow_step(na, nb, fa, fb, acc);
+#pragma unroll
+            for (int o = 0; o < 4; o++) red[wave][o][lane] = sum_diagonals<kSmallDiagonals>([&](int d) { return acc[d][o]; }, 0);
+        } else {
+            v4i acc[kSmallWideDiagonals];
+#pragma unroll
+            for (int d = 0; d < kSmallWideDiagonals; d++) acc[d] = v4i{ 0, 0, 0, 0 };
+            if (na <= 5) small_step<5, 9>(fa, fb, acc);
             else if (nb <= 5) small_step<9, 5>(fa, fb, acc);
             else small_step<9, 9>(fa, fb, acc);
-        }
 #pragma unroll
-        for (int o = 0; o < 4; o++)
-            red[wave][o][lane] = wide ? sum_diagonals<kSmallWideDiagonals>([&](int d) { return acc[d][o]; }, 0) : sum_diagonals<kSmallDiagonals>([&](int d) { return narrow[d][o]; }, 0);
+            for (int o = 0; o < 4; o++) red[wave][o][lane] = sum_diagonals<kSmallWideDiagonals>([&](int d) { return acc[d][o]; }, 0);
+        }
     } else {
         v4i acc[kSmallDiagonals];
 #pragma unroll
