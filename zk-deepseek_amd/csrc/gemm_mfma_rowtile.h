@@ -1,8 +1,8 @@
 // Products of many rows with a B that is small next to them (a KV cache against the queries of a whole prompt, one head's
 // weights): B is split into digit planes by a pass in front (b_planes_kernel), A by this kernel itself, row tile by row tile.
 //   * A workgroup owns 64 rows of A at a time.  It reads them once, splits them into digit planes in a slot of scratch memory of
-//     its own (where its loads find them in the caches: a slot is written and read by one workgroup only), and multiplies
-//     all tile columns, or a part of them, from there.  A share of the next row tile is split behind every tile.  As a pass
+//     its own (a slot is written and read by one workgroup only; the slots outgrow the L2s, and the cache behind those serves the loads), and
+//     multiplies all tile columns, or a part of them, from there.  A share of the next row tile is split behind every tile.  As a pass
 //     of its own the split writes its planes to memory and reads them back: 435 of 2500 us of the attention core on 1024
 //     tokens.
 //   * Two workgroups of four wavefronts share a compute unit, and nothing ties them to one another: while one splits, or combines
@@ -12,10 +12,12 @@
 //     unit's LDS leaves three to five stages, so a stage is loaded again as soon as its fragments are in registers.
 // Row tiles whose later steps hold nothing but zeros in A (the probabilities of a causal prompt: a token's rows end at its
 // own position) end there; the split sees it.
-// What bounds it: power.  131072 rows x [1024,512], (3,4) digits: 630 us with neither stores nor splits (2.6 POP/s of i8
-// products, at 1.7-2.0 GHz), 595 with every load at one address on top; the stores add 105 and the splits 110-130,
-// overlapped or not.  Whole calls, pass over A and pipelined kernel / this, both on one device: 131072 x [1024,512] 874 / 818-840 us,
-// x [1024,64] 262 / 236, values of 1024 causal tokens 642 / 562-574, 31104 x [243,512] 86 / 81.
+// What bounds it: stores and splits that the steps do not hide, and the steps themselves.  131072 rows x [1024,512], (3,4) digits, 780-790
+// us: 630 with neither stores nor splits (2.6 POP/s of i8 products, what the pipelined kernel reaches on ready planes), 595 with every load at
+// one address on top; the stores add 105 and the splits 110-130, overlapped or not.  As a whole the matrix pipe is busy 53 % of the
+// time at 1.88 GHz, for the values of 1024 causal tokens 33 % at 2.17 GHz; each tile column reads the planes of A again from beyond
+// the L2s (1.6 GB beside 0.54 of A).  Whole calls, pass over A and pipelined kernel / this, both on one device, medians of six runs in turn: 131072 x
+// [1024,512] 876 / 833 us (869-885 / 827-896), x [1024,64] 266 / 239, values of 1024 causal tokens 643 / 579, 31104 x [243,512] 85 / 76.
 #pragma once
 #include "gemm_mfma_pipe.h"
 
