@@ -1343,9 +1343,9 @@ def test_rmsnorm_residual_fusion(K, oracle, N, k, w32, inplace):
 
 
 @pytest.mark.parametrize("M", [64, 65, 256, 257])
-@pytest.mark.parametrize("N,bits", [(513, 31), (2048, 55), (2049, 31), (5001, 20), (7168, 31), (8192, 62)])
+@pytest.mark.parametrize("N,bits", [(513, 31), (1024, 31), (1025, 20), (1026, 62), (2047, 31), (2048, 55), (2049, 31), (5001, 20), (7168, 31), (8192, 62)])
 def test_rmsnorm_row_counts_next_to_the_lines(K, oracle, M, N, bits):
-    """few rows take a thousand threads each: both sides of each line, odd lengths, statistics of one digit to six"""
+    """few rows take as many threads as pay, 256 to a thousand: both sides of each line, odd lengths, statistics of one digit to six"""
     rng = np.random.default_rng(M * N)
     X, Y, W = rand_i64(rng, (M, N), bits), rand_i64(rng, (M, N), 22), rng.integers(1 << 5, 1 << 20, size=(N,), dtype=np.int32)
     Xe, Ce, rmse = oracle.RMS_Norm_residual_int64(X, Y, 8, W, 1, N)

@@ -564,12 +564,15 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
         else { if (vec) ZK_RMS_LAUNCH2(THREADS, EPT, WPE, true, false); else ZK_RMS_LAUNCH2(THREADS, EPT, WPE, false, false); }      \
     } while (0)
     // Rows that have a compute unit to themselves take as many threads as it gives them, and a shorter chain of elements each: one
-    // row of 7168 with residual 11.3 -> 9.6 us, of 1536 6.2 -> 5.6; 256 rows of 7168 12.5 -> 11.6, of 5001 14.7 -> 11.1 (384 rows of
-    // 7168 11.5 -> 15.6: two to a unit).
+    // row of 7168 with residual 11.3 -> 9.6 us; 256 rows of 7168 12.5 -> 11.6, of 5001 14.7 -> 11.1 (384 rows of 7168 11.5 -> 15.6: two to a
+    // unit).  Short rows gain no more from it than the reduction over more wavefronts costs: 256 threads of eight elements / 512 of four / 1024
+    // of two, kernel alone, mean of 1 to 64 rows: up to 1024 elements 4.7 / 4.9 / 5.4 us (with residual 4.6 / 5.0 / 5.4), 1025 to 2048 5.3 / 5.1 / 5.5
+    // (5.1 / 5.3 / 5.6), of odd length 5.7 / 5.3 / 5.5.
+    const bool apart = vec && !res && M <= 16 && N > 22528;
     if (N <= 512) ZK_RMS_LAUNCH(256, 2, 1);
-    else if (M <= 64 && N <= 2048) ZK_RMS_LAUNCH(1024, 2, 1);
+    else if (N <= 2048 && !(M <= 64 && N > 1024)) ZK_RMS_LAUNCH(256, 8, 1);
+    else if (N <= 2048) ZK_RMS_LAUNCH(512, 4, 1);
     else if (M <= (N <= 4096 ? 64 : 256) && N <= 8192) ZK_RMS_LAUNCH(1024, 8, 1);
-    else if (N <= 2048) ZK_RMS_LAUNCH(256, 8, 1);
     else if (N <= 4096) ZK_RMS_LAUNCH(512, 8, 1);
     else if (N <= 8192) ZK_RMS_LAUNCH(512, 16, 6);
     else if (N <= 16384) ZK_RMS_LAUNCH(1024, 16, 1);
@@ -578,7 +581,7 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
     // 500 rows of 24576 54.0 / 42.2, of 18431 71.2 / 45.1.  A few of the longest, where nothing overlaps the spills and the second
     // kernel's several workgroups per row are worth their launch, keep the two: 1 row of 24576 13.8 / 15.3, 2 rows 13.2 / 14.4, 16 rows
     // 13.9 / 14.6, 24 rows 16.8 / 16.1 (of 20480 13.7 / 11.5; with residual 16 rows 21.0 / 17.4)
-    else if (N <= 24576 && M <= 65535 && !(M <= 16 && N > 22528 && vec && !res)) ZK_RMS_LAUNCH(1024, 24, 1);
+    else if (N <= 24576 && M <= 65535 && !apart) ZK_RMS_LAUNCH(1024, 24, 1);
     else {
         if (!apply_rows_ok(name, M)) return;          // before the residual sum or the statistic is written
         const int64_t *src = A;
