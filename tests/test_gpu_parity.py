@@ -1355,9 +1355,10 @@ def test_rmsnorm_row_counts_next_to_the_lines(K, oracle, M, N, bits):
     assert np.array_equal(rms[:M].numpy(), rmse) and np.array_equal(host(C), Ce)
 
 
-@pytest.mark.parametrize("M,N", [(1, 24576), (16, 22528), (16, 22530), (17, 22530), (17, 24576)])
+@pytest.mark.parametrize("M,N", [(1, 24576), (16, 22528), (16, 22530), (17, 22530), (17, 24576), (256, 16386), (257, 16386),
+                                 (257, 24576), (272, 18432), (273, 18432)])
 def test_rmsnorm_few_of_the_longest_rows(K, oracle, M, N):
-    """a statistic and a product of their own, or one kernel: both sides of the line, and residual and odd rows beside it"""
+    """a few rows, and a few more than there are compute units: a statistic and a product of their own, or one kernel: both sides of the line, and residual and odd rows beside it"""
     rng = np.random.default_rng(M * N)
     for n in (N, N - 1):
         X, W = rand_i64(rng, (M, n), 31), rand_i64(rng, (n,), 20)

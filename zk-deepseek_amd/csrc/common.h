@@ -14,6 +14,7 @@ enum ErrorCode { kOk = 0, kBadArgument = 1, kLaunchFailure = 2, kUnsupportedSize
 void set_error(int code, const char *fmt, ...);
 // hipGetLastError() after a launch; records kLaunchFailure and returns false on failure.
 bool check_launch(const char *what);
+int device_cus();                          // compute units of the current device
 
 // Errors detected on the device: a pinned host flag per kind (null when pinned memory is not to be had) that a kernel
 // sets to 1; zk_last_error() turns a set flag into a recorded error.

@@ -99,8 +99,6 @@ void gemm_valu_launch(const GemmDesc &d, GuardArgs *guard = nullptr);
 // guessed.  Returns false (nothing launched) for any other descriptor.
 bool gemm_gemv_launch(const GemmDesc &d);
 
-int device_cus();                          // compute units of the current device
-
 // Small products in one launch, nothing guessed (gemm_small.hip).  Returns false (nothing launched) for any other descriptor.
 bool gemm_small_launch(const GemmDesc &d);
 long gemm_small_calls();                   // launches so far

@@ -556,6 +556,7 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
     }
     const bool vec = N % 2 == 0 && (align & 15) == 0;
     const dim3 grid((unsigned)M);
+    const int cus = device_cus();
 #define ZK_RMS_LAUNCH2(THREADS, EPT, WPE, VEC, RES) \
     rms_fused_kernel<WT, THREADS, EPT, VEC, VEC || WPE < 4 ? WPE : 4, RES><<<grid, dim3(THREADS), 0, 0>>>(A, W, rms, C, N, eps, dim, r)
 #define ZK_RMS_LAUNCH(THREADS, EPT, WPE)                                                   \
@@ -568,7 +569,7 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
     // unit).  Short rows gain no more from it than the reduction over more wavefronts costs: 256 threads of eight elements / 512 of four / 1024
     // of two, kernel alone, mean of 1 to 64 rows: up to 1024 elements 4.7 / 4.9 / 5.4 us (with residual 4.6 / 5.0 / 5.4), 1025 to 2048 5.3 / 5.1 / 5.5
     // (5.1 / 5.3 / 5.6), of odd length 5.7 / 5.3 / 5.5.
-    const bool apart = vec && !res && M <= 16 && N > 22528;
+    const bool apart = vec && !res && ((M <= 16 && N > 22528) || (M > cus && M <= cus + cus / 16));
     if (N <= 512) ZK_RMS_LAUNCH(256, 2, 1);
     else if (N <= 2048 && !(M <= 64 && N > 1024)) ZK_RMS_LAUNCH(256, 8, 1);
     else if (N <= 2048) ZK_RMS_LAUNCH(512, 4, 1);
@@ -580,7 +581,9 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
     // kernels, as below / this, us: 1 row of 18432 10.5 / 9.9, 64 rows 17.3 / 13.7, 500 rows 42.6 / 33.1, with residual 74.6 / 56.3;
     // 500 rows of 24576 54.0 / 42.2, of 18431 71.2 / 45.1.  A few of the longest, where nothing overlaps the spills and the second
     // kernel's several workgroups per row are worth their launch, keep the two: 1 row of 24576 13.8 / 15.3, 2 rows 13.2 / 14.4, 16 rows
-    // 13.9 / 14.6, 24 rows 16.8 / 16.1 (of 20480 13.7 / 11.5; with residual 16 rows 21.0 / 17.4)
+    // 13.9 / 14.6, 24 rows 16.8 / 16.1 (of 20480 13.7 / 11.5; with residual 16 rows 21.0 / 17.4).  So do a few rows more than there are compute
+    // units, which would be a second round nearly empty: 257 rows of 18432 26.8 / 28.9, of 24576 34.0 / 35.8, 272 rows 34.9 / 35.6, 288 rows
+    // 36.5 / 36.2
     else if (N <= 24576 && M <= 65535 && !apart) ZK_RMS_LAUNCH(1024, 24, 1);
     else {
         if (!apply_rows_ok(name, M)) return;          // before the residual sum or the statistic is written
