@@ -2027,7 +2027,7 @@ def test_converters(K, oracle):
 
 
 @pytest.mark.parametrize("rows,cols", [(300, 4), (1, 1024), (129, 12), (257, 2052), (2051, 2052), (513, 8200), (100, 16384),
-                                       (1, 5), (131, 5), (300, 6), (129, 129), (257, 1027), (2053, 2051), (3, 1), (5, 3)])
+                                       (1, 5), (131, 5), (300, 6), (129, 129), (1, 511), (73, 7), (57, 9), (257, 1027), (2053, 2051), (3, 1), (5, 3)])
 def test_fp8_quantisation_over_ends_of_rows(K, oracle, rows, cols):
     """workgroups take the pieces of the matrix one after the other, whatever its rows: rows of one piece, ends of rows and of
     scale blocks inside a workgroup's stretch, a last stretch that is not whole, one and two pieces per thread,

@@ -143,7 +143,11 @@ static void for_stretches(long pieces, Launch launch)
     for (long b = 0; b < blocks; b += kMost) launch(dim3((unsigned)(blocks - b < kMost ? blocks - b : kMost)), b * per_block, two);
 }
 
-// element by element: rows of one to three weights, and pointers that are not aligned to the vectors
+constexpr long kPiecesMin = 512;
+
+// element by element: rows of one to three weights, matrices so small that a thread per piece is a longer chain for nothing (in
+// pieces / so, kernel alone, us: 1 x 7 1.55 / 1.36, 1 x 101 1.60 / 1.36, 1 x 333 1.60 / 1.48, but 128 x 5 1.46 / 1.72, 1 x 1537 1.68 / 2.20), and
+// pointers that are not aligned to the vectors
 __global__ __launch_bounds__(256) void fp8_to_int32_kernel(const uint8_t *__restrict__ w, const float *__restrict__ scale,
                                                            int32_t *__restrict__ out, long n, int cols, int scale_cols, float mult)
 {
@@ -211,7 +215,7 @@ void fp8_block_scaled_to_int32(const uint8_t *w, const float *scale, int32_t *ou
             if (two) zk::fp8_to_int32_vec_kernel<2><<<grid, dim3(256), 0, 0>>>(wp, scale, op, begin, n / 4, ppr, scale_cols, mult);
             else zk::fp8_to_int32_vec_kernel<1><<<grid, dim3(256), 0, 0>>>(wp, scale, op, begin, n / 4, ppr, scale_cols, mult);
         });
-    } else if (cols >= 4 && ((uintptr_t)w & 3) == 0 && ((uintptr_t)out & 15) == 0) {
+    } else if (cols >= 4 && n >= zk::kPiecesMin && ((uintptr_t)w & 3) == 0 && ((uintptr_t)out & 15) == 0) {
         zk::for_stretches(n / 4, [&](dim3 grid, long begin, bool two) {
             if (two) zk::fp8_to_int32_any_kernel<2><<<grid, dim3(256), 0, 0>>>(w, scale, out, begin, n, cols, scale_cols, mult);
             else zk::fp8_to_int32_any_kernel<1><<<grid, dim3(256), 0, 0>>>(w, scale, out, begin, n, cols, scale_cols, mult);
