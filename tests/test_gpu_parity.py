@@ -119,6 +119,21 @@ def test_gemm_two_depths_per_step(K, oracle, bits_a, bits_w, digits, w32):
     K.lib.zk_gemm_set_path(0)
 
 
+@pytest.mark.parametrize("w32", [False, True])
+@pytest.mark.parametrize("M", [129, 160, 161, 193, 224, 225, 256])
+def test_gemm_last_row_tile_on_planes(K, oracle, M, w32):
+    """A from planes on 128x64 tiles: the last row tile has one to four live groups of 32 rows, whose wavefronts alone load
+    blocks of A; one, two and three steps of 64 k, the last of them partial"""
+    rng = np.random.default_rng(M * 2 + w32)
+    for Kd, bits_a, bits_w, digits in ((64, 20, 28, (3, 4)), (130, 28, 28, (4, 4)), (191, 28, 20, (4, 3))):
+        A = rand_i64(rng, (1, M, Kd), bits_a)
+        W = rand_i32(rng, (8260, Kd), bits_w) if w32 else rand_i64(rng, (8260, Kd), bits_w)
+        for _ in range(2):      # (a first call may run on digits remembered for other operands at these addresses)
+            _gemm_case(K, oracle, 2, A, W, 1, 1, 23)
+        assert K.gemm_last_plan()[1:] == digits
+    K.lib.zk_gemm_set_path(0)
+
+
 @pytest.mark.parametrize("Kd", [14432, 14464, 16384, 18432])
 def test_gemm_long_k_with_nine_digit_operands(K, oracle, Kd):
     """the int32 accumulators of the MFMA path hold min(NA, NB) * K * 2^14 up to 0x7F000000 (the epilogue hands carries from

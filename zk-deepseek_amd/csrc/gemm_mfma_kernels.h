@@ -591,6 +591,10 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
     constexpr int A_IT = APL ? 1 : (A_ITEMS + T - 1) / T, B_IT = BPL ? 1 : (B_ITEMS + T - 1) / T;
     constexpr int A_CHUNKS = KK * A_BLOCKS * 64, A_CIT = APL ? (A_CHUNKS + T - 1) / T : 1;
     constexpr int B_CHUNKS = KK * B_BLOCKS * 64, B_CIT = BPL ? (B_CHUNKS + T - 1) / T : 1;
+    // Where the blocks of A's planes come out even, a wavefront loads those of its own rows (and of the depth that its column
+    // group has the number of): one without rows then loads its share of B alone.
+    constexpr bool OWN_ROWS = APL && WM == 1 && WVM > 1 && KK == WVN;
+    static_assert(!OWN_ROWS || A_CIT == NA, "two depths of 32 rows between the wavefronts of a row");
     static_assert(!BPL || (!B32 && !BKM && !BRS), "prepared planes of B go with the int64 forms (and are made for the kernel's KK: the owned-k order depends on it)");
     int64_t sa[A_IT][8], sb[B_IT][8];
     v4i pa[A_CIT], pb[B_CIT];
@@ -616,7 +620,8 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
             const bool live = A_CHUNKS % T == 0 || c < A_CHUNKS;
             const int cc0 = live ? c : 0;
             // LDS order inside a stage is [kk][sub][digit]; planes are [sub][ks32][digit]
-            const int kk = cc0 / (A_BLOCKS * 64), cc = cc0 - kk * (A_BLOCKS * 64);
+            const int kk = OWN_ROWS ? wn : cc0 / (A_BLOCKS * 64);
+            const int cc = OWN_ROWS ? (wm * NA + it) * 64 + lane : cc0 - kk * (A_BLOCKS * 64);
             const int sub_i = cc / (NA * 64), within = cc - sub_i * (NA * 64);
             a_pl[it] = p.a_planes + (((long)g * p.a_msub + (m0 >> 5) + sub_i) * p.a_ksteps + kk) * (NA * 1024) + within * 16;
             pl_dst[it] = live ? kk * SUBSTAGE + cc * 16 : DUMMY;
@@ -681,12 +686,14 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
     constexpr int B_N = BPL ? B_CIT : B_IT;          // items (or chunks of planes) of B per thread
 
     // FAST: the whole step lies inside K and the pointers allow 16-byte loads: no guards at all.
-    auto fetch = [&](int ks, auto fast_tag, auto part_tag) {
+    // WITH_A: false in a wavefront whose rows of A nobody multiplies.
+    auto fetch = [&](int ks, auto fast_tag, auto part_tag, auto a_tag) {
+        constexpr bool WITH_A = decltype(a_tag)::value;
         constexpr bool FAST = decltype(fast_tag)::value;
         constexpr int PART = decltype(part_tag)::value;
         constexpr int B_LO = PART == 1 ? B_N / 2 : 0, B_HI = PART == 0 ? B_N / 2 : B_N;
         const int k0 = ks * BK;
-        if (PART == 1) {
+        if (PART == 1 || !WITH_A) {
         } else if (APL) {
 #pragma unroll
             for (int it = 0; it < A_CIT; it++)
@@ -728,10 +735,11 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
     };
 
     // staged elements -> digits -> LDS stage `buf`, fragment order
-    auto stash = [&](int buf, auto part_tag) {
+    auto stash = [&](int buf, auto part_tag, auto a_tag) {
+        constexpr bool WITH_A = decltype(a_tag)::value;
         constexpr int PART = decltype(part_tag)::value;
         constexpr int B_LO = PART == 1 ? B_N / 2 : 0, B_HI = PART == 0 ? B_N / 2 : B_N;
-        if (PART == 1) {
+        if (PART == 1 || !WITH_A) {
         } else if (APL) {
 #pragma unroll
             for (int it = 0; it < A_CIT; it++)
@@ -846,22 +854,24 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
     };
 
     // prologue: stage 0 holds the first step, the staging registers hold the second
-    if (ks_begin < full_steps) fetch(ks_begin, std::true_type(), PAll()); else fetch(ks_begin, std::false_type(), PAll());
+    if (ks_begin < full_steps) fetch(ks_begin, std::true_type(), PAll(), std::true_type()); else fetch(ks_begin, std::false_type(), PAll(), std::true_type());
     track(PAll());
-    stash(0, PAll());
+    stash(0, PAll(), std::true_type());
     if (ks_begin + 1 < ks_end) {
-        if (ks_begin + 1 < full_steps) fetch(ks_begin + 1, std::true_type(), PAll()); else fetch(ks_begin + 1, std::false_type(), PAll());
+        if (ks_begin + 1 < full_steps) fetch(ks_begin + 1, std::true_type(), PAll(), std::true_type()); else fetch(ks_begin + 1, std::false_type(), PAll(), std::true_type());
     }
     __syncthreads();
     int ks = ks_begin;
     const int fast_end = full_steps < ks_end ? full_steps : ks_end;
-    // (411 rows x [18432,7168] int32, (4,4): 846 -> 805 us.  The 128x128 tiles keep the one loop: with two, the registers of
+    // (411 rows x [18432,7168] int32, (4,4): 846 -> 805 us, and 824 -> 803 on another device without its share of
+    // A's planes, too; 192 rows 427 -> 418, 300 rows 619 -> 606.  The 128x128 tiles keep the one loop: with two, the registers of
     // the hot one were dealt worse and 512 x 7168 x 18432 went from 622 to 634.)
     if (WM == 1 && WVM > 1 && !rows_live) {
+        typedef std::integral_constant<bool, !OWN_ROWS> DeadA;
         auto dead_step = [&](int step, auto fast_tag) {
-            stash(((step - ks_begin) & 1) ^ 1, PAll());
+            stash(((step - ks_begin) & 1) ^ 1, PAll(), DeadA());
             track(PAll());
-            if (step + 2 < ks_end) fetch(step + 2, fast_tag, PAll());
+            if (step + 2 < ks_end) fetch(step + 2, fast_tag, PAll(), DeadA());
             __syncthreads();
         };
         for (; ks + 2 < fast_end; ks++) dead_step(ks, std::true_type());
@@ -924,7 +934,7 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
                 v4i fa[WM][NA], fb[WN][NB];
                 load_frags(cur, 0, fa, fb);
                 mfma_slice(I0(), IF(), fa, fb);
-                stash(cur ^ 1, PFirst());
+                stash(cur ^ 1, PFirst(), std::true_type());
 #pragma unroll
                 for (int i = 0; i < MFMAS; i++) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -933,14 +943,14 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 track(PFirst());
-                if (ks + 2 < ks_end) fetch(ks + 2, fast_tag, PFirst());
+                if (ks + 2 < ks_end) fetch(ks + 2, fast_tag, PFirst(), std::true_type());
                 __builtin_amdgcn_sched_barrier(0);
             }
             {
                 v4i fa[WM][NA], fb[WN][NB];
                 load_frags(cur, 1, fa, fb);
                 mfma_slice(I0(), IF(), fa, fb);
-                stash(cur ^ 1, PSecond());
+                stash(cur ^ 1, PSecond(), std::true_type());
 #pragma unroll
                 for (int i = 0; i < MFMAS; i++) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -949,7 +959,7 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 track(PSecond());
-                if (ks + 2 < ks_end) fetch(ks + 2, fast_tag, PSecond());
+                if (ks + 2 < ks_end) fetch(ks + 2, fast_tag, PSecond(), std::true_type());
             }
             __syncthreads();
             return;
@@ -965,7 +975,7 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
         mfma_slice(I0(), IH(), fa, fb);
         __builtin_amdgcn_sched_barrier(0);
         mfma_slice(IH(), IF(), fa, fb);
-        stash(cur ^ 1, PAll());
+        stash(cur ^ 1, PAll(), std::true_type());
 #pragma unroll
         for (int i = 0; i < MFMAS - MFMAS / 2; i++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -974,7 +984,7 @@ __device__ __forceinline__ void gemm_mfma_block(const MfmaParams &p, const int b
         }
         __builtin_amdgcn_sched_barrier(0);
         track(PAll());
-        if (ks + 2 < ks_end) fetch(ks + 2, fast_tag, PAll());
+        if (ks + 2 < ks_end) fetch(ks + 2, fast_tag, PAll(), std::true_type());
         __syncthreads();
     };
 
