@@ -1671,10 +1671,12 @@ def test_silu_mul_q23_fusion(K, oracle, shape, keep):
         assert np.array_equal(host(S), se)
 
 
-# (the shapes with 2..16 groups of 8, 16 or 32 experts run on the lane-per-group kernel, the others on the wave-wide one;
+# (128, 256 and 512 experts in a power of two of groups run on the kernel for few tokens up to 8192 of them, other shapes with
+#  2..16 groups of 8, 16 or 32 experts, and those beyond 8192 tokens, on the lane-per-group kernel, the others on the wave-wide one;
 #  (64, 8, 2, 40) and (32, 2, 1, 20) ask for more winners than the kept groups hold, so masked experts win too)
 GATE_SHAPES = [(256, 8, 4, 8), (16, 4, 2, 4), (64, 1, 1, 6), (96, 3, 3, 5), (512, 8, 3, 8), (1024, 16, 5, 64), (7, 1, 1, 7),
-               (512, 16, 4, 6), (64, 4, 2, 9), (64, 8, 2, 40), (32, 2, 1, 20), (128, 16, 16, 64), (64, 2, 2, 3)]
+               (512, 16, 4, 6), (64, 4, 2, 9), (64, 8, 2, 40), (32, 2, 1, 20), (128, 16, 16, 64), (64, 2, 2, 3),
+               (128, 1, 1, 64), (256, 1, 1, 5), (128, 64, 20, 64), (256, 32, 1, 9), (512, 2, 1, 3), (512, 64, 3, 30)]
 
 
 @pytest.mark.parametrize("E,G,KG,K_", GATE_SHAPES)
@@ -1682,7 +1684,7 @@ GATE_SHAPES = [(256, 8, 4, 8), (16, 4, 2, 4), (64, 1, 1, 6), (96, 3, 3, 5), (512
 def test_gate_route(K, oracle, E, G, KG, K_, with_bias):
     """routing of Gate.forward on the device against the oracle, ties included (coarse scores tie often)"""
     rng = np.random.default_rng(E * 3 + G + with_bias)
-    # (beyond 8192 tokens the lane-per-group kernel switches from four lanes per group to one)
+    # (up to 8192 tokens a token has more lanes than beyond)
     for T, hi in ((1, 1 << 23), (77, 1 << 23), (300, 12), (1031, 1 << 23), (8200, 1 << 23), (8195, 9)):
         scores = rng.integers(1, hi, size=(T, E), dtype=np.int64)
         bias = rng.integers(-(hi >> 3) - 1, (hi >> 3) + 1, size=E, dtype=np.int64).astype(np.int32) if with_bias else None

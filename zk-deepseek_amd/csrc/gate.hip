@@ -38,8 +38,52 @@ __device__ __forceinline__ int64_t floordiv64(int64_t a, int64_t b)
 {
     if (b == 0) return 0;
     int64_t q = tdiv64(a, b);
-    if ((a % b != 0) && ((a < 0) != (b < 0))) q--;
+    if ((uint64_t)q * (uint64_t)b != (uint64_t)a && ((a < 0) != (b < 0))) q--;
     return q;
+}
+
+// The values of a lane and of its partner OFF lanes away, as a reduction over 1, 2, 4 ... lanes needs them (lanes that have met
+// already hold the same): through the vector pipe alone, where a shuffle goes through LDS.  Within sixteen lanes by row permutes
+// (neighbours, pairs, mirrored eights, mirrored sixteens), beyond by swapping rows of sixteen and halves of the wavefront.
+template <int OFF>
+__device__ __forceinline__ void lane_pair(int64_t v, int64_t &a, int64_t &b)
+{
+    const unsigned lo = (unsigned)(uint64_t)v, hi = (unsigned)((uint64_t)v >> 32);
+    if constexpr (OFF <= 8) {
+        constexpr int CTRL = OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : OFF == 4 ? 0x141 : 0x140;
+        const unsigned ol = (unsigned)__builtin_amdgcn_update_dpp(0, (int)lo, CTRL, 0xF, 0xF, true);
+        const unsigned oh = (unsigned)__builtin_amdgcn_update_dpp(0, (int)hi, CTRL, 0xF, 0xF, true);
+        a = v;
+        b = (int64_t)((uint64_t)oh << 32 | ol);
+    } else {
+        const auto l = OFF == 16 ? __builtin_amdgcn_permlane16_swap(lo, lo, false, false) : __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const auto h = OFF == 16 ? __builtin_amdgcn_permlane16_swap(hi, hi, false, false) : __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        a = (int64_t)((uint64_t)h[0] << 32 | l[0]);
+        b = (int64_t)((uint64_t)h[1] << 32 | l[1]);
+    }
+}
+template <int OFF>
+__device__ __forceinline__ int64_t lane_max(int64_t v)
+{
+    int64_t a, b;
+    lane_pair<OFF>(v, a, b);
+    return a > b ? a : b;
+}
+// the two largest of both sides: the larger first, then the best of the rest
+template <int OFF>
+__device__ __forceinline__ void lane_best2(int64_t &b1, int64_t &b2)
+{
+    int64_t a1, o1, a2, o2;
+    lane_pair<OFF>(b1, a1, o1);
+    lane_pair<OFF>(b2, a2, o2);
+    const int64_t lo = a1 > o1 ? o1 : a1, rest = a2 > o2 ? a2 : o2;
+    b1 = a1 > o1 ? a1 : o1;
+    b2 = lo > rest ? lo : rest;
+}
+__device__ __forceinline__ int64_t from_lane(int64_t v, int lane)      // (the same lane for the whole wavefront)
+{
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(uint64_t)v, lane), hi = (unsigned)__builtin_amdgcn_readlane((int)((uint64_t)v >> 32), lane);
+    return (int64_t)((uint64_t)hi << 32 | lo);
 }
 
 constexpr int64_t kMasked = -((int64_t)1 << 42);
@@ -147,7 +191,8 @@ __global__ __launch_bounds__(256) void gate_route_kernel(const int64_t *__restri
 // from l * GS on in registers, LPG neighbouring lanes make up a group.  The groups' two best, the masking and most of the
 // arg-max over a token's experts (GS comparisons per lane, log2(LT) exchanges) stay inside a lane; the wave-wide form
 // above pays six exchanges per group and per winner.  LPG = 1 gives the most tokens per wavefront (throughput when
-// there are many tokens), LPG = 4 the shorter chain of dependent work per token (latency when there are few).
+// there are many tokens), LPG = 4 the shorter chain of dependent work per token (few tokens of up to 64 experts; more experts:
+// gate_route_few_kernel).
 template <int GS, int LPG, int NG, bool FUSED>
 __global__ __launch_bounds__(256) void gate_route_groups_kernel(const int64_t *__restrict__ scores, const int64_t *__restrict__ lut,
                                                                 int64_t *__restrict__ sig, const int32_t *__restrict__ bias,
@@ -249,6 +294,107 @@ __global__ __launch_bounds__(256) void gate_route_groups_kernel(const int64_t *_
     }
 }
 
+// Tokens up to which a token has a wavefront to itself.  What bounds one token is the chain of dependent work, what bounds many
+// their instructions.  Whole calls with sigmoid, lane groups / a wavefront per token (10.1 us is what the host takes): 256 experts in 8
+// groups, 256 tokens 13.2 / 10.2 us, 4096 17.1 / 13.7, 8192 24.2 / 22.5; 512 experts in 8 groups, which had six exchanges
+// through LDS per group and winner, 1 token 23.9 / 10.2, 8192 118 / 38; 128 in 8 groups 4096 12.0 / 10.5, 8192 15.7 / 16.3.
+// The launch for one token and 256 experts: 13-17 -> 7.6 us.
+constexpr int kFewTokens = 8192;
+
+// Few tokens: a wavefront each, EPL consecutive experts per lane, 64 / n_groups lanes per group (a power of two).  What takes
+// the time is the chain of dependent work per token, so nothing in it leaves the registers: maxima go through lane_pair, a
+// winner's lane is found by a ballot (the lowest lane, and in it the lowest expert, wins a tie) and its unbiased score is read
+// from that lane; the sigmoid's table waits in LDS, loaded beside the logits.
+template <int EPL, bool FUSED>
+__global__ __launch_bounds__(64) void gate_route_few_kernel(const int64_t *__restrict__ scores, const int64_t *__restrict__ lut,
+                                                            int64_t *__restrict__ sig, const int32_t *__restrict__ bias,
+                                                            int64_t *__restrict__ weights, int64_t *__restrict__ indices,
+                                                            int64_t *__restrict__ raw, int n_groups, int topk_groups, int topk)
+{
+    __shared__ int64_t table[256];
+    const int lane = threadIdx.x;
+    const long tok = blockIdx.x;
+    const int64_t *row = scores + (tok * 64 + lane) * EPL;
+    int64_t orig[EPL], s[EPL];
+#pragma unroll
+    for (int j = 0; j < EPL; j += 2) {
+        const i64x2g v = *reinterpret_cast<const i64x2g *>(row + j);
+        orig[j] = v.x;
+        orig[j + 1] = v.y;
+    }
+    int add[EPL];
+#pragma unroll
+    for (int j = 0; j < EPL; j++) add[j] = bias ? bias[lane * EPL + j] : 0;
+    if (FUSED) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) table[lane + 64 * q] = lut[lane + 64 * q];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < EPL; j++) orig[j] = act_one<23, true>(orig[j], table);
+        if (sig) {
+#pragma unroll
+            for (int j = 0; j < EPL; j += 2) *reinterpret_cast<i64x2g *>(sig + (tok * 64 + lane) * EPL + j) = i64x2g{ orig[j], orig[j + 1] };
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < EPL; j++) s[j] = (int64_t)((uint64_t)orig[j] + (uint64_t)(int64_t)add[j]);
+
+    if (n_groups > 1) {
+        // the group's score: its two largest biased scores (its largest without bias); then the group's rank
+        const int lanes = 64 / n_groups, g = lane / lanes;
+        int64_t b1 = s[0], b2 = INT64_MIN;
+#pragma unroll
+        for (int j = 1; j < EPL; j++) {
+            const bool first_j = s[j] > b1;
+            const int64_t lower = first_j ? b1 : s[j];
+            b1 = first_j ? s[j] : b1;
+            b2 = lower > b2 ? lower : b2;
+        }
+        if (lanes > 1) lane_best2<1>(b1, b2);
+        if (lanes > 2) lane_best2<2>(b1, b2);
+        if (lanes > 4) lane_best2<4>(b1, b2);
+        if (lanes > 8) lane_best2<8>(b1, b2);
+        if (lanes > 16) lane_best2<16>(b1, b2);
+        const int64_t gs = bias ? (int64_t)((uint64_t)b1 + (uint64_t)b2) : b1;
+        int rank = 0;
+        for (int h = 0; h < n_groups; h++) {
+            const int64_t o = from_lane(gs, h * lanes);
+            if (o > gs || (o == gs && h < g)) rank++;
+        }
+        if (rank >= topk_groups) {
+#pragma unroll
+            for (int j = 0; j < EPL; j++) s[j] = kMasked;
+        }
+    }
+
+    unsigned taken = 0;                                    // bit j: s[j] has won already
+    int64_t wsum = 0, my_w = 0;                            // lane i < topk keeps winner i
+    int my_idx = 0;
+    for (int i = 0; i < topk; i++) {
+        int64_t v = INT64_MIN, w = 0;
+        int slot = -1;
+#pragma unroll
+        for (int j = 0; j < EPL; j++) {
+            const bool better_j = !((taken >> j) & 1) && (slot < 0 || s[j] > v);
+            v = better_j ? s[j] : v;
+            w = better_j ? orig[j] : w;
+            slot = better_j ? j : slot;
+        }
+        const int64_t best = lane_max<32>(lane_max<16>(lane_max<8>(lane_max<4>(lane_max<2>(lane_max<1>(v))))));
+        const int owner = __ffsll((unsigned long long)__ballot(slot >= 0 && v == best)) - 1;
+        w = from_lane(w, owner);
+        wsum = (int64_t)((uint64_t)wsum + (uint64_t)w);
+        const int idx = owner * EPL + __builtin_amdgcn_readlane(slot, owner);
+        if (lane == owner) taken |= 1u << slot;
+        if (lane == i) { my_w = w; my_idx = idx; }
+    }
+    if (lane >= topk) return;
+    if (raw) raw[tok * topk + lane] = my_w;
+    const int64_t w = floordiv64((int64_t)((uint64_t)my_w << 23), wsum);           // (w * 2^23) // sum  (model.py:1203)
+    weights[tok * topk + lane] = (int64_t)((uint64_t)w * 5ull) >> 1;                // w * 5 // 2         (model.py:1208)
+    indices[tok * topk + lane] = my_idx;
+}
+
 template <bool FUSED>
 static void gate_launch(const char *name, const int64_t *scores, const int64_t *lut, int64_t *sig, const int32_t *bias,
                         int64_t *weights, int64_t *indices, int64_t *raw, int T, int E, int n_groups, int topk_groups, int topk)
@@ -264,13 +410,22 @@ static void gate_launch(const char *name, const int64_t *scores, const int64_t *
     const int gsize = E / n_groups;
     const bool aligned = (((uintptr_t)scores | (uintptr_t)sig) & 15) == 0;
     const bool pow2 = (n_groups & (n_groups - 1)) == 0;
+    if (aligned && pow2 && T <= kFewTokens && (E == 128 || E == 256 || E == 512) && gsize >= E / 64) {
+#define ZK_GATE_F(EPL) gate_route_few_kernel<EPL, FUSED><<<dim3((unsigned)T), dim3(64), 0, 0>>>(scores, lut, sig, bias, weights, indices, raw, n_groups, topk_groups, topk)
+        if (E == 128) ZK_GATE_F(2);
+        else if (E == 256) ZK_GATE_F(4);
+        else ZK_GATE_F(8);
+#undef ZK_GATE_F
+        check_launch(name);
+        return;
+    }
     if (aligned && pow2 && n_groups >= 2 && (gsize == 32 || gsize == 16 || gsize == 8) && n_groups <= 16) {
-        // few tokens: four lanes per group (the chain of dependent work per token is what takes the time); many: one
-        const bool spread = T <= 8192;
+        // (what the kernel for few tokens does not take: four lanes per group up to 64 experts; else one)
+        const bool spread = T <= kFewTokens && E <= 64;
         const int per_wave = 64 / (n_groups * (spread ? 4 : 1));
         const dim3 grid((unsigned)((T + 4 * per_wave - 1) / (4 * per_wave))), block(256);
 #define ZK_GATE_G(GS, LPG, NG) gate_route_groups_kernel<GS, LPG, NG, FUSED><<<grid, block, 0, 0>>>(scores, lut, sig, bias, weights, indices, raw, T, topk_groups, topk)
-#define ZK_GATE_NG(GSIZE, NG) do { if (spread) ZK_GATE_G(GSIZE / 4, 4, NG); else ZK_GATE_G(GSIZE, 1, NG); } while (0)
+#define ZK_GATE_NG(GSIZE, NG) do { if constexpr (GSIZE * NG <= 64) { if (spread) { ZK_GATE_G(GSIZE / 4, 4, NG); break; } } ZK_GATE_G(GSIZE, 1, NG); } while (0)
 #define ZK_GATE_GS(GSIZE) do { if (n_groups == 2) ZK_GATE_NG(GSIZE, 2); else if (n_groups == 4) ZK_GATE_NG(GSIZE, 4); \
                                else if (n_groups == 8) ZK_GATE_NG(GSIZE, 8); else ZK_GATE_NG(GSIZE, 16); } while (0)
         if (gsize == 32) ZK_GATE_GS(32);
