@@ -1370,6 +1370,36 @@ def test_rmsnorm_row_counts_next_to_the_lines(K, oracle, M, N, bits):
     assert np.array_equal(rms[:M].numpy(), rmse) and np.array_equal(host(C), Ce)
 
 
+@pytest.mark.parametrize("M", [1, 2, 32, 33])
+@pytest.mark.parametrize("N,off", [(4096, 0), (4097, 0), (4098, 0), (6143, 1), (6145, 0), (7168, 1), (8191, 0), (8192, 0)])
+def test_rmsnorm_few_rows_on_several_compute_units(K, oracle, M, N, off):
+    """up to 32 rows of 4097 to 8192 elements: four workgroups per row, each storing a quarter of it; not where what is stored
+    overlaps what is read (the sum over its first operand, the result over its row)"""
+    rng = np.random.default_rng(M * 31 + N)
+    A, Y = rand_i64(rng, (M, N), 31), rand_i64(rng, (M, N), 22)
+    W = rng.integers(1 << 18, 1 << 20, size=(N,), dtype=np.int32)
+    A[M - 1], Y[M - 1] = 0, 0                       # a row without a statistic of its own
+    Ce, rms_e = oracle.RMS_Norm_int64(A, W, 1, N)
+    X = A + (Y << 8)
+    Xe, rms_x = oracle.RMS_Norm_int64(X, W, 1, N)
+
+    def shifted(a):
+        t = torch.empty(a.size + 2, dtype=torch.int64, device="cuda")[off:off + a.size].view(M, N)
+        return t.copy_(dev(a))
+    w, stat, out, xo = dev(W), torch.empty(M, dtype=torch.int64, device="cuda"), shifted(A), shifted(A)
+    lib, ptr = K.lib, lambda t: t.data_ptr()
+    for a in (shifted(A), out):                      # the second: the result over the row
+        lib.rms_norm_fused_32(ptr(a), ptr(w), ptr(stat), ptr(out), M, N, 1, N)
+        assert np.array_equal(host(out), Ce) and np.array_equal(host(stat), rms_e[:M])
+        out = out.copy_(dev(A)) if a is not out else out
+    y = shifted(Y)
+    for a in (shifted(A), xo):                       # the second: the sum over its first operand
+        xo.copy_(dev(A))
+        lib.rms_norm_residual_fused_32(ptr(a), ptr(y), 8, ptr(w), ptr(xo), ptr(stat), ptr(out), M, N, 1, N)
+        assert np.array_equal(host(xo), X) and np.array_equal(host(out), Xe) and np.array_equal(host(stat), rms_x[:M])
+    K._check("rms_norm")
+
+
 @pytest.mark.parametrize("M,N", [(1, 24576), (16, 22528), (16, 22530), (17, 22530), (17, 24576), (256, 16386), (257, 16386),
                                  (257, 24576), (272, 18432), (273, 18432)])
 def test_rmsnorm_few_of_the_longest_rows(K, oracle, M, N):

@@ -42,26 +42,6 @@ __device__ __forceinline__ int64_t floordiv64(int64_t a, int64_t b)
     return q;
 }
 
-// The values of a lane and of its partner OFF lanes away, as a reduction over 1, 2, 4 ... lanes needs them (lanes that have met
-// already hold the same): through the vector pipe alone, where a shuffle goes through LDS.  Within sixteen lanes by row permutes
-// (neighbours, pairs, mirrored eights, mirrored sixteens), beyond by swapping rows of sixteen and halves of the wavefront.
-template <int OFF>
-__device__ __forceinline__ void lane_pair(int64_t v, int64_t &a, int64_t &b)
-{
-    const unsigned lo = (unsigned)(uint64_t)v, hi = (unsigned)((uint64_t)v >> 32);
-    if constexpr (OFF <= 8) {
-        constexpr int CTRL = OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : OFF == 4 ? 0x141 : 0x140;
-        const unsigned ol = (unsigned)__builtin_amdgcn_update_dpp(0, (int)lo, CTRL, 0xF, 0xF, true);
-        const unsigned oh = (unsigned)__builtin_amdgcn_update_dpp(0, (int)hi, CTRL, 0xF, 0xF, true);
-        a = v;
-        b = (int64_t)((uint64_t)oh << 32 | ol);
-    } else {
-        const auto l = OFF == 16 ? __builtin_amdgcn_permlane16_swap(lo, lo, false, false) : __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
-        const auto h = OFF == 16 ? __builtin_amdgcn_permlane16_swap(hi, hi, false, false) : __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-        a = (int64_t)((uint64_t)h[0] << 32 | l[0]);
-        b = (int64_t)((uint64_t)h[1] << 32 | l[1]);
-    }
-}
 template <int OFF>
 __device__ __forceinline__ int64_t lane_max(int64_t v)
 {

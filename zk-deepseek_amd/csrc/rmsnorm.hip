@@ -59,16 +59,28 @@ struct SquareSum {
     }
 };
 
-__device__ __forceinline__ U192 wave_sum_u192(U192 a)
+template <int OFF>
+__device__ __forceinline__ void lane_add_u192(U192 &a)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        U192 o;
-        o.w0 = (uint64_t)__shfl_xor((long long)a.w0, off, kWave);
-        o.w1 = (uint64_t)__shfl_xor((long long)a.w1, off, kWave);
-        o.w2 = (uint64_t)__shfl_xor((long long)a.w2, off, kWave);
-        u192_add(a, o);
-    }
+    U192 b;
+    int64_t x, y;
+    lane_pair<OFF>((int64_t)a.w0, x, y); a.w0 = (uint64_t)x; b.w0 = (uint64_t)y;
+    lane_pair<OFF>((int64_t)a.w1, x, y); a.w1 = (uint64_t)x; b.w1 = (uint64_t)y;
+    lane_pair<OFF>((int64_t)a.w2, x, y); a.w2 = (uint64_t)x; b.w2 = (uint64_t)y;
+    u192_add(a, b);
+}
+
+// the sum over groups of LANES lanes (a power of two), in every lane.  (Through shuffles, which take turns in LDS, and with the
+// wavefronts' sums added one after the other, before / now, us: 1 row of 7168 6.7 / 5.9, 500 rows of 512 4.9 / 4.4, 16 rows of 2048 5.2 / 4.3.)
+template <int LANES>
+__device__ __forceinline__ U192 lanes_sum_u192(U192 a)
+{
+    if (LANES > 1) lane_add_u192<1>(a);
+    if (LANES > 2) lane_add_u192<2>(a);
+    if (LANES > 4) lane_add_u192<4>(a);
+    if (LANES > 8) lane_add_u192<8>(a);
+    if (LANES > 16) lane_add_u192<16>(a);
+    if (LANES > 32) lane_add_u192<32>(a);
     return a;
 }
 
@@ -265,14 +277,11 @@ constexpr int kRmsThreads = 256;
 template <int THREADS>
 __device__ __forceinline__ U192 block_sum_u192(U192 acc, U192 *red)
 {
-    acc = wave_sum_u192(acc);
+    acc = lanes_sum_u192<64>(acc);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (lane == 0) red[wave] = acc;
     __syncthreads();
-    U192 tot = red[0];
-#pragma unroll
-    for (int w = 1; w < THREADS / 64; w++) u192_add(tot, red[w]);
-    return tot;
+    return lanes_sum_u192<THREADS / 64>(red[lane % (THREADS / 64)]);
 }
 
 typedef int v4i_r __attribute__((ext_vector_type(4)));
@@ -408,16 +417,22 @@ __device__ __forceinline__ void store_pair(int64_t *p, int64_t x, int64_t y, boo
 // spills again and does not.  Rows that are not VEC spill at 80 already and run two (500 rows of 8191 24.1 -> 17.2 us).
 // RES: the row that is normalised is A + Y * 2^k (wrapping int64 arithmetic, as the tensor ops of the reference's
 // residual connection, inference/model.py:1465, 1472), and that sum is also stored to Xout (which may be A itself).
+// PARTS: workgroups per row.  Each takes the statistic of the whole row and stores one pair of every thread: a row that is alone on the
+// device is bound by what one compute unit's vector pipes do, and most of that is the exact division of its elements.  Nothing that
+// is stored may overlap what the other workgroups of the row still read (rows_overlap).
 struct RmsResidual { const int64_t *Y; int64_t *Xout; int k; };
 
-template <typename WT, int THREADS, int EPT, bool VEC, int WPE, bool RES>
+template <typename WT, int THREADS, int EPT, bool VEC, int WPE, bool RES, int PARTS = 1>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void rms_fused_kernel(const int64_t *A, const WT *__restrict__ W,
                                                                 int64_t *__restrict__ rms, int64_t *__restrict__ C,
                                                                 int N, int64_t eps, int64_t dim, RmsResidual res)
 {
     __shared__ U192 red[THREADS / 64];
     __shared__ int64_t rms_s;
-    const long row = blockIdx.x;
+    static_assert(PARTS == 1 || PARTS == EPT / 2, "a part is one pair of every thread");
+    const long row = PARTS > 1 ? blockIdx.x / PARTS : blockIdx.x;
+    const int part = PARTS > 1 ? blockIdx.x % PARTS : 0;
+    const auto mine = [&](int j) { return PARTS == 1 || j == part; };
     const int64_t *a = A + row * N;
     int64_t v[EPT];
     // The weights travel with the row, up to eight elements a thread: no load is left for after the barrier.  Where several rows share a compute unit
@@ -436,7 +451,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) 
         if (i < N) {
             const bool both = VEC || i + 1 < N;
             const v4i_r t = load_pair<VEC>(a + i, both);
-            if (!W_LATE) {
+            if (!W_LATE && mine(j)) {
                 const WPair<WT> w = both ? load_w_pair(W, i, w_vec) : WPair<WT>{ W[i], 0 };
                 if (W_LDS) w_s[j * THREADS + threadIdx.x] = w;
                 else wp[j] = w;
@@ -449,7 +464,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) 
                 const uint64_t y1 = ((uint64_t)(uint32_t)u[3] << 32) | (uint32_t)u[2];
                 v[2 * j] = (int64_t)((uint64_t)v[2 * j] + (y0 << res.k));
                 v[2 * j + 1] = (int64_t)((uint64_t)v[2 * j + 1] + (y1 << res.k));
-                store_pair<VEC>(res.Xout + row * N + i, v[2 * j], v[2 * j + 1], both);
+                if (mine(j)) store_pair<VEC>(res.Xout + row * N + i, v[2 * j], v[2 * j + 1], both);
             }
             sq.add(v[2 * j]);
             sq.add(v[2 * j + 1]);
@@ -459,7 +474,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) 
     if (threadIdx.x == 0) {
         int64_t r = rms_finalize(tot, eps, dim);
         rms_s = r;
-        rms[row] = r;
+        if (part == 0) rms[row] = r;
     }
     __syncthreads();
     const int64_t r = rms_s;
@@ -474,7 +489,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) 
 #pragma unroll
     for (int j = 0; j < EPT / 2; j++) {
         const int i = (j * THREADS + threadIdx.x) * 2;
-        if (i < N) {
+        if (mine(j) && i < N) {
             const bool both = VEC || i + 1 < N;
             bool ok0, ok1;
             const WPair<WT> w = weights(i, j, both);
@@ -540,6 +555,12 @@ __global__ __launch_bounds__(256) void residual_add_kernel(const int64_t *A, con
         Xout[i] = (int64_t)((uint64_t)A[i] + ((uint64_t)Y[i] << k));
 }
 
+static bool rows_overlap(const void *a, const void *b, long bytes)
+{
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return x < y + (uintptr_t)bytes && y < x + (uintptr_t)bytes;
+}
+
 template <typename WT>
 static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_t *rms, int64_t *C, int M, int N,
                          int64_t eps, int64_t dim, const RmsResidual *res = nullptr)
@@ -557,6 +578,13 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
     const bool vec = N % 2 == 0 && (align & 15) == 0;
     const dim3 grid((unsigned)M);
     const int cus = device_cus();
+#define ZK_RMS_SPLIT2(THREADS, EPT, VEC, RES) \
+    rms_fused_kernel<WT, THREADS, EPT, VEC, 1, RES, EPT / 2><<<dim3((unsigned)M * (EPT / 2)), dim3(THREADS), 0, 0>>>(A, W, rms, C, N, eps, dim, r)
+#define ZK_RMS_SPLIT(THREADS, EPT)                                                         \
+    do {                                                                                   \
+        if (res) { if (vec) ZK_RMS_SPLIT2(THREADS, EPT, true, true); else ZK_RMS_SPLIT2(THREADS, EPT, false, true); }    \
+        else { if (vec) ZK_RMS_SPLIT2(THREADS, EPT, true, false); else ZK_RMS_SPLIT2(THREADS, EPT, false, false); }      \
+    } while (0)
 #define ZK_RMS_LAUNCH2(THREADS, EPT, WPE, VEC, RES) \
     rms_fused_kernel<WT, THREADS, EPT, VEC, VEC || WPE < 4 ? WPE : 4, RES><<<grid, dim3(THREADS), 0, 0>>>(A, W, rms, C, N, eps, dim, r)
 #define ZK_RMS_LAUNCH(THREADS, EPT, WPE)                                                   \
@@ -570,7 +598,13 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
     // of two, kernel alone, mean of 1 to 64 rows: up to 1024 elements 4.7 / 4.9 / 5.4 us (with residual 4.6 / 5.0 / 5.4), 1025 to 2048 5.3 / 5.1 / 5.5
     // (5.1 / 5.3 / 5.6), of odd length 5.7 / 5.3 / 5.5.
     const bool apart = vec && !res && ((M <= 16 && N > 22528) || (M > cus && M <= cus + cus / 16));
-    if (N <= 512) ZK_RMS_LAUNCH(256, 2, 1);
+    const long bytes = (long)M * N * 8;
+    const bool split = !rows_overlap(C, A, bytes) && (!res || (!rows_overlap(C, r.Y, bytes) && !rows_overlap(C, r.Xout, bytes) && !rows_overlap(r.Xout, A, bytes) && !rows_overlap(r.Xout, r.Y, bytes)));
+    // Few long rows go to four compute units each.  One workgroup / four, us: 1 row of 7168 5.9 / 5.1, with residual 6.8 / 5.6, of 8191
+    // 6.7 / 5.4 and 7.4 / 5.8; 16 rows of 7168 6.7 / 6.4 and 7.7 / 7.1; 32 rows 6.7 / 6.6 and 7.9 / 7.7; 64 rows 6.9 / 7.0 and 8.0 / 8.1, of 8191
+    // with residual 8.5 / 8.7; rows of 2049, whose pairs do not go round a second time, level or slower.
+    if (split && N > 4096 && N <= 8192 && M <= 32) ZK_RMS_SPLIT(1024, 8);
+    else if (N <= 512) ZK_RMS_LAUNCH(256, 2, 1);
     else if (N <= 2048 && !(M <= 64 && N > 1024)) ZK_RMS_LAUNCH(256, 8, 1);
     else if (N <= 2048) ZK_RMS_LAUNCH(512, 4, 1);
     else if (M <= (N <= 4096 ? 64 : 256) && N <= 8192) ZK_RMS_LAUNCH(1024, 8, 1);
@@ -598,6 +632,8 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
         if (check_launch(name)) launch_apply<WT>(name, src, W, rms, C, M, N);
         return;
     }
+#undef ZK_RMS_SPLIT
+#undef ZK_RMS_SPLIT2
 #undef ZK_RMS_LAUNCH
 #undef ZK_RMS_LAUNCH2
     check_launch(name);
