@@ -42,13 +42,6 @@ __device__ __forceinline__ int64_t floordiv64(int64_t a, int64_t b)
     return q;
 }
 
-template <int OFF>
-__device__ __forceinline__ int64_t lane_max(int64_t v)
-{
-    int64_t a, b;
-    lane_pair<OFF>(v, a, b);
-    return a > b ? a : b;
-}
 // the two largest of both sides: the larger first, then the best of the rest
 template <int OFF>
 __device__ __forceinline__ void lane_best2(int64_t &b1, int64_t &b2)
@@ -360,7 +353,7 @@ __global__ __launch_bounds__(64) void gate_route_few_kernel(const int64_t *__res
             w = better_j ? orig[j] : w;
             slot = better_j ? j : slot;
         }
-        const int64_t best = lane_max<32>(lane_max<16>(lane_max<8>(lane_max<4>(lane_max<2>(lane_max<1>(v))))));
+        const int64_t best = wave_max_i64(v);
         const int owner = __ffsll((unsigned long long)__ballot(slot >= 0 && v == best)) - 1;
         w = from_lane(w, owner);
         wsum = (int64_t)((uint64_t)wsum + (uint64_t)w);

@@ -49,8 +49,8 @@ inline int guard_parts(long seen_count, long grid)
     return (int)(n < 1 ? 1 : (n > most ? most : n));
 }
 
-// by whole workgroups of at most 1024 threads, number `part` of g.parts
-__device__ __forceinline__ void guard_report(const GuardArgs &g, int part)
+// by whole workgroups of at most 1024 threads, number `part` of g.parts; `verdict`: what the verdict word holds
+__device__ __forceinline__ void guard_report(const GuardArgs &g, int part, unsigned verdict)
 {
     __shared__ int report_red[16];
     unsigned a = 0, b = 0;
@@ -71,12 +71,12 @@ __device__ __forceinline__ void guard_report(const GuardArgs &g, int part)
         }
     }
     unsigned ab = a << 16 | b;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const unsigned o = (unsigned)__shfl_xor((int)ab, off, kWave);
-        const unsigned oa = o >> 16, ob = o & 0xFFFFu, ma = ab >> 16, mb = ab & 0xFFFFu;
-        ab = (oa > ma ? oa : ma) << 16 | (ob > mb ? ob : mb);
-    }
+    wave_steps([&](auto off) {
+        unsigned x, y;
+        lane_pair<decltype(off)::value>(ab, x, y);
+        const unsigned xa = x >> 16, xb = x & 0xFFFFu, ya = y >> 16, yb = y & 0xFFFFu;
+        ab = (xa > ya ? xa : ya) << 16 | (xb > yb ? xb : yb);
+    });
     if ((threadIdx.x & 63) == 0) report_red[threadIdx.x >> 6] = (int)ab;
     __syncthreads();
     if (threadIdx.x != 0) return;
@@ -86,8 +86,7 @@ __device__ __forceinline__ void guard_report(const GuardArgs &g, int part)
         a = (o >> 16) > a ? (o >> 16) : a;
         b = (o & 0xFFFFu) > b ? (o & 0xFFFFu) : b;
     }
-    const unsigned v = __atomic_load_n(g.verdict, __ATOMIC_RELAXED);
-    if (g.host) __hip_atomic_store(g.host + part, (unsigned long long)g.seq << 32 | v << 16 | b << 8 | a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (g.host) __hip_atomic_store(g.host + part, (unsigned long long)g.seq << 32 | verdict << 16 | b << 8 | a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (g.next && part == 0) __atomic_store_n(g.next, 0u, __ATOMIC_RELAXED);
 }
 

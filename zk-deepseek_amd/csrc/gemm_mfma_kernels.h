@@ -182,11 +182,11 @@ __device__ __forceinline__ int digits_i32(int lo, int hi)
 
 __device__ __forceinline__ int wave_max_i32(int v)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const int o = __shfl_xor(v, off, kWave);
-        v = o > v ? o : v;
-    }
+    wave_steps([&](auto off) {
+        unsigned a, b;
+        lane_pair<decltype(off)::value>((unsigned)v, a, b);
+        v = (int)a > (int)b ? (int)a : (int)b;
+    });
     return v;
 }
 
@@ -427,7 +427,7 @@ __global__ __launch_bounds__(256) void b_planes_kernel(BPlanesParams p)
 }
 
 // The report of a launch that has no guarded launch behind it (its caller waits for the digits instead).
-static __global__ __launch_bounds__(256) void digits_report_kernel(GuardArgs g) { guard_report(g, 0); }
+static __global__ __launch_bounds__(256) void digits_report_kernel(GuardArgs g) { guard_report(g, 0, __atomic_load_n(g.verdict, __ATOMIC_RELAXED)); }
 
 // One output from its D int32 diagonals: init + sum_d dg(d) * 2^(8d) as the words of a 128-bit sum.  A diagonal keeps its
 // low byte and hands the rest to the next one, so everything is 32-bit: two instructions per diagonal and a byte permute
@@ -1061,7 +1061,7 @@ template <int NA, int NB, int WVM, int WVN, int WM, int WN, int KK, bool B32, bo
 __global__ __launch_bounds__(64 * WVM * WVN) void gemm_mfma_guarded_kernel(MfmaParams p)
 {
     const unsigned verdict = __atomic_load_n(p.guard.verdict, __ATOMIC_RELAXED);            // (the same for every thread of the launch)
-    if ((int)blockIdx.x < p.guard.parts) guard_report(p.guard, (int)blockIdx.x);
+    if ((int)blockIdx.x < p.guard.parts) guard_report(p.guard, (int)blockIdx.x, verdict);
     if (verdict == 0) return;
     if (verdict == 1 && (NA > 5 || NB > 5)) {
         // five digits cover both operands (every workgroup that met a wider element would have raised the verdict to 2): a

@@ -363,7 +363,7 @@ __global__ __launch_bounds__(64 * kR16Waves) void gemm_rows16_kernel(Rows16Param
 {
     if (p.guard.verdict) {
         const unsigned verdict = __atomic_load_n(p.guard.verdict, __ATOMIC_RELAXED);       // (the same for every thread of the launch)
-        if ((int)blockIdx.x < p.guard.parts) guard_report(p.guard, (int)blockIdx.x);
+        if ((int)blockIdx.x < p.guard.parts) guard_report(p.guard, (int)blockIdx.x, verdict);
         if (verdict == 0) return;
     }
     for (unsigned item = blockIdx.x; item < p.items; item += gridDim.x) {

@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256) void gemm_valu_kernel(ValuParams p)
     const int tid = threadIdx.x;
     if (p.guard.verdict) {
         const unsigned verdict = __atomic_load_n(p.guard.verdict, __ATOMIC_RELAXED);
-        if ((int)blockIdx.x < p.guard.parts) guard_report(p.guard, (int)blockIdx.x);
+        if ((int)blockIdx.x < p.guard.parts) guard_report(p.guard, (int)blockIdx.x, verdict);
         if (verdict == 0) return;
     }
     for (long tile = blockIdx.x; tile < p.tiles; tile += gridDim.x) {
@@ -178,6 +178,18 @@ void gemm_valu_launch(const GemmDesc &d, GuardArgs *guard)
     p.guard = guard ? *guard : GuardArgs();
     if (d.b32) { if (kmajor) launch2<true, true>(p, grid, rescale); else launch2<true, false>(p, grid, rescale); }
     else { if (kmajor) launch2<false, true>(p, grid, rescale); else launch2<false, false>(p, grid, rescale); }
+}
+
+// sum over a wavefront, in every lane
+__device__ __forceinline__ u128 wave_sum_u128(u128 v)
+{
+    wave_steps([&](auto off) {
+        uint64_t al, bl, ah, bh;
+        lane_pair<decltype(off)::value>((uint64_t)v, al, bl);
+        lane_pair<decltype(off)::value>((uint64_t)(v >> 64), ah, bh);
+        v = ((u128)ah << 64 | al) + ((u128)bh << 64 | bl);
+    });
+    return v;
 }
 
 // ---- one or two rows of A: a matrix-vector product -----------------------------------------------------------
@@ -317,12 +329,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(ValuParams p)
 #pragma unroll
         for (int m = 0; m < MR; m++) {
             if (SPLIT) acc[c][m] = (shi[c][m].total() << 32) + slo[c][m].total();
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                const uint64_t lo = (uint64_t)__shfl_xor((long long)(uint64_t)acc[c][m], off, 64);
-                const uint64_t hi = (uint64_t)__shfl_xor((long long)(uint64_t)(acc[c][m] >> 64), off, 64);
-                acc[c][m] += ((u128)hi << 64) | lo;
-            }
+            acc[c][m] = wave_sum_u128(acc[c][m]);
         }
     if (WPC > 1) {
         if (lane == 0)
@@ -449,12 +456,7 @@ __global__ __launch_bounds__(64 * kStagedWaves) void gemv32_staged_kernel(ValuPa
 #pragma unroll
         for (int c = 0; c < CPW; c++) {
             u128 sum = (u128)((i128)acc[m][c][0] + ((i128)acc[m][c][1] << 21) + ((i128)acc[m][c][2] << 42));
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                const uint64_t lo = (uint64_t)__shfl_xor((long long)(uint64_t)sum, off, 64);
-                const uint64_t hi = (uint64_t)__shfl_xor((long long)(uint64_t)(sum >> 64), off, 64);
-                sum += ((u128)hi << 64) | lo;
-            }
+            sum = wave_sum_u128(sum);
             if (lane == 0 && n_first + c < p.N) {
                 sum += (u128)(i128)p.init;
                 const long o = (long)g * p.sC + (long)m * p.ldc + n_first + c;

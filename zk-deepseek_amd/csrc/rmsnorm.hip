@@ -62,12 +62,12 @@ struct SquareSum {
 template <int OFF>
 __device__ __forceinline__ void lane_add_u192(U192 &a)
 {
-    U192 b;
-    int64_t x, y;
-    lane_pair<OFF>((int64_t)a.w0, x, y); a.w0 = (uint64_t)x; b.w0 = (uint64_t)y;
-    lane_pair<OFF>((int64_t)a.w1, x, y); a.w1 = (uint64_t)x; b.w1 = (uint64_t)y;
-    lane_pair<OFF>((int64_t)a.w2, x, y); a.w2 = (uint64_t)x; b.w2 = (uint64_t)y;
-    u192_add(a, b);
+    U192 x, y;
+    lane_pair<OFF>(a.w0, x.w0, y.w0);
+    lane_pair<OFF>(a.w1, x.w1, y.w1);
+    lane_pair<OFF>(a.w2, x.w2, y.w2);
+    u192_add(x, y);
+    a = x;
 }
 
 // the sum over groups of LANES lanes (a power of two), in every lane.  (Through shuffles, which take turns in LDS, and with the
