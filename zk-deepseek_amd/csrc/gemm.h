@@ -43,8 +43,11 @@ struct GuardArgs {
 // One workgroup for every 1024 words of `seen` (a load or four per thread), at most 32: a product of 131072 rows leaves
 // 50000 words, for which one workgroup took 44 us.
 constexpr int kGuardParts = 32;
+// kReported in place of the count: a launch in between has left the report.
+constexpr long kReported = -1;
 inline int guard_parts(long seen_count, long grid)
 {
+    if (seen_count == kReported) return 0;
     const long n = (seen_count + 1023) / 1024, most = grid < kGuardParts ? grid : kGuardParts;
     return (int)(n < 1 ? 1 : (n > most ? most : n));
 }

@@ -1002,17 +1002,27 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
                 return kFailed;
             }
         }
+        // no waiting: a guarded launch redoes the product if the verdict is raised, the digits seen follow later
+        GuardArgs guard = {};
+        if (speculate) {
+            guard = make_guard((p.seen ? blocks : 0) + plane_wgs + b_plane_wgs);
+            if (!p.seen) guard.seen += blocks;
+        }
         if (p.split > 1) {
-            (pipe.fn ? pipe.finish : inst->finish)<<<dim3((unsigned)((total - p.main_tiles) * p.finish_rq)), dim3((unsigned)inst->threads), 0, 0>>>(p);
+            if (speculate) {
+                guard.parts = guard_parts(guard.seen_count, kGuardParts);
+                p.guard = guard;
+            }
+            (pipe.fn ? pipe.finish : inst->finish)<<<dim3((unsigned)((total - p.main_tiles) * p.finish_rq + p.guard.parts)), dim3((unsigned)inst->threads), 0, 0>>>(p);
             if (hipGetLastError() != hipSuccess) { set_error(kLaunchFailure, "gemm: split finish launch failed"); return kFailed; }
         }
         *limbs_a = inst->na;
         *limbs_b = inst->nb;
         if (speculate) {
-            // no waiting: a guarded launch redoes the product if the verdict is raised, the digits seen follow later
-            GuardArgs guard = make_guard((p.seen ? blocks : 0) + plane_wgs + b_plane_wgs);
-            if (!p.seen) guard.seen += blocks;
-            if (const Outcome got = launch_guarded_fallback(d, p, b_shift, &guard)) return got;
+            GuardArgs behind = guard;
+            if (p.split > 1) behind.seen_count = kReported;
+            if (const Outcome got = launch_guarded_fallback(d, p, b_shift, &behind)) return got;
+            if (p.split <= 1) guard.parts = behind.parts;
             guard_taken(guard, key_a, key_b, prep ? prep->nb : 0);       // (the slots are shared with the grouped launches, which set it too)
             return kDone;
         }
