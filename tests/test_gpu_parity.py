@@ -1000,10 +1000,10 @@ def test_row_tiles_where_their_stores_are_the_slower_ones(K, oracle, rows, N, Kd
 
 
 @pytest.mark.parametrize("heads,cols,k", [(5, 1, 1), (16, 16, 63), (17, 15, 64), (33, 70, 65), (128, 779, 512), (128, 512, 779), (128, 512, 1024),
-                                          (256, 256, 2048), (31, 1200, 2047)])
+                                          (256, 256, 2048), (31, 1200, 2047), (128, 600, 255), (128, 600, 257), (120, 544, 1023)])
 def test_attention_of_few_positions_in_one_launch(K, oracle, heads, cols, k):
     """scores and values of at most two rounds of 16 x 16 tiles: edges of tiles, of steps of 64 k and of the eight wavefronts
-    that share K, rows off the 16-byte grid, batches, every digit count from 3 to 9 with single elements that need more than
+    that share K (four where the tiles are more than the compute units), rows off the 16-byte grid, batches, every digit count from 3 to 9 with single elements that need more than
     the rest, the largest magnitudes"""
     rng = np.random.default_rng(heads * 4096 + cols + k)
     for bits_a, bits_b in ((19, 21), (27, 28), (36, 35), (36, 60), (62, 22), (63, 63)):
@@ -1241,6 +1241,20 @@ def test_activation_unaligned_pointers(K, oracle):
     C = torch.empty_like(dev(x))
     K.silu_q23(R, C)
     assert np.array_equal(host(C), oracle.silu_q23(x))
+
+
+@pytest.mark.parametrize("n,off", [(509, 0), (512, 0), (515, 0), (1 << 20, 1), ((1 << 20) + 1, 1), ((1 << 20) - 1, 0)])
+def test_activation_vectors_per_thread(K, oracle, n, off):
+    """one vector (or element) a thread up to 2^20 of them, four beyond (tensors off the 16-byte grid); odd ends"""
+    rng = np.random.default_rng(n + off)
+    x, u = rng.integers(-(20 << 23), 20 << 23, size=(1, 1, n), dtype=np.int64), rng.integers(-(1 << 40), 1 << 40, size=(1, 1, n), dtype=np.int64)
+    place = lambda a: torch.empty(n + 2, dtype=torch.int64, device="cuda")[off:off + n].view(1, 1, n).copy_(dev(a))
+    R, U, C = place(x), place(u), place(x)
+    K.silu_q23(R, C)
+    se, ce = oracle.silu_mul_q23(x, u)
+    assert np.array_equal(host(C), se)
+    K.silu_mul_q23(R, U, C)
+    assert np.array_equal(host(C), ce)
 
 
 def test_activation_dense_ffn_shape(K, oracle):
