@@ -3,10 +3,10 @@
 //
 // On the general kernel such a product is three dependent launches (tiles cut along K, the sum of the slices, the guarded
 // launch behind a guess of digit counts) of 4 to 11 us each.  Here a workgroup owns a tile of 16 x 16 outputs and all of K: its
-// eight wavefronts take every eighth step of 64 k, load their fragments straight into registers (the four lanes of a
+// eight (or four) wavefronts take every eighth (fourth) step of 64 k, load their fragments straight into registers (the four lanes of a
 // row read 64 contiguous bytes per load), take the digit counts that those need (3, 4 or 5 per operand, gemm_frag16.h),
 // split, multiply, and meet in LDS with their 128-bit sums.  A wavefront that meets values beyond five digits (2^38 and up)
-// multiplies its share again with nine digits.  Where a wavefront has one step at most (K up to 512) that step's elements are still in
+// multiplies its share again with nine digits.  Where a wavefront has one step at most (K up to 512, or 256) that step's elements are still in
 // its registers: a cache of 44 bits, share read again / this, us a call, 128 rows x [512,7] n-contiguous 8.9 / 6.3, x [512,300]
 // 9.4 / 6.5, x [779,512] k-contiguous 20.9 / 13.2 (the first had become slower than on the general kernel).
 #include "gemm_frag16.h"
@@ -23,11 +23,11 @@ struct SmallParams {
     int64_t init;
 };
 
-constexpr int kSmallWaves = 8, kSmallTile = 16, kSmallDiagonals = 9, kSmallWideDiagonals = 16;   // of five digits a side, of nine (what lies at 2^128 and above does not matter)
+constexpr int kSmallTile = 16, kSmallDiagonals = 9, kSmallWideDiagonals = 16;   // of five digits a side, of nine (what lies at 2^128 and above does not matter)
 // Where it pays, against the general and the 16-row kernels over 250 shapes of 5 to 600 rows and 16 to 2048 columns (those / this, us):
 // one round of tiles 0.3-0.8 of their time up to K = 2048 (128 rows x [512,779] n-contiguous 20.0 / 8.9, 50 x [94,321] (5,5)
 // 24.9 / 7.1, 32 x [1513,759] 23.2 / 8.7, 274 x [161,2145] 22.6 / 16.2) and level at 4000; two rounds up to K = 1024 (128 x
-// [779,512] 18.8 / 11.7, 128 x [1024,512] 19.4 / 12.1; 66 x [1398,1454] 26.5 / 30.4); three rounds no longer (256 x [779,512]
+// [779,512] 18.8 / 10.4, 128 x [1024,512] 19.4 / 10.9; 66 x [1398,1454] 26.5 / 30.4); three rounds no longer (256 x [779,512]
 // 19.4 / 21.1).  Offered to it are scores and values of up to eight positions (kFewPositions).
 constexpr int kSmallMaxK = 2048, kSmallMaxKTwoRounds = 1024;
 
@@ -76,10 +76,10 @@ __device__ __forceinline__ void load_elements(RawFrag<false> &f, const int64_t *
 }
 
 // BKM: B is contiguous along n.  ONE: no wavefront has more than one step
-template <bool BKM, bool ONE>
-__global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(SmallParams p)
+template <bool BKM, bool ONE, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2))) void gemm_small_kernel(SmallParams p)
 {
-    __shared__ Words red[kSmallWaves][4][64];
+    __shared__ Words red[WAVES][4][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, q = lane >> 4;
     const int per_batch = p.tiles_m * p.tiles_n;
     const int g = blockIdx.x / per_batch, rem = blockIdx.x - g * per_batch;
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(SmallParam
         v4i acc[kSmallDiagonals];
 #pragma unroll
         for (int d = 0; d < kSmallDiagonals; d++) acc[d] = v4i{ 0, 0, 0, 0 };
-        for (int ks = wave; ks < steps; ks += kSmallWaves) {
+        for (int ks = wave; ks < steps; ks += WAVES) {
             RawFrag<false> fa;
             RawFrag<false> fb;
             load(ks, fa, fb);
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(SmallParam
             small_narrow_step(na, nb, fa, fb, acc);
         }
         // (5 pairs x 64 products of 2^14 a step)
-        static_assert((kSmallMaxK / 64 + kSmallWaves - 1) / kSmallWaves * 5L * 64 * 16384 <= kMaxDiagonal, "the int32 accumulators hold a wavefront's share");
+        static_assert((kSmallMaxK / 64 + WAVES - 1) / WAVES * 5L * 64 * 16384 <= kMaxDiagonal, "the int32 accumulators hold a wavefront's share");
 #pragma unroll
         for (int o = 0; o < 4; o++) red[wave][o][lane] = sum_diagonals<kSmallDiagonals>([&](int d) { return acc[d][o]; }, 0);
     }
@@ -170,13 +170,13 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(SmallParam
         v4i acc[D];
 #pragma unroll
         for (int d = 0; d < D; d++) acc[d] = v4i{ 0, 0, 0, 0 };
-        for (int ks = wave; ks < steps; ks += kSmallWaves) {
+        for (int ks = wave; ks < steps; ks += WAVES) {
             RawFrag<false> fa_raw;
             RawFrag<false> fb_raw;
             load(ks, fa_raw, fb_raw);
             small_step<9, 9>(fa_raw, fb_raw, acc);
         }
-        static_assert((kSmallMaxK / 64 + kSmallWaves - 1) / kSmallWaves * 9L * 64 * 16384 <= kMaxDiagonal, "and of nine digits");
+        static_assert((kSmallMaxK / 64 + WAVES - 1) / WAVES * 9L * 64 * 16384 <= kMaxDiagonal, "and of nine digits");
 #pragma unroll
         for (int o = 0; o < 4; o++) red[wave][o][lane] = sum_diagonals<D>([&](int d) { return acc[d][o]; }, 0);
     }
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void gemm_small_kernel(SmallParam
     if (wave >= 4 || m >= p.M || n >= p.N) return;
     u128 s = (u128)(i128)p.init;
 #pragma unroll
-    for (int w = 0; w < kSmallWaves; w++) {
+    for (int w = 0; w < WAVES; w++) {
         const Words t = red[w][wave][lane];
         s += (u128)((uint64_t)t.w[3] << 32 | t.w[2]) << 64 | ((uint64_t)t.w[1] << 32 | t.w[0]);
     }
@@ -206,13 +206,16 @@ bool gemm_small_launch(const GemmDesc &d)
     p.lda = d.lda; p.sA = d.sA; p.ldbn = d.ldbn; p.ldbk = d.ldbk; p.sB = d.sB; p.ldc = d.ldc; p.sC = d.sC;
     p.M = d.M; p.N = d.N; p.K = d.K; p.shift = d.shift; p.init = d.init;
     p.tiles_m = (int)tiles_m; p.tiles_n = (int)tiles_n;
-    const dim3 grid((unsigned)tiles), block(64 * kSmallWaves);
-    const bool one = d.K <= 64 * kSmallWaves;
-    if (d.ldbk != 1) {
-        if (one) gemm_small_kernel<true, true><<<grid, block, 0, 0>>>(p);
-        else gemm_small_kernel<true, false><<<grid, block, 0, 0>>>(p);
-    } else if (one) gemm_small_kernel<false, true><<<grid, block, 0, 0>>>(p);
-    else gemm_small_kernel<false, false><<<grid, block, 0, 0>>>(p);
+    const dim3 grid((unsigned)tiles);
+    // More tiles than compute units: four wavefronts each, two workgroups to a unit (their registers leave room for no more than two of
+    // four), so that all tiles run at once and one loads while the other multiplies.  Eight / four wavefronts, us: 128 rows x [779,512] 11.7 / 10.4, x
+    // [779,64] 6.5 / 6.1, x [1024,576] 15.9 / 13.3, n-contiguous x [1024,779] 18.0 / 14.9, 256 rows x [512,779] 15.2 / 11.9.
+    const int waves = tiles > device_cus() ? 4 : 8;
+    const bool one = d.K <= 64 * waves;
+#define ZK_SMALL(BKM) do { if (waves == 4) { if (one) gemm_small_kernel<BKM, true, 4><<<grid, dim3(256), 0, 0>>>(p); else gemm_small_kernel<BKM, false, 4><<<grid, dim3(256), 0, 0>>>(p); } \
+                           else if (one) gemm_small_kernel<BKM, true, 8><<<grid, dim3(512), 0, 0>>>(p); else gemm_small_kernel<BKM, false, 8><<<grid, dim3(512), 0, 0>>>(p); } while (0)
+    if (d.ldbk != 1) ZK_SMALL(true); else ZK_SMALL(false);
+#undef ZK_SMALL
     g_small_calls++;
     return true;
 }
