@@ -753,6 +753,25 @@ def test_einsums_seeded_random_problems(K, oracle, seed):
 
 
 # ---------------------------------------------------------------------------------- einsums -----
+@pytest.mark.parametrize("bits_a,bits_b,digits", [(20, 28, (3, 4)), (28, 20, (4, 3)), (28, 28, (4, 4))])
+def test_einsums_of_a_short_k_on_small_tiles(K, oracle, bits_a, bits_b, digits):
+    """64x64 tiles, two workgroups to a compute unit: K around one, two and eight steps of 64, rows and columns around the tiles' edges, one B
+    per head in either layout and a shared one against many rows"""
+    rng = np.random.default_rng(bits_a * 64 + bits_b)
+
+    def both(fn, A, B, c):
+        for _ in range(2):      # (a first call may run on digits remembered for other operands at these addresses)
+            got = host(getattr(K, fn)(dev(A), dev(B), c))
+            assert np.array_equal(got, getattr(oracle, fn)(A, B, c)), (fn, A.shape, B.shape)
+        assert K.gemm_last_plan()[1:] == digits, (fn, A.shape, B.shape)
+    for H, M, D, C in ((64, 66, 63, 260), (64, 129, 64, 257), (128, 65, 65, 300), (128, 193, 128, 130)):
+        both("einsum_bshd_hdc_bshc", rand_i64(rng, (1, M, H, D), bits_a), rand_i32(rng, (H, D, C), bits_b), 30)
+    for H, M, D, C in ((64, 66, 260, 64), (128, 129, 65, 129), (128, 192, 65, 250), (48, 193, 129, 511), (128, 130, 66, 512)):
+        both("einsum_bshc_hdc_bshd", rand_i64(rng, (1, M, H, C), bits_a), rand_i32(rng, (H, D, C), bits_b), 30)
+    for M, T, D in ((129, 193, 64), (128, 256, 63), (131, 200, 1)):
+        both("einsum_bshc_btc_bsht", rand_i64(rng, (1, M, 128, D), bits_a), rand_i64(rng, (1, T, D), bits_b), 21)
+
+
 @pytest.mark.parametrize("path", PATHS)
 @pytest.mark.parametrize("bits", [20, 40, 63])
 def test_einsums(K, oracle, path, bits):

@@ -53,6 +53,7 @@ static const Instance *instances(int *count)
         mfma_instances_narrow(t);
         mfma_instances_mid(t);
         mfma_instances_wide(t);
+        mfma_instances_short(t);
         mfma_instances_both(t);
         mfma_instances_pruned(t);
         mfma_instances_rows32(t);
@@ -76,7 +77,7 @@ static const Instance *pick_instance(int na, int nb, bool b32, bool skinny, int 
     const Instance *best = nullptr;
     long best_cost = 0;
     for (int i = 0; i < count; i++) {
-        if (t[i].na < na || t[i].nb < nb || t[i].skinny != skinny || t[i].alt) continue;
+        if (t[i].na < na || t[i].nb < nb || t[i].skinny != skinny || t[i].alt || t[i].short_k) continue;
         if (t[i].dmax < 16 && t[i].dmax < need_diag) continue;
         if (exact_nb && (t[i].nb != exact_nb || t[i].kk != exact_kk)) continue;
         if (variant >= 0 && !t[i].fn[variant]) continue;
@@ -595,6 +596,30 @@ static int rowtile_parts(const GemmDesc &d, int na, int nb, int bn, int cus)
     return parts;
 }
 
+// The 64x64 form of an instance with 128x64 tiles, for a K of a few steps.  A tile is then bound by its first loads and its epilogue, and
+// a workgroup of eight wavefronts has its compute unit to itself, so nothing runs beside them; of these workgroups of four two run to a unit, one
+// loading while the other combines and stores, and fewer rows are padding.  What it costs is B split twice as often.
+// 128x64 tiles / this, us, all with A split in the kernel but the last.  One B per head, int32 n-contiguous, 128 heads [128,512]: 129 rows
+// (3,4) 54.6 / 45.5, 192 rows (4,4) 64.0 / 52.6, 243 rows 65.4 / 61.5, 300 rows 84.6 / 74.1, 384 rows 113 / 108; 64 heads [64,300], 65 rows 16.0 /
+// 14.2; not where they fill two rounds at most (64 heads [128,512], 65 rows 20.7 / 21.2, 16 heads, 192 rows 13.4 / 14.4).  k-contiguous, 128
+// heads, K = 512, 128 columns: 192 rows 44.6 / 38.7, 243 rows 49.5 / 46.7, 500 rows 124 / 110; not in one round (64 heads 25.1 / 26.1), nor up
+// to 128 rows (70 rows 25.9 / 26.8).  A shared B of many columns: not at K = 512 (20480 rows x [160,512] 43.2 / 44.8), but tall at K = 64, where the
+// pass that splits A in front goes as well: 25600 rows x [200,64] 31.1 / 25.9, 31104 x [243,64] 35.4 / 27.8.  With (3,3) digits, 128x128
+// tiles, it is slower throughout (243 rows of 128 heads [128,512] 52.7 / 59.4).
+static const Instance *short_k_tiles(const Instance *inst, const GemmDesc &d, int cus)
+{
+    const long tiles_n = (d.N + 63) / 64, tiles = (long)((d.M + 127) / 128) * tiles_n * d.G;
+    if (inst->bm != 128 || inst->bn != 64 || inst->dmax != 16) return inst;
+    const bool heads = d.G > 1 && d.sB != 0 && (d.K <= 64 ? tiles >= cus : d.K <= 128 ? tiles > 2L * cus : d.K <= 512 && d.M > 128 && 2 * tiles >= 3L * cus);
+    const bool tall = d.K <= 64 && d.M >= kPipeMinRows && tiles_n >= 4;
+    if (!heads && !tall) return inst;
+    int count;
+    const Instance *t = instances(&count);
+    for (int i = 0; i < count; i++)
+        if (t[i].short_k && t[i].na == inst->na && t[i].nb == inst->nb) return t + i;
+    return inst;
+}
+
 // B[g][k][n] (n contiguous) -> out[g][n][k]: 32x32 tiles through LDS, both sides coalesced
 __global__ __launch_bounds__(256) void b_rows_kernel(const int64_t *__restrict__ B, long ldbk, long sB, int64_t *__restrict__ out, int N, int K)
 {
@@ -788,6 +813,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
                 if (p.col_parts) { rowtile = rowtile_form(inst->na, inst->nb); pipe = PipeForm{}; }
             }
         }
+        if (!prep && !pre_b && b_shift == 0) inst = short_k_tiles(inst, d, g_cache.cus);
         bool b_copied = false;
         if (kmajor && !pre_b && b_copy_pays(d, inst->nb, b_batches)) {
             // (without memory for the copy the n-contiguous kernels run as they are)
@@ -836,7 +862,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         const bool in_step = small_split > 1 && (small_split % 8 == 0 || 8 % small_split == 0);
         const bool few_columns = p.tiles_n <= 4 && (inst->na > 3 || in_step);
         const bool long_slices = !few_columns && (long)steps * 32 * inst->kk >= 800L * (small_split > 1 ? small_split : 1);
-        const bool use_planes = !rowtile.fn && (pre_b || (planes_fit && !by_columns && !inst->skinny && (prep || (p.tiles_n >= g_switches.planes_min_tiles_n && (total >= g_cache.cus || long_slices)))));
+        const bool use_planes = !rowtile.fn && !inst->short_k && (pre_b || (planes_fit && !by_columns && !inst->skinny && (prep || (p.tiles_n >= g_switches.planes_min_tiles_n && (total >= g_cache.cus || long_slices)))));
         if (b_shift && (by_columns || !inst->skinny)) return kDeclined;
         const int variant = pre_b ? kB64PlanesBoth : prep ? (inst->skinny ? kB64FlyBPlanes : kB64PlanesBoth)
                           : b_shift ? (d.b32 ? kB32FlyRs : kB64FlyRs)

@@ -1053,6 +1053,13 @@ __global__ __launch_bounds__(64 * WVM * WVN) void gemm_mfma_kernel(MfmaParams p)
     gemm_mfma_block<NA, NB, WVM, WVN, WM, WN, KK, B32, BKM, APL, GRP, BRS, DMAX, BPL>(p, (int)blockIdx.x);
 }
 
+// The same product on 64x64 tiles of four wavefronts, two workgroups to a compute unit (see short_k_tiles in gemm_mfma.hip).
+template <int NA, int NB, int KK, bool B32, bool BKM>
+__global__ __launch_bounds__(256, 2) void gemm_mfma_short_kernel(MfmaParams p)
+{
+    gemm_mfma_block<NA, NB, 2, 2, 1, 1, KK, B32, BKM, false>(p, (int)blockIdx.x);
+}
+
 // The same product behind a guard word: nothing happens unless *p.guard is non-zero (the verdict of the speculative launch
 // in front of it: its digit counts did not cover the operands), and then the grid, one workgroup per compute unit, walks
 // the workgroup ids of an ordinary launch.  A guarded launch almost always finds nothing to do, and thousands of
@@ -1180,6 +1187,7 @@ struct Instance {
     bool skinny;                 // 32-row tiles for M <= 32
     int dmax;                    // diagonals from this one up are left out (16: none but the 2^128 one)
     bool alt;                    // 128x64 tiles for digit counts that also have 128x128 ones: taken by launch size (see smaller_tiles)
+    bool short_k;                // 64x64 tiles for digit counts that also have larger ones: taken by K (see short_k_tiles)
     MfmaKernel fn[kVariants];
     PlanesKernel planes[2];      // [b32]: the owned-k pattern follows the element size of B
     FinishKernel finish;         // adds up the partial sums of split tail tiles
@@ -1217,6 +1225,7 @@ static Instance make_instance()
     s.skinny = SKINNY;
     s.dmax = DMAX;
     s.alt = TILE == kTile128x64;
+    s.short_k = false;
     for (int v = 0; v < kVariants; v++) s.fn[v] = nullptr;
     s.guarded[0][0] = s.guarded[0][1] = s.guarded[1][0] = s.guarded[1][1] = nullptr;
     // every operand fits nine digits, every int32 five: these instances can stand behind any speculative launch
@@ -1275,7 +1284,25 @@ static Instance make_instance()
     return s;
 }
 
+// 64x64 tiles, A always split on the fly
+template <int NA, int NB, int KK>
+static Instance make_short_instance()
+{
+    static_assert(NA + NB <= 8, "two workgroups' LDS and registers fit a compute unit up to seven diagonals");
+    Instance s = {};
+    s.na = NA; s.nb = NB; s.bm = 64; s.bn = 64; s.threads = 256; s.kk = KK;
+    s.dmax = 16;
+    s.short_k = true;
+    s.fn[kB64Fly] = gemm_mfma_short_kernel<NA, NB, KK, false, false>;
+    s.fn[kB64KmajorFly] = gemm_mfma_short_kernel<NA, NB, KK, false, true>;
+    s.fn[kB32Fly] = gemm_mfma_short_kernel<NA, NB, KK, true, false>;
+    s.fn[kB32KmajorFly] = gemm_mfma_short_kernel<NA, NB, KK, true, true>;
+    s.finish = gemm_split_finish_kernel<2, 2, 1, 1>;
+    return s;
+}
+
 // the instance lists of the translation units
+void mfma_instances_short(std::vector<Instance> &out);
 void mfma_instances_narrow(std::vector<Instance> &out);
 void mfma_instances_mid(std::vector<Instance> &out);
 void mfma_instances_wide(std::vector<Instance> &out);
