@@ -187,9 +187,18 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const int64_t *__restr
     const long t = blockIdx.y;
     for (int n = blockIdx.x * 256 + threadIdx.x; n < N; n += gridDim.x * 256) {
         uint64_t acc = 0;
-        for (int k = 0; k < K; k++) {
-            const int64_t v = ye[(long)pos[t * K + k] * N + n];
-            acc += (uint64_t)((int64_t)((uint64_t)v * (uint64_t)w[t * K + k]) >> shift);
+        // (eight slots' loads under way together: one after the other, each waits for its position and then for its row, and one token's
+        // sum lives on that.  256 tokens of 8 slots, 7168 elements, 21.0 -> 20.0 us a call, 300 tokens 24.6 -> 22.7, one to 32 tokens 7.1 -> 6.5)
+        for (int k0 = 0; k0 < K; k0 += 8) {
+            int64_t v[8], wk[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int k = k0 + j < K ? k0 + j : K - 1;
+                v[j] = ye[(long)pos[t * K + k] * N + n];
+                wk[j] = k0 + j < K ? w[t * K + k] : 0;
+            }
+#pragma unroll
+            for (int j = 0; j < 8; j++) acc += (uint64_t)((int64_t)((uint64_t)v[j] * (uint64_t)wk[j]) >> shift);
         }
         y[t * N + n] = (int64_t)acc;
     }
