@@ -1838,6 +1838,21 @@ def test_moe_dispatch_reports_indices_outside_the_experts(K, oracle, monkeypatch
     assert np.array_equal(host(y), ye)
 
 
+@pytest.mark.parametrize("Kr", [1, 7, 8, 9, 16, 17])
+def test_moe_combine_slots_in_eights(K, Kr):
+    """the weighted sum over slots taken eight at a time, products that wrap, floor shift, columns past whole workgroups"""
+    rng = np.random.default_rng(Kr)
+    T, N, E = 3, 515, 40
+    idx = np.stack([rng.permutation(E)[:Kr] for _ in range(T)]).astype(np.int64)
+    d = K.moe_dispatch(dev(idx), E)
+    ye, w = rand_i64(rng, (T * Kr, N), 62), rand_i64(rng, (T, Kr), 40)
+    pos = host(d["pos"]).reshape(T, Kr)
+    want = np.zeros((T, N), dtype=np.int64)
+    for k in range(Kr):
+        want += (ye[pos[:, k]] * w[:, k:k + 1]) >> 23
+    assert np.array_equal(host(K.moe_combine(dev(ye), dev(w), d, T)), want)
+
+
 @pytest.mark.parametrize("path", PATHS)
 @pytest.mark.parametrize("w32", [False, True])
 @pytest.mark.parametrize("bits", [(20, 16), (37, 30), (50, 31)])
