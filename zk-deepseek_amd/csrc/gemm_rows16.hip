@@ -373,7 +373,7 @@ __global__ __launch_bounds__(64 * kR16Waves) void gemm_rows16_kernel(Rows16Param
 }
 
 // Adds the slots of every output tile, applies rounding term and shift, stores C and R.  Four threads share an output
-// (each adds every fourth slice with all its loads under way at once, then the four meet through shuffles): the launch
+// (each adds every fourth slice with all its loads under way at once, then the four meet by row permutes): the launch
 // is a chain of one load latency, not of one per slice.
 template <bool B32>
 __global__ __launch_bounds__(256) void gemm_rows16_finish_kernel(Rows16Params p)
@@ -400,13 +400,15 @@ __global__ __launch_bounds__(256) void gemm_rows16_finish_kernel(Rows16Params p)
         for (int j = 0; j < 8; j++) s += t[j];
     }
     uint64_t lo = (uint64_t)s, hi = (uint64_t)(s >> 64);
-#pragma unroll
-    for (int off = 1; off < 4; off <<= 1) {
-        const uint64_t olo = (uint64_t)__shfl_xor((long long)lo, off, 64), ohi = (uint64_t)__shfl_xor((long long)hi, off, 64);
-        const uint64_t tlo = lo + olo;
-        hi += ohi + (tlo < lo ? 1 : 0);
-        lo = tlo;
-    }
+    auto add_pair = [&](auto off) {
+        uint64_t alo, blo, ahi, bhi;
+        lane_pair<decltype(off)::value>(lo, alo, blo);
+        lane_pair<decltype(off)::value>(hi, ahi, bhi);
+        lo = alo + blo;
+        hi = ahi + bhi + (lo < alo ? 1 : 0);
+    };
+    add_pair(std::integral_constant<int, 1>());
+    add_pair(std::integral_constant<int, 2>());
     if (part != 0 || m >= p.M || n >= p.N) return;
     const uint64_t ilo = (uint64_t)p.init, ihi = (uint64_t)(p.init >> 63);
     const uint64_t flo = lo + ilo;
