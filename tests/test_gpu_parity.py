@@ -1019,12 +1019,21 @@ def test_row_tiles_where_their_stores_are_the_slower_ones(K, oracle, rows, N, Kd
 
 
 @pytest.mark.parametrize("heads,cols,k", [(5, 1, 1), (16, 16, 63), (17, 15, 64), (33, 70, 65), (128, 779, 512), (128, 512, 779), (128, 512, 1024),
-                                          (256, 256, 2048), (31, 1200, 2047), (128, 600, 255), (128, 600, 257), (120, 544, 1023)])
+                                          (256, 256, 2048), (31, 1200, 2047), (128, 600, 255), (128, 600, 257), (120, 544, 1023),
+                                          (64, 500, 511), (64, 500, 512), (64, 500, 513), (60, 250, 300)])
 def test_attention_of_few_positions_in_one_launch(K, oracle, heads, cols, k):
     """scores and values of at most two rounds of 16 x 16 tiles: edges of tiles, of steps of 64 k and of the eight wavefronts
     that share K (four where the tiles are more than the compute units), rows off the 16-byte grid, batches, every digit count from 3 to 9 with single elements that need more than
-    the rest, the largest magnitudes"""
+    the rest, in a wavefront's first step, in a later one or in the last, the largest magnitudes"""
     rng = np.random.default_rng(heads * 4096 + cols + k)
+    for at in sorted({0, min(k - 1, 256), k // 2, k - 1}):
+        a, b = rand_i64(rng, (1, 1, heads, k), 27), rand_i64(rng, (1, cols, k), 21)
+        a[0, 0, heads // 2, at], b[0, cols // 3, at] = -(1 << 44), (1 << 41) + 3
+        for wide_a, wide_b in ((True, True), (True, False), (False, True)):
+            x, y = a if wide_a else np.clip(a, -(1 << 27), 1 << 27), b if wide_b else np.clip(b, -(1 << 21), 1 << 21)
+            assert np.array_equal(host(K.einsum_bshc_btc_bsht(dev(x), dev(y), 23)), oracle.einsum_bshc_btc_bsht(x, y, 23)), (at, wide_a, wide_b)
+            v = np.ascontiguousarray(y.transpose(0, 2, 1))
+            assert np.array_equal(host(K.einsum_bsht_btc_bshc(dev(x), dev(v), 23)), oracle.einsum_bsht_btc_bshc(x, v, 23)), (at, wide_a, wide_b)
     for bits_a, bits_b in ((19, 21), (27, 28), (36, 35), (36, 60), (62, 22), (63, 63)):
         B, S = (2, 3) if heads * cols < 3000 else (1, 1)
         a, b = rand_i64(rng, (B, S, heads, k), bits_a), rand_i64(rng, (B, cols, k), bits_b)

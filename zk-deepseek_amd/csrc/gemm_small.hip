@@ -5,10 +5,12 @@
 // launch behind a guess of digit counts) of 4 to 11 us each.  Here a workgroup owns a tile of 16 x 16 outputs and all of K: its
 // eight (or four) wavefronts take every eighth (fourth) step of 64 k, load their fragments straight into registers (the four lanes of a
 // row read 64 contiguous bytes per load), take the digit counts that those need (3, 4 or 5 per operand, gemm_frag16.h),
-// split, multiply, and meet in LDS with their 128-bit sums.  A wavefront that meets values beyond five digits (2^38 and up)
-// multiplies its share again with nine digits.  Where a wavefront has one step at most (K up to 512, or 256) that step's elements are still in
-// its registers: a cache of 44 bits, share read again / this, us a call, 128 rows x [512,7] n-contiguous 8.9 / 6.3, x [512,300]
-// 9.4 / 6.5, x [779,512] k-contiguous 20.9 / 13.2 (the first had become slower than on the general kernel).
+// split, multiply, and meet in LDS with their 128-bit sums.  A wavefront that meets values beyond five digits (2^38 and up) goes on with
+// nine digits for the side that needs them, from the step it holds.  Its share read again with nine digits on both sides / so, a cache of 44 bits, us
+// a call: 128 rows x [779,512] k-contiguous 14.8 / 11.4 (13.2 with eight wavefronts of one step each), x [779,576] 16.5 / 13.2, x
+// [300,576] 12.1 / 8.8, n-contiguous x [576,512] 12.9 / 9.8, x [576,779] 16.3 / 14.2.  Narrow values are level (n-contiguous 0.05-0.2 us more).
+// Where no wavefront has more than one step (K up to 512, or 256) there is no loop around it: narrow and 44 bits, loop / this, 128 rows x
+// [512,257] n-contiguous 5.8 / 4.9 and 6.8 / 5.9, x [300,512] k-contiguous 7.2 / 6.9 and 8.2 / 7.6.
 #include "gemm_frag16.h"
 
 #include <atomic>
@@ -58,6 +60,16 @@ __device__ __forceinline__ void small_narrow_step(int na, int nb, const RawFrag<
     case 7: small_step<5, 4>(fa, fb, acc); break;
     default: small_step<5, 5>(fa, fb, acc); break;
     }
+}
+
+__device__ __forceinline__ u128 words_value(const Words &t) { return (u128)((uint64_t)t.w[3] << 32 | t.w[2]) << 64 | ((uint64_t)t.w[1] << 32 | t.w[0]); }
+
+// any width
+__device__ __forceinline__ void small_wide_step(int na, int nb, const RawFrag<false> &fa, const RawFrag<false> &fb, v4i (&acc)[kSmallWideDiagonals])
+{
+    if (na <= 5) small_step<5, 9>(fa, fb, acc);
+    else if (nb <= 5) small_step<9, 5>(fa, fb, acc);
+    else small_step<9, 9>(fa, fb, acc);
 }
 
 // A fragment element by element: byte b of the fragment is k = frag_k(q, b) of the step, `lane_at` the lane's offset with its
@@ -115,7 +127,17 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
         }
     };
     // accumulator register r of lane (li, q) holds row 4*q + r, column li of the tile
-    bool wide = false;
+    auto store_sums = [&](auto &acc) {
+        constexpr int D = sizeof(acc) / sizeof(v4i);
+#pragma unroll
+        for (int o = 0; o < 4; o++) red[wave][o][lane] = sum_diagonals<D>([&](int d) { return acc[d][o]; }, 0);
+    };
+    // HELD: the step that shows values beyond five digits outlives the loop in its registers.  Eight wavefronts with B contiguous along n read
+    // their share again instead: holding it costs them 0.15 us of 8.6 on 128 rows x [512,779] of narrow values (it would save 2.4 of 12.1 with
+    // 44 bits), and values are narrow in the model.
+    constexpr bool HELD = !BKM || WAVES == 4;
+    // (5 pairs, of nine digits 9, x 64 products of 2^14 a step)
+    static_assert((kSmallMaxK / 64 + WAVES - 1) / WAVES * 9L * 64 * 16384 <= kMaxDiagonal, "the int32 accumulators hold a wavefront's share");
     if (ONE) {
         RawFrag<false> fa, fb;
         int na = 0, nb = 0;
@@ -124,8 +146,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
             na = wave_digits(magnitude_or<false>(fa));
             nb = wave_digits(magnitude_or<false>(fb));
         }
-        // (each width adds up its own sums: with a choice between the two sets of accumulators in front of the sums a call takes 12.6 us
-        // on 128 rows x [779,512], now 11.7, and with 44 bits 14.3, now 13.2)
+        // (each width adds up its own sums: with a choice between the two sets of accumulators in front of the sums a call took 0.9 us
+        // more, 128 rows x [779,512] on eight wavefronts)
         if (na == 0) {
 #pragma unroll
             for (int o = 0; o < 4; o++) red[wave][o][lane] = Words{};
@@ -134,51 +156,69 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
 #pragma unroll
             for (int d = 0; d < kSmallDiagonals; d++) acc[d] = v4i{ 0, 0, 0, 0 };
             small_narrow_step(na, nb, fa, fb, acc);
-#pragma unroll
-            for (int o = 0; o < 4; o++) red[wave][o][lane] = sum_diagonals<kSmallDiagonals>([&](int d) { return acc[d][o]; }, 0);
+            store_sums(acc);
         } else {
             v4i acc[kSmallWideDiagonals];
 #pragma unroll
             for (int d = 0; d < kSmallWideDiagonals; d++) acc[d] = v4i{ 0, 0, 0, 0 };
-            if (na <= 5) small_step<5, 9>(fa, fb, acc);
-            else if (nb <= 5) small_step<9, 5>(fa, fb, acc);
-            else small_step<9, 9>(fa, fb, acc);
+            small_wide_step(na, nb, fa, fb, acc);
+            store_sums(acc);
+        }
+    } else if constexpr (HELD) {
+        v4i acc[kSmallDiagonals];
 #pragma unroll
-            for (int o = 0; o < 4; o++) red[wave][o][lane] = sum_diagonals<kSmallWideDiagonals>([&](int d) { return acc[d][o]; }, 0);
+        for (int d = 0; d < kSmallDiagonals; d++) acc[d] = v4i{ 0, 0, 0, 0 };
+        RawFrag<false> fa, fb;
+        int na = 0, nb = 0, ks = wave;
+        for (; ks < steps; ks += WAVES) {
+            load(ks, fa, fb);
+            na = wave_digits(magnitude_or<false>(fa));
+            nb = wave_digits(magnitude_or<false>(fb));
+            if (na > 5 || nb > 5) break;
+            small_narrow_step(na, nb, fa, fb, acc);
+        }
+        if (ks >= steps) {
+            store_sums(acc);
+        } else {
+            // (the sums so far are the lower diagonals of the wide ones)
+            v4i wide[kSmallWideDiagonals];
+#pragma unroll
+            for (int d = 0; d < kSmallWideDiagonals; d++) wide[d] = d < kSmallDiagonals ? acc[d] : v4i{ 0, 0, 0, 0 };
+            for (;;) {
+                small_wide_step(na, nb, fa, fb, wide);
+                ks += WAVES;
+                if (ks >= steps) break;
+                load(ks, fa, fb);
+                na = wave_digits(magnitude_or<false>(fa));
+                nb = wave_digits(magnitude_or<false>(fb));
+            }
+            store_sums(wide);
         }
     } else {
         v4i acc[kSmallDiagonals];
 #pragma unroll
         for (int d = 0; d < kSmallDiagonals; d++) acc[d] = v4i{ 0, 0, 0, 0 };
+        bool wide = false;
         for (int ks = wave; ks < steps; ks += WAVES) {
-            RawFrag<false> fa;
-            RawFrag<false> fb;
+            RawFrag<false> fa, fb;
             load(ks, fa, fb);
             const int na = wave_digits(magnitude_or<false>(fa));
             const int nb = wave_digits(magnitude_or<false>(fb));
             if (na > 5 || nb > 5) { wide = true; break; }
             small_narrow_step(na, nb, fa, fb, acc);
         }
-        // (5 pairs x 64 products of 2^14 a step)
-        static_assert((kSmallMaxK / 64 + WAVES - 1) / WAVES * 5L * 64 * 16384 <= kMaxDiagonal, "the int32 accumulators hold a wavefront's share");
+        store_sums(acc);
+        if (wide) {
+            v4i wacc[kSmallWideDiagonals];
 #pragma unroll
-        for (int o = 0; o < 4; o++) red[wave][o][lane] = sum_diagonals<kSmallDiagonals>([&](int d) { return acc[d][o]; }, 0);
-    }
-    if (!ONE && wide) {
-        // wider than five digits: this wavefront's steps once more with nine
-        constexpr int D = kSmallWideDiagonals;
-        v4i acc[D];
-#pragma unroll
-        for (int d = 0; d < D; d++) acc[d] = v4i{ 0, 0, 0, 0 };
-        for (int ks = wave; ks < steps; ks += WAVES) {
-            RawFrag<false> fa_raw;
-            RawFrag<false> fb_raw;
-            load(ks, fa_raw, fb_raw);
-            small_step<9, 9>(fa_raw, fb_raw, acc);
+            for (int d = 0; d < kSmallWideDiagonals; d++) wacc[d] = v4i{ 0, 0, 0, 0 };
+            for (int ks = wave; ks < steps; ks += WAVES) {
+                RawFrag<false> fa, fb;
+                load(ks, fa, fb);
+                small_step<9, 9>(fa, fb, wacc);
+            }
+            store_sums(wacc);
         }
-        static_assert((kSmallMaxK / 64 + WAVES - 1) / WAVES * 9L * 64 * 16384 <= kMaxDiagonal, "and of nine digits");
-#pragma unroll
-        for (int o = 0; o < 4; o++) red[wave][o][lane] = sum_diagonals<D>([&](int d) { return acc[d][o]; }, 0);
     }
     __syncthreads();
     const int m = m0 + 4 * q + (wave & 3), n = n0 + li;
@@ -186,8 +226,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2)))
     u128 s = (u128)(i128)p.init;
 #pragma unroll
     for (int w = 0; w < WAVES; w++) {
-        const Words t = red[w][wave][lane];
-        s += (u128)((uint64_t)t.w[3] << 32 | t.w[2]) << 64 | ((uint64_t)t.w[1] << 32 | t.w[0]);
+        s += words_value(red[w][wave][lane]);
     }
     const uint64_t lo = (uint64_t)s, hi = (uint64_t)(s >> 64);
     p.C[(long)g * p.sC + (long)m * p.ldc + n] = (int64_t)((lo >> p.shift) | ((hi << 1) << (63 - p.shift)));
