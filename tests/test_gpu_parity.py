@@ -1847,7 +1847,7 @@ def test_moe_dispatch_reports_indices_outside_the_experts(K, oracle, monkeypatch
     assert np.array_equal(host(y), ye)
 
 
-@pytest.mark.parametrize("Kr", [1, 7, 8, 9, 16, 17])
+@pytest.mark.parametrize("Kr", [1, 2, 3, 4, 5, 6, 7, 8, 9, 15, 16, 18])
 def test_moe_combine_slots_in_eights(K, Kr):
     """the weighted sum over slots taken eight at a time, products that wrap, floor shift, columns past whole workgroups"""
     rng = np.random.default_rng(Kr)

@@ -179,27 +179,42 @@ __global__ __launch_bounds__(256) void moe_gather_kernel(const int64_t *__restri
     }
 }
 
+// the terms of S slots of one element, all their loads under way together
+template <int S>
+__device__ __forceinline__ uint64_t combine_slots(const int64_t *__restrict__ ye, const int64_t *__restrict__ w, const int *__restrict__ pos,
+                                                  int N, int n, int shift)
+{
+    int64_t v[S], wk[S];
+#pragma unroll
+    for (int j = 0; j < S; j++) {
+        v[j] = ye[(long)pos[j] * N + n];
+        wk[j] = w[j];
+    }
+    uint64_t acc = 0;
+#pragma unroll
+    for (int j = 0; j < S; j++) acc += (uint64_t)((int64_t)((uint64_t)v[j] * (uint64_t)wk[j]) >> shift);
+    return acc;
+}
+
 // y[t][n] = sum_k (ye[pos[t][k]][n] * w[t][k]) >> shift   (wrapping products and sums, floor shift: model.py:1379)
+// Slots one after the other wait for their position and then for their row, and one token's sum lives on that; loads for slots that are not
+// there cost as much as the others.  So a piece of what is beyond whole eights, and then eights.  One after the other / always eight / so, rows
+// of 7168, kernels alone, us: 256 tokens of 1 slot 5.4 / 10.5 / 5.4, 2 slots 8.5 / 10.8 / 8.1, 3 slots 10.9 / 11.4 / 10.5, 8 slots 20.3 / 19.8 /
+// 20.1, 9 slots 22.0 / 21.2 / 21.0; one token of 1, 8 and 9 slots 1.95 / 2.28 / 1.94, 2.73 / 2.20 / 2.02 and 2.93 / 2.83 / 2.23; 2000 tokens of 2
+// slots 71 / 93 / 65.
+// REST: slots beyond whole eights
+template <int REST>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const int64_t *__restrict__ ye, const int64_t *__restrict__ w,
                                                           const int *__restrict__ pos, int64_t *__restrict__ y, int K, int N,
                                                           int shift)
 {
     const long t = blockIdx.y;
+    const int64_t *wt = w + t * K;
+    const int *pt = pos + t * K;
     for (int n = blockIdx.x * 256 + threadIdx.x; n < N; n += gridDim.x * 256) {
         uint64_t acc = 0;
-        // (eight slots' loads under way together: one after the other, each waits for its position and then for its row, and one token's
-        // sum lives on that.  256 tokens of 8 slots, 7168 elements, 21.0 -> 20.0 us a call, 300 tokens 24.6 -> 22.7, one to 32 tokens 7.1 -> 6.5)
-        for (int k0 = 0; k0 < K; k0 += 8) {
-            int64_t v[8], wk[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int k = k0 + j < K ? k0 + j : K - 1;
-                v[j] = ye[(long)pos[t * K + k] * N + n];
-                wk[j] = k0 + j < K ? w[t * K + k] : 0;
-            }
-#pragma unroll
-            for (int j = 0; j < 8; j++) acc += (uint64_t)((int64_t)((uint64_t)v[j] * (uint64_t)wk[j]) >> shift);
-        }
+        if constexpr (REST > 0) acc = combine_slots<REST>(ye, wt, pt, N, n, shift);
+        for (int k = REST; k < K; k += 8) acc += combine_slots<8>(ye, wt + k, pt + k, N, n, shift);
         y[t * N + n] = (int64_t)acc;
     }
 }
@@ -259,7 +274,18 @@ void moe_combine(const int64_t *ye, const int64_t *weights, const int *sorted_po
     if (bx > 32) bx = 32;
     for (long t0 = 0; t0 < T; t0 += 65535) {
         const long nt = T - t0 < 65535 ? T - t0 : 65535;
-        zk::moe_combine_kernel<<<dim3((unsigned)bx, (unsigned)nt), dim3(256), 0, 0>>>(ye, weights + t0 * K, sorted_pos + t0 * K, y + t0 * N, K, N, shift);
+#define ZK_COMBINE(REST) zk::moe_combine_kernel<REST><<<dim3((unsigned)bx, (unsigned)nt), dim3(256), 0, 0>>>(ye, weights + t0 * K, sorted_pos + t0 * K, y + t0 * N, K, N, shift)
+        switch (K % 8) {
+        case 0: ZK_COMBINE(0); break;
+        case 1: ZK_COMBINE(1); break;
+        case 2: ZK_COMBINE(2); break;
+        case 3: ZK_COMBINE(3); break;
+        case 4: ZK_COMBINE(4); break;
+        case 5: ZK_COMBINE(5); break;
+        case 6: ZK_COMBINE(6); break;
+        default: ZK_COMBINE(7); break;
+        }
+#undef ZK_COMBINE
     }
     zk::check_launch(name);
 }
