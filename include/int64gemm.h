@@ -169,6 +169,8 @@ void gate_route_q23(const int64_t *scores, const int32_t *bias, int64_t *weights
 void gate_sigmoid_route_q23(const int64_t *logits, const int64_t *lut, const int32_t *bias, int64_t *scores,
                             int64_t *weights, int64_t *indices, int64_t *raw_weights, int T, int E, int n_groups,
                             int topk_groups, int topk);
+/* How many of the routings so far gave every token a wavefront of its own (128, 256 or 512 experts, few tokens). */
+long zk_gate_wave_calls(void);
 
 /* Witness dump writer (replaces the reference's saveTensor, inference/model.py:94-102: a synchronous .cpu() copy and
  * file write per tensor, ~30 per layer).  zk_dump_device queues the raw bytes of `bytes` bytes of contiguous device

@@ -1743,8 +1743,9 @@ def test_silu_mul_q23_fusion(K, oracle, shape, keep):
         assert np.array_equal(host(S), se)
 
 
-# (128, 256 and 512 experts in a power of two of groups run on the kernel for few tokens up to 8192 of them, other shapes with
-#  2..16 groups of 8, 16 or 32 experts, and those beyond 8192 tokens, on the lane-per-group kernel, the others on the wave-wide one;
+# (128, 256 and 512 experts in a power of two of groups run on the kernel for few tokens up to 4096 to 8192 of them, see
+#  test_gate_route_on_both_sides_of_its_lines, other shapes with 2..16 groups of 8, 16 or 32 experts, and those beyond, on the lane-group
+#  kernel, the others on the wave-wide one;
 #  (64, 8, 2, 40) and (32, 2, 1, 20) ask for more winners than the kept groups hold, so masked experts win too)
 GATE_SHAPES = [(256, 8, 4, 8), (16, 4, 2, 4), (64, 1, 1, 6), (96, 3, 3, 5), (512, 8, 3, 8), (1024, 16, 5, 64), (7, 1, 1, 7),
                (512, 16, 4, 6), (64, 4, 2, 9), (64, 8, 2, 40), (32, 2, 1, 20), (128, 16, 16, 64), (64, 2, 2, 3),
@@ -1788,6 +1789,27 @@ def test_gate_sigmoid_route(K, oracle, E, G, KG, K_, with_bias):
             assert np.array_equal(host(idx), ie), "indices"
             assert np.array_equal(host(raw), re_), "gathered scores"
             assert np.array_equal(host(w), we), "weights"
+
+
+@pytest.mark.parametrize("E,G,KG,K_,sigmoid,line", [(128, 8, 4, 6, False, 4096), (128, 4, 2, 32, False, 5120), (256, 8, 4, 8, False, 5120), (256, 8, 4, 32, False, 7168),
+                                                    (128, 4, 2, 6, True, 7168), (128, 8, 4, 40, True, 7168), (256, 8, 4, 8, True, 8192), (128, 16, 16, 6, False, 8192),
+                                                    (256, 16, 4, 8, True, 8192), (512, 16, 8, 8, False, 8192), (256, 4, 2, 8, True, 8192), (128, 64, 20, 6, False, 8192)])
+def test_gate_route_on_both_sides_of_its_lines(K, oracle, E, G, KG, K_, sigmoid, line):
+    """a wavefront per token up to a number of tokens, four lanes per group from there to 8192, one lane per group or the whole wavefront beyond"""
+    rng = np.random.default_rng(E + G + K_)
+    bias = rng.integers(-3, 4, size=E, dtype=np.int64).astype(np.int32)
+    for T in sorted({line, line + 1, 8192, 8193}):
+        x = rng.integers(1, 40, size=(T, E), dtype=np.int64)
+        raw = torch.empty((T, K_), dtype=torch.int64, device="cuda")
+        before = K.lib.zk_gate_wave_calls()
+        if sigmoid:
+            _, w, idx = K.gate_sigmoid_route(dev(x), dev(bias), G, KG, K_, raw)
+            we, ie, re_ = oracle.gate_route(oracle.sigmoid_q23(x[None])[0], bias, G, KG, K_)
+        else:
+            w, idx = K.gate_route(dev(x), dev(bias), G, KG, K_, raw)
+            we, ie, re_ = oracle.gate_route(x, bias, G, KG, K_)
+        assert np.array_equal(host(idx), ie) and np.array_equal(host(raw), re_) and np.array_equal(host(w), we), T
+        assert K.lib.zk_gate_wave_calls() == before + (T <= line), T
 
 
 def _routing(rng, T, E, Kr):

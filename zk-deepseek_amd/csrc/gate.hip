@@ -10,6 +10,8 @@
 #include "act_one.h"
 #include "../../include/int64gemm.h"
 
+#include <atomic>
+
 namespace zk {
 
 struct Best { int64_t v; int idx; };
@@ -164,8 +166,7 @@ __global__ __launch_bounds__(256) void gate_route_kernel(const int64_t *__restri
 // from l * GS on in registers, LPG neighbouring lanes make up a group.  The groups' two best, the masking and most of the
 // arg-max over a token's experts (GS comparisons per lane, log2(LT) exchanges) stay inside a lane; the wave-wide form
 // above pays six exchanges per group and per winner.  LPG = 1 gives the most tokens per wavefront (throughput when
-// there are many tokens), LPG = 4 the shorter chain of dependent work per token (few tokens of up to 64 experts; more experts:
-// gate_route_few_kernel).
+// there are many tokens), LPG = 4 the shorter chain of dependent work per token (fewer tokens; the fewest: gate_route_few_kernel).
 template <int GS, int LPG, int NG, bool FUSED>
 __global__ __launch_bounds__(256) void gate_route_groups_kernel(const int64_t *__restrict__ scores, const int64_t *__restrict__ lut,
                                                                 int64_t *__restrict__ sig, const int32_t *__restrict__ bias,
@@ -267,12 +268,24 @@ __global__ __launch_bounds__(256) void gate_route_groups_kernel(const int64_t *_
     }
 }
 
-// Tokens up to which a token has a wavefront to itself.  What bounds one token is the chain of dependent work, what bounds many
-// their instructions.  Whole calls with sigmoid, lane groups / a wavefront per token (10.1 us is what the host takes): 256 experts in 8
-// groups, 256 tokens 13.2 / 10.2 us, 4096 17.1 / 13.7, 8192 24.2 / 22.5; 512 experts in 8 groups, which had six exchanges
-// through LDS per group and winner, 1 token 23.9 / 10.2, 8192 118 / 38; 128 in 8 groups 4096 12.0 / 10.5, 8192 15.7 / 16.3.
-// The launch for one token and 256 experts: 13-17 -> 7.6 us.
+// Tokens up to which a token has a wavefront to itself, or four lanes per group.  What bounds one token is the chain of dependent work,
+// what bounds many their instructions.
+// (One token of 256 experts in 8 groups, with sigmoid, in the lane groups / as a wavefront 12.4 / 7.0 us; of 512, which had six exchanges through LDS per group
+// and winner, 24.0 / 9.8, 8192 tokens 119 / 38.)
 constexpr int kFewTokens = 8192;
+
+// ... and the line between the two, where the lane groups have the shape: a wavefront to a token is ahead while the chain is what counts, the
+// lane groups once there are more wavefronts than the device runs at once, sooner without the sigmoid and its table.  Kernels alone, with
+// bias, lane groups / a wavefront, us.  Without sigmoid, 6 winners: 128 experts in 8 groups, 4096 tokens 8.8 / 8.0, 6144 9.3 / 10.1, 8192 10.5 /
+// 12.1, in 4 groups 8.4 / 7.7, 9.2 / 9.7, 9.3 / 11.7; 256 in 8 groups 10.0 / 9.3, 11.2 / 11.7, 12.9 / 14.0, of 32 winners 7168 tokens 42.6 / 38.1.
+// With it: 128 in 8 groups 10.9 / 9.6, 12.2 / 12.2, 14.1 / 14.8; 256 in 8 groups 15.9 / 12.7, 19.3 / 16.6, 22.5 / 20.8.  In 16 groups a wavefront is ahead all
+// through (128 experts, 8192 tokens 21.6 / 16.0, 256 25.3 / 21.8; 512 37.0 / 36.4, without sigmoid 23.3 / 24.2 with bias, 22.3 / 17.5 without).
+static int wave_per_token_up_to(int E, int gsize, int topk, bool fused)
+{
+    if (E == 512 || gsize == 8 || (E == 256 && gsize == 16)) return kFewTokens;
+    if (fused) return E == 256 ? kFewTokens : 7168;
+    return E == 256 ? (topk <= 8 ? 5120 : 7168) : (topk <= 8 ? 4096 : 5120);
+}
 
 // Few tokens: a wavefront each, EPL consecutive experts per lane, 64 / n_groups lanes per group (a power of two).  What takes
 // the time is the chain of dependent work per token, so nothing in it leaves the registers: maxima go through lane_pair, a
@@ -368,6 +381,8 @@ __global__ __launch_bounds__(64) void gate_route_few_kernel(const int64_t *__res
     indices[tok * topk + lane] = my_idx;
 }
 
+static std::atomic<long> g_gate_wave_calls(0);
+
 template <bool FUSED>
 static void gate_launch(const char *name, const int64_t *scores, const int64_t *lut, int64_t *sig, const int32_t *bias,
                         int64_t *weights, int64_t *indices, int64_t *raw, int T, int E, int n_groups, int topk_groups, int topk)
@@ -383,22 +398,25 @@ static void gate_launch(const char *name, const int64_t *scores, const int64_t *
     const int gsize = E / n_groups;
     const bool aligned = (((uintptr_t)scores | (uintptr_t)sig) & 15) == 0;
     const bool pow2 = (n_groups & (n_groups - 1)) == 0;
-    if (aligned && pow2 && T <= kFewTokens && (E == 128 || E == 256 || E == 512) && gsize >= E / 64) {
+    const bool lane_groups = aligned && pow2 && n_groups >= 2 && (gsize == 32 || gsize == 16 || gsize == 8) && n_groups <= 16;
+    if (aligned && pow2 && T <= (lane_groups ? wave_per_token_up_to(E, gsize, topk, FUSED) : kFewTokens) && (E == 128 || E == 256 || E == 512) && gsize >= E / 64) {
 #define ZK_GATE_F(EPL) gate_route_few_kernel<EPL, FUSED><<<dim3((unsigned)T), dim3(64), 0, 0>>>(scores, lut, sig, bias, weights, indices, raw, n_groups, topk_groups, topk)
         if (E == 128) ZK_GATE_F(2);
         else if (E == 256) ZK_GATE_F(4);
         else ZK_GATE_F(8);
 #undef ZK_GATE_F
+        g_gate_wave_calls++;
         check_launch(name);
         return;
     }
-    if (aligned && pow2 && n_groups >= 2 && (gsize == 32 || gsize == 16 || gsize == 8) && n_groups <= 16) {
-        // (what the kernel for few tokens does not take: four lanes per group up to 64 experts; else one)
-        const bool spread = T <= kFewTokens && E <= 64;
+    if (lane_groups) {
+        // what the kernel for few tokens does not take: four lanes per group while tokens are few, then one
+        const bool spread = T <= kFewTokens;
         const int per_wave = 64 / (n_groups * (spread ? 4 : 1));
         const dim3 grid((unsigned)((T + 4 * per_wave - 1) / (4 * per_wave))), block(256);
 #define ZK_GATE_G(GS, LPG, NG) gate_route_groups_kernel<GS, LPG, NG, FUSED><<<grid, block, 0, 0>>>(scores, lut, sig, bias, weights, indices, raw, T, topk_groups, topk)
-#define ZK_GATE_NG(GSIZE, NG) do { if constexpr (GSIZE * NG <= 64) { if (spread) { ZK_GATE_G(GSIZE / 4, 4, NG); break; } } ZK_GATE_G(GSIZE, 1, NG); } while (0)
+        // (groups of 8, 16 and 32 out of more than 64, 128 and 256 experts come here with many tokens only)
+#define ZK_GATE_NG(GSIZE, NG) do { if constexpr (GSIZE * NG <= (GSIZE == 32 ? 256 : GSIZE == 16 ? 128 : 64)) { if (spread) { ZK_GATE_G(GSIZE / 4, 4, NG); break; } } ZK_GATE_G(GSIZE, 1, NG); } while (0)
 #define ZK_GATE_GS(GSIZE) do { if (n_groups == 2) ZK_GATE_NG(GSIZE, 2); else if (n_groups == 4) ZK_GATE_NG(GSIZE, 4); \
                                else if (n_groups == 8) ZK_GATE_NG(GSIZE, 8); else ZK_GATE_NG(GSIZE, 16); } while (0)
         if (gsize == 32) ZK_GATE_GS(32);
@@ -435,3 +453,5 @@ extern "C" void gate_sigmoid_route_q23(const int64_t *logits, const int64_t *lut
 {
     zk::gate_launch<true>("gate_sigmoid_route_q23", logits, lut, scores, bias, weights, indices, raw_weights, T, E, n_groups, topk_groups, topk);
 }
+
+extern "C" long zk_gate_wave_calls(void) { return zk::g_gate_wave_calls; }
