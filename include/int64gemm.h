@@ -252,9 +252,11 @@ long zk_gemm_grouped_streamed_calls(void);
  * prepared with zk_gemm_prepare_weights, and a B that is small next to the product, with A split by a pass in front or by the
  * kernel itself; ZK_NO_PIPE=1 switches them off). */
 long zk_gemm_pipe_calls(void);
-/* How many of those ran on the kernel that splits A itself (ZK_NO_ROWTILE=1 leaves their A to the pass in front), and how many
- * launches so far were small products done in one launch (scores and values of up to eight positions). */
+/* How many of those ran on the kernel that splits A itself (ZK_NO_ROWTILE=1 leaves their A to the pass in front), how many GEMM
+ * launches so far ran on 64x64 tiles (a short K), and how many were small products done in one launch (scores and values of up to
+ * eight positions). */
 long zk_gemm_rowtile_calls(void);
+long zk_gemm_short_calls(void);
 long zk_gemm_small_calls(void);
 /* No reference counterpart: model weights do not change between calls, so a weight matrix W[N,K] (int64, or int32 with
  * b32 != 0; groups == 0, B = the device pointer later passed as B) or all the matrices of a device table of pointers

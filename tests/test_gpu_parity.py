@@ -756,20 +756,42 @@ def test_einsums_seeded_random_problems(K, oracle, seed):
 @pytest.mark.parametrize("bits_a,bits_b,digits", [(20, 28, (3, 4)), (28, 20, (4, 3)), (28, 28, (4, 4))])
 def test_einsums_of_a_short_k_on_small_tiles(K, oracle, bits_a, bits_b, digits):
     """64x64 tiles, two workgroups to a compute unit: K around one, two and eight steps of 64, rows and columns around the tiles' edges, one B
-    per head in either layout and a shared one against many rows"""
+    per head in either layout and a shared one against many rows; and a shape on the other side of each line that keeps 128x64 tiles"""
     rng = np.random.default_rng(bits_a * 64 + bits_b)
 
-    def both(fn, A, B, c):
+    def both(fn, A, B, c, short=1):
+        expected = getattr(oracle, fn)(A, B, c)
         for _ in range(2):      # (a first call may run on digits remembered for other operands at these addresses)
+            before = K.lib.zk_gemm_short_calls()
             got = host(getattr(K, fn)(dev(A), dev(B), c))
-            assert np.array_equal(got, getattr(oracle, fn)(A, B, c)), (fn, A.shape, B.shape)
-        assert K.gemm_last_plan()[1:] == digits, (fn, A.shape, B.shape)
-    for H, M, D, C in ((64, 66, 63, 260), (64, 129, 64, 257), (128, 65, 65, 300), (128, 193, 128, 130)):
-        both("einsum_bshd_hdc_bshc", rand_i64(rng, (1, M, H, D), bits_a), rand_i32(rng, (H, D, C), bits_b), 30)
-    for H, M, D, C in ((64, 66, 260, 64), (128, 129, 65, 129), (128, 192, 65, 250), (48, 193, 129, 511), (128, 130, 66, 512)):
-        both("einsum_bshc_hdc_bshd", rand_i64(rng, (1, M, H, C), bits_a), rand_i32(rng, (H, D, C), bits_b), 30)
-    for M, T, D in ((129, 193, 64), (128, 256, 63), (131, 200, 1)):
-        both("einsum_bshc_btc_bsht", rand_i64(rng, (1, M, 128, D), bits_a), rand_i64(rng, (1, T, D), bits_b), 21)
+            assert np.array_equal(got, expected), (fn, A.shape, B.shape)
+        assert K.gemm_last_plan()[1:] == digits and K.lib.zk_gemm_short_calls() == before + short, (fn, A.shape, B.shape)
+    for H, M, D, C, short in ((64, 66, 63, 260, 1), (64, 129, 64, 257, 1), (128, 65, 65, 300, 1), (128, 193, 128, 130, 1), (128, 192, 260, 130, 1),
+                              (128, 193, 260, 130, 0), (64, 129, 128, 256, 0)):
+        both("einsum_bshd_hdc_bshc", rand_i64(rng, (1, M, H, D), bits_a), rand_i32(rng, (H, D, C), bits_b), 30, short)
+    for H, M, D, C, short in ((64, 66, 260, 64, 1), (128, 129, 65, 129, 1), (128, 192, 65, 250, 1), (128, 193, 129, 511, 1), (128, 130, 66, 512, 1),
+                              (48, 193, 129, 511, 0), (128, 193, 129, 513, 0)):
+        both("einsum_bshc_hdc_bshd", rand_i64(rng, (1, M, H, C), bits_a), rand_i32(rng, (H, D, C), bits_b), 30, short)
+    for M, T, D, short in ((129, 193, 64, 1), (128, 256, 63, 1), (131, 200, 1, 1), (127, 256, 63, 0), (129, 192, 64, 0), (128, 256, 65, 0)):
+        both("einsum_bshc_btc_bsht", rand_i64(rng, (1, M, 128, D), bits_a), rand_i64(rng, (1, T, D), bits_b), 21, short)
+
+
+@pytest.mark.parametrize("cols,short", [(2000, 1), (2020, 0)])
+def test_small_tiles_up_to_what_the_memory_side_cache_holds(K, oracle, cols, short):
+    """16384 rows whose A and outputs are just below, and just beyond, 252 MB"""
+    rng = np.random.default_rng(cols)
+    a, b = rand_i64(rng, (1, 128, 128, 8), 20), rand_i64(rng, (1, cols, 8), 28)
+    oracle.set_threads(oracle.max_threads())
+    try:
+        expected = oracle.einsum_bshc_btc_bsht(a, b, 21)
+    finally:
+        oracle.set_threads(1)
+    da, db = dev(a), dev(b)
+    for _ in range(2):
+        before = K.lib.zk_gemm_short_calls()
+        got = K.einsum_bshc_btc_bsht(da, db, 21)
+        assert np.array_equal(host(got), expected)
+    assert K.gemm_last_plan()[1:] == (3, 4) and K.lib.zk_gemm_short_calls() == before + short
 
 
 @pytest.mark.parametrize("path", PATHS)

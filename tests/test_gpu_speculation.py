@@ -428,6 +428,37 @@ def test_stale_guess_per_head_einsums(K, oracle):
                         lambda: (oracle.einsum_bshc_hdc_bshd(o.h, w2.h, 31),), [o, w2], pokes)
 
 
+@pytest.mark.parametrize("bits_w", [28, 20])
+def test_stale_guess_on_small_tiles(K, oracle, oracle_threads, bits_w):
+    """the 64x64 tiles for a short K, one B per head in either layout: wide elements in the first and the last tile, in the rows and columns of a
+    tile's edge, int32 weights that outgrow three digits, and operands wide throughout"""
+    rng = np.random.default_rng(43 + bits_w)
+    H, S = 64, 129
+    for fn, D, Cc in (("einsum_bshd_hdc_bshc", 64, 257), ("einsum_bshc_hdc_bshd", 257, 60)):
+        a = Operand(rand_i64(rng, (1, S, H, 64 if Cc == 257 else Cc), 28))
+        w = Operand(rand_i32(rng, (H, D, Cc), bits_w))
+
+        def call():
+            before = K.lib.zk_gemm_short_calls()
+            out = getattr(K, fn)(a.d, w.d, 30)
+            call.short = K.lib.zk_gemm_short_calls() == before + 1
+            return (out,)
+
+        def poked(poke):
+            def f():
+                assert call.short, "the narrow call is expected on the small tiles"
+                poke()
+            return f
+
+        def widen():
+            a.h[...] = rand_i64(rng, a.h.shape, 63)
+            a.d.copy_(torch.from_numpy(a.h))
+        pokes = [lambda: a.poke((0, S - 1, H - 1, a.h.shape[-1] - 1), WIDE), lambda: a.poke((0, 64, 0, 0), -WIDE), lambda: a.poke((0, 0, 31, 33), 1 << 62), widen]
+        if bits_w == 20:
+            pokes += [lambda: w.poke((H - 1, D - 1, Cc - 1), 1 << 30), lambda: w.poke((0, 0, 0), -(1 << 30)), lambda: w.poke((17, D // 2, 1), 1 << 24)]
+        _stale_guess_rounds(K, call, lambda: (getattr(oracle, fn)(a.h, w.h, 30),), [a, w], [poked(p) for p in pokes])
+
+
 @pytest.mark.parametrize("M", [20, 200])
 def test_stale_guess_prepared_weights(K, oracle, M):
     """B from prepared digit planes (its digit count is exact, nothing of it is tracked): activations that outgrow the

@@ -300,12 +300,13 @@ static bool wait_digits(long first, long seen_count, int *need_a, int *need_b)
 }
 
 static int g_last_pairs = 0, g_last_prepared = 0;
-static long g_streamed_calls = 0, g_pipe_calls = 0, g_rowtile_calls = 0;
+static long g_streamed_calls = 0, g_pipe_calls = 0, g_rowtile_calls = 0, g_short_calls = 0;
 int gemm_mfma_last_pairs() { return g_last_pairs; }
 int gemm_mfma_last_prepared() { return g_last_prepared; }
 long gemm_mfma_grouped_streamed_calls() { return g_streamed_calls; }
 long gemm_mfma_pipe_calls() { return g_pipe_calls; }
 long gemm_mfma_rowtile_calls() { return g_rowtile_calls; }
+long gemm_mfma_short_calls() { return g_short_calls; }
 
 long gemm_mfma_guard_hits()
 {
@@ -604,14 +605,24 @@ static int rowtile_parts(const GemmDesc &d, int na, int nb, int bn, int cus)
 // 14.2; not where they fill two rounds at most (64 heads [128,512], 65 rows 20.7 / 21.2, 16 heads, 192 rows 13.4 / 14.4).  k-contiguous, 128
 // heads, K = 512, 128 columns: 192 rows 44.6 / 38.7, 243 rows 49.5 / 46.7, 500 rows 124 / 110; not in one round (64 heads 25.1 / 26.1), nor up
 // to 128 rows (70 rows 25.9 / 26.8).  A shared B of many columns: not at K = 512 (20480 rows x [160,512] 43.2 / 44.8), but tall at K = 64, where the
-// pass that splits A in front goes as well: 25600 rows x [200,64] 31.1 / 25.9, 31104 x [243,64] 35.4 / 27.8.  With (3,3) digits, 128x128
-// tiles, it is slower throughout (243 rows of 128 heads [128,512] 52.7 / 59.4).
+// pass that splits A in front goes as well: 25600 rows x [200,64] 31.1 / 25.9, 31104 x [243,64] 35.4 / 27.8, and at any K below (64000 x [277,8]
+// 64.6 / 56.1, 19968 x [960,48] 63.3 / 57.7).  With (3,3) digits, 128x128 tiles, it is slower throughout (243 rows of 128 heads [128,512] 52.7 / 59.4).
+// Splitting B twice as often shows where nothing is won by it, n-contiguous and K > 256, (4,4), [512,512]: rows that fill their tiles in
+// rounds that fill the device, 32 heads 243 rows 48.3 / 50.7, 384 rows 70.1 / 73.7, 64 heads 243 rows 91.3 / 95.3; half a last round is enough to
+// win (48 heads, 384 rows x [256,512] 67.0 / 61.9), and so are many rounds (64 heads, 500 rows 201 / 190; 256 columns from four: 128 heads, 500
+// rows x [128,512] 128 / 119).  And two workgroups store at a lower rate than one where A and the outputs are more than the memory-side cache holds next to
+// each other (256 MB): K <= 64 and k-contiguous or tall, 16384 x [1924,32] (242 MB) 84.1 / 80.5, 64000 x [621,24] (315) 107 / 123, 19968 x
+// [2328,16] (357) 117 / 137, with remainder 65536 x [243,64] (275) 72.6 / 82.3, 16 heads, 8000 rows x [300,64] (355) 131 / 144.
 static const Instance *short_k_tiles(const Instance *inst, const GemmDesc &d, int cus)
 {
     const long tiles_n = (d.N + 63) / 64, tiles = (long)((d.M + 127) / 128) * tiles_n * d.G;
     if (inst->bm != 128 || inst->bn != 64 || inst->dmax != 16) return inst;
-    const bool heads = d.G > 1 && d.sB != 0 && (d.K <= 64 ? tiles >= cus : d.K <= 128 ? tiles > 2L * cus : d.K <= 512 && d.M > 128 && 2 * tiles >= 3L * cus);
-    const bool tall = d.K <= 64 && d.M >= kPipeMinRows && tiles_n >= 4;
+    const bool in_cache = (double)d.G * d.M * (8.0 * d.K + (d.R ? 16.0 : 8.0) * d.N) <= 252.0 * (1 << 20);
+    const long last = tiles % cus;
+    const bool gaps = (d.M - 1) % 128 < 64 || (last != 0 && 2 * last <= cus) || tiles > (d.N <= 256 ? 3L : 6L) * cus;
+    const bool heads = d.G > 1 && d.sB != 0 && (d.K <= 64 ? tiles >= cus && (in_cache || d.ldbk != 1) : d.K <= 128 ? tiles > 2L * cus
+                       : d.K <= 512 && d.M > 128 && 2 * tiles >= 3L * cus && (d.K <= 256 || d.ldbk == 1 || gaps));
+    const bool tall = d.K <= 64 && d.M >= kPipeMinRows && tiles_n >= 4 && in_cache;
     if (!heads && !tall) return inst;
     int count;
     const Instance *t = instances(&count);
@@ -1020,6 +1031,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
         g_last_prepared = prep ? 1 : 0;
         if (pipe.fn || rowtile.fn) g_pipe_calls++;
         if (rowtile.fn) g_rowtile_calls++;
+        if (inst->short_k) g_short_calls++;
         {
             const hipError_t err = hipGetLastError();
             if (err != hipSuccess) {
