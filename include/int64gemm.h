@@ -133,6 +133,8 @@ void rms_norm_residual_fused_32(const int64_t *X, const int64_t *Y, int k, const
                                 int64_t *C, int M, int N, int64_t eps, int64_t dim);
 void rms_norm_residual_fused_64(const int64_t *X, const int64_t *Y, int k, const int64_t *W, int64_t *Xout, int64_t *rms,
                                 int64_t *C, int M, int N, int64_t eps, int64_t dim);
+/* How many of the fused norms so far took several workgroups per row (few long rows, nothing stored over anything that is read). */
+long zk_rms_split_calls(void);
 
 /* 1: softmax_q19/q21 also overwrite R with the per-element weights, as the reference's kernels do
  * (inference/int64_gemm.cu:708,729 and :629,650).  0 (default): R is left untouched. */

@@ -1452,15 +1452,46 @@ def test_rmsnorm_few_rows_on_several_compute_units(K, oracle, M, N, off):
         return t.copy_(dev(a))
     w, stat, out, xo = dev(W), torch.empty(M, dtype=torch.int64, device="cuda"), shifted(A), shifted(A)
     lib, ptr = K.lib, lambda t: t.data_ptr()
+    several = N > 4096 and M <= 32
     for a in (shifted(A), out):                      # the second: the result over the row
+        before = lib.zk_rms_split_calls()
         lib.rms_norm_fused_32(ptr(a), ptr(w), ptr(stat), ptr(out), M, N, 1, N)
+        assert lib.zk_rms_split_calls() == before + (several and a is not out)
         assert np.array_equal(host(out), Ce) and np.array_equal(host(stat), rms_e[:M])
         out = out.copy_(dev(A)) if a is not out else out
     y = shifted(Y)
     for a in (shifted(A), xo):                       # the second: the sum over its first operand
         xo.copy_(dev(A))
+        before = lib.zk_rms_split_calls()
         lib.rms_norm_residual_fused_32(ptr(a), ptr(y), 8, ptr(w), ptr(xo), ptr(stat), ptr(out), M, N, 1, N)
+        assert lib.zk_rms_split_calls() == before + (several and a is not xo)
         assert np.array_equal(host(xo), X) and np.array_equal(host(out), Xe) and np.array_equal(host(stat), rms_x[:M])
+    K._check("rms_norm")
+
+
+@pytest.mark.parametrize("N", [4098, 7168, 8191])
+def test_rmsnorm_of_one_row_over_its_own_operands(K, oracle, N):
+    """a row that one workgroup holds in its registers may be stored over its weights, at any offset, and its statistic over the row or the
+    residual: such calls keep that one workgroup"""
+    rng = np.random.default_rng(N)
+    A, Y, W = rand_i64(rng, (1, N), 31), rand_i64(rng, (1, N), 22), rng.integers(1 << 18, 1 << 20, size=(N,), dtype=np.int64)
+    Ce, rms_e = oracle.RMS_Norm_int64(A, W, 1, N)
+    Xe, Cx, rms_x = oracle.RMS_Norm_residual_int64(A, Y, 8, W, 1, N)
+    lib, ptr = K.lib, lambda t: t.data_ptr()
+    before = lib.zk_rms_split_calls()
+    for off in (-1300, -2, 1, 2048):
+        a, buf, stat = dev(A), torch.zeros(N + 4096, dtype=torch.int64, device="cuda"), torch.empty(1, dtype=torch.int64, device="cuda")
+        w, c = buf[2048:2048 + N].copy_(dev(W)), buf[2048 + off:2048 + off + N]
+        lib.rms_norm_fused_64(ptr(a), ptr(w), ptr(stat), ptr(c), 1, N, 1, N)
+        assert np.array_equal(host(c), Ce[0]) and int(stat[0]) == rms_e[0], off
+    for at in (0, N // 2, N - 1):
+        a, w, c, x = dev(A), dev(W), torch.empty((1, N), dtype=torch.int64, device="cuda"), torch.empty((1, N), dtype=torch.int64, device="cuda")
+        lib.rms_norm_fused_64(ptr(a), ptr(w), ptr(a[0, at:]), ptr(c), 1, N, 1, N)
+        assert np.array_equal(host(c), Ce) and int(a[0, at]) == rms_e[0], at
+        a, y = dev(A), dev(Y)
+        lib.rms_norm_residual_fused_64(ptr(a), ptr(y), 8, ptr(w), ptr(x), ptr(y[0, at:]), ptr(c), 1, N, 1, N)
+        assert np.array_equal(host(x), Xe) and np.array_equal(host(c), Cx) and int(y[0, at]) == rms_x[0], at
+    assert lib.zk_rms_split_calls() == before
     K._check("rms_norm")
 
 

@@ -8,6 +8,8 @@
 #include "common.h"
 #include "../../include/int64gemm.h"
 
+#include <atomic>
+
 namespace zk {
 
 // ---- 192-bit unsigned accumulator -------------------------------------------------------------
@@ -419,7 +421,7 @@ __device__ __forceinline__ void store_pair(int64_t *p, int64_t x, int64_t y, boo
 // residual connection, inference/model.py:1465, 1472), and that sum is also stored to Xout (which may be A itself).
 // PARTS: workgroups per row.  Each takes the statistic of the whole row and stores one pair of every thread: a row that is alone on the
 // device is bound by what one compute unit's vector pipes do, and most of that is the exact division of its elements.  Nothing that
-// is stored may overlap what the other workgroups of the row still read (rows_overlap).
+// is stored may overlap what the other workgroups of the row still read or store (spans_overlap).
 struct RmsResidual { const int64_t *Y; int64_t *Xout; int k; };
 
 template <typename WT, int THREADS, int EPT, bool VEC, int WPE, bool RES, int PARTS = 1>
@@ -555,10 +557,20 @@ __global__ __launch_bounds__(256) void residual_add_kernel(const int64_t *A, con
         Xout[i] = (int64_t)((uint64_t)A[i] + ((uint64_t)Y[i] << k));
 }
 
-static bool rows_overlap(const void *a, const void *b, long bytes)
+static std::atomic<long> g_rms_split_calls(0);
+
+// Whether anything that a norm stores overlaps something that it reads or stores elsewhere.
+struct Span { const void *at; size_t bytes; };
+static bool spans_overlap(const Span *out, int outs, const Span *in, int ins)
 {
-    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
-    return x < y + (uintptr_t)bytes && y < x + (uintptr_t)bytes;
+    const auto meet = [](const Span &a, const Span &b) { return (uintptr_t)a.at < (uintptr_t)b.at + b.bytes && (uintptr_t)b.at < (uintptr_t)a.at + a.bytes; };
+    for (int i = 0; i < outs; i++) {
+        for (int j = 0; j < ins; j++)
+            if (meet(out[i], in[j])) return true;
+        for (int j = 0; j < i; j++)
+            if (meet(out[i], out[j])) return true;
+    }
+    return false;
 }
 
 template <typename WT>
@@ -598,12 +610,16 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
     // of two, kernel alone, mean of 1 to 64 rows: up to 1024 elements 4.7 / 4.9 / 5.4 us (with residual 4.6 / 5.0 / 5.4), 1025 to 2048 5.3 / 5.1 / 5.5
     // (5.1 / 5.3 / 5.6), of odd length 5.7 / 5.3 / 5.5.
     const bool apart = vec && !res && ((M <= 16 && N > 22528) || (M > cus && M <= cus + cus / 16));
-    const long bytes = (long)M * N * 8;
-    const bool split = !rows_overlap(C, A, bytes) && (!res || (!rows_overlap(C, r.Y, bytes) && !rows_overlap(C, r.Xout, bytes) && !rows_overlap(r.Xout, A, bytes) && !rows_overlap(r.Xout, r.Y, bytes)));
     // Few long rows go to four compute units each.  One workgroup / four, us: 1 row of 7168 5.9 / 5.1, with residual 6.8 / 5.6, of 8191
     // 6.7 / 5.4 and 7.4 / 5.8; 16 rows of 7168 6.7 / 6.4 and 7.7 / 7.1; 32 rows 6.7 / 6.6 and 7.9 / 7.7; 64 rows 6.9 / 7.0 and 8.0 / 8.1, of 8191
     // with residual 8.5 / 8.7; rows of 2049, whose pairs do not go round a second time, level or slower.
-    if (split && N > 4096 && N <= 8192 && M <= 32) ZK_RMS_SPLIT(1024, 8);
+    bool split = N > 4096 && N <= 8192 && M <= 32;
+    if (split) {
+        const size_t bytes = (size_t)M * N * 8;
+        const Span out[3] = { { C, bytes }, { rms, (size_t)M * 8 }, { r.Xout, bytes } }, in[3] = { { A, bytes }, { W, (size_t)N * sizeof(WT) }, { r.Y, bytes } };
+        split = !spans_overlap(out, res ? 3 : 2, in, res ? 3 : 2);
+    }
+    if (split) { ZK_RMS_SPLIT(1024, 8); g_rms_split_calls++; }
     else if (N <= 512) ZK_RMS_LAUNCH(256, 2, 1);
     else if (N <= 2048 && !(M <= 64 && N > 1024)) ZK_RMS_LAUNCH(256, 8, 1);
     else if (N <= 2048) ZK_RMS_LAUNCH(512, 4, 1);
@@ -642,6 +658,8 @@ static void launch_fused(const char *name, const int64_t *A, const WT *W, int64_
 }  // namespace zk
 
 extern "C" {
+
+long zk_rms_split_calls(void) { return zk::g_rms_split_calls; }
 
 void rms_norm_32(const int64_t *A, const int32_t *W, const int64_t *rms, int64_t *C, int seqLen, int Dim)
 {

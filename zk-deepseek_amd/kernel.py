@@ -80,6 +80,7 @@ lib.zk_gemm_pipe_calls.restype = ctypes.c_long
 lib.zk_gemm_rowtile_calls.restype = ctypes.c_long
 lib.zk_gemm_short_calls.restype = ctypes.c_long
 lib.zk_gemm_small_calls.restype = ctypes.c_long
+lib.zk_rms_split_calls.restype = ctypes.c_long
 lib.zk_gate_wave_calls.restype = ctypes.c_long
 lib.softmax_q19_scores.argtypes = [_vp] * 6 + [_ci] * 4 + [ctypes.c_longlong] * 2
 lib.silu_mul_q23.argtypes = [_vp] * 5 + [_ci] * 3
