@@ -260,6 +260,9 @@ long zk_gemm_pipe_calls(void);
 long zk_gemm_rowtile_calls(void);
 long zk_gemm_short_calls(void);
 long zk_gemm_small_calls(void);
+/* How many products cut along K have left the digit counts that they saw with the sum of their slices (the others leave them
+ * with the guarded launch). */
+long zk_gemm_sum_reports(void);
 /* No reference counterpart: model weights do not change between calls, so a weight matrix W[N,K] (int64, or int32 with
  * b32 != 0; groups == 0, B = the device pointer later passed as B) or all the matrices of a device table of pointers
  * (groups > 0, B = the table later passed to int64_grouped_bmm_launcher) can be split into base-256 digit planes ONCE.

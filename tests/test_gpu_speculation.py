@@ -428,6 +428,24 @@ def test_stale_guess_per_head_einsums(K, oracle):
                         lambda: (oracle.einsum_bshc_hdc_bshd(o.h, w2.h, 31),), [o, w2], pokes)
 
 
+@pytest.mark.parametrize("shape,w32,reports", [((1, 70, 1000, 64), False, 1), ((1, 243, 4096, 512), True, 1), ((2, 130, 900, 150), True, 1), ((1, 300, 64, 2000), False, 0)])
+def test_stale_guess_reported_with_the_sum_of_slices(K, oracle, oracle_threads, shape, w32, reports):
+    """a product cut along K leaves its report with the sum of the slices, from one workgroup and from several, others with the guarded
+    launch: what a wide element needed reaches the next call either way, and so does what a narrow one did not"""
+    Bd, M, Kd, N = shape
+    rng = np.random.default_rng(sum(shape))
+    A = Operand(rand_i64(rng, (Bd, M, Kd), 20))
+    W = Operand(rand_i32(rng, (N, Kd), 16) if w32 else rand_i64(rng, (N, Kd), 16))
+
+    def call():
+        before = K.lib.zk_gemm_sum_reports()
+        out = K.int64_bmm_broadcast(A.d, W.d, 1, 1, 29)
+        assert K.lib.zk_gemm_sum_reports() == before + reports
+        return out
+    pokes = [lambda: A.poke((Bd - 1, M - 1, Kd - 1), WIDE), lambda: A.poke((0, 0, 0), 1 << 62), lambda: W.poke((N - 1, 0), (1 << 30) if w32 else -WIDE)]
+    _stale_guess_rounds(K, call, lambda: oracle.int64_bmm_broadcast(A.h, W.h, 1, 1, 29), [A, W], pokes)
+
+
 @pytest.mark.parametrize("bits_w", [28, 20])
 def test_stale_guess_on_small_tiles(K, oracle, oracle_threads, bits_w):
     """the 64x64 tiles for a short K, one B per head in either layout: wide elements in the first and the last tile, in the rows and columns of a

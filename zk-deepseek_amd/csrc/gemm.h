@@ -134,6 +134,7 @@ long gemm_mfma_grouped_streamed_calls();   // grouped launches so far that ran o
 long gemm_mfma_pipe_calls();               // launches so far that ran on the software-pipelined kernels for planes on both sides
 long gemm_mfma_rowtile_calls();            // ... and those of them on the kernel that splits A itself (gemm_mfma_rowtile.h)
 long gemm_mfma_short_calls();              // launches so far on the 64x64 tiles for a short K
+long gemm_mfma_sum_reports();              // reports so far that left with the sum of a product's slices
 
 // Grouped product: the rows of A and C form one contiguous segment per group and every group has its own
 // k-contiguous B[N,K] (the experts of a MoE layer after the tokens have been sorted by expert):

@@ -295,6 +295,7 @@ long zk_gemm_grouped_streamed_calls(void) { return zk::gemm_mfma_grouped_streame
 long zk_gemm_pipe_calls(void) { return zk::gemm_mfma_pipe_calls(); }
 long zk_gemm_rowtile_calls(void) { return zk::gemm_mfma_rowtile_calls(); }
 long zk_gemm_short_calls(void) { return zk::gemm_mfma_short_calls(); }
+long zk_gemm_sum_reports(void) { return zk::gemm_mfma_sum_reports(); }
 long zk_gemm_small_calls(void) { return zk::gemm_small_calls(); }
 
 int zk_gemm_last_prepared(void) { return zk::g_last_digits ? zk::gemm_mfma_last_prepared() : 0; }

@@ -300,13 +300,14 @@ static bool wait_digits(long first, long seen_count, int *need_a, int *need_b)
 }
 
 static int g_last_pairs = 0, g_last_prepared = 0;
-static long g_streamed_calls = 0, g_pipe_calls = 0, g_rowtile_calls = 0, g_short_calls = 0;
+static long g_streamed_calls = 0, g_pipe_calls = 0, g_rowtile_calls = 0, g_short_calls = 0, g_sum_reports = 0;
 int gemm_mfma_last_pairs() { return g_last_pairs; }
 int gemm_mfma_last_prepared() { return g_last_prepared; }
 long gemm_mfma_grouped_streamed_calls() { return g_streamed_calls; }
 long gemm_mfma_pipe_calls() { return g_pipe_calls; }
 long gemm_mfma_rowtile_calls() { return g_rowtile_calls; }
 long gemm_mfma_short_calls() { return g_short_calls; }
+long gemm_mfma_sum_reports() { return g_sum_reports; }
 
 long gemm_mfma_guard_hits()
 {
@@ -1050,6 +1051,7 @@ int gemm_mfma_launch(const GemmDesc &d, int *limbs_a, int *limbs_b)
             if (speculate) {
                 guard.parts = guard_parts(guard.seen_count, kGuardParts);
                 p.guard = guard;
+                g_sum_reports++;
             }
             (pipe.fn ? pipe.finish : inst->finish)<<<dim3((unsigned)((total - p.main_tiles) * p.finish_rq + p.guard.parts)), dim3((unsigned)inst->threads), 0, 0>>>(p);
             if (hipGetLastError() != hipSuccess) { set_error(kLaunchFailure, "gemm: split finish launch failed"); return kFailed; }

@@ -79,6 +79,7 @@ lib.zk_gemm_grouped_streamed_calls.restype = ctypes.c_long
 lib.zk_gemm_pipe_calls.restype = ctypes.c_long
 lib.zk_gemm_rowtile_calls.restype = ctypes.c_long
 lib.zk_gemm_short_calls.restype = ctypes.c_long
+lib.zk_gemm_sum_reports.restype = ctypes.c_long
 lib.zk_gemm_small_calls.restype = ctypes.c_long
 lib.zk_rms_split_calls.restype = ctypes.c_long
 lib.zk_gate_wave_calls.restype = ctypes.c_long
